@@ -200,6 +200,20 @@ def test_key_split_chunks(p1a, kv_type, Hq, Hkv, D, p0, T):
         assert ma < 2e-3 and rl < 1e-3, (t, ma, rl)
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,p0,T", [(3, 1, 64, 4000, 33), (2, 2, 64, 33000, 1), (5, 1, 128, 3000, 7), (1, 1, 256, 40000, 130), (24, 4, 256, 3500, 512)])
+def test_key_split_merge_edges(p1a, Hq, Hkv, D, p0, T):
+    """the merge takes several rows per workgroup and eight splits at a time: row counts that do not fill the last workgroup,
+    two splits up to the most a shape takes, splits past the last tile of the first rows"""
+    ks = p1a.prefill_key_splits(T, p0, Hq)
+    assert ks > 1, ks
+    pool = Pool(p1a, O.KV_F16, Hq, Hkv, D, 6, [p0 + T], seed=p0 + D)
+    q, _, _, gate = I.qkv(p0 + 1, 1, T, Hq, Hkv, D, f16_inputs=True)
+    rows = np.unique(np.r_[0, T // 2, T - 1])
+    ref = O.attn_rows(pool.host_seq(0), q[rows], (p0 + rows).astype(np.int32), Hq, D ** -0.5, gate=gate[rows])
+    out = run_prefill(p1a, pool.dev_seq(0), q, T, p0, Hq, D ** -0.5, gate=gate)
+    check(out[rows], ref, f"key-split merge {Hq}/{Hkv}/{D} p0 {p0} T {T} splits {ks}")
+
+
 def test_key_split_plan():
     """the split count is a function of the shape and the device only: none for chunks that fill the device or contexts too
     short to share out, several for a short chunk over a long context; the scratch size says what it holds"""
