@@ -190,11 +190,11 @@ int p1a_attn_prefill(const float *q, const p1a_kv *c, float *out, const float *g
  * roundup(2 * roundup(p0 + T, 16) * Hkv * D * 2, 256) + (key splits > 1 ? roundup(T * Hq * splits * 8, 256) + T * Hq * splits * D * 4 : 0).
  * Replaces attn_fold_scratch_bytes (src/fast/attn_fold.cuh:19). */
 size_t p1a_attn_prefill_scratch_bytes(int T, int p0, int Hq, int Hkv, int D);
-/* Key splits a prefill call of this shape takes on the current device (1 = none). A chunk of few token blocks over a long
- * context (the last chunk of a prompt, a short turn of a long chat) would occupy T/128 * Hq workgroups, each walking every
- * key; its keys are then dealt to several workgroups per (token block, q head) and the partials merged (the nsplit of
- * attn_fold, src/fast/attn_fold.cuh:19-26, chosen by the library). The count depends on (T, p0, Hq) and the device's CU
- * count only, never on the scratch passed or on the state of the stream; partials that do not fit the caller's scratch
+/* Key splits a prefill call of this shape takes at most on the current device (1 = none). A chunk of few query rows over a
+ * long context (the last chunk of a prompt, a short turn of a long chat) would occupy T * Hq / 128 workgroups, each walking
+ * every key; its keys are then dealt to several workgroups per (block of 128 rows, kv head) and the partials merged (the
+ * nsplit of attn_fold, src/fast/attn_fold.cuh:19-26, chosen by the library). The count depends on (T, p0, Hq) and the
+ * device's CU count only - what a call takes also on Hkv, which rounds its row blocks up - never on the scratch passed or on the state of the stream; partials that do not fit the caller's scratch
  * live in buffers the library keeps per (device, stream) for this purpose (never freed before p1a_release). They cannot
  * be allocated during stream capture: such a call is refused with P1A_E_SCRATCH unless p1a_warmup_prefill (or an eager
  * call of the shape) came first. */

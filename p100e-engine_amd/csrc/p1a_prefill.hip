@@ -1,7 +1,9 @@
 // Chunked causal prefill attention over a paged f16 / q8_0 / q4_0 KV cache for gfx950 (MI355X).
 //
-// One workgroup (4 waves, one per SIMD, 512 registers each) owns 128 consecutive query tokens of ONE q head; wave w owns
-// 32 of them as the N = 32 columns of v_mfma_f32_32x32x16_f16 tiles. Keys are walked in tiles of 64, kept in LDS as f16
+// One workgroup (4 waves, one per SIMD, 512 registers each) owns 128 consecutive query ROWS of one kv head - row r is token
+// r / GQA under q head r % GQA of the group; wave w owns 32 of them as the N = 32 columns of v_mfma_f32_32x32x16_f16 tiles.
+// (Rows, not the tokens of one q head: a chunk of few tokens fills its blocks - 77 tokens under 6 heads are 4 blocks, not
+// 6 - and a block spans 128 / GQA tokens, so fewer of the keys it walks are behind the diagonal for most of its rows.) Keys are walked in tiles of 64, kept in LDS as f16
 // (two K and two V tiles). f16 rows of 512 bytes are moved from global memory straight into LDS
 // (global_load_lds_dwordx4); everything else is fetched into registers with 16-byte loads off a wave-uniform page base,
 // dequantized and stored to the same LDS places.
@@ -19,7 +21,7 @@
 // rounded P that multiplies V. The reference maximum of a row moves lazily (only when the row maximum has grown
 // by more than 2^RESCALE_STEP), so the accumulators are rescaled a handful of times per row. Keys above a row's
 // diagonal are masked; the sigmoid output gate is applied in the epilogue.
-// Workgroup order: the q heads of one kv head, for one token block, get consecutive dispatch slots on the same XCD,
+// Workgroup order: GQA consecutive row blocks of one kv head (128 tokens) get consecutive dispatch slots on the same XCD,
 // so they stream the same K/V tiles through one L2.
 #include "p1a_common.hpp"
 
@@ -29,7 +31,7 @@ namespace p1a {
 size_t prefill_stage_bytes(int n, int Hkv, int D);
 namespace {
 
-constexpr int BM = 128;   // query tokens per workgroup
+constexpr int BM = 128;   // query rows per workgroup
 constexpr int BN = 64;    // keys per tile
 constexpr int NTHR = 256;
 constexpr float NEG_INF = -__builtin_inff();
@@ -75,8 +77,10 @@ struct pf_params {
     int T, p0, Hq, Hkv, GQA;
     int n_rows;   // positions the cache holds (contiguous caches: rows that may be read)
     float qscale;
-    int nblk;     // token blocks
-    // key splits: with nks > 1 workgroup (block, head, ks) walks its share of the block's tiles and leaves an unnormalised
+    int R;        // query rows of a kv head: T * GQA
+    int nblk;     // row blocks of a kv head
+    int nbg;      // groups of GQA row blocks
+    // key splits: with nks > 1 workgroup (block, kv head, ks) walks its share of the block's tiles and leaves an unnormalised
     // partial (O relative to m, and (m, l)) per row in part_o [T*Hq][nks][D] / part_ml [T*Hq][nks][2] for the merge
     int nks;
     float * part_o;
@@ -230,27 +234,26 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 31, g = lane >> 5;
-    // blockIdx.x -> (token block, kv head, q head of the group): the GQA heads of one (block, kv head) share an XCD
+    // blockIdx.x -> (group of GQA row blocks, kv head, block of the group): the blocks of a group share an XCD
     const int id = blockIdx.x, xcd = id & 7, slot = id >> 3;
-    // (with key splits a unit is (key split, token block, kv head): the splits spread over the XCDs like the blocks do)
+    // (with key splits a unit is (key split, group, kv head): the splits spread over the XCDs like the groups do)
     const int vunit = (slot / P.GQA) * 8 + xcd, hh = slot % P.GQA;
-    const int nunits = P.nblk * P.Hkv;
+    const int nunits = P.nbg * P.Hkv;
     if (vunit >= nunits * P.nks) return;
     const int ksp = vunit / nunits, unit = vunit - ksp * nunits;
     // longest blocks (most keys) first
-    const int tb = P.nblk - 1 - unit / P.Hkv, hk = unit % P.Hkv;
-    const int h = hk * P.GQA + hh;
+    const int rb = (P.nbg - 1 - unit / P.Hkv) * P.GQA + hh, hk = unit % P.Hkv;
+    if (rb >= P.nblk) return;                                 // (the last group need not be full)
 
-    const int tok0 = tb * BM;                                 // first token of the block
-    const int wtok0 = tok0 + 32 * wave;                       // first token of this wave
-    const int my_tok = wtok0 + c;                             // this lane's query row
-    const bool live = my_tok < P.T;
-    const int my_pos = P.p0 + (live ? my_tok : P.T - 1);
-    const int pmax = P.p0 + min(P.T, tok0 + BM) - 1;          // last position any row of the block sees
-    const int wave_pmin = P.p0 + wtok0;                       // smallest limit among this wave's rows
-    const int wave_pmax = P.p0 + min(P.T - 1, wtok0 + 31);
-    const bool wave_live = wtok0 < P.T;
-    const int ntiles_all = pmax / BN + 1;                     // tiles the block sees
+    const int row0 = rb * BM;                                 // first row of the block
+    const int my_row = row0 + 32 * wave + c;                  // this lane's query row
+    const bool live = my_row < P.R;
+    const int my_tok = (live ? my_row : P.R - 1) / P.GQA;
+    const int my_pos = P.p0 + my_tok;
+    const int pmax = P.p0 + (min(P.R, row0 + BM) - 1) / P.GQA;   // last position any row of the block sees
+    // a row -> its index among the T * Hq rows of q, out, gate and the partials
+    auto row_index = [&](int r) { const int t = r / P.GQA; return (size_t) t * P.Hq + (size_t) hk * P.GQA + (r - t * P.GQA); };
+    const int ntiles_all = pmax / BN + 1;                        // tiles the block sees
     // this workgroup's share of them: tiles tile_a .. tile_a + ntiles - 1
     int tile_a = 0, ntiles = ntiles_all;
     if (P.nks > 1) {
@@ -259,7 +262,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
         ntiles = min(tps, ntiles_all - tile_a);
         if (ntiles <= 0) {   // nothing left for this split: an empty partial (the merge skips it)
             if (g == 0 && live) {
-                float * ml = P.part_ml + (((size_t) my_tok * P.Hq + h) * P.nks + ksp) * 2;
+                float * ml = P.part_ml + (row_index(my_row) * P.nks + ksp) * 2;
                 ml[0] = NEG_INF;
                 ml[1] = 0.f;
             }
@@ -279,7 +282,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     // hand-issued ones, so asking earlier would put the two latencies in a row): one latency, not two.)
     auto load_q = [&]() {
         float4 qa[C::NKS], qb[C::NKS];
-        const float * qr = P.q + ((size_t) (live ? my_tok : 0) * P.Hq + h) * D;
+        const float * qr = P.q + (live ? row_index(my_row) : 0) * D;
 #pragma unroll
         for (int ks = 0; ks < C::NKS; ++ks) {
             qa[ks] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -703,15 +706,15 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (also: no tile load is left in flight)
     if (P.nks > 1) {   // one of several key splits: the unnormalised partial of every row, for the merge
         if (g == 0 && live) {
-            float * ml = P.part_ml + (((size_t) my_tok * P.Hq + h) * P.nks + ksp) * 2;
+            float * ml = P.part_ml + (row_index(my_row) * P.nks + ksp) * 2;
             ml[0] = m_run;
             ml[1] = l_own;
         }
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-            const int tok = tok0 + 32 * (r ? wave ^ 1 : wave) + c;
-            if (tok >= P.T) continue;
-            float * orow = P.part_o + (((size_t) tok * P.Hq + h) * P.nks + ksp) * D;
+            const int row = row0 + 32 * (r ? wave ^ 1 : wave) + c;
+            if (row >= P.R) continue;
+            float * orow = P.part_o + (row_index(row) * P.nks + ksp) * D;
 #pragma unroll
             for (int dt = 0; dt < HD; ++dt)
 #pragma unroll
@@ -728,8 +731,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     if (P.gate) {
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-            const int tok = tok0 + 32 * (r ? wave ^ 1 : wave) + c;
-            const float * grow = P.gate + ((size_t) min(tok, P.T - 1) * P.Hq + h) * D;
+            const float * grow = P.gate + row_index(min(row0 + 32 * (r ? wave ^ 1 : wave) + c, P.R - 1)) * D;
 #pragma unroll
             for (int dt = 0; dt < HD; ++dt)
 #pragma unroll
@@ -738,10 +740,10 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     }
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
-        const int tok = tok0 + 32 * (r ? wave ^ 1 : wave) + c;
-        if (tok >= P.T) continue;
+        const int row = row0 + 32 * (r ? wave ^ 1 : wave) + c;
+        if (row >= P.R) continue;
         const float inv = 1.0f / (r ? l_par : l_own);
-        float * orow = P.out + ((size_t) tok * P.Hq + h) * D;
+        float * orow = P.out + row_index(row) * D;
 #pragma unroll
         for (int dt = 0; dt < HD; ++dt)
 #pragma unroll
@@ -777,7 +779,7 @@ int launch_pf_g(const pf_params & P, hipStream_t s) {
         }
         attr_set.fetch_or(bit, std::memory_order_release);
     }
-    const int units = P.nblk * P.Hkv * P.nks;
+    const int units = P.nbg * P.Hkv * P.nks;
     const int slots = ((units + 7) / 8) * P.GQA;
     prefill_k<KT, D, GROUPED, DMA><<<slots * 8, NTHR, lds, s>>>(P);
     return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
@@ -845,19 +847,30 @@ __global__ void __launch_bounds__(256) dq_k(const char * kc, const char * vc, kv
 }
 }   // namespace
 
-// Key splits of a call: a chunk of few token blocks over a long context would leave most of the device idle (one
-// workgroup per block and q head, each walking every tile), so the tiles of a block are dealt to nks workgroups and the
+// Key splits of a call: a chunk of few row blocks over a long context would leave most of the device idle (one
+// workgroup per block and kv head, each walking every tile), so the tiles of a block are dealt to nks workgroups and the
 // partials merged. Chosen from the shape and the device alone (never from what scratch the caller brought: the result
-// bits depend on the split): the count that minimises rounds of workgroups x tiles per workgroup, a split being at least
-// 8 tiles and paying about 6 tiles' worth of set-up and partial traffic; 1 unless that saves 15 %.
-int prefill_key_splits(int T, int p0, int Hq, int cus) {
-    const long units = (long) ((T + BM - 1) / BM) * Hq, nt = (p0 + T - 1) / BN + 1;
+// bits depend on the split): the count that minimises, in units of a tile step, rounds of workgroups x (tiles per
+// workgroup + 6 for its set-up and partial stores) + the merge (its launch, 2, and its read of the partials, 1 per 6900
+// rows and split); a split is at least 8 tiles; 1 unless that saves 15 %.
+static int plan_splits(long units, int T, int p0, int Hq, int cus) {
+    const long nt = (p0 + T - 1) / BN + 1;
     if (cus < 1) cus = 1;
-    auto cost = [&](long k) { return ((units * k + cus - 1) / cus) * ((nt + k - 1) / k + 6); };
+    auto cost = [&](long k) {
+        const long c = ((units * k + cus - 1) / cus) * ((nt + k - 1) / k + 6);
+        return k > 1 ? c + 2 + (long) T * Hq * k / 6900 : c;
+    };
     long best = 1, cbest = cost(1);
     for (long k = 2; k <= 64 && nt / k >= 8; ++k)
         if (cost(k) < cbest) { best = k; cbest = cost(k); }
     return cbest * 100 <= cost(1) * 85 ? (int) best : 1;
+}
+// The split slots a shape reserves, whatever its GQA: planned for the fewest row blocks T * Hq rows can make. The count a
+// call uses is planned from the blocks it really has (each kv head's last block need not be full): at most as many.
+int prefill_key_splits(int T, int p0, int Hq, int cus) { return plan_splits(((long) T * Hq + BM - 1) / BM, T, p0, Hq, cus); }
+static int used_key_splits(int T, int p0, int Hq, int Hkv, int cus) {
+    const int most = prefill_key_splits(T, p0, Hq, cus), k = plan_splits(((long) T * (Hq / Hkv) + BM - 1) / BM * Hkv, T, p0, Hq, cus);
+    return k < most ? k : most;
 }
 size_t prefill_part_bytes_o(int T, int Hq, int D, int nks) { return nks > 1 ? (size_t) T * Hq * nks * D * 4 : 0; }
 size_t prefill_part_bytes_ml(int T, int Hq, int nks) { return nks > 1 ? (((size_t) T * Hq * nks * 2 * 4) + 255) & ~(size_t) 255 : 0; }
@@ -880,7 +893,9 @@ int launch_prefill(const p1a_kv & c, const float * q, float * out, const float *
     P.T = T; P.p0 = p0; P.Hq = Hq; P.Hkv = c.Hkv; P.GQA = Hq / c.Hkv;
     P.n_rows = c.n_ctx;
     P.qscale = scale * 1.4426950408889634f;
-    P.nblk = (T + BM - 1) / BM;
+    P.R = T * P.GQA;
+    P.nblk = (P.R + BM - 1) / BM;
+    P.nbg = (P.nblk + P.GQA - 1) / P.GQA;
     P.nks = 1; P.part_o = nullptr; P.part_ml = nullptr;
     // the caller's scratch: first the f16 staging copy of a quantized cache (when it fits), then the split partials (when
     // they fit behind it); partials that do not fit go to the library's own per-stream buffers
@@ -892,7 +907,7 @@ int launch_prefill(const p1a_kv & c, const float * q, float * out, const float *
     void * stage_own = nullptr;
     if (c.type != P1A_KV_F16 && !stage_caller) stage_own = stage_scratch(s, prefill_stage_bytes(n, c.Hkv, c.D));
     const bool stage = stage_caller || stage_own;
-    const int nks = prefill_key_splits(T, p0, Hq, cu_count());
+    const int nks = used_key_splits(T, p0, Hq, c.Hkv, cu_count());
     if (nks > 1) {
         const size_t bo = prefill_part_bytes_o(T, Hq, c.D, nks), bm = prefill_part_bytes_ml(T, Hq, nks);
         if (aligned && scratch_bytes >= used + bm + bo) {

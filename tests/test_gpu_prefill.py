@@ -200,6 +200,17 @@ def test_key_split_chunks(p1a, kv_type, Hq, Hkv, D, p0, T):
         assert ma < 2e-3 and rl < 1e-3, (t, ma, rl)
 
 
+@pytest.mark.parametrize("Hq,Hkv,T,p0", [(10, 2, 26, 0), (10, 2, 25, 70), (7, 1, 37, 3), (12, 2, 64, 64), (16, 1, 9, 500), (3, 3, 129, 0), (24, 4, 22, 2100)])
+def test_row_blocks(p1a, Hq, Hkv, T, p0):
+    """a block of 128 query rows holds tokens x q heads of one kv head: blocks that end inside a token, last blocks of one to
+    all rows, groups of blocks that are not full, one head per kv head"""
+    pool = Pool(p1a, O.KV_F16, Hq, Hkv, 256, 4, [p0 + T], seed=T + p0)
+    q, _, _, gate = I.qkv(T, 1, T, Hq, Hkv, 256, f16_inputs=True)
+    ref = O.attn_rows(pool.host_seq(0), q, (p0 + np.arange(T)).astype(np.int32), Hq, 1 / 16, gate=gate)
+    out = run_prefill(p1a, pool.dev_seq(0), q, T, p0, Hq, 1 / 16, gate=gate)
+    check(out, ref, f"row blocks {Hq}/{Hkv} p0 {p0} T {T}")
+
+
 @pytest.mark.parametrize("Hq,Hkv,D,p0,T", [(3, 1, 64, 4000, 33), (2, 2, 64, 33000, 1), (5, 1, 128, 3000, 7), (1, 1, 256, 40000, 130), (24, 4, 256, 3500, 512)])
 def test_key_split_merge_edges(p1a, Hq, Hkv, D, p0, T):
     """the merge takes several rows per workgroup and eight splits at a time: row counts that do not fill the last workgroup,
