@@ -3,8 +3,9 @@
 // One workgroup (4 waves, one per SIMD, 512 registers each) owns 128 consecutive query ROWS of one kv head - row r is token
 // r / GQA under q head r % GQA of the group; wave w owns 32 of them as the N = 32 columns of v_mfma_f32_32x32x16_f16 tiles.
 // (Rows, not the tokens of one q head: a chunk of few tokens fills its blocks - 77 tokens under 6 heads are 4 blocks, not
-// 6 - and a block spans 128 / GQA tokens, so fewer of the keys it walks are behind the diagonal for most of its rows.) Keys are walked in tiles of 64, kept in LDS as f16
-// (two K and two V tiles). f16 rows of 512 bytes are moved from global memory straight into LDS
+// 6 - and a block spans 128 / GQA tokens, so fewer of the keys it walks are behind the diagonal for most of its rows. 24 / 4
+// heads of 256, q8_0: 77 tokens behind 16000 88.7 -> 79.7 us for the whole call; a full chunk, 4096 behind 28672, the same.)
+// Keys are walked in tiles of 64, kept in LDS as f16 (two K and two V tiles). f16 rows of 512 bytes are moved from global memory straight into LDS
 // (global_load_lds_dwordx4); everything else is fetched into registers with 16-byte loads off a wave-uniform page base,
 // dequantized and stored to the same LDS places.
 //   S^T = K Q^T : A = K rows straight from LDS (ds_read_b128), B = Q^T held in accumulation registers (pre-multiplied
@@ -250,6 +251,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     const bool live = my_row < P.R;
     const int my_tok = (live ? my_row : P.R - 1) / P.GQA;
     const int my_pos = P.p0 + my_tok;
+    const int wave_vis = __builtin_amdgcn_readfirstlane(my_pos);  // every row of this wave sees the positions up to here
     const int pmax = P.p0 + (min(P.R, row0 + BM) - 1) / P.GQA;   // last position any row of the block sees
     // a row -> its index among the T * Hq rows of q, out, gate and the partials
     auto row_index = [&](int r) { const int t = r / P.GQA; return (size_t) t * P.Hq + (size_t) hk * P.GQA + (r - t * P.GQA); };
@@ -315,12 +317,17 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     // multiplies V. 16 vector instructions in the shadow of the S^T products instead of four more matrix instructions
     // per tile (-1.3 % of the call). Kept per (key half, lane half) and added up once, in a fixed order, at the end.
     float lp[2] = {0.f, 0.f};
+    // The reference maximum of the own row (-inf: no visible key yet) rides in the S^T products as the value they accumulate
+    // on: they deliver S - m, and exp2 takes them as they are.
     float m_run = NEG_INF;
+    f16x neg_m;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
+        neg_m[i] = 0.f;
 #pragma unroll
         for (int dt = 0; dt < HD; ++dt) { o[0][dt][i] = 0.f; o[1][dt][i] = 0.f; }
     }
+    asm volatile("" : "+v"(neg_m));                          // (16 registers of one value: not to be rebuilt at every use)
     // exchange areas behind the tile stages: P^T of every wave (BN / 16 k-steps x 64 lanes x 16 bytes), then one float
     // per query row (rescale factor during the loop, denominator at the end)
     char * const xbase = lds + 2 * L::STAGE_B + (S::SCALES_VIA_LDS ? 2 * 4 * 16 * S::SB : 0);
@@ -558,24 +565,30 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
         } else gp_k = group_pages(tile_of(it + 3));                    // entries for the K fetch at the end of this step
         f16x s[2] = {s_next[0], s_next[1]};                            // S^T(it), masked; mloc = its row maximum
 
-        // Lazy reference maximum: m_run follows the row maximum only when it has grown by more than RESCALE_STEP, so P
-        // stays below 2^RESCALE_STEP (well inside f16) and the accumulators are rescaled a handful of times per row
-        // instead of at every tile. A row that has seen no visible key yet (m_run = -inf) just adopts the maximum.
+        // Lazy reference maximum: m_run follows the row maximum (mloc, relative to it) only when that has grown by more than
+        // RESCALE_STEP, so P stays below 2^RESCALE_STEP (well inside f16) and the accumulators are rescaled a handful of times
+        // per row instead of at every tile. A row that has seen no visible key yet just adopts its first maximum (mloc = -inf
+        // never moves anything; the exponentials of such a row are 0).
         const bool fresh = m_run == NEG_INF;
-        const bool move = mloc > m_run + RESCALE_STEP || fresh;      // mloc = -inf never moves anything
-        const float mnew = (move && mloc != NEG_INF) ? mloc : m_run;
-        const bool dead = mnew == NEG_INF;
-        const float alpha = (fresh || mnew == m_run) ? 1.0f : __builtin_amdgcn_exp2f(m_run - mnew);
-        m_run = mnew;
-        const float msub = dead ? 0.0f : mnew;                       // a row with no visible key yet: exp2(-inf - 0) = 0
-        lp[0] *= alpha;
-        lp[1] *= alpha;
-        if (__builtin_expect(__any(alpha != 1.0f), 0)) {
+        const bool move = mloc > RESCALE_STEP || (fresh && mloc != NEG_INF);
+        float alpha = 1.0f;
+        if (__builtin_expect(__any(move), 0)) {
+            const float shift = move ? mloc : 0.0f;
+            if (move) {
+                alpha = fresh ? 1.0f : __builtin_amdgcn_exp2f(-shift);   // (fresh: nothing accumulated)
+                m_run = (fresh ? 0.0f : m_run) + shift;
+            }
+            lp[0] *= alpha;
+            lp[1] *= alpha;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
+                neg_m[i] = m_run == NEG_INF ? 0.0f : -m_run;
+                s[0][i] -= shift;
+                s[1][i] -= shift;
 #pragma unroll
                 for (int dt = 0; dt < HD; ++dt) o[0][dt][i] *= alpha;
             }
+            asm volatile("" : "+v"(neg_m));
         }
         // ---- stream 1: S^T(it+1) on the matrix pipe; stream 2: P^T(it) = exp2(S^T(it) - m) on the vector pipe ----
         // Written step by step, one MFMA per step, with a scheduling fence after each: the LDS read of the K fragment
@@ -599,11 +612,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
                 }
             }
             const int u = k / C::NKS;
-            if (k % C::NKS == 0) {
-#pragma unroll
-                for (int i = 0; i < 16; ++i) s_next[u][i] = 0.f;
-            }
-            s_next[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[k], qf[k % C::NKS], s_next[u], 0, 0, 0);
+            s_next[u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fr[k], qf[k % C::NKS], k % C::NKS ? s_next[u] : neg_m, 0, 0, 0);
             if constexpr (SVL) {   // the scales of the raw tiles fetched one step ago: through LDS to the lanes that use them
                 if (k == NQK - 4) { park_sblk(ksc, sk); park_sblk(vsc, sv); }
                 if (k == NQK - 2) { pick_scales(rk, ksc); pick_scales(rv, vsc); }
@@ -611,7 +620,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
 #pragma unroll
             for (int v = 0; v < VPS; ++v) {
                 const int idx = k * VPS + v, su = idx >> 4, i = idx & 15;
-                s[su][i] = __builtin_amdgcn_exp2f(s[su][i] - msub);
+                s[su][i] = __builtin_amdgcn_exp2f(s[su][i]);
                 if (idx & 1) {   // packed conversion (round to nearest even), two values per instruction
                     const h2 pr = __builtin_convertvector(f2v{s[su][i - 1], s[su][i]}, h2);
                     lp[su] = __builtin_amdgcn_fdot2(pr, one2, lp[su], false);
@@ -670,7 +679,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
                 }
                 o[1][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pp[ps], o[1][dt], 0, 0, 0);
 #pragma unroll
-                for (int v = 0; v < MPS; ++v) mloc = mask_max(s_next, k0n, f * MPS + v, mloc);
+                for (int v = 0; v < MPS; ++v) mloc = fmaxf(mloc, s_next[(f * MPS + v) >> 4][(f * MPS + v) & 15]);
 #pragma unroll
                 for (int pt = DMA ? NP : f * NP / NFR; pt < (f + 1) * NP / NFR; ++pt) {
                     const int item = pt / S::PARTS, part = pt % S::PARTS;
@@ -678,6 +687,14 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
                     else               S::store_part(rv, st_nxt + L::KT_B, L::VB, tid, item - S::NPT, part);       // V(it+1) over V(it-1)
                 }
                 __builtin_amdgcn_sched_barrier(0);
+            }
+            // A tile that every row of the wave sees whole - all but the last few of a block - is not masked: the 64 compares
+            // and selects run for the others only, out of line (with S - m straight from the products 257 -> 127 vector
+            // instructions a tile, 4096 tokens behind 28672 3182 -> 3060 us)
+            if (__builtin_expect(k0n + BN - 1 > wave_vis, 0)) {
+                mloc = NEG_INF;
+#pragma unroll
+                for (int idx = 0; idx < 32; ++idx) mloc = mask_max(s_next, k0n, idx, mloc);
             }
         }
 
