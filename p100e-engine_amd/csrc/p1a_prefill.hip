@@ -27,6 +27,7 @@
 #include "p1a_common.hpp"
 
 #include <atomic>
+#include <type_traits>
 
 namespace p1a {
 size_t prefill_stage_bytes(int n, int Hkv, int D);
@@ -223,6 +224,10 @@ __device__ __forceinline__ uint32_t lds_addr(const char * p) { return (uint32_t)
 // 64 lanes x 16 bytes, global (scalar base + 32-bit lane offset) -> LDS at `lds` + 16 * lane, no registers in between
 __device__ __forceinline__ void dma16(const char * sbase, uint32_t voff, uint32_t lds) {
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(voff), "s"(sbase), "s"(lds) : "memory", "m0");
+}
+// the same to `lds` + a constant: one scalar instruction per load
+__device__ __forceinline__ void dma16_at(const char * sbase, uint32_t voff, uint32_t lds, int at) {
+    asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(voff), "s"(sbase), "s"(lds), "i"(at) : "memory", "m0", "scc");
 }
 
 template <uint32_t KT, int D, bool GROUPED, bool DMA>
@@ -466,9 +471,10 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     // Workgroups that share a kv head would otherwise walk the keys in lock-step and ask one L2 channel for the same
     // line at the same instant. Each starts at its own tile and wraps around (softmax does not care about key order);
     // the q heads of one group stay one tile apart, so all but the first still find the tile in L2.
-    // Steps past the last one (the pipeline looks up to three tiles ahead) repeat the last tile; nothing uses them.
+    // Steps past the last one (the pipeline looks up to four tiles ahead) wrap around as well; nothing uses them.
     const int rot = (int) (((unsigned) unit * 29u + (unsigned) hh) % (unsigned) ntiles);
-    auto tile_of = [&](int it) { const int t = min(it, ntiles - 1) + rot; return tile_a + (t >= ntiles ? t - ntiles : t); };
+    auto tile_after = [&](int tile) { return tile + 1 == tile_a + ntiles ? tile_a : tile + 1; };
+    const int tile0 = tile_a + rot, tile1 = tile_after(tile0), tile2 = tile_after(tile1);
 
     // S^T of one tile: 32-key halves u = 0, 1
     auto qk = [&](const char * kt, f16x (&s)[2]) {
@@ -486,14 +492,16 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     };
 
     // ---- LDS-direct tile loads (DMA): wave w moves the 8 blocks of its 16-key group; instruction j takes keys j and
-    // j + 8 of the group (lanes 0-31 / 32-63, 16 bytes of the row each): a scalar base that advances by one row per
-    // instruction and ONE loop-invariant lane offset. Rows past the last position are fetched as they are (the group lies
+    // j + 8 of the group (lanes 0-31 / 32-63, 16 bytes of the row each): the group's base and a loop-invariant lane offset per
+    // instruction - eight registers that spare the loop two 64-bit scalar additions a load. Rows past the last position are fetched as they are (the group lies
     // inside one page, or inside the cache when it is contiguous - the host checks): as K they only make scores that the
     // mask replaces; as V they are overwritten with zeros in LDS once the tile has landed (P = 0 times anything finite).
-    const uint32_t dma_vo = (uint32_t) (8 * g) * (uint32_t) P.pg.rowb + (uint32_t) (lane & 31) * 16u;
-    auto dma_block = [&](const char * cache, const gbases & gb, char * dst_tile, int bstride, int j) {
-        dma16(cache + gb.go + (size_t) j * P.pg.rowb, dma_vo, lds_addr(dst_tile + (8 * wave + j) * bstride));
-    };
+    uint32_t dma_vo[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) dma_vo[j] = (uint32_t) (8 * g + j) * (uint32_t) P.pg.rowb + (uint32_t) (lane & 31) * 16u;
+    const uint32_t k_dst = lds_addr(lds) + 8 * wave * L::KB, v_dst = lds_addr(lds) + L::KT_B + 8 * wave * L::VB;   // this wave's blocks of stage 0
+    auto dma_k = [&](const gbases & gb, int stage, int j) { dma16_at(P.kc + gb.go, dma_vo[j], k_dst, stage * L::STAGE_B + j * L::KB); };
+    auto dma_v = [&](const gbases & gb, int stage, int j) { dma16_at(P.vc + gb.go, dma_vo[j], v_dst, stage * L::STAGE_B + j * L::VB); };
     auto zero_v_tail = [&](int tile, char * vtile) {
         if (tile != last_tile) return;
         const int room = pmax - (last_tile * BN + 16 * wave);             // the wave's last key that exists (< 0: none)
@@ -504,39 +512,45 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     // ---- prologue: K(0), V(0), K(1) in LDS; (staged through registers: V(1) and K(2) on their way); S^T(0) ----
     typename S::raw rk, rv;
     sblk sk, sv;                                           // scale blocks that belong to rk, rv
-    gbases gb_prev;                                        // group bases of the tile whose V is fetched next
-    gpages gp_ahead;                                       // (DMA) table entry of the K tile fetched in the next step
+    // group bases of the V tile and (DMA) the K tile that the next step fetches, table entry of the K tile of the one after
+    gbases gb_v, gb_k;
+    gpages gp_ahead;
     if constexpr (DMA) {
-        gpages g0 = group_pages(tile_of(0)), g1 = group_pages(tile_of(1));
-        const gbases b0 = group_bases(tile_of(0), g0);
-        gb_prev = group_bases(tile_of(1), g1);
-        gp_ahead = group_pages(tile_of(2));
+        gpages g0 = group_pages(tile0), g1 = group_pages(tile1), g2 = group_pages(tile2);
+        const gbases b0 = group_bases(tile0, g0);
+        gb_v = group_bases(tile1, g1);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) dma_block(P.kc, b0, lds, L::KB, j);
+        for (int j = 0; j < 8; ++j) dma_k(b0, 0, j);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) dma_block(P.vc, b0, lds + L::KT_B, L::VB, j);
+        for (int j = 0; j < 8; ++j) dma_v(b0, 0, j);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) dma_block(P.kc, gb_prev, lds + L::STAGE_B, L::KB, j);
+        for (int j = 0; j < 8; ++j) dma_k(gb_v, 1, j);
+        gb_k = group_bases(tile2, g2);
+        gp_ahead = group_pages(tile_after(tile2));
         load_q();
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        zero_v_tail(tile_of(0), lds + L::KT_B);
+        zero_v_tail(tile0, lds + L::KT_B);
     } else {
-        gpages g0 = group_pages(tile_of(0)), g1 = group_pages(tile_of(1)), g2 = group_pages(tile_of(2));
-        const gbases b0 = group_bases(tile_of(0), g0), b1 = group_bases(tile_of(1), g1);
-        gb_prev = group_bases(tile_of(2), g2);
-        fetch_tile(rk, P.kc, ksc, tile_of(0), b0);
-        fetch_tile(rv, P.vc, vsc, tile_of(0), b0);
+        gpages g0 = group_pages(tile0), g1 = group_pages(tile1), g2 = group_pages(tile2);
+        const gbases b0 = group_bases(tile0, g0), b1 = group_bases(tile1, g1);
+        gb_v = group_bases(tile2, g2);
+        fetch_tile(rk, P.kc, ksc, tile0, b0);
+        fetch_tile(rv, P.vc, vsc, tile0, b0);
         store_tile<S>(rk, lds, L::KB, tid);
         store_tile<S>(rv, lds + L::KT_B, L::VB, tid);
-        fetch_tile(rk, P.kc, ksc, tile_of(1), b1);
+        fetch_tile(rk, P.kc, ksc, tile1, b1);
         store_tile<S>(rk, lds + L::STAGE_B, L::KB, tid);
-        load_tile(rv, P.vc, tile_of(1), b1);
-        load_tile(rk, P.kc, tile_of(2), gb_prev);
-        if constexpr (SVL) { sv = load_sblk(P.vc, tile_of(1), b1); sk = load_sblk(P.kc, tile_of(2), gb_prev); }
+        load_tile(rv, P.vc, tile1, b1);
+        load_tile(rk, P.kc, tile2, gb_v);
+        if constexpr (SVL) { sv = load_sblk(P.vc, tile1, b1); sk = load_sblk(P.kc, tile2, gb_v); }
     }
     __syncthreads();
-    f16x s_next[2];
-    qk(lds, s_next);
+    // S^T of two tiles: that of the tile in hand and that of the next, taking turns. (DMA: a step is written out twice, so that
+    // neither the values nor the LDS addresses of the two stages have to be moved about. A step is then 64 matrix and 346
+    // other instructions instead of 461 - one wave per SIMD issues one in four clocks - and its maximum and denominator
+    // sums sit beside matrix instructions instead of behind the last one: 3060 -> 2860 us for 4096 tokens behind 28672.)
+    f16x s_a[2], s_b[2];
+    qk(lds, s_a);
     // Masking and the row maximum of a tile are done one step ahead of its softmax (in the shadow of the O^T products of
     // the tile before it): value i of half u of a lane's S^T column is key k0 + key_of(u, i) + 4 g of the lane's own row.
     auto mask_max = [&](f16x (&sv_)[2], int k0_, int idx, float m) {
@@ -548,29 +562,26 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     auto row_max = [&](float m) { return max_swap32(m); };
     float mloc = NEG_INF;
 #pragma unroll
-    for (int idx = 0; idx < 32; ++idx) mloc = mask_max(s_next, tile_of(0) * BN, idx, mloc);
+    for (int idx = 0; idx < 32; ++idx) mloc = mask_max(s_a, tile0 * BN, idx, mloc);
     mloc = row_max(mloc);
     // (the first step overwrites K(0) while it runs; every wave has to be done reading it)
     if constexpr (DMA) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
-    for (int it = 0; it < ntiles; ++it) {
-        const int k0 = tile_of(it) * BN;
-        char * const st_cur = lds + (it & 1) * L::STAGE_B;             // holds K(it) (done with) and V(it)
-        char * const st_nxt = lds + ((it + 1) & 1) * L::STAGE_B;       // holds K(it+1); V(it-1) is done with
+    int tile_c = tile0, tile_n = tile1, tile_nn = tile2;      // the tiles of this step, the next and the one after
+    auto step = [&](auto par, f16x (&s)[2], f16x (&s_next)[2]) {   // s: S^T of this step's tile, masked; mloc: its row maximum
+        const int ST = par;
+        char * const st_cur = lds + ST * L::STAGE_B;                   // holds K(it) (done with) and V(it)
+        char * const st_nxt = lds + (1 - ST) * L::STAGE_B;             // holds K(it+1); V(it-1) is done with
+        const int k0n = tile_n * BN;
         gpages gp_k;
-        gbases gb_dma;
-        if constexpr (DMA) {
-            gb_dma = group_bases(tile_of(it + 2), gp_ahead);           // K(it+2) goes over K(it), V(it+1) over V(it-1):
-            gp_ahead = group_pages(tile_of(it + 3));                   // requested between the S^T steps below
-        } else gp_k = group_pages(tile_of(it + 3));                    // entries for the K fetch at the end of this step
-        f16x s[2] = {s_next[0], s_next[1]};                            // S^T(it), masked; mloc = its row maximum
+        if constexpr (!DMA) gp_k = group_pages(tile_after(tile_nn));   // entries for the K fetch at the end of this step
 
         // Lazy reference maximum: m_run follows the row maximum (mloc, relative to it) only when that has grown by more than
         // RESCALE_STEP, so P stays below 2^RESCALE_STEP (well inside f16) and the accumulators are rescaled a handful of times
         // per row instead of at every tile. A row that has seen no visible key yet just adopts its first maximum (mloc = -inf
         // never moves anything; the exponentials of such a row are 0).
         const bool fresh = m_run == NEG_INF;
-        const bool move = mloc > RESCALE_STEP || (fresh && mloc != NEG_INF);
+        const bool move = mloc > (fresh ? NEG_INF : RESCALE_STEP);
         float alpha = 1.0f;
         if (__builtin_expect(__any(move), 0)) {
             const float shift = move ? mloc : 0.0f;
@@ -607,8 +618,8 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
             if constexpr (DMA) {   // one tile load every other step: K(it+2) first (it is needed first), then V(it+1)
                 if (k % 2 == 0) {
                     const int j = k / 2;
-                    if (j < 8) dma_block(P.kc, gb_dma, st_cur, L::KB, j);
-                    else if (j < 16) dma_block(P.vc, gb_prev, st_nxt + L::KT_B, L::VB, j - 8);
+                    if (j < 8) dma_k(gb_k, ST, j);                     // over K(it)
+                    else if (j < 16) dma_v(gb_v, 1 - ST, j - 8);       // over V(it-1)
                 }
             }
             const int u = k / C::NKS;
@@ -624,6 +635,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
                 if (idx & 1) {   // packed conversion (round to nearest even), two values per instruction
                     const h2 pr = __builtin_convertvector(f2v{s[su][i - 1], s[su][i]}, h2);
                     lp[su] = __builtin_amdgcn_fdot2(pr, one2, lp[su], false);
+                    asm volatile("" : "+v"(lp[su]));   // (here, in the shadow of this product, not at the end of the step)
                     pb[idx >> 3][(idx & 7) - 1] = pr[0];
                     pb[idx >> 3][idx & 7] = pr[1];
                 }
@@ -646,21 +658,31 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
                          __builtin_amdgcn_ds_read_tr16_b64_v4i16((s4 __attribute__((address_space(3))) *) (p0_ + L::v_hi(f / HD)))};
         };
         vfrag vf[NFR];
+        if constexpr (!DMA) {
 #pragma unroll
-        for (int f = 0; f < PF_V && f < NFR; ++f) vf[f] = vread(f);
+            for (int f = 0; f < PF_V && f < NFR; ++f) vf[f] = vread(f);
+        }
         // ---- hand P^T and the rescale factor of the own rows to the partner ----
 #pragma unroll
         for (int ps = 0; ps < BN / 16; ++ps) *reinterpret_cast<h8 *>(px_own + (ps * 64 + lane) * 16) = pb[ps];
-        if (g == 0) ax_own[c] = alpha;
+        ax_own[c] = alpha;                                    // (both lane halves: the same value)
+        // (the V(it) loads of the previous step are older than this step's 16: they have landed when 16 are left)
+        if constexpr (DMA) {
+            asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+            zero_v_tail(tile_c, st_cur + L::KT_B);
+        }
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         // ---- stream 1: O^T += V^T(it) P^T on the matrix pipe; stream 2: masking and row maximum of S^T(it+1) (and K(it+2),
         // V(it+1) -> f16 tiles in LDS when they are staged through registers) ----
         {
+            if constexpr (DMA) {
+#pragma unroll
+                for (int f = 0; f < PF_V && f < NFR; ++f) vf[f] = vread(f);
+            }
             const float alpha_p = ax_par[c];                                      // (needed before the partner's first product)
             h8 pp[BN / 16];
             constexpr int MPS = 32 / NFR;                                          // next tile's values masked per step
             static_assert(32 % NFR == 0, "mask slices must tile the 32 values of a lane");
-            const int k0n = tile_of(it + 1) * BN;
             mloc = NEG_INF;
             pp[0] = *reinterpret_cast<const h8 *>(px_par + lane * 16);
 #pragma unroll
@@ -680,6 +702,11 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
                 o[1][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pp[ps], o[1][dt], 0, 0, 0);
 #pragma unroll
                 for (int v = 0; v < MPS; ++v) mloc = fmaxf(mloc, s_next[(f * MPS + v) >> 4][(f * MPS + v) & 15]);
+                asm volatile("" : "+v"(mloc));
+                if constexpr (DMA) {   // where the next step's tiles come from
+                    if (f == 1) { gb_v = gb_k; gb_k = group_bases(tile_after(tile_nn), gp_ahead); }
+                    if (f == 2) gp_ahead = group_pages(tile_after(tile_after(tile_nn)));
+                }
 #pragma unroll
                 for (int pt = DMA ? NP : f * NP / NFR; pt < (f + 1) * NP / NFR; ++pt) {
                     const int item = pt / S::PARTS, part = pt % S::PARTS;
@@ -702,18 +729,34 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
         // ---- raw loads of K(it+3), V(it+2): one whole step to arrive. Issued back to back: a vector memory instruction
         // holds the wave for as long as the CU's address path needs for it, wherever it is placed ----
         if constexpr (DMA) {
-            gb_prev = gb_dma;
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // this step's tile loads have landed
-            zero_v_tail(tile_of(it + 1), st_nxt + L::KT_B);
+            asm volatile("s_waitcnt vmcnt(8)" ::: "memory");        // K(it+2) has landed; V(it+1) has until the next exchange
         } else {
-            const gbases gb_k = group_bases(tile_of(it + 3), gp_k);
-            load_tile(rk, P.kc, tile_of(it + 3), gb_k);
-            load_tile(rv, P.vc, tile_of(it + 2), gb_prev);
-            if constexpr (SVL) { sk = load_sblk(P.kc, tile_of(it + 3), gb_k); sv = load_sblk(P.vc, tile_of(it + 2), gb_prev); }
-            gb_prev = gb_k;
+            const int tile_3 = tile_after(tile_nn);
+            const gbases gb_3 = group_bases(tile_3, gp_k);
+            load_tile(rk, P.kc, tile_3, gb_3);
+            load_tile(rv, P.vc, tile_nn, gb_v);
+            if constexpr (SVL) { sk = load_sblk(P.kc, tile_3, gb_3); sv = load_sblk(P.vc, tile_nn, gb_v); }
+            gb_v = gb_3;
         }
+        tile_c = tile_n;
+        tile_n = tile_nn;
+        tile_nn = tile_after(tile_nn);
         // LDS stores retired, then the barrier (without the global-memory fence of __syncthreads())
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    };
+    if constexpr (DMA) {
+        for (int it = 0;;) {
+            step(std::integral_constant<int, 0>{}, s_a, s_b);
+            if (++it == ntiles) break;
+            step(std::integral_constant<int, 1>{}, s_b, s_a);
+            if (++it == ntiles) break;
+        }
+    } else {   // (staged through registers there are none left for two copies)
+        for (int it = 0; it < ntiles; ++it) {
+            step(it & 1, s_a, s_b);
+            s_a[0] = s_b[0];
+            s_a[1] = s_b[1];
+        }
     }
 
     // ---- epilogue: the pair swaps denominators, then each wave normalises, gates and stores its half of the dims of
