@@ -468,13 +468,13 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
         }
     };
 
-    // Workgroups that share a kv head would otherwise walk the keys in lock-step and ask one L2 channel for the same
-    // line at the same instant. Each starts at its own tile and wraps around (softmax does not care about key order);
-    // the q heads of one group stay one tile apart, so all but the first still find the tile in L2.
-    // Steps past the last one (the pipeline looks up to four tiles ahead) wrap around as well; nothing uses them.
-    const int rot = (int) (((unsigned) unit * 29u + (unsigned) hh) % (unsigned) ntiles);
-    auto tile_after = [&](int tile) { return tile + 1 == tile_a + ntiles ? tile_a : tile + 1; };
-    const int tile0 = tile_a + rot, tile1 = tile_after(tile0), tile2 = tile_after(tile1);
+    // Every workgroup walks its tiles in ascending order: those that share a kv head then ask for a tile within a step of
+    // one another and find it in L2. (Each used to start at a tile of its own, to keep them off one L2 channel; the tiles then
+    // came from the Infinity Cache: 4096 tokens behind 28672 2815 -> 2740 us without, 77 behind 16000 73.5 -> 69.6.)
+    // Steps past the last one (the pipeline looks up to four tiles ahead) wrap around; nothing uses them.
+    const int tile_z = tile_a + ntiles - 1;
+    auto tile_after = [&](int tile) { return tile == tile_z ? tile_a : tile + 1; };
+    const int tile0 = tile_a, tile1 = tile_after(tile0), tile2 = tile_after(tile1);
 
     // S^T of one tile: 32-key halves u = 0, 1
     auto qk = [&](const char * kt, f16x (&s)[2]) {
