@@ -43,29 +43,36 @@ template <int D> struct pf_cfg {
     static constexpr int NDT = D / 32;         // 32-dim tiles of O^T
 };
 
-// Where the f16 tiles sit in LDS: in blocks of two rows (2 x 2 D bytes, then padding). Block (key & 7) + 8 (key >> 4)
-// holds key in its half (key >> 3) & 1 - two keys of the same 16-key group. For D = 256 a block is exactly what one
-// global_load_lds_dwordx4 moves (64 lanes x 16 bytes to 1 KB of consecutive LDS), and one page base serves it; tiles
-// staged through registers use the same places. The padding puts the rows that are read together into disjoint banks:
-// S^T row c of half u is the key of block 16 u + (c & 15), half c >> 4 (16 consecutive lanes: 16 blocks, 4 banks
-// apart); the transposing V reads take 4 consecutive blocks of one half (16 banks apart). Every read address is
-// (per-lane base) + (compile-time offset).
+// Where the f16 tiles sit in LDS: in blocks of 1 KB - RPB = 2, 4 or 8 rows of 512, 256 or 128 bytes - and padding. A block is
+// exactly what one global_load_lds_dwordx4 moves (64 lanes x 16 bytes to consecutive LDS); its rows are keys of one 16-key
+// group, so one page base serves it: group q of the tile has the NJ = 16 / RPB blocks NJ q .. , key k of it sits in block
+// NJ q + k % NJ, slot k / NJ. Tiles staged through registers use the same places. The padding (K 16 bytes, V 64) puts
+// the rows that are read together into disjoint banks: 16 consecutive rows of an S^T operand are 16 blocks 4 banks apart
+// (D = 64: 8 blocks, and two slots 32 banks apart), the four rows of a transposing V read 4 blocks 16 banks apart. So row
+// c of half u of S^T is block c % NB (NB = 64 / RPB blocks; D = 256: + 16 u), slot (c / NB) + u (32 / NB) - which key that is
+// follows - and the rows of O^T's operand follow from the order of the S^T values. Every read address is (per-lane base)
+// + (compile-time offset).
 template <int D> struct pf_lay {
     static constexpr int RB = 2 * D;                            // bytes of a row
-    static constexpr int KB = 2 * RB + 16, VB = 2 * RB + 64;   // block strides
-    static constexpr int KT_B = 32 * KB, VT_B = 32 * VB;
+    static constexpr int RPB = 1024 / RB, NJ = 16 / RPB, NB = BN / RPB;
+    static constexpr int KB = 1024 + 16, VB = 1024 + 64;        // block strides
+    static constexpr int KT_B = NB * KB, VT_B = NB * VB;
     static constexpr int STAGE_B = KT_B + VT_B;
-    static __device__ __forceinline__ int key_off(int key, int bstride) { return ((key & 7) + 8 * (key >> 4)) * bstride + ((key >> 3) & 1) * RB; }
+    static __device__ __forceinline__ int key_off(int key, int bstride) { return (NJ * (key >> 4) + key % NJ) * bstride + (key & 15) / NJ * RB; }
+    // row r (0 .. 31) of half u: its block and slot
+    static constexpr __host__ __device__ int block(int u, int r) { return D == 256 ? 16 * u + (r & 15) : r % NB; }
+    static constexpr __host__ __device__ int slot(int u, int r) { return D == 256 ? r >> 4 : r / NB + u * (32 / NB); }
     // S^T operand rows: lane base of row c, offset of half u
-    static __device__ __forceinline__ int k_lane(int c) { return (c & 15) * KB + (c >> 4) * RB; }
-    static constexpr int k_half(int u) { return 16 * u * KB; }
-    // which key of the tile value i of half u of a lane's S^T column is, without the lane's 4 g
-    static constexpr int key_of(int u, int i) { return 32 * u + 16 * ((i >> 2) & 1) + 8 * (i >> 3) + (i & 3); }
-    // V^T operand of k-step ps: rows r = 4 g + kk (lane part), then the step's two row groups:
-    // keys 32 (ps / 2) + 8 (ps % 2) + r and the same + 16
+    static __device__ __forceinline__ int k_lane(int c) { return block(0, c) * KB + slot(0, c) * RB; }
+    static constexpr int k_half(int u) { return block(u, 0) * KB + slot(u, 0) * RB; }
+    // which key of the tile value i of half u of a lane's S^T column is: key_of(u, i) + KG g (row 8 (i / 4) + 4 g + i % 4)
+    static constexpr __host__ __device__ int key_at(int u, int r) { return 16 * (block(u, r) / NJ) + block(u, r) % NJ + NJ * slot(u, r); }
+    static constexpr int key_of(int u, int i) { return key_at(u, 8 * (i >> 2) + (i & 3)); }
+    static constexpr int KG = key_at(0, 4) - key_at(0, 0);
+    // V^T operand of k-step ps (half ps / 2 of the tile): rows 16 (ps % 2) + 4 g + kk (lane part: 4 g + kk), and the same + 8
     static __device__ __forceinline__ int v_lane(int r) { return r * VB; }
-    static constexpr int v_lo(int ps) { return 16 * (ps >> 1) * VB + (ps & 1) * RB; }
-    static constexpr int v_hi(int ps) { return v_lo(ps) + 8 * VB; }
+    static constexpr int v_lo(int ps) { return block(ps >> 1, 16 * (ps & 1)) * VB + slot(ps >> 1, 16 * (ps & 1)) * RB; }
+    static constexpr int v_hi(int ps) { return block(ps >> 1, 16 * (ps & 1) + 8) * VB + slot(ps >> 1, 16 * (ps & 1) + 8) * RB; }
 };
 
 
@@ -230,9 +237,20 @@ __device__ __forceinline__ void dma16_at(const char * sbase, uint32_t voff, uint
     asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(voff), "s"(sbase), "s"(lds), "i"(at) : "memory", "m0", "scc");
 }
 
+// D <= 128: a wave keeps all the dims of its own 32 rows (the V^T reads are few enough), so no P^T changes hands, no barrier
+// stands between the two products, and a workgroup fits twice on a CU: 68 KB of LDS, 256 registers. One workgroup's
+// set-up, epilogue and tile latency then run beside the other's products - at D = 128 a tile's products take about as long
+// as a tile takes to arrive. Measured with f16, 32 / 8 heads of 128 (registers -> LDS as pairs, LDS-direct as pairs, LDS-direct
+// solo): 4096 tokens behind 12000 1227, 1029, 868 us (1.09 PFLOP/s); the first 2003 tokens 71, 59, 53 us; D = 64, 16 / 2 heads,
+// 4096 behind 12000: 318, 319 (pairs), 275 us.
+constexpr bool pf_solo(int D, bool dma) { return dma && D <= 128; }
+
+template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
+
 template <uint32_t KT, int D, bool GROUPED, bool DMA>
-__global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
-    static_assert(!DMA || (KT == P1A_KV_F16 && GROUPED && D == 256), "the LDS-direct loads are laid out for f16 rows of 512 bytes");
+__global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const pf_params P) {
+    static_assert(!DMA || (KT == P1A_KV_F16 && GROUPED), "the LDS-direct loads move f16 rows, a 16-key group at a time");
+    constexpr bool PAIR = !pf_solo(D, DMA);
     using C = pf_cfg<D>;
     using L = pf_lay<D>;
     using S = stager<KT, D>;
@@ -304,7 +322,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
                         (half_t) (b.x * s), (half_t) (b.y * s), (half_t) (b.z * s), (half_t) (b.w * s)};
             // Q stays in accumulation registers for the whole kernel: the matrix instructions read them in place, and
             // the vector registers are left to the tiles in flight
-            asm volatile("" : "+a"(qf[ks]));
+            if constexpr (PAIR) asm volatile("" : "+a"(qf[ks]));
         }
     };
     if constexpr (!DMA) load_q();
@@ -313,10 +331,11 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     // (tiles HD * (w & 1) ..) for ALL 64 rows: a V^T fragment read from LDS then feeds two MFMAs (own rows, partner's
     // rows) instead of one, which halves the transposing reads - the slowest LDS traffic of the kernel. The price is
     // that P^T (and the rare rescale factors) of the partner come through LDS, behind one more barrier per tile.
-    constexpr int HD = C::NDT / 2;                            // dim tiles per wave
-    static_assert(C::NDT % 2 == 0, "the dims split over a pair of waves");
-    const int dh = wave & 1;                                  // which half of the dims
-    f16x o[2][HD];                                            // [0]: own rows, [1]: the partner's rows
+    constexpr int NR = PAIR ? 2 : 1;                          // row blocks a wave accumulates
+    constexpr int HD = C::NDT / NR;                           // dim tiles per wave
+    static_assert(C::NDT % NR == 0, "the dims split over a pair of waves");
+    const int dh = PAIR ? wave & 1 : 0;                       // which half of the dims
+    f16x o[NR][HD];                                            // [0]: own rows, [1]: the partner's rows
     // softmax denominator of the own rows: this lane's share, per key half of a tile - the sum of the ROUNDED P values
     // (a packed dot product with ones, fp32 accumulation: v_dot2 keeps f16 denormals), so that it matches what
     // multiplies V. 16 vector instructions in the shadow of the S^T products instead of four more matrix instructions
@@ -330,7 +349,9 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     for (int i = 0; i < 16; ++i) {
         neg_m[i] = 0.f;
 #pragma unroll
-        for (int dt = 0; dt < HD; ++dt) { o[0][dt][i] = 0.f; o[1][dt][i] = 0.f; }
+        for (int dt = 0; dt < HD; ++dt)
+#pragma unroll
+            for (int r = 0; r < NR; ++r) o[r][dt][i] = 0.f;
     }
     asm volatile("" : "+v"(neg_m));                          // (16 registers of one value: not to be rebuilt at every use)
     // exchange areas behind the tile stages: P^T of every wave (BN / 16 k-steps x 64 lanes x 16 bytes), then one float
@@ -491,22 +512,23 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
         }
     };
 
-    // ---- LDS-direct tile loads (DMA): wave w moves the 8 blocks of its 16-key group; instruction j takes keys j and
-    // j + 8 of the group (lanes 0-31 / 32-63, 16 bytes of the row each): the group's base and a loop-invariant lane offset per
-    // instruction - eight registers that spare the loop two 64-bit scalar additions a load. Rows past the last position are fetched as they are (the group lies
+    // ---- LDS-direct tile loads (DMA): wave w moves the NJ blocks of its 16-key group; instruction j takes the keys j, j + NJ,
+    // ... of the group (16 bytes of a row per lane): the group's base and a loop-invariant lane offset per
+    // instruction - registers that spare the loop two 64-bit scalar additions a load. Rows past the last position are fetched as they are (the group lies
     // inside one page, or inside the cache when it is contiguous - the host checks): as K they only make scores that the
     // mask replaces; as V they are overwritten with zeros in LDS once the tile has landed (P = 0 times anything finite).
-    uint32_t dma_vo[8];
+    constexpr int NJ = L::NJ, LPR = 64 / L::RPB;              // loads per tile and wave; lanes per row
+    uint32_t dma_vo[NJ];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) dma_vo[j] = (uint32_t) (8 * g + j) * (uint32_t) P.pg.rowb + (uint32_t) (lane & 31) * 16u;
-    const uint32_t k_dst = lds_addr(lds) + 8 * wave * L::KB, v_dst = lds_addr(lds) + L::KT_B + 8 * wave * L::VB;   // this wave's blocks of stage 0
+    for (int j = 0; j < NJ; ++j) dma_vo[j] = (uint32_t) (NJ * (lane / LPR) + j) * (uint32_t) P.pg.rowb + (uint32_t) (lane % LPR) * 16u;
+    const uint32_t k_dst = lds_addr(lds) + NJ * wave * L::KB, v_dst = lds_addr(lds) + L::KT_B + NJ * wave * L::VB;   // this wave's blocks of stage 0
     auto dma_k = [&](const gbases & gb, int stage, int j) { dma16_at(P.kc + gb.go, dma_vo[j], k_dst, stage * L::STAGE_B + j * L::KB); };
     auto dma_v = [&](const gbases & gb, int stage, int j) { dma16_at(P.vc + gb.go, dma_vo[j], v_dst, stage * L::STAGE_B + j * L::VB); };
     auto zero_v_tail = [&](int tile, char * vtile) {
         if (tile != last_tile) return;
         const int room = pmax - (last_tile * BN + 16 * wave);             // the wave's last key that exists (< 0: none)
         for (int kg = max(room + 1, 0); kg < 16; ++kg)
-            *reinterpret_cast<u2v *>(vtile + L::key_off(16 * wave + kg, L::VB) + lane * 8) = u2v{0u, 0u};
+            if (lane * 8 < L::RB) *reinterpret_cast<u2v *>(vtile + L::key_off(16 * wave + kg, L::VB) + lane * 8) = u2v{0u, 0u};
     };
 
     // ---- prologue: K(0), V(0), K(1) in LDS; (staged through registers: V(1) and K(2) on their way); S^T(0) ----
@@ -520,11 +542,11 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
         const gbases b0 = group_bases(tile0, g0);
         gb_v = group_bases(tile1, g1);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) dma_k(b0, 0, j);
+        for (int j = 0; j < NJ; ++j) dma_k(b0, 0, j);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) dma_v(b0, 0, j);
+        for (int j = 0; j < NJ; ++j) dma_v(b0, 0, j);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) dma_k(gb_v, 1, j);
+        for (int j = 0; j < NJ; ++j) dma_k(gb_v, 1, j);
         gb_k = group_bases(tile2, g2);
         gp_ahead = group_pages(tile_after(tile2));
         load_q();
@@ -552,10 +574,10 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     f16x s_a[2], s_b[2];
     qk(lds, s_a);
     // Masking and the row maximum of a tile are done one step ahead of its softmax (in the shadow of the O^T products of
-    // the tile before it): value i of half u of a lane's S^T column is key k0 + key_of(u, i) + 4 g of the lane's own row.
+    // the tile before it): value i of half u of a lane's S^T column is key k0 + key_of(u, i) + KG g of the lane's own row.
     auto mask_max = [&](f16x (&sv_)[2], int k0_, int idx, float m) {
         const int su = idx >> 4, i = idx & 15;
-        sv_[su][i] = L::key_of(su, i) <= my_pos - k0_ - 4 * g ? sv_[su][i] : NEG_INF;
+        sv_[su][i] = L::key_of(su, i) <= my_pos - k0_ - L::KG * g ? sv_[su][i] : NEG_INF;
         return fmaxf(m, sv_[su][i]);
     };
     // both lane halves of a row -> the row's maximum
@@ -618,8 +640,8 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
             if constexpr (DMA) {   // one tile load every other step: K(it+2) first (it is needed first), then V(it+1)
                 if (k % 2 == 0) {
                     const int j = k / 2;
-                    if (j < 8) dma_k(gb_k, ST, j);                     // over K(it)
-                    else if (j < 16) dma_v(gb_v, 1 - ST, j - 8);       // over V(it-1)
+                    if (j < NJ) dma_k(gb_k, ST, j);                    // over K(it)
+                    else if (j < 2 * NJ) dma_v(gb_v, 1 - ST, j - NJ);  // over V(it-1)
                 }
             }
             const int u = k / C::NKS;
@@ -644,7 +666,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
         }
         // ---- O^T += V^T(it) P^T: set-up. V(it) has been in LDS since the last barrier, so its first fragments are asked
         // for ahead of the exchange: their latency hides behind it ----
-        // Slot e of lane half g in k-step ps is key 32 (ps / 2) + 8 (ps % 2) + 4 g + e (e < 4), or that + 16 for e - 4
+        // Slot e of lane half g in k-step ps is row 16 (ps % 2) + 4 g + e (e < 4) of half ps / 2, or row + 8 for e - 4
         const int i16 = lane & 15, blk = lane >> 4;        // 16-lane block: dims 16 (blk & 1) .., lane half blk >> 1 == g
         const int kk = i16 >> 2, jq = i16 & 3;
         const char * vbase = st_cur + L::KT_B + L::v_lane(4 * g + kk) + (16 * (blk & 1) + 4 * jq) * 2 + dh * HD * 64;
@@ -658,48 +680,55 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
                          __builtin_amdgcn_ds_read_tr16_b64_v4i16((s4 __attribute__((address_space(3))) *) (p0_ + L::v_hi(f / HD)))};
         };
         vfrag vf[NFR];
-        if constexpr (!DMA) {
+        if constexpr (!PAIR || !DMA) {
 #pragma unroll
             for (int f = 0; f < PF_V && f < NFR; ++f) vf[f] = vread(f);
         }
-        // ---- hand P^T and the rescale factor of the own rows to the partner ----
+        if constexpr (PAIR) {
+            // ---- hand P^T and the rescale factor of the own rows to the partner ----
 #pragma unroll
-        for (int ps = 0; ps < BN / 16; ++ps) *reinterpret_cast<h8 *>(px_own + (ps * 64 + lane) * 16) = pb[ps];
-        ax_own[c] = alpha;                                    // (both lane halves: the same value)
-        // (the V(it) loads of the previous step are older than this step's 16: they have landed when 16 are left)
-        if constexpr (DMA) {
-            asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
-            zero_v_tail(tile_c, st_cur + L::KT_B);
+            for (int ps = 0; ps < BN / 16; ++ps) *reinterpret_cast<h8 *>(px_own + (ps * 64 + lane) * 16) = pb[ps];
+            ax_own[c] = alpha;                                    // (both lane halves: the same value)
+            // (the V(it) loads of the previous step are older than this step's 2 NJ: they have landed when those are left)
+            if constexpr (DMA) {
+                wait_vm<2 * NJ>();
+                zero_v_tail(tile_c, st_cur + L::KT_B);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         }
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         // ---- stream 1: O^T += V^T(it) P^T on the matrix pipe; stream 2: masking and row maximum of S^T(it+1) (and K(it+2),
         // V(it+1) -> f16 tiles in LDS when they are staged through registers) ----
         {
-            if constexpr (DMA) {
+            if constexpr (PAIR && DMA) {
 #pragma unroll
                 for (int f = 0; f < PF_V && f < NFR; ++f) vf[f] = vread(f);
             }
-            const float alpha_p = ax_par[c];                                      // (needed before the partner's first product)
+            float alpha_p = 1.0f;
             h8 pp[BN / 16];
+            if constexpr (PAIR) {
+                alpha_p = ax_par[c];                                              // (needed before the partner's first product)
+                pp[0] = *reinterpret_cast<const h8 *>(px_par + lane * 16);
+            }
             constexpr int MPS = 32 / NFR;                                          // next tile's values masked per step
             static_assert(32 % NFR == 0, "mask slices must tile the 32 values of a lane");
             mloc = NEG_INF;
-            pp[0] = *reinterpret_cast<const h8 *>(px_par + lane * 16);
 #pragma unroll
             for (int f = 0; f < NFR; ++f) {
                 if (f + PF_V < NFR) vf[f + PF_V] = vread(f + PF_V);
                 const int ps = f / HD, dt = f % HD;
-                if (dt == 0 && ps + 1 < BN / 16) pp[ps + 1] = *reinterpret_cast<const h8 *>(px_par + ((ps + 1) * 64 + lane) * 16);
+                if (PAIR && dt == 0 && ps + 1 < BN / 16) pp[ps + 1] = *reinterpret_cast<const h8 *>(px_par + ((ps + 1) * 64 + lane) * 16);
                 const h4 l4 = __builtin_bit_cast(h4, vf[f].lo), h4_ = __builtin_bit_cast(h4, vf[f].hi);
                 const h8 a = {l4[0], l4[1], l4[2], l4[3], h4_[0], h4_[1], h4_[2], h4_[3]};
                 o[0][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pb[ps], o[0][dt], 0, 0, 0);
-                if (f == 0 && __builtin_expect(__any(alpha_p != 1.0f), 0)) {       // the partner's rows moved their reference maximum
+                if constexpr (PAIR) {
+                    if (f == 0 && __builtin_expect(__any(alpha_p != 1.0f), 0)) {   // the partner's rows moved their reference maximum
 #pragma unroll
-                    for (int i = 0; i < 16; ++i)
+                        for (int i = 0; i < 16; ++i)
 #pragma unroll
-                        for (int d2 = 0; d2 < HD; ++d2) o[1][d2][i] *= alpha_p;
+                            for (int d2 = 0; d2 < HD; ++d2) o[1][d2][i] *= alpha_p;
+                    }
+                    o[1][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pp[ps], o[1][dt], 0, 0, 0);
                 }
-                o[1][dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pp[ps], o[1][dt], 0, 0, 0);
 #pragma unroll
                 for (int v = 0; v < MPS; ++v) mloc = fmaxf(mloc, s_next[(f * MPS + v) >> 4][(f * MPS + v) & 15]);
                 asm volatile("" : "+v"(mloc));
@@ -729,7 +758,11 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
         // ---- raw loads of K(it+3), V(it+2): one whole step to arrive. Issued back to back: a vector memory instruction
         // holds the wave for as long as the CU's address path needs for it, wherever it is placed ----
         if constexpr (DMA) {
-            asm volatile("s_waitcnt vmcnt(8)" ::: "memory");        // K(it+2) has landed; V(it+1) has until the next exchange
+            if constexpr (PAIR) wait_vm<NJ>();                      // K(it+2) has landed; V(it+1) has until the next exchange
+            else {
+                wait_vm<0>();
+                zero_v_tail(tile_n, st_nxt + L::KT_B);
+            }
         } else {
             const int tile_3 = tile_after(tile_nn);
             const gbases gb_3 = group_bases(tile_3, gp_k);
@@ -762,7 +795,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
     // ---- epilogue: the pair swaps denominators, then each wave normalises, gates and stores its half of the dims of
     // all 64 rows. Lane (row c, half g) holds dims 32 dt + 8 (i / 4) + 4 g + (i % 4) of tile dt ----
     const float l_own = (lp[0] + __shfl_xor(lp[0], 32)) + (lp[1] + __shfl_xor(lp[1], 32));
-    if (g == 0) ax_own[c] = l_own;
+    if constexpr (PAIR) { if (g == 0) ax_own[c] = l_own; }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (also: no tile load is left in flight)
     if (P.nks > 1) {   // one of several key splits: the unnormalised partial of every row, for the merge
         if (g == 0 && live) {
@@ -771,7 +804,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
             ml[1] = l_own;
         }
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
+        for (int r = 0; r < NR; ++r) {
             const int row = row0 + 32 * (r ? wave ^ 1 : wave) + c;
             if (row >= P.R) continue;
             float * orow = P.part_o + (row_index(row) * P.nks + ksp) * D;
@@ -784,13 +817,13 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
         }
         return;
     }
-    const float l_par = ax_par[c];
+    const float l_par = PAIR ? ax_par[c] : 0.f;
     // (the gate values of both row blocks are asked for before the first is used: one memory round trip, not one per 16
     // bytes or per block)
-    f4 gt[2][HD][4];
+    f4 gt[NR][HD][4];
     if (P.gate) {
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
+        for (int r = 0; r < NR; ++r) {
             const float * grow = P.gate + row_index(min(row0 + 32 * (r ? wave ^ 1 : wave) + c, P.R - 1)) * D;
 #pragma unroll
             for (int dt = 0; dt < HD; ++dt)
@@ -799,7 +832,7 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
         }
     }
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
+    for (int r = 0; r < NR; ++r) {
         const int row = row0 + 32 * (r ? wave ^ 1 : wave) + c;
         if (row >= P.R) continue;
         const float inv = 1.0f / (r ? l_par : l_own);
@@ -825,7 +858,8 @@ __global__ void __launch_bounds__(NTHR, 1) prefill_k(const pf_params P) {
 template <uint32_t KT, int D, bool GROUPED, bool DMA = false>
 int launch_pf_g(const pf_params & P, hipStream_t s) {
     using L = pf_lay<D>;
-    const int lds = 2 * L::STAGE_B + (stager<KT, D>::SCALES_VIA_LDS ? 2 * 4 * 16 * stager<KT, D>::SB : 0) + 4 * (BN / 16) * 64 * 16 + 4 * 32 * 4;
+    const int lds = 2 * L::STAGE_B + (stager<KT, D>::SCALES_VIA_LDS ? 2 * 4 * 16 * stager<KT, D>::SB : 0) +
+                    (pf_solo(D, DMA) ? 0 : 4 * (BN / 16) * 64 * 16 + 4 * 32 * 4);
     // (the attribute belongs to the function on ONE device: remembered per device, set again on another)
     static std::atomic<uint32_t> attr_set{0};
     int dev = 0;
@@ -847,7 +881,7 @@ int launch_pf_g(const pf_params & P, hipStream_t s) {
 template <uint32_t KT, int D>
 int launch_pf(const pf_params & P, hipStream_t s) {
     const bool grouped = !P.pg.pt || P.pg.psh >= 4;
-    if constexpr (KT == P1A_KV_F16 && D == 256) {
+    if constexpr (KT == P1A_KV_F16) {
         // (rows of whole 16-byte units at 16-byte aligned addresses: what a 16-byte load per lane needs)
         // and whole 16-key groups that can be read: always inside a page; inside a contiguous cache when it holds them
         const bool groups_ok = P.pg.pt || ((P.p0 + P.T - 1) | 15) < P.n_rows;

@@ -144,6 +144,32 @@ def test_rows_past_the_last_position_are_never_weighted(p1a, kv_type, p0, T):
     assert np.array_equal(out2.cpu().numpy(), out)
 
 
+@pytest.mark.parametrize("kv_type", TYPES)
+@pytest.mark.parametrize("Hq,Hkv,D,p0,T", [(8, 2, 128, 0, 37), (4, 4, 128, 700, 130), (6, 1, 64, 61, 3), (8, 2, 64, 0, 200), (8, 8, 128, 63, 1)])
+def test_small_heads_take_the_same_bits_whichever_way_tiles_come(p1a, kv_type, Hq, Hkv, D, p0, T):
+    """D = 64 / 128: tiles loaded straight into LDS (16-position pages, or the f16 copy of a quantized cache) by workgroups of
+    independent waves, and tiles staged through registers by pairs of waves (8-position pages, dequantization in the kernel):
+    the same bits, the oracle's values, and nothing of what lies past the last position (NaN here)"""
+    n, outs = p0 + T, []
+    q, _, _, gate = I.qkv(n, 1, T, Hq, Hkv, D, f16_inputs=True)
+    for psh in (4, 3):
+        pool = Pool(p1a, kv_type, Hq, Hkv, D, psh, [n], seed=n + D, n_layers=1, layer=0)
+        c, rb, ps = pool.dev_seq(0), O.row_bytes(kv_type, Hkv, D), 1 << psh
+        page, first = int(pool.tabs[(n - 1) >> psh]), ((n - 1) & (ps - 1)) + 1
+        for base in (0, ps * rb):
+            o = page * c.pstride + base + first * rb
+            pool.dpool[o:o + (ps - first) * rb] = 0xff if kv_type != O.KV_F16 else 0x7e
+        for limit in ((1 << 30,) if kv_type == O.KV_F16 else (1 << 30, 0)):
+            p1a.set_prefill_staging_limit(limit)
+            try:
+                outs.append(run_prefill(p1a, c, q, T, p0, Hq, D ** -0.5, gate=gate))
+            finally:
+                p1a.set_prefill_staging_limit(1 << 30)
+    for o in outs[1:]:
+        assert np.array_equal(o, outs[0])
+    check(outs[0], O.attn_rows(pool.host_seq(0), q, (p0 + np.arange(T)).astype(np.int32), Hq, D ** -0.5, gate=gate), f"small heads {kv_type} {Hq}/{Hkv}/{D} p0 {p0} T {T}")
+
+
 def test_f16_contiguous_and_small_pages_take_the_same_bits(p1a):
     """f16, D = 256: a contiguous cache that ends right behind the last position (whole 16-key groups cannot be fetched:
     the register-staged kernel runs), one with room (tiles loaded straight into LDS) and 16-position pages must agree
