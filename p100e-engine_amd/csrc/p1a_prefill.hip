@@ -87,7 +87,9 @@ struct pf_params {
     int n_rows;   // positions the cache holds (contiguous caches: rows that may be read)
     float qscale;
     int R;        // query rows of a kv head: T * GQA
-    int nblk;     // row blocks of a kv head
+    uint32_t gqa_magic;   // floor(2^32 / GQA) (2^32 - 1 for GQA = 1)
+    int rpw;      // rows of a wave: 32, or 16 or 8 (a call of few blocks)
+    int nblk;     // row blocks (4 rpw rows) of a kv head
     int nbg;      // groups of GQA row blocks
     // key splits: with nks > 1 workgroup (block, kv head, ks) walks its share of the block's tiles and leaves an unnormalised
     // partial (O relative to m, and (m, l)) per row in part_o [T*Hq][nks][D] / part_ml [T*Hq][nks][2] for the merge
@@ -269,16 +271,23 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
     const int rb = (P.nbg - 1 - unit / P.Hkv) * P.GQA + hh, hk = unit % P.Hkv;
     if (rb >= P.nblk) return;                                 // (the last group need not be full)
 
-    const int row0 = rb * BM;                                 // first row of the block
-    const int my_row = row0 + 32 * wave + c;                  // this lane's query row
-    const bool live = my_row < P.R;
-    const int my_tok = (live ? my_row : P.R - 1) / P.GQA;
+    const int row0 = rb * 4 * P.rpw;                          // first row of the block
+    const int wrow0 = row0 + P.rpw * wave;                    // first row of this wave
+    const int wrows = min(P.rpw, P.R - wrow0);                // how many it has (<= 0: none)
+    const int my_row = wrow0 + c;                             // this lane's query row
+    const bool live = c < wrows;
+    // row -> token (the multiplication is at most one short)
+    auto tok_of = [&](int r) {
+        const int t = (int) __umulhi((uint32_t) r, P.gqa_magic);
+        return r - t * P.GQA >= P.GQA ? t + 1 : t;
+    };
+    const int my_tok = tok_of(min(my_row, P.R - 1));
     const int my_pos = P.p0 + my_tok;
     const int wave_vis = __builtin_amdgcn_readfirstlane(my_pos);  // every row of this wave sees the positions up to here
-    const int pmax = P.p0 + (min(P.R, row0 + BM) - 1) / P.GQA;   // last position any row of the block sees
+    const int pmax = P.p0 + tok_of(min(P.R, row0 + 4 * P.rpw) - 1);   // last position any row of the block sees
     // a row -> its index among the T * Hq rows of q, out, gate and the partials
-    auto row_index = [&](int r) { const int t = r / P.GQA; return (size_t) t * P.Hq + (size_t) hk * P.GQA + (r - t * P.GQA); };
-    const int ntiles_all = pmax / BN + 1;                        // tiles the block sees
+    auto row_index = [&](int r) { const int t = tok_of(r); return (size_t) t * P.Hq + (size_t) hk * P.GQA + (r - t * P.GQA); };
+    const int ntiles_all = pmax / BN + 1;                         // tiles the block sees
     // this workgroup's share of them: tiles tile_a .. tile_a + ntiles - 1
     int tile_a = 0, ntiles = ntiles_all;
     if (P.nks > 1) {
@@ -301,31 +310,45 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
 
     // ---- Q^T operands (B: k = 16 dims per step, n = query row): lane (row c, half g) holds dims 16 ks + 8 g .. + 7 ----
     h8 qf[C::NKS];
-    // (all the loads first, then the conversions: a load that is waited for before the next one is asked for costs a
-    // memory round trip each - 16 of them in a row were most of what a workgroup spent outside its key loop. With
-    // LDS-direct tiles the rows are asked for right behind the first tiles (the compiler drains its own loads in front of
-    // hand-issued ones, so asking earlier would put the two latencies in a row): one latency, not two.)
-    auto load_q = [&]() {
-        float4 qa[C::NKS], qb[C::NKS];
-        const float * qr = P.q + (live ? row_index(my_row) : 0) * D;
+    // fp32 rows of q, out, gate and the partials are moved whole, 16 bytes per lane in memory order: RPI rows of LPF lanes per
+    // instruction, NRI instructions for 32 rows (a lane's own operands are 32 bytes of each of 32 rows per instruction: four
+    // times the cache lines; 300 tokens, 24 / 4 heads of 256: 25.1 -> 24.8 us, with short blocks 17.6)
+    constexpr int LPF = D / 4, RPI = 64 / LPF, NRI = 32 / RPI, N8 = 8 / RPI;   // (N8: instructions of 8 rows)
+    const int wlast = wrows > 0 ? wrows - 1 : P.R - 1 - wrow0;   // the row that stands in for those past the wave's last
+    auto row_at = [&](int i) { return i * RPI + lane / LPF; };   // the row of the wave that this lane moves in instruction i
+    // the wave's Q rows -> f16 row images at `img` (rows padded by 16 bytes) -> operands. All loads first, then the conversions.
+    auto load_q = [&](char * img, auto && between) {
+        constexpr int QRS = 2 * D + 16;
+        float4 a[NRI];
+        auto fetch = [&](int i) { a[i] = *reinterpret_cast<const float4 *>(P.q + row_index(wrow0 + min(row_at(i), wlast)) * D + 4 * (lane % LPF)); };
 #pragma unroll
-        for (int ks = 0; ks < C::NKS; ++ks) {
-            qa[ks] = make_float4(0.f, 0.f, 0.f, 0.f);
-            qb[ks] = qa[ks];
-            if (live) { qa[ks] = *reinterpret_cast<const float4 *>(qr + 16 * ks + 8 * g); qb[ks] = *reinterpret_cast<const float4 *>(qr + 16 * ks + 8 * g + 4); }
+        for (int i = 0; i < N8; ++i) fetch(i);
+#pragma unroll
+        for (int i = N8; i < NRI; ++i) a[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (P.rpw > 8) {
+#pragma unroll
+            for (int i = N8; i < NRI; ++i) fetch(i);
         }
+        between();
+        const float s = P.qscale;
+#pragma unroll
+        for (int i = 0; i < NRI; ++i)
+            *reinterpret_cast<h4 *>(img + (i * RPI + lane / LPF) * QRS + (lane % LPF) * 8) = h4{(half_t) (a[i].x * s), (half_t) (a[i].y * s), (half_t) (a[i].z * s), (half_t) (a[i].w * s)};
 #pragma unroll
         for (int ks = 0; ks < C::NKS; ++ks) {
-            const float4 a = qa[ks], b = qb[ks];
-            const float s = P.qscale;
-            qf[ks] = h8{(half_t) (a.x * s), (half_t) (a.y * s), (half_t) (a.z * s), (half_t) (a.w * s),
-                        (half_t) (b.x * s), (half_t) (b.y * s), (half_t) (b.z * s), (half_t) (b.w * s)};
+            qf[ks] = *reinterpret_cast<const h8 *>(img + c * QRS + ks * 32 + g * 16);
             // Q stays in accumulation registers for the whole kernel: the matrix instructions read them in place, and
             // the vector registers are left to the tiles in flight
             if constexpr (PAIR) asm volatile("" : "+a"(qf[ks]));
         }
     };
-    if constexpr (!DMA) load_q();
+    // where the images go before the tiles need the room: with LDS-direct tiles, whose K is on its way by then, two waves' into
+    // each V stage (D = 64: the padded rows have an area behind the stages)
+    char * const q_img = !DMA ? lds + wave * 32 * (2 * D + 16) : D == 64 ? lds + 2 * L::STAGE_B + wave * 32 * (2 * D + 16) : lds + (wave >> 1) * L::STAGE_B + L::KT_B + (wave & 1) * 32 * (2 * D + 16);
+    if constexpr (!DMA) {
+        load_q(q_img, [] {});
+        __syncthreads();                                      // (the tiles that follow go over the images)
+    }
 
     // Waves pair up for O^T: the pair (w, w ^ 1) shares its 64 query rows, each wave accumulating HALF the dims
     // (tiles HD * (w & 1) ..) for ALL 64 rows: a V^T fragment read from LDS then feeds two MFMAs (own rows, partner's
@@ -541,17 +564,17 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
         gpages g0 = group_pages(tile0), g1 = group_pages(tile1), g2 = group_pages(tile2);
         const gbases b0 = group_bases(tile0, g0);
         gb_v = group_bases(tile1, g1);
+        load_q(q_img, [&] {
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) dma_k(b0, 0, j);
+            for (int j = 0; j < NJ; ++j) dma_k(b0, 0, j);
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) dma_v(b0, 0, j);
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) dma_k(gb_v, 1, j);
+            for (int j = 0; j < NJ; ++j) dma_k(gb_v, 1, j);
+        });
         gb_k = group_bases(tile2, g2);
         gp_ahead = group_pages(tile_after(tile2));
-        load_q();
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        zero_v_tail(tile0, lds + L::KT_B);
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) dma_v(b0, 0, j);         // (over the Q images, which every wave is done with)
     } else {
         gpages g0 = group_pages(tile0), g1 = group_pages(tile1), g2 = group_pages(tile2);
         const gbases b0 = group_bases(tile0, g0), b1 = group_bases(tile1, g1);
@@ -566,7 +589,7 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
         load_tile(rk, P.kc, tile2, gb_v);
         if constexpr (SVL) { sv = load_sblk(P.vc, tile1, b1); sk = load_sblk(P.kc, tile2, gb_v); }
     }
-    __syncthreads();
+    if constexpr (!DMA) __syncthreads();
     // S^T of two tiles: that of the tile in hand and that of the next, taking turns. (DMA: a step is written out twice, so that
     // neither the values nor the LDS addresses of the two stages have to be moved about. A step is then 64 matrix and 346
     // other instructions instead of 461 - one wave per SIMD issues one in four clocks - and its maximum and denominator
@@ -587,7 +610,13 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
     for (int idx = 0; idx < 32; ++idx) mloc = mask_max(s_a, tile0 * BN, idx, mloc);
     mloc = row_max(mloc);
     // (the first step overwrites K(0) while it runs; every wave has to be done reading it)
-    if constexpr (DMA) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if constexpr (DMA) {
+        if constexpr (!PAIR) {                                // (pairs wait for V(0) at their first exchange)
+            wait_vm<0>();
+            zero_v_tail(tile0, lds + L::KT_B);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
 
     int tile_c = tile0, tile_n = tile1, tile_nn = tile2;      // the tiles of this step, the next and the one after
     auto step = [&](auto par, f16x (&s)[2], f16x (&s_next)[2]) {   // s: S^T of this step's tile, masked; mloc: its row maximum
@@ -797,61 +826,77 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
     const float l_own = (lp[0] + __shfl_xor(lp[0], 32)) + (lp[1] + __shfl_xor(lp[1], 32));
     if constexpr (PAIR) { if (g == 0) ax_own[c] = l_own; }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // (also: no tile load is left in flight)
-    if (P.nks > 1) {   // one of several key splits: the unnormalised partial of every row, for the merge
-        if (g == 0 && live) {
-            float * ml = P.part_ml + (row_index(my_row) * P.nks + ksp) * 2;
-            ml[0] = m_run;
-            ml[1] = l_own;
-        }
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-            const int row = row0 + 32 * (r ? wave ^ 1 : wave) + c;
-            if (row >= P.R) continue;
-            float * orow = P.part_o + (row_index(row) * P.nks + ksp) * D;
+    const float l_par = PAIR ? ax_par[c] : 0.f;
+    const bool part = P.nks > 1;   // one of several key splits: the unnormalised partial of every row, for the merge
+    if (part && g == 0 && live) {
+        float * ml = P.part_ml + (row_index(my_row) * P.nks + ksp) * 2;
+        ml[0] = m_run;
+        ml[1] = l_own;
+    }
+    // (a device full of workgroups, two on a CU: each lane the 16 bytes it holds of its row, which the other workgroup covers; 1 - 2 %
+    // better there than the way below, but 11.2 against 9.7 us for 40 tokens behind 100)
+    if (!PAIR && P.rpw == 32) {
+        const float inv = part ? 1.0f : 1.0f / l_own;
+        const size_t rr = row_index(min(my_row, P.R - 1));
+        f4 gt[HD][4];
+        if (P.gate && !part)
 #pragma unroll
             for (int dt = 0; dt < HD; ++dt)
 #pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4)
-                    *reinterpret_cast<f4 *>(orow + 32 * (dh * HD + dt) + 8 * q4 + 4 * g) =
-                        f4{o[r][dt][4 * q4], o[r][dt][4 * q4 + 1], o[r][dt][4 * q4 + 2], o[r][dt][4 * q4 + 3]};
+                for (int q4 = 0; q4 < 4; ++q4) gt[dt][q4] = *reinterpret_cast<const f4 *>(P.gate + rr * D + 32 * dt + 8 * q4 + 4 * g);
+        if (live) {
+            float * orow = part ? P.part_o + (rr * P.nks + ksp) * D : P.out + rr * D;
+#pragma unroll
+            for (int dt = 0; dt < HD; ++dt)
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4) {
+                    f4 v = {o[0][dt][4 * q4] * inv, o[0][dt][4 * q4 + 1] * inv, o[0][dt][4 * q4 + 2] * inv, o[0][dt][4 * q4 + 3] * inv};
+                    if (P.gate && !part)
+#pragma unroll
+                        for (int x = 0; x < 4; ++x) v[x] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * gt[dt][q4][x]));
+                    *reinterpret_cast<f4 *>(orow + 32 * dt + 8 * q4 + 4 * g) = v;
+                }
         }
         return;
     }
-    const float l_par = PAIR ? ax_par[c] : 0.f;
-    // (the gate values of both row blocks are asked for before the first is used: one memory round trip, not one per 16
-    // bytes or per block)
-    f4 gt[NR][HD][4];
-    if (P.gate) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r) {
-            const float * grow = P.gate + row_index(min(row0 + 32 * (r ? wave ^ 1 : wave) + c, P.R - 1)) * D;
-#pragma unroll
-            for (int dt = 0; dt < HD; ++dt)
-#pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4) gt[r][dt][q4] = *reinterpret_cast<const f4 *>(grow + 32 * (dh * HD + dt) + 8 * q4 + 4 * g);
-        }
-    }
+    // through LDS, where a row is put together (4 D bytes and 16 of padding; the tiles are done with), to whole rows in memory
+    constexpr int ORS = 4 * D + 16;
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
-        const int row = row0 + 32 * (r ? wave ^ 1 : wave) + c;
-        if (row >= P.R) continue;
-        const float inv = 1.0f / (r ? l_par : l_own);
-        float * orow = P.out + row_index(row) * D;
+        const float inv = part ? 1.0f : 1.0f / (r ? l_par : l_own);
+        char * const orow = lds + (32 * (r ? wave ^ 1 : wave) + c) * ORS + dh * HD * 128 + 16 * g;
 #pragma unroll
         for (int dt = 0; dt < HD; ++dt)
 #pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-                const int d0 = 32 * (dh * HD + dt) + 8 * q4 + 4 * g;
-                f4 rr = {o[r][dt][4 * q4] * inv, o[r][dt][4 * q4 + 1] * inv, o[r][dt][4 * q4 + 2] * inv, o[r][dt][4 * q4 + 3] * inv};
-                if (P.gate) {
-                    // sigmoid through the hardware exponential and reciprocal (each within an ulp or two; exact at g = 0): the
-                    // library's full-range expf and IEEE division are some twenty instructions per value, 128 values per lane
+            for (int q4 = 0; q4 < 4; ++q4)
+                *reinterpret_cast<f4 *>(orow + 128 * dt + 32 * q4) = f4{o[r][dt][4 * q4] * inv, o[r][dt][4 * q4 + 1] * inv, o[r][dt][4 * q4 + 2] * inv, o[r][dt][4 * q4 + 3] * inv};
+    }
+    const char * const img = lds + (32 * wave + lane / LPF) * ORS + (lane % LPF) * 16;
+    const int d4 = 4 * (lane % LPF);
 #pragma unroll
-                    for (int x = 0; x < 4; ++x)
-                        rr[x] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * gt[r][dt][q4][x]));
-                }
-                *reinterpret_cast<f4 *>(orow + d0) = rr;
-            }
+    for (int i0 = 0; i0 < NRI; i0 += N8) {
+        f4 gt[N8], v[N8];
+        if (P.gate && !part) {
+#pragma unroll
+            for (int i = 0; i < N8; ++i) gt[i] = *reinterpret_cast<const f4 *>(P.gate + row_index(wrow0 + min(row_at(i0 + i), wlast)) * D + d4);
+        }
+        if (PAIR && i0 == 0) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < N8; ++i) v[i] = *reinterpret_cast<const f4 *>(img + (i0 + i) * RPI * ORS);
+        if (P.gate && !part) {
+            // sigmoid through the hardware exponential and reciprocal (each within an ulp or two; exact at g = 0): the
+            // library's full-range expf and IEEE division are some twenty instructions per value, 128 values per lane
+#pragma unroll
+            for (int i = 0; i < N8; ++i)
+#pragma unroll
+                for (int x = 0; x < 4; ++x) v[i][x] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * gt[i][x]));
+        }
+#pragma unroll
+        for (int i = 0; i < N8; ++i) {
+            const size_t row = row_index(wrow0 + row_at(i0 + i));
+            if (row_at(i0 + i) < wrows) *reinterpret_cast<f4 *>((part ? P.part_o + (row * P.nks + ksp) * D : P.out + row * D) + d4) = v[i];
+        }
+        if ((i0 + N8) * RPI >= wrows) break;
     }
 }
 
@@ -859,7 +904,8 @@ template <uint32_t KT, int D, bool GROUPED, bool DMA = false>
 int launch_pf_g(const pf_params & P, hipStream_t s) {
     using L = pf_lay<D>;
     const int lds = 2 * L::STAGE_B + (stager<KT, D>::SCALES_VIA_LDS ? 2 * 4 * 16 * stager<KT, D>::SB : 0) +
-                    (pf_solo(D, DMA) ? 0 : 4 * (BN / 16) * 64 * 16 + 4 * 32 * 4);
+                    (pf_solo(D, DMA) ? (D == 64 ? BM * (2 * D + 16) : 0) : 4 * (BN / 16) * 64 * 16 + 4 * 32 * 4);
+    static_assert(BM * (4 * D + 16) <= 2 * L::STAGE_B + 4 * (BN / 16) * 64 * 16, "the output rows fit where the tiles and P^T were");
     // (the attribute belongs to the function on ONE device: remembered per device, set again on another)
     static std::atomic<uint32_t> attr_set{0};
     int dev = 0;
@@ -966,6 +1012,15 @@ static int used_key_splits(int T, int p0, int Hq, int Hkv, int cus) {
     const int most = prefill_key_splits(T, p0, Hq, cus), k = plan_splits(((long) T * (Hq / Hkv) + BM - 1) / BM * Hkv, T, p0, Hq, cus);
     return k < most ? k : most;
 }
+// Rows of a block: 128, halved (down to 32) while the call would still leave half of the device without a workgroup. A
+// workgroup's set-up and epilogue are bound by its own CU's memory path (some 20 bytes a clock: 128 rows of q, gate and out
+// take 11 us), its key loop takes the same time however many of its rows are live. 85 tokens behind 126, 24 / 4 heads of 256:
+// 22.8 -> 15.4 us (20.8 when a block was 128 tokens of one head), the first 69 tokens of 4 / 1 heads 22.4 -> 15.4.
+static int block_rows(int R, int Hkv, int nks, int cus) {
+    int b = BM;
+    while (b > 32 && 2L * ((R + b - 1) / b) * Hkv * nks <= cus) b /= 2;
+    return b;
+}
 size_t prefill_part_bytes_o(int T, int Hq, int D, int nks) { return nks > 1 ? (size_t) T * Hq * nks * D * 4 : 0; }
 size_t prefill_part_bytes_ml(int T, int Hq, int nks) { return nks > 1 ? (((size_t) T * Hq * nks * 2 * 4) + 255) & ~(size_t) 255 : 0; }
 void prefill_part_need(int T, int p0, int Hq, int D, size_t & bytes_o, size_t & bytes_ml) {
@@ -988,8 +1043,7 @@ int launch_prefill(const p1a_kv & c, const float * q, float * out, const float *
     P.n_rows = c.n_ctx;
     P.qscale = scale * 1.4426950408889634f;
     P.R = T * P.GQA;
-    P.nblk = (P.R + BM - 1) / BM;
-    P.nbg = (P.nblk + P.GQA - 1) / P.GQA;
+    P.gqa_magic = (uint32_t) ((P.GQA == 1 ? (1ull << 32) - 1 : (1ull << 32) / (unsigned) P.GQA));
     P.nks = 1; P.part_o = nullptr; P.part_ml = nullptr;
     // the caller's scratch: first the f16 staging copy of a quantized cache (when it fits), then the split partials (when
     // they fit behind it); partials that do not fit go to the library's own per-stream buffers
@@ -1010,6 +1064,9 @@ int launch_prefill(const p1a_kv & c, const float * q, float * out, const float *
         } else if (!split_scratch(s, bo, bm, P.part_o, P.part_ml)) return P1A_E_SCRATCH;   // (the split count fixes the result bits: never fewer splits for want of room)
     }
     P.nks = nks;
+    P.rpw = block_rows(P.R, c.Hkv, nks, cu_count()) / 4;
+    P.nblk = (P.R + 4 * P.rpw - 1) / (4 * P.rpw);
+    P.nbg = (P.nblk + P.GQA - 1) / P.GQA;
     auto finish = [&](int rc) {
         if (rc != P1A_OK || P.nks == 1) return rc;
         return launch_merge(P.part_o, P.part_ml, out, gate, P.nks, c.D, Hq, T, s);
