@@ -128,6 +128,9 @@ struct decode_args {
     void * qbuf;          // optional: a16 activation buffer of the (gated) output, [T][Hq*D] values
 };
 int launch_decode(const p1a_kv & c, const decode_args & a, hipStream_t s);
+// the split kernel for the caches dec_mfma_k does not take, and the positions of one of its units
+int launch_decode_any(const p1a_kv & c, const decode_args & a, int rows_per_group, int nsplit, hipStream_t s);
+int decode_any_unit(int D);
 int decode_rows_per_group(const p1a_kv & c, int Hq, int want);
 int decode_nsplit(const p1a_kv & c, int Hq, int nsplit_req, int cus);
 void decode_scratch_need(const p1a_kv & c, int Hq, int rows, int rows_per_group, int nsplit_req, int cus,

@@ -836,92 +836,6 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     }
 }
 
-// ---- generic path: any D % 32 == 0 (<= 512), any GQA, every type; one wave per (split stream, q head, row) ----
-template <uint32_t KT>
-__device__ __forceinline__ float kv_elem(const char * head, int D, int d) {
-    if constexpr (KT == P1A_KV_F16) return (float) reinterpret_cast<const half_t *>(head)[d];
-    else if constexpr (KT == P1A_KV_Q8_0) {
-        const float sc = (float) reinterpret_cast<const half_t *>(head)[d >> 5];
-        return sc * (float) reinterpret_cast<const int8_t *>(head + (D / 32) * 2)[d];
-    } else {
-        const char * b = head + (d >> 5) * 18;
-        const float sc = (float) *reinterpret_cast<const half_t *>(b);
-        const int i = d & 31;
-        const uint32_t by = (uint8_t) b[2 + (i & 15)];
-        return (float) ((int) (i < 16 ? (by & 15) : (by >> 4)) - 8) * sc;
-    }
-}
-
-struct gen_params {
-    const float * q;
-    const char * kc;
-    const char * vc;
-    float * part_o;
-    float * part_ml;
-    kv_view pg;
-    int p0;
-    const int32_t * p0_dev;
-    const int32_t * pos_rows;
-    int RG, Hq, Hkv, D;
-    float qscale;
-    int nsplit;
-};
-
-constexpr int GEN_MAXV = 8;   // dims per lane: D <= 512
-
-template <uint32_t KT>
-__global__ void __launch_bounds__(256) dec_generic_k(const gen_params P) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int h = blockIdx.y, t = blockIdx.z, D = P.D;
-    const int hk = h / (P.Hq / P.Hkv);
-    const int pos = P.pos_rows ? P.pos_rows[t] : (P.p0_dev ? *P.p0_dev : P.p0) + t;
-    const int grow = P.pos_rows ? (t / P.RG) * P.RG : 0;   // the row whose page table the group uses
-    const int32_t * ptab = kv_tab(P.pg, grow);
-    const size_t hb = KT == P1A_KV_F16 ? (size_t) D * 2 : KT == P1A_KV_Q8_0 ? (size_t) (D / 32) * 34 : (size_t) (D / 32) * 18;
-    const int nv = D / 64 + (D % 64 ? 1 : 0);
-    float qv[GEN_MAXV], acc[GEN_MAXV];
-    const float * qr = P.q + ((size_t) t * P.Hq + h) * D;
-#pragma unroll
-    for (int x = 0; x < GEN_MAXV; ++x) {
-        const int d = x * 64 + lane;
-        qv[x] = (x < nv && d < D) ? (float) (half_t) (qr[d] * P.qscale) : 0.f;
-        acc[x] = 0.f;
-    }
-    float m = NEG_INF, l = 0.f;
-    const int sp = blockIdx.x * 4 + wave, NS = P.nsplit * 4;
-    for (int j = sp; j <= pos; j += NS) {
-        const size_t o = kv_off_tab(P.pg, ptab, j) + (size_t) hk * hb;
-        float dot = 0.f;
-#pragma unroll
-        for (int x = 0; x < GEN_MAXV; ++x) {
-            const int d = x * 64 + lane;
-            if (x < nv && d < D) dot += qv[x] * kv_elem<KT>(P.kc + o, D, d);
-        }
-#pragma unroll
-        for (int w = 32; w > 0; w >>= 1) dot += __shfl_xor(dot, w);
-        const float mn = fmaxf(m, dot);
-        const float a = __builtin_amdgcn_exp2f(m - mn), p = __builtin_amdgcn_exp2f(dot - mn);
-        l = l * a + p;
-#pragma unroll
-        for (int x = 0; x < GEN_MAXV; ++x) {
-            const int d = x * 64 + lane;
-            if (x < nv && d < D) acc[x] = acc[x] * a + p * kv_elem<KT>(P.vc + o, D, d);
-        }
-        m = mn;
-    }
-    const size_t row = (size_t) t * P.Hq + h;
-    float * po = P.part_o + (row * NS + sp) * D;
-#pragma unroll
-    for (int x = 0; x < GEN_MAXV; ++x) {
-        const int d = x * 64 + lane;
-        if (x < nv && d < D) po[d] = acc[x];
-    }
-    if (lane == 0) {
-        P.part_ml[(row * NS + sp) * 2] = m;
-        P.part_ml[(row * NS + sp) * 2 + 1] = l;
-    }
-}
-
 // ---- merge of the split partials, in a fixed order, with the fused sigmoid gate ----
 // out[row][d] = sum_s 2^(m_s - M) O_s[d] / sum_s 2^(m_s - M) l_s; empty streams (m = -inf or l = 0) are skipped.
 // One workgroup of 256 threads per (row, 128 dims): thread = (slice of the splits, 4 dims); slice k folds splits k, k + 8,
@@ -1066,12 +980,12 @@ __global__ void __launch_bounds__(256) sigmoid_mul_k(float * __restrict__ x, con
 // The MFMA kernel needs 16-byte aligned head rows (f16: D in {64, 128, 256}; q8_0 / q4_0: D == 256), 16-byte aligned
 // bases and strides, pages of >= 16 positions and GQA <= 16; q8_0 / q4_0 at D = 64 or 128 (head rows of whole dwords)
 // take its staged build, which fetches 4 bytes per lane and only needs 4-byte alignment. Everything else takes the
-// generic kernel.
+// kernel of p1a_decode_any.hip.
 struct dec_plan {
     bool mfma;
     int GQA, NW, NT, RG;
     int nsplit;    // split streams
-    int NS;        // partials per output row (what merge_k folds)
+    int NS;        // partials per output row the scratch is sized for (at least nsplit, what merge_k folds)
 };
 
 bool mfma_ok(const p1a_kv & c, int GQA) {
@@ -1091,9 +1005,14 @@ dec_plan make_plan(const p1a_kv & c, int Hq, int rows_per_group, int nsplit_req,
     if (!p.mfma) {
         p.NW = 4; p.NT = 1;
         p.RG = rows_per_group < 1 ? 1 : rows_per_group;   // no sharing here: the group only selects the page table
+        // the scratch such a call asks for (4 partials for every 2 CUs per q head) is part of what callers size and
+        // allocate by; one workgroup per CU needs no more of them than that
         int n = nsplit_req > 0 ? nsplit_req : 2 * cus / Hq;
-        p.nsplit = n < 1 ? 1 : (n > 1024 ? 1024 : n);
-        p.NS = p.nsplit * 4;
+        n = n < 1 ? 1 : (n > 1024 ? 1024 : n);
+        p.NS = n * 4;
+        if (nsplit_req <= 0) n = cus / c.Hkv < p.NS ? cus / c.Hkv : p.NS;
+        if (n >= 8) n &= ~7;
+        p.nsplit = n < 1 ? 1 : n;
         return p;
     }
     const int cap = 32 / p.GQA < 4 ? 32 / p.GQA : 4;
@@ -1192,20 +1111,11 @@ int launch_decode(const p1a_kv & c, const decode_args & a, hipStream_t s) {
         else if (c.D == 128) rc = launch_mfma<P1A_KV_F16, 128>(c, a, pl, s);
         else rc = launch_mfma<P1A_KV_F16, 64>(c, a, pl, s);
     } else {
-        gen_params P;
-        P.q = a.q; P.kc = (const char *) c.k; P.vc = (const char *) c.v;
-        P.part_o = a.part_o; P.part_ml = a.part_ml; P.pg = view_of(c);
-        P.p0 = a.p0; P.p0_dev = a.p0_dev; P.pos_rows = a.pos_rows; P.RG = pl.RG;
-        P.Hq = a.Hq; P.Hkv = c.Hkv; P.D = c.D; P.qscale = a.scale * 1.4426950408889634f; P.nsplit = pl.nsplit;
-        const dim3 grid(pl.nsplit, a.Hq, a.T);
-        if (c.type == P1A_KV_F16) dec_generic_k<P1A_KV_F16><<<grid, 256, 0, s>>>(P);
-        else if (c.type == P1A_KV_Q8_0) dec_generic_k<P1A_KV_Q8_0><<<grid, 256, 0, s>>>(P);
-        else dec_generic_k<P1A_KV_Q4_0><<<grid, 256, 0, s>>>(P);
-        rc = hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+        rc = launch_decode_any(c, a, pl.RG, pl.nsplit, s);
     }
     if (rc != P1A_OK || a.skip_merge) return rc;
-    merge_k<<<dim3(a.T * a.Hq, (c.D + MRG_DIMS - 1) / MRG_DIMS), 256, 0, s>>>(a.part_o, a.part_ml, a.out, a.gate, pl.NS, c.D, a.qbuf, a.Hq, a.T,
-                                                       pl.mfma ? a.pos_rows : nullptr, 32 * pl.NW);
+    merge_k<<<dim3(a.T * a.Hq, (c.D + MRG_DIMS - 1) / MRG_DIMS), 256, 0, s>>>(a.part_o, a.part_ml, a.out, a.gate, pl.nsplit, c.D, a.qbuf, a.Hq, a.T,
+                                                       a.pos_rows, pl.mfma ? 32 * pl.NW : decode_any_unit(c.D));
     return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
 }
 
