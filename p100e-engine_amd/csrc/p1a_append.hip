@@ -24,6 +24,11 @@ __device__ __forceinline__ float xor8_max(float a) {
     return a;
 }
 
+template <int CTRL> __device__ __forceinline__ float dpp(float x) {
+    const int xi = __builtin_bit_cast(int, x);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(xi, xi, CTRL, 0xf, 0xf, false));
+}
+
 __device__ __forceinline__ uint16_t f16_bits(float f) {
     const half_t h = (half_t) f;   // v_cvt_f16_f32, round-to-nearest-even
     return __builtin_bit_cast(uint16_t, h);
@@ -192,6 +197,17 @@ inline double det_log(double x) {
     const double lm = (2.0 * s) * p;
     return (double) e * LN2_HI + ((double) e * LN2_LO + lm);
 }
+// interleaved M-RoPE (src/fast/mrope.cuh:25-33): pair j rotates by the position of the stream its sector selects
+__device__ __forceinline__ int pair_pos(const mrope_view & mr, const int32_t * pos, int t, int j) {
+    if (!mr.p) return pos[t];
+    const int sector = j % mr.sect;
+    int st;
+    if (sector % 3 == 1 && sector < 3 * mr.s1) st = 1;
+    else if (sector % 3 == 2 && sector < 3 * mr.s2) st = 2;
+    else if (sector % 3 == 0 && sector < 3 * mr.s0) st = 0;
+    else return 0;
+    return mr.p[(size_t) st * mr.stride + t];
+}
 template <uint32_t KT>
 __global__ void __launch_bounds__(64) prep_k(const float * __restrict__ qg, const float * __restrict__ k,
                                              const float * __restrict__ v, const float * __restrict__ qn,
@@ -246,17 +262,6 @@ __global__ void __launch_bounds__(64) prep_k(const float * __restrict__ qg, cons
     const int half = n_rot >> 1, hl = half >> 2;
     const bool lo = i < hl, rot = i < 2 * hl;
     const int partner = lo ? i + hl : i - hl;
-    // interleaved M-RoPE (src/fast/mrope.cuh:25-33): pair j rotates by the position of the stream its sector selects
-    auto pair_pos = [&](int j) {
-        if (!mr.p) return pos[t];
-        const int sector = j % mr.sect;
-        int st;
-        if (sector % 3 == 1 && sector < 3 * mr.s1) st = 1;
-        else if (sector % 3 == 2 && sector < 3 * mr.s2) st = 2;
-        else if (sector % 3 == 0 && sector < 3 * mr.s0) st = 0;
-        else return 0;
-        return mr.p[(size_t) st * mr.stride + t];
-    };
     // the angle tables of the head: pair j is computed once, by lane j & 63 (slot j >> 6), and handed round by shuffle
     float tc[2] = {1.f, 1.f}, tsn[2] = {0.f, 0.f};
 #pragma unroll
@@ -264,7 +269,7 @@ __global__ void __launch_bounds__(64) prep_k(const float * __restrict__ qg, cons
         const int jj = i + 64 * sl;
         if (jj < half) {
             const float inv = (float) det_exp(((-2.0 * (double) jj) / (double) n_rot) * ln_base);
-            const float theta = (float) pair_pos(jj) * inv;
+            const float theta = (float) pair_pos(mr, pos, t, jj) * inv;
             det_sincos((double) theta, tc[sl], tsn[sl]);
         }
     }
@@ -286,6 +291,117 @@ __global__ void __launch_bounds__(64) prep_k(const float * __restrict__ qg, cons
         if (live) reinterpret_cast<float4 *>(q + ((size_t) t * Hq + h) * D)[i] = r;
     } else {
         write_head(kc, h, r);
+    }
+}
+
+// The same for calls of many tokens, which one wave per (head, token) spent on the angles - some 250 double operations,
+// repeated by each of the token's heads - instead of on moving q, gate, k and v: a workgroup takes a token, works its angles
+// out once (thread j pair j) and its groups of G lanes (the power of two at or above D / 4: 64 / G heads to a wave) walk the
+// heads, the rows of the next one requested while one is normed, rotated and written. Every operation and its order are
+// prep_k's: the lanes past a head add zeros there, and a balanced tree of equal partial sums does not care how they travel.
+// Bound by memory, and by the latency of a head's turn where the call is small: 24 / 4 heads of 256, 4096 tokens (424 MB)
+// 93 -> 74 us = 5.7 TB/s (a 200 MB copy: 5.4), 512 tokens 16.2 -> 12.2 us; 32 / 8 of 128, 2003 tokens 60 -> 27 us; 8 / 8 of
+// 64, 4096 tokens 49 -> 17 us. NT: q | gate rows read past the caches - worth it once they do not stay there anyway (2003
+// tokens of 24 heads of 256, 98 MB: 44.7 -> 40.7 us; 512 tokens, 25 MB: 12.2 -> 14.8 us).
+template <uint32_t KT, int G, bool NT>
+__global__ void __launch_bounds__(512) prep_rows_k(const float * __restrict__ qg, const float * __restrict__ k,
+                                                   const float * __restrict__ v, const float * __restrict__ qn,
+                                                   const float * __restrict__ kn, const int32_t * __restrict__ pos,
+                                                   float * __restrict__ q, float * __restrict__ gate, char * kc, char * vc, int p0,
+                                                   int Hq, int Hkv, int D, int n_rot, double ln_base, float eps, int ldq, int ldk,
+                                                   int ldv, kv_view pg, mrope_view mr) {
+    __shared__ __attribute__((aligned(16))) float tc[128], tsn[128];
+    const int t = blockIdx.x, i = threadIdx.x % G, H = Hq + 2 * Hkv, step = (int) blockDim.x / G;
+    const bool live = 4 * i < D;
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+    auto load = [&](int b, f4 & a, f4 & gt) {
+        a = gt = zero;
+        if (b >= H || !live) return;
+        const float * src = b < Hq ? qg + (size_t) t * ldq + (size_t) b * 2 * D
+                          : b < Hq + Hkv ? k + (size_t) t * ldk + (size_t) (b - Hq) * D : v + (size_t) t * ldv + (size_t) (b - Hq - Hkv) * D;
+        const f4 * x = reinterpret_cast<const f4 *>(src) + i;
+        a = NT ? __builtin_nontemporal_load(x) : *x;
+        if (b < Hq) gt = NT ? __builtin_nontemporal_load(x + D / 4) : x[D / 4];
+    };
+    int b = threadIdx.x / G;
+    f4 a, gt;
+    load(b, a, gt);
+    f4 wq = zero, wk = zero;
+    if (qn && live) wq = reinterpret_cast<const f4 *>(qn)[i];
+    if (kn && live) wk = reinterpret_cast<const f4 *>(kn)[i];
+    const int half = n_rot >> 1, hl = half >> 2;
+    if ((int) threadIdx.x < half) {
+        const int jj = threadIdx.x;
+        const float inv = (float) det_exp(((-2.0 * (double) jj) / (double) n_rot) * ln_base);
+        const float theta = (float) pair_pos(mr, pos, t, jj) * inv;
+        det_sincos((double) theta, tc[jj], tsn[jj]);
+    }
+    const int row = p0 < 0 ? pos[t] : p0 + t;
+    const size_t o = kv_off_tab(pg, kv_tab(pg, t), row);
+    const int nb = D / 32, blk = i >> 3, j8 = i & 7;
+    __syncthreads();
+    const bool lo = i < hl, rot = i < 2 * hl;
+    const int partner = (threadIdx.x & 63) - i + (rot ? (lo ? i + hl : i - hl) : i);
+    f4 c4 = {1.f, 1.f, 1.f, 1.f}, s4_ = {0.f, 0.f, 0.f, 0.f};
+    if (rot) {
+        const int jj = 4 * (lo ? i : i - hl);
+        c4 = *reinterpret_cast<const f4 *>(tc + jj);
+        s4_ = *reinterpret_cast<const f4 *>(tsn + jj);
+    }
+    for (; b < H; b += step) {
+        f4 an, gn;
+        load(b + step, an, gn);
+        const bool isq = b < Hq;
+        float x[4] = {a[0], a[1], a[2], a[3]};
+        if (b < Hq + Hkv) {
+            float ss = a[0] * a[0];
+            ss = ss + a[1] * a[1];
+            ss = ss + a[2] * a[2];
+            ss = ss + a[3] * a[3];
+            ss = ss + dpp<0xB1>(ss);      // lane ^ 1
+            ss = ss + dpp<0x4E>(ss);      // lane ^ 2
+            ss = ss + dpp<0x141>(ss);     // the other quad of 8
+            if constexpr (G >= 16) ss = ss + dpp<0x140>(ss);   // the other 8 of 16
+            if constexpr (G >= 32) ss = ss + __shfl_xor(ss, 16);
+            if constexpr (G >= 64) ss = ss + __shfl_xor(ss, 32);
+            const float sc = 1.0f / sqrtf(ss / (float) D + eps);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = x[e] * sc;
+            const f4 ww = isq ? wq : wk;
+            if (isq ? qn != nullptr : kn != nullptr) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = x[e] * ww[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float other = __shfl(x[e], partner);
+                if (rot) {
+                    const float x0 = lo ? x[e] : other, x1 = lo ? other : x[e];
+                    const float p0_ = x0 * (lo ? c4[e] : s4_[e]), p1_ = x1 * (lo ? s4_[e] : c4[e]);
+                    x[e] = lo ? p0_ - p1_ : p0_ + p1_;
+                }
+            }
+        }
+        const float4 r = make_float4(x[0], x[1], x[2], x[3]);
+        if (isq) {
+            if (live) {
+                const size_t at = ((size_t) t * Hq + b) * D;
+                __builtin_nontemporal_store(gt, reinterpret_cast<f4 *>(gate + at) + i);   // (wanted again only behind the attention)
+                reinterpret_cast<float4 *>(q + at)[i] = r;
+            }
+        } else {
+            const int h = b < Hq + Hkv ? b - Hq : b - Hq - Hkv;
+            char * const cache = b < Hq + Hkv ? kc : vc;
+            if constexpr (KT == P1A_KV_F16) {
+                if (live) reinterpret_cast<h4 *>(cache + o + (size_t) h * D * 2)[i] = h4{(half_t) r.x, (half_t) r.y, (half_t) r.z, (half_t) r.w};
+            } else if constexpr (KT == P1A_KV_Q8_0) {
+                if (live) q8_block(r, j8, cache + o + (size_t) h * nb * 34, blk, nb);
+            } else {
+                if (live) q4_block(r, j8, cache + o + ((size_t) h * nb + blk) * 18);
+            }
+        }
+        a = an;
+        gt = gn;
     }
 }
 
@@ -380,9 +496,28 @@ int launch_prep(const p1a_kv & c, const float * qg, const float * k, const float
                 const int32_t * pos, float * q, float * gate, int p0, int T, int Hq, int n_rot, float freq_base, float eps,
                 int ldq, int ldk, int ldv, const mrope_view & mr, hipStream_t s) {
     const kv_view pg = view_of(c);
-    const dim3 grid(Hq + 2 * c.Hkv, T);
     char * kc = (char *) c.k, * vc = (char *) c.v;
     const double ln_base = det_log((double) freq_base);
+    // One wave per (head, token) until those waves fill three quarters of what the device holds (8192): 24 / 4 heads of 256
+    // are equal there (128 tokens 6.5 against 8.0 us, 256 tokens 10.5 against 9.6), 32 / 8 of 128 6.8 against 6.4.
+    const int H = Hq + 2 * c.Hkv;
+    if ((long long) T * H >= 6144) {
+        // 8 waves to a token, or 4 where two turns of those see all heads
+#define P1A_PREP_ROWS(KT_, G_) do { const int th_ = H > 2 * (256 / G_) ? 512 : 256; \
+            if (nt) prep_rows_k<KT_, G_, true><<<T, th_, 0, s>>>(P1A_PREP_ARGS); else prep_rows_k<KT_, G_, false><<<T, th_, 0, s>>>(P1A_PREP_ARGS); } while (0)
+#define P1A_PREP_ARGS qg, k, v, q_norm, k_norm, pos, q, gate, kc, vc, p0, Hq, c.Hkv, c.D, n_rot, ln_base, eps, ldq, ldk, ldv, pg, mr
+#define P1A_PREP_ROWS_G(KT_) do { if (c.D > 128) P1A_PREP_ROWS(KT_, 64); else if (c.D > 64) P1A_PREP_ROWS(KT_, 32); else if (c.D > 32) P1A_PREP_ROWS(KT_, 16); \
+                                  else P1A_PREP_ROWS(KT_, 8); } while (0)
+        const bool nt = (size_t) T * Hq * c.D * 8 >= (size_t) 80 << 20;
+        if (c.type == P1A_KV_F16) P1A_PREP_ROWS_G(P1A_KV_F16);
+        else if (c.type == P1A_KV_Q8_0) P1A_PREP_ROWS_G(P1A_KV_Q8_0);
+        else P1A_PREP_ROWS_G(P1A_KV_Q4_0);
+#undef P1A_PREP_ROWS_G
+#undef P1A_PREP_ARGS
+#undef P1A_PREP_ROWS
+        return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+    }
+    const dim3 grid(H, T);
 #define P1A_PREP(KT_) prep_k<KT_><<<grid, 64, 0, s>>>(qg, k, v, q_norm, k_norm, pos, q, gate, kc, vc, p0, Hq, c.Hkv, c.D, n_rot, \
                                                       ln_base, eps, ldq, ldk, ldv, pg, mr)
     if (c.type == P1A_KV_F16) P1A_PREP(P1A_KV_F16);

@@ -198,3 +198,67 @@ def test_mrope_positions(p1a, kv_type):
     with pytest.raises(p1a.P1AError, match="M-RoPE"):
         p1a.attn_prep(dev(qg), dev(k), dev(v), dev(qn), dev(kn), dev(pos), q2, gate, c2, -1, T, Hq, n_rot, base, eps,
                       mrope=(dev(mp), T + 3, (11, 11, 10), 0))
+
+
+@pytest.mark.parametrize("kv_type", TYPES)
+@pytest.mark.parametrize("Hq,Hkv,D,n_rot,by_pos", [(24, 4, 256, 64, False), (2, 1, 256, 256, True), (5, 1, 192, 184, False), (32, 8, 128, 128, True),
+                                                   (4, 2, 96, 96, False), (6, 3, 64, 0, True), (7, 1, 32, 8, False)])
+def test_calls_of_many_tokens(p1a, kv_type, Hq, Hkv, D, n_rot, by_pos):
+    """a call large enough for the workgroup-per-token kernel (64, 32, 16 and 8 lanes to a head, dead lanes at D = 192 and 96):
+    the oracle's bits, and those of the same rows in calls of one token (one wave per head), strided inputs, no norm weight
+    where n_rot is 0"""
+    base, eps = 1e6, 1e-6
+    T = 16384 // (Hq + 2 * Hkv) + 1
+    p0, n_ctx = 11, T + 16
+    qg, k, v, qn, kn = make(D + n_rot + Hq, T, Hq, Hkv, D)
+    if n_rot == 0:
+        qn = kn = None
+    pos = (p0 + np.arange(T)).astype(np.int32)
+    if by_pos:
+        pos = pos[I.rng(5).permutation(T)].copy()
+    host = O.HostKV.contiguous(kv_type, n_ctx, Hkv, D)
+    q_ref, gate_ref = O.attn_prep(host, qg, k, v, qn, kn, pos, -1 if by_pos else p0, Hq, n_rot, base, eps)
+    c = p1a.KVCache.contiguous(kv_type, n_ctx, Hkv, D)
+    c1 = p1a.KVCache.contiguous(kv_type, n_ctx, Hkv, D)
+    ldq, ldk, ldv = Hq * 2 * D + 8, Hkv * D + 4, Hkv * D + 12
+
+    def strided(a, ld):
+        buf = np.full((T, ld), 7.0, np.float32)
+        buf[:, : a[0].size] = a.reshape(T, -1)
+        return dev(buf)
+    dqg, dk, dv, dpos = strided(qg, ldq), strided(k, ldk), strided(v, ldv), dev(pos)
+    dqn, dkn = (None if x is None else dev(x) for x in (qn, kn))
+    q, gate = torch.zeros((T, Hq, D), device="cuda"), torch.zeros((T, Hq * D), device="cuda")
+    p1a.attn_prep(dqg, dk, dv, dqn, dkn, dpos, q, gate, c, -1 if by_pos else p0, T, Hq, n_rot, base, eps, ldq=ldq, ldk=ldk, ldv=ldv)
+    assert np.array_equal(gate.cpu().numpy(), gate_ref)
+    assert np.array_equal(q.cpu().numpy().view(np.int32), q_ref.view(np.int32))
+    assert np.array_equal(c._keep[0].cpu().numpy(), host.k)
+    assert np.array_equal(c._keep[1].cpu().numpy(), host.v)
+    for t in (0, T // 2, T - 1):
+        q1, g1 = torch.zeros((1, Hq, D), device="cuda"), torch.zeros((1, Hq * D), device="cuda")
+        p1a.attn_prep(dqg[t:], dk[t:], dv[t:], dqn, dkn, dpos[t:], q1, g1, c1, -1 if by_pos else p0 + t, 1, Hq, n_rot, base, eps, ldq=ldq, ldk=ldk, ldv=ldv)
+        assert torch.equal(q1[0], q[t]) and torch.equal(g1[0], gate[t])
+
+
+@pytest.mark.parametrize("Hq,D,n_rot", [(24, 256, 64), (8, 128, 128)])
+def test_mrope_in_a_call_of_many_tokens(p1a, Hq, D, n_rot):
+    """interleaved M-RoPE positions through the workgroup-per-token kernel: the bits of one-token calls"""
+    Hkv, sect = 2, (11, 11, 10)
+    T = 16384 // (Hq + 2 * Hkv) + 3
+    g = I.rng(9)
+    qg, k, v, qn, kn = make(3, T, Hq, Hkv, D)
+    mr = dev(np.ascontiguousarray(g.integers(0, 5000, (3, T)).astype(np.int32)))
+    pos = dev(np.arange(T, dtype=np.int32))
+    dqg, dk, dv, dqn, dkn = (dev(x) for x in (qg, k, v, qn, kn))
+    out = []
+    for step in (T, 1):
+        c = p1a.KVCache.contiguous(O.KV_Q8_0, T, Hkv, D)
+        q, gate = torch.zeros((T, Hq, D), device="cuda"), torch.zeros((T, Hq * D), device="cuda")
+        for a in (range(0, T, step) if step == T else (0, 1, T - 2, T - 1)):
+            n = min(step, T - a)
+            p1a.attn_prep(dqg[a:], dk[a:], dv[a:], dqn, dkn, pos[a:], q[a:a + n], gate[a:a + n], c, a, n, Hq, n_rot, 1e6, 1e-6,
+                          mrope=(mr[:, a:a + n].contiguous(), n, sect, 32))
+        out.append((q, gate, c._keep[0].reshape(T, -1), c._keep[1].reshape(T, -1)))
+    for x, y in zip(*out):
+        for t in (0, 1, T - 2, T - 1):
+            assert torch.equal(x[t], y[t]), t
