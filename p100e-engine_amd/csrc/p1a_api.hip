@@ -179,6 +179,7 @@ int decode_call(const float * q, const p1a_kv * c, float * out, const float * ga
     a.rows_per_group = decode_rows_per_group(*c, Hq, pos_rows ? (rows_per_seq < 1 ? 1 : rows_per_seq) : T);
     // a sequence's rows must split into whole groups, or a group would mix two sequences
     while (pos_rows && rows_per_seq > 1 && rows_per_seq % a.rows_per_group) --a.rows_per_group;
+    a.rows_per_seq = pos_rows ? (rows_per_seq < 1 ? 1 : rows_per_seq) : 1 << 30;
     a.nsplit = nsplit_req();
     a.cus = cu_count();
     a.skip_merge = split_only;

@@ -117,6 +117,7 @@ struct decode_args {
     const int32_t * p0_dev;
     const int32_t * pos_rows;
     int rows_per_group;   // rows sharing one KV read
+    int rows_per_seq;     // rows of one sequence (1 << 30 without per-row positions: all of them)
     int Hq;
     float scale;
     int nsplit;           // requested split streams (0 = default for the device)

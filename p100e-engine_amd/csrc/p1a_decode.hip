@@ -78,6 +78,7 @@ struct dec_params {
     int T, RG, Hq, Hkv, GQA;
     float qscale;     // softmax scale * log2(e)
     int nsplit;       // split streams
+    int GPS;          // row groups of a sequence
     int hkv_sh;       // log2(Hkv) when Hkv is a power of two, else -1
     int npt;          // page-table entries of one sequence (ceil(n_ctx / page positions)); 0 = contiguous
 };
@@ -200,14 +201,18 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     const int lane = threadIdx.x & 63, wave = rfl(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
     // blockIdx.x -> (split stream, head group). Workgroups are dealt to the 8 XCDs round-robin by linear index, so
-    // the kv heads of one split stream (which share cache lines) are given the same index mod 8.
+    // the kv heads of one split stream (which share cache lines) are given the same index mod 8. Sequence r of a batch
+    // starts on XCD r mod 8 (all of its row groups, which read the same keys): sequences fill the streams from 0 up, and
+    // with stream s on XCD s mod 8 in each of them the low XCDs had the work of all short ones. A layer of 32 sequences
+    // (24 / 4 heads of 256, q8_0, prep and merge included), each of 256 keys - 128 live workgroups, all on XCD 0 - 43 -> 29
+    // us, of 1024 keys 47 -> 39, of 2048 (eight streams) 51 both ways; of 300 ... 5000 keys 57 -> 48.
     const int HG = P.Hkv;
     int split, hg;
     if ((P.nsplit & 7) == 0) {
         const int i = blockIdx.x, j = i >> 3;
         const int jq = P.hkv_sh >= 0 ? j >> P.hkv_sh : j / HG;
         hg = j - jq * HG;
-        split = jq * 8 + (i & 7);
+        split = jq * 8 + ((i - (P.GPS == 1 ? (int) blockIdx.y : (int) blockIdx.y / P.GPS)) & 7);
     } else {
         split = blockIdx.x / HG;
         hg = blockIdx.x - split * HG;
@@ -1043,6 +1048,7 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hi
     P.p0 = a.p0; P.p0_dev = a.p0_dev; P.pos_rows = a.pos_rows;
     P.T = a.T; P.RG = pl.RG; P.Hq = a.Hq; P.Hkv = c.Hkv; P.GQA = pl.GQA;
     P.qscale = a.scale * 1.4426950408889634f; P.nsplit = pl.nsplit;
+    P.GPS = a.rows_per_seq > pl.RG ? a.rows_per_seq / pl.RG : 1;
     P.hkv_sh = -1;
     for (int sh = 0; sh < 16; ++sh) if ((1 << sh) == c.Hkv) P.hkv_sh = sh;
     P.npt = c.pt ? (int) (((long long) c.n_ctx + (1LL << c.psh) - 1) >> c.psh) : 0;

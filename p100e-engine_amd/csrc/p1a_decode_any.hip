@@ -41,6 +41,7 @@ struct any_params {
     int RG, Hq, Hkv, GQA, D;
     float qscale;     // softmax scale * log2(e)
     int nsplit;
+    int SQ;           // rows of a sequence (1 << 30: all rows are one sequence's)
 };
 
 // a load through the scalar cache at a wave-uniform address (page tables and positions do not change while a kernel runs)
@@ -78,12 +79,13 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
     const int nb = EX ? NBM : P.D >> 5, D = nb * 32;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
-    // the kv heads of one split stream share cache lines: given the same index mod 8 they sit on one XCD
+    // the kv heads of one split stream share cache lines: given the same index mod 8 they sit on one XCD, and
+    // sequence r of a batch starts on XCD r mod 8 (short ones only fill the first streams: p1a_decode.hip)
     int split, hk;
     if ((P.nsplit & 7) == 0) {
         const int i = blockIdx.x, j = i >> 3, jq = j / P.Hkv;
         hk = j - jq * P.Hkv;
-        split = jq * 8 + (i & 7);
+        split = jq * 8 + ((i - (int) blockIdx.z / P.SQ) & 7);
     } else {
         split = blockIdx.x / P.Hkv;
         hk = blockIdx.x - split * P.Hkv;
@@ -370,6 +372,7 @@ int launch_decode_any(const p1a_kv & c, const decode_args & a, int rows_per_grou
     P.part_o = a.part_o; P.part_ml = a.part_ml; P.pg = view_of(c);
     P.p0 = a.p0; P.p0_dev = a.p0_dev; P.pos_rows = a.pos_rows; P.RG = rows_per_group;
     P.Hq = a.Hq; P.Hkv = c.Hkv; P.GQA = a.Hq / c.Hkv; P.D = c.D; P.qscale = a.scale * 1.4426950408889634f; P.nsplit = nsplit;
+    P.SQ = a.rows_per_seq;
     const dim3 grid(nsplit * c.Hkv, (P.GQA + 15) / 16, a.T);
     if (c.type == P1A_KV_F16) launch_kt<P1A_KV_F16>(P, grid, s);
     else if (c.type == P1A_KV_Q8_0) launch_kt<P1A_KV_Q8_0>(P, grid, s);
