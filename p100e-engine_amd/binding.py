@@ -174,12 +174,24 @@ def _check(rc, what):
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()     # (the c_void_p argument takes the number as it is)
+
+
+_torch = _raw_stream = _device = None
 
 
 def _stream():
-    import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream's handle. A call on little data is bound by what the host does around its launches, and half of
+    that was torch.cuda.current_stream(), which builds a Stream object; the handle alone is asked for once torch has a device."""
+    global _torch, _raw_stream, _device
+    if _torch is None:
+        import torch
+        _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        _device = getattr(torch._C, "_cuda_getDevice", None)
+        _torch = torch
+    if _raw_stream is None or _device is None or not _torch.cuda.is_initialized():
+        return _torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_device())
 
 
 class KVCache:
@@ -190,6 +202,8 @@ class KVCache:
     does (tests/fast_sessions_test.cu:75,91-92) - one layer selected by the k / v base pointers, a slot by its
     page-table row. (The engine's own pool layout is class Pool's.)
     """
+
+    _pt_off = 0          # first page-table entry of a slot's view
 
     def __init__(self, kv_type, n_ctx, Hkv, D, k, v, pt=None, rtab=None, psh=0, pstride=0, keep=()):
         self.type, self.n_ctx, self.Hkv, self.D = kv_type, n_ctx, Hkv, D
@@ -232,14 +246,9 @@ class KVCache:
         return c
 
     def struct(self):
-        s = p1a_kv()
-        s.type, s.n_ctx, s.Hkv, s.D = self.type, self.n_ctx, self.Hkv, self.D
-        s.k, s.v = self.k, self.v
-        off = getattr(self, "_pt_off", 0)
-        s.pt = None if self.pt is None else self.pt.data_ptr() + 4 * off
-        s.rtab = None if self.rtab is None else self.rtab.data_ptr()
-        s.psh, s.pstride = self.psh, self.pstride
-        return s
+        pt, rtab = self.pt, self.rtab
+        return p1a_kv(self.type, self.n_ctx, self.Hkv, self.D, self.k, self.v, None if pt is None else pt.data_ptr() + 4 * self._pt_off,
+                      None if rtab is None else rtab.data_ptr(), self.psh, self.pstride)
 
 
 def kv_append(c, k, v, p0, T):
@@ -273,8 +282,8 @@ def attn_prep(qg, k, v, q_norm, k_norm, pos, q, gate, c, p0, T, Hq, n_rot, freq_
                                          ctypes.byref(c.struct()), p0, T, Hq, n_rot, freq_base, eps, ldq, ldk, ldv,
                                          _ptr(mp), stride, s0, s1, s2, sect, _stream()), "attn_prep")
         return
-    _check(lib().p1a_attn_prep(_ptr(qg), _ptr(k), _ptr(v), _ptr(q_norm), _ptr(k_norm), _ptr(pos), _ptr(q), _ptr(gate),
-                               ctypes.byref(c.struct()), p0, T, Hq, n_rot, freq_base, eps, ldq, ldk, ldv, _stream()), "attn_prep")
+    _check(lib().p1a_attn_prep(_ptr(qg), _ptr(k), _ptr(v), _ptr(q_norm), _ptr(k_norm), _ptr(pos), _ptr(q), _ptr(gate), c.struct(), p0, T, Hq,
+                               n_rot, freq_base, eps, ldq, ldk, ldv, _stream()), "attn_prep")
 
 
 def attn_decode(q, c, out, T, p0, Hq, scale, gate=None):

@@ -140,6 +140,11 @@ int nsplit_req() {
 
 // the decode split buffers of a head shape: P1A_MAX_ROWS rows, the largest need over the KV types and row groupings
 void decode_footprint(int Hq, int Hkv, int D, size_t & need_o, size_t & need_ml) {
+    // (two dozen plans, about 1 us: the last answer of a thread is kept with all that it depends on)
+    struct memo { int Hq, Hkv, D, req, cus; size_t o, ml; };
+    static thread_local memo last = {0, 0, 0, 0, 0, 0, 0};
+    const int req = nsplit_req(), cus = cu_count();
+    if (last.Hq == Hq && last.Hkv == Hkv && last.D == D && last.req == req && last.cus == cus) { need_o = last.o; need_ml = last.ml; return; }
     p1a_kv c;
     memset(&c, 0, sizeof c);
     c.Hkv = Hkv; c.D = D;
@@ -153,10 +158,11 @@ void decode_footprint(int Hq, int Hkv, int D, size_t & need_o, size_t & need_ml)
                 size_t o, m;
                 c.type = ty;
                 c.k = c.v = (void *) base;
-                decode_scratch_need(c, Hq, P1A_MAX_ROWS, rg, nsplit_req(), cu_count(), o, m);
+                decode_scratch_need(c, Hq, P1A_MAX_ROWS, rg, req, cus, o, m);
                 if (o > need_o) need_o = o;
                 if (m > need_ml) need_ml = m;
             }
+    last = memo{Hq, Hkv, D, req, cus, need_o, need_ml};
 }
 
 // ext / ext_bytes: split scratch brought by the caller of this function (the allocation-free entry point); nullptr = the
