@@ -22,7 +22,7 @@
 // rounded P that multiplies V. The reference maximum of a row moves lazily (only when the row maximum has grown
 // by more than 2^RESCALE_STEP), so the accumulators are rescaled a handful of times per row. Keys above a row's
 // diagonal are masked; the sigmoid output gate is applied in the epilogue.
-// Workgroup order: GQA consecutive row blocks of one kv head (128 tokens) get consecutive dispatch slots on the same XCD,
+// Workgroup order: up to GQA consecutive row blocks of one kv head (128 tokens) get consecutive dispatch slots on the same XCD,
 // so they stream the same K/V tiles through one L2.
 #include "p1a_common.hpp"
 
@@ -90,7 +90,9 @@ struct pf_params {
     uint32_t gqa_magic;   // floor(2^32 / GQA) (2^32 - 1 for GQA = 1)
     int rpw;      // rows of a wave: 32, or 16 or 8 (a call of few blocks)
     int nblk;     // row blocks (4 rpw rows) of a kv head
-    int nbg;      // groups of GQA row blocks
+    int nbg;      // groups of row blocks
+    int bpg;      // blocks of a group
+    int run;      // key splits: consecutive workgroups of an XCD (0: groups in turn)
     // key splits: with nks > 1 workgroup (block, kv head, ks) walks its share of the block's tiles and leaves an unnormalised
     // partial (O relative to m, and (m, l)) per row in part_o [T*Hq][nks][D] / part_ml [T*Hq][nks][2] for the merge
     int nks;
@@ -260,15 +262,17 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c = lane & 31, g = lane >> 5;
-    // blockIdx.x -> (group of GQA row blocks, kv head, block of the group): the blocks of a group share an XCD
+    // blockIdx.x -> (group of row blocks, kv head, block of the group): the blocks of a group share an XCD. Groups are dealt to
+    // the XCDs in turn; with key splits a unit is (key split, kv head) with all of its row blocks, and an XCD may take a run of
+    // `run` consecutive workgroups instead of whole units
     const int id = blockIdx.x, xcd = id & 7, slot = id >> 3;
-    // (with key splits a unit is (key split, group, kv head): the splits spread over the XCDs like the groups do)
-    const int vunit = (slot / P.GQA) * 8 + xcd, hh = slot % P.GQA;
+    const int lin = P.run ? xcd * P.run + slot : ((slot / P.bpg) * 8 + xcd) * P.bpg + slot % P.bpg;
+    const int vunit = lin / P.bpg, hh = lin - vunit * P.bpg;
     const int nunits = P.nbg * P.Hkv;
     if (vunit >= nunits * P.nks) return;
     const int ksp = vunit / nunits, unit = vunit - ksp * nunits;
     // longest blocks (most keys) first
-    const int rb = (P.nbg - 1 - unit / P.Hkv) * P.GQA + hh, hk = unit % P.Hkv;
+    const int rb = (P.nbg - 1 - unit / P.Hkv) * P.bpg + hh, hk = unit % P.Hkv;
     if (rb >= P.nblk) return;                                 // (the last group need not be full)
 
     const int row0 = rb * 4 * P.rpw;                          // first row of the block
@@ -920,7 +924,7 @@ int launch_pf_g(const pf_params & P, hipStream_t s) {
         attr_set.fetch_or(bit, std::memory_order_release);
     }
     const int units = P.nbg * P.Hkv * P.nks;
-    const int slots = ((units + 7) / 8) * P.GQA;
+    const int slots = P.run ? P.run : ((units + 7) / 8) * P.bpg;
     prefill_k<KT, D, GROUPED, DMA><<<slots * 8, NTHR, lds, s>>>(P);
     return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
 }
@@ -1066,7 +1070,16 @@ int launch_prefill(const p1a_kv & c, const float * q, float * out, const float *
     P.nks = nks;
     P.rpw = block_rows(P.R, c.Hkv, nks, cu_count()) / 4;
     P.nblk = (P.R + 4 * P.rpw - 1) / (4 * P.rpw);
-    P.nbg = (P.nblk + P.GQA - 1) / P.GQA;
+    // Groups of at most GQA blocks, as even as can be: a group's missing blocks are workgroups that find nothing to do, but
+    // each takes a compute unit's LDS before it can say so, and the blocks behind it wait. A key-split call is planned to fill
+    // the device in so many rounds, and a unit too many on one XCD (three blocks a unit, 84 units: 33 workgroups on an XCD of
+    // 32 compute units) is a round more: the XCDs take equal runs of workgroups where whole units in turn would not be
+    // equal. q8_0, 64 tokens behind 16000 (24 / 4 heads of 256) 83 -> 63 us, 17 behind 16000 (32 / 8) 132 -> 72, 85 behind 16000
+    // (16 / 2) 79 -> 54. (Runs everywhere: 39 -> 43 us for 8 / 8 heads, 32 behind 5000, whose units in turn are equal.)
+    P.nbg = nks > 1 ? 1 : (P.nblk + P.GQA - 1) / P.GQA;
+    P.bpg = (P.nblk + P.nbg - 1) / P.nbg;
+    const int units = P.nbg * c.Hkv * nks, even = (units * P.bpg + 7) / 8;
+    P.run = nks > 1 && (units + 7) / 8 * P.bpg > even ? even : 0;
     auto finish = [&](int rc) {
         if (rc != P1A_OK || P.nks == 1) return rc;
         return launch_merge(P.part_o, P.part_ml, out, gate, P.nks, c.D, Hq, T, s);
