@@ -1025,6 +1025,19 @@ static int block_rows(int R, int Hkv, int nks, int cus) {
     while (b > 32 && 2L * ((R + b - 1) / b) * Hkv * nks <= cus) b /= 2;
     return b;
 }
+// A quantized cache is converted inside the kernel, without a copy, where few row blocks would share the copy: one block
+// makes every tile exactly once either way. A copy costs its bytes (about 0.5 us per million values of K and V each), the
+// conversion in the kernel some 1.5 us per tile of a workgroup (q8_0 a little more: two loads a key), and those are few only
+// while the splits spread them. Measured
+// copy / inside, us, q8_0 and q4_0: one block, 8 / 8 heads of 256 behind 28000 124 / 61 and 146 / 62, 24 / 4 behind 5000 41 / 38 and
+// 43 / 38, behind 2000 31 / 33 and 32 / 33; three, 24 / 4 behind 16000 63 / 56 and 69 / 56; four, 51 / 49 behind 10000 and 41 / 42
+// behind 5000; six, 86 / 90 behind 16000. At D <= 128 the kernel on a copy also has two workgroups to a CU: one block 44 / 34
+// (8 / 8 of 128 behind 16000), two (32 / 8) 55 / 70.
+static bool convert_inside(const p1a_kv & c, int R, int n) {
+    const int blocks = (R + BM - 1) / BM;
+    if (c.pt && c.psh < 4) return false;                      // (a page lookup per key: measured nowhere as good)
+    return blocks <= (c.D == 256 ? 4 : 1) && (long long) n * c.Hkv * c.D >= (c.type == P1A_KV_Q8_0 ? 4000000LL : 2500000LL) * blocks;
+}
 size_t prefill_part_bytes_o(int T, int Hq, int D, int nks) { return nks > 1 ? (size_t) T * Hq * nks * D * 4 : 0; }
 size_t prefill_part_bytes_ml(int T, int Hq, int nks) { return nks > 1 ? (((size_t) T * Hq * nks * 2 * 4) + 255) & ~(size_t) 255 : 0; }
 void prefill_part_need(int T, int p0, int Hq, int D, size_t & bytes_o, size_t & bytes_ml) {
@@ -1053,11 +1066,12 @@ int launch_prefill(const p1a_kv & c, const float * q, float * out, const float *
     // they fit behind it); partials that do not fit go to the library's own per-stream buffers
     const int n = p0 + T;
     const bool aligned = scratch && !((uintptr_t) scratch & 255);
-    const bool stage_caller = c.type != P1A_KV_F16 && aligned && scratch_bytes >= prefill_stage_bytes(n, c.Hkv, c.D);
+    const bool want_copy = c.type != P1A_KV_F16 && !convert_inside(c, P.R, n);
+    const bool stage_caller = want_copy && aligned && scratch_bytes >= prefill_stage_bytes(n, c.Hkv, c.D);
     const size_t used = stage_caller ? (prefill_stage_bytes(n, c.Hkv, c.D) + 255) & ~(size_t) 255 : 0;
     // no room in the caller's scratch (the reference's attn_prefill brings none): the library's own staging copy, if it has one
     void * stage_own = nullptr;
-    if (c.type != P1A_KV_F16 && !stage_caller) stage_own = stage_scratch(s, prefill_stage_bytes(n, c.Hkv, c.D));
+    if (want_copy && !stage_caller) stage_own = stage_scratch(s, prefill_stage_bytes(n, c.Hkv, c.D));
     const bool stage = stage_caller || stage_own;
     const int nks = used_key_splits(T, p0, Hq, c.Hkv, cu_count());
     if (nks > 1) {
@@ -1086,7 +1100,7 @@ int launch_prefill(const p1a_kv & c, const float * q, float * out, const float *
     };
 #define PF(KT_) finish(c.D == 256 ? launch_pf<KT_, 256>(P, s) : c.D == 128 ? launch_pf<KT_, 128>(P, s) : launch_pf<KT_, 64>(P, s))
     if (c.type == P1A_KV_F16) return PF(P1A_KV_F16);
-    // A quantized cache with enough caller scratch: convert the visible positions to f16 once (tens of microseconds, the
+    // A quantized cache with room for a copy: convert the visible positions to f16 once (tens of microseconds, the
     // copy stays in the Infinity Cache) and run the f16 kernel on it - every workgroup then skips the dequantization it
     // would otherwise repeat per 128 query rows. Same tiles, same products, same bits as the direct kernel.
     if (stage) {

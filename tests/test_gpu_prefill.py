@@ -339,3 +339,24 @@ def test_sequence_selected_through_the_row_table(p1a, kv_type):
     p1a.kv_fill_random(pool.devkv.with_rows(rt), 10, 600, 5)
     torch.cuda.synchronize()
     assert np.array_equal(pool.dpool.cpu().numpy(), pool.host.pool)
+
+
+@pytest.mark.parametrize("kv_type", TYPES)
+@pytest.mark.parametrize("Hq,Hkv,D,p0,T", [(24, 4, 256, 3660, 64), (8, 8, 256, 2100, 100), (24, 4, 256, 5000, 40), (16, 2, 128, 3000, 50), (8, 8, 128, 3900, 21)])
+def test_long_contexts_of_few_row_blocks(p1a, kv_type, Hq, Hkv, D, p0, T):
+    """key-split calls of one to four row blocks a kv head: equal runs of workgroups per XCD where whole units in turn would
+    not be equal (7 splits of 3 blocks), and the quantized cache converted inside the kernel from a size on (pages of 16
+    positions) or copied (pages of 8, always): the same bits each way and the oracle's values"""
+    n, outs = p0 + T, []
+    q, _, _, gate = I.qkv(n, 1, T, Hq, Hkv, D, f16_inputs=True)
+    for psh in (3, 4):
+        pool = Pool(p1a, kv_type, Hq, Hkv, D, psh, [n], seed=n + D, n_layers=1, layer=0)
+        for limit in ((1 << 30,) if kv_type == O.KV_F16 else (1 << 30, 0)):
+            p1a.set_prefill_staging_limit(limit)
+            try:
+                outs.append(run_prefill(p1a, pool.dev_seq(0), q, T, p0, Hq, D ** -0.5, gate=gate))
+            finally:
+                p1a.set_prefill_staging_limit(1 << 30)
+    for o in outs[1:]:
+        assert np.array_equal(o, outs[0])
+    check(outs[0], O.attn_rows(pool.host_seq(0), q, (p0 + np.arange(T)).astype(np.int32), Hq, D ** -0.5, gate=gate), f"few blocks {kv_type} {Hq}/{Hkv}/{D} p0 {p0} T {T}")
