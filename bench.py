@@ -209,8 +209,8 @@ def extras(p1a, torch, stream, Hq, Hkv, D, psh, scale, top, cpu):
     ex["prep_4rows_q8_0_us"] = round(sec * 1e6, 2)
     del kv, c, q, gate, out
     # q8_0 at head_dim 128 (head rows that are not whole 16-byte chunks): raw tiles fetched 4 bytes per lane and converted
-    # to f16 tiles by their wave, then the f16 MFMA kernel; and head_dim 96, which only the generic
-    # one-wave-per-(stream, head, row) kernel takes, so that "correct, slow" has a number
+    # to f16 tiles by their wave, then the f16 MFMA kernel; and head_dim 96, which the kernel
+    # for any shape takes
     for Dx, tag in ((128, "staged_q8_0_D128_32K"), (96, "generic_q8_0_D96_32K")):
         kvg, ppg = build_pool(p1a, torch, p1a.KV_Q8_0, Hq, Hkv, Dx, psh, 32768, 1, seed=25)
         qg_ = normed((1, Hq, Dx))

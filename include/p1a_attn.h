@@ -195,10 +195,10 @@ size_t p1a_attn_prefill_scratch_bytes(int T, int p0, int Hq, int Hkv, int D);
  * long context (the last chunk of a prompt, a short turn of a long chat) would occupy T * Hq / 128 workgroups, each walking
  * every key; its keys are then dealt to several workgroups per (block of 128 rows, kv head) and the partials merged (the
  * nsplit of attn_fold, src/fast/attn_fold.cuh:19-26, chosen by the library). The count depends on (T, p0, Hq) and the
- * device's CU count only - what a call takes also on Hkv, which rounds its row blocks up - never on the scratch passed or on the state of the stream; partials that do not fit the caller's scratch
- * live in buffers the library keeps per (device, stream) for this purpose (never freed before p1a_release). They cannot
- * be allocated during stream capture: such a call is refused with P1A_E_SCRATCH unless p1a_warmup_prefill (or an eager
- * call of the shape) came first. */
+ * device's CU count only - what a call takes also on Hkv, which rounds its row blocks up - never on the scratch passed or on
+ * the state of the stream; partials that do not fit the caller's scratch live in buffers the library keeps per (device,
+ * stream) for this purpose (never freed before p1a_release). They cannot be allocated during stream capture: such a call
+ * is refused with P1A_E_SCRATCH unless p1a_warmup_prefill (or an eager call of the shape) came first. */
 int p1a_attn_prefill_key_splits(int T, int p0, int Hq);
 /* Largest f16 staging copy the library keeps per (device, stream) for p1a_attn_prefill calls without caller scratch
  * (bytes; 0 = never: such calls convert inside the kernel). No counterpart in the reference. */
