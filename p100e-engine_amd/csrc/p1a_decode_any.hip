@@ -11,8 +11,12 @@
 //   S^T = K Q^T, 16 keys x 16 columns at a time. f16 keys and the integer codes of quantized ones are f16 operands as they
 //   are; the products are exact in fp32, and a block's scale multiplies its fp32 partial result.
 //   O^T = V^T P^T. Quantized: the codes are exact in bf16, and P * scale (fp32) is cut into three bf16 pieces of 8 bits - all
-//   24 of its mantissa - so the three products add up to the fp32 one. f16: P carries a factor 2^15 and is cut into two
-//   f16 pieces (22 bits), neither of them zero or negative unless P is zero, so that an infinite V stays infinite.
+//   24 of its mantissa - so the three products add up to the fp32 one. f16: P carries a factor 2^15. Where every P of a tile
+//   that is not zero is at least 1, it is cut into three f16 pieces, 11, 11 and the 2 to 4 bits left: exact (the last bit of
+//   such a P is 2^-23, f16 ends at 2^-24) and each above zero, so that an infinite V stays infinite. A tile with a smaller P
+//   takes fp32 matrix products, at a fifth of the rate: pieces would end at 2^-39 of the largest weight, where fp32 does not,
+//   and thousands of light keys with a large V are more than the result. (24 / 4 heads of 256 in pages of 4, 8 sequences x 4
+//   rows of 2500 keys, two pieces whatever P is 104 us, as it is 104, fp32 products throughout 122; 24 / 4 of 96 39 and 42.)
 // Data movement
 //   A lane reads what it feeds to the products straight into registers: 8 consecutive values (16 / 8 / 4 bytes) of its key
 //   per K block, 2 consecutive dims (4 / 2 bytes; q4_0: one byte, dims c and c + 16) of 4 keys per V block. Only the
@@ -66,6 +70,11 @@ __device__ __forceinline__ void codes4(uint32_t x, float off, uint32_t & a, uint
     a = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, perm(0x64646464u, x, 0x04010400u)) - o);
     b = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, perm(0x64646464u, x, 0x04030402u)) - o);
 }
+
+// the fp32 value below x > 0 (0 for 0)
+__device__ __forceinline__ float below(float x) { return asf(__builtin_elementwise_sub_sat(asu(x), 1u)); }
+// two values to f16, towards zero
+__device__ __forceinline__ h2 cut2(float x, float y) { return __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(x, y)); }
 
 // NBM: the most 32-dim blocks of a head this build takes; EX: exactly that many
 template <uint32_t KT, int NBM, bool EX, int NW>
@@ -248,27 +257,43 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
                         for (int b = 0; b < NBM; ++b) vr[b][i] = 0;
                     }
             }
-            h4 ph, pl;
+            if (__builtin_expect(__any((p[0] < 1.f && p[0] > 0.f) || (p[1] < 1.f && p[1] > 0.f) || (p[2] < 1.f && p[2] > 0.f) || (p[3] < 1.f && p[3] > 0.f)), 0)) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                // cut, not rounded: the rest is not negative
-                float f = asf(asu(p[i]) & 0xffffe000u);
-                if (p[i] > 0.f) f = fmaxf(f, 0x1p-24f);
-                const half_t h = (half_t) f;
-                float r = p[i] - (float) h;
-                if (p[i] > 0.f) r = fmaxf(r, 0x1p-24f);
-                ph[i] = h;
-                pl[i] = (half_t) r;
-            }
+                for (int b = 0; b < NBM; ++b) {
+                    if (!EX && b >= nb) continue;
 #pragma unroll
-            for (int b = 0; b < NBM; ++b) {
-                if (!EX && b >= nb) continue;
+                    for (int i = 0; i < 4; ++i) {             // keys 4 g + i of the four lane groups
+                        uint32_t w = vr[b][i];
+                        asm volatile("" : "+v"(w));           // (here, one at a time: 512 registers do not hold all of them as fp32)
+                        const h2 v = __builtin_bit_cast(h2, w);
+                        o[b][0] = __builtin_amdgcn_mfma_f32_16x16x4f32((float) v[0], p[i], o[b][0], 0, 0, 0);
+                        o[b][1] = __builtin_amdgcn_mfma_f32_16x16x4f32((float) v[1], p[i], o[b][1], 0, 0, 0);
+                    }
+                }
+            } else {
+                h4 pc[3];                                     // the largest f16 value below what is left, twice, and the rest
 #pragma unroll
-                for (int x = 0; x < 2; ++x) {
-                    const uint32_t sel = x ? 0x07060302u : 0x05040100u;
-                    const i2 a = {(int) perm(vr[b][1], vr[b][0], sel), (int) perm(vr[b][3], vr[b][2], sel)};
-                    o[b][x] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(h4, a), pl, o[b][x], 0, 0, 0);
-                    o[b][x] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(h4, a), ph, o[b][x], 0, 0, 0);
+                for (int i = 0; i < 4; i += 2) {
+                    float r0 = p[i], r1 = p[i + 1];
+#pragma unroll
+                    for (int k = 0; k < 3; ++k) {
+                        const h2 h = k < 2 ? cut2(below(r0), below(r1)) : cut2(r0, r1);
+                        pc[k][i] = h[0];
+                        pc[k][i + 1] = h[1];
+                        r0 -= (float) h[0];
+                        r1 -= (float) h[1];
+                    }
+                }
+#pragma unroll
+                for (int b = 0; b < NBM; ++b) {
+                    if (!EX && b >= nb) continue;
+#pragma unroll
+                    for (int x = 0; x < 2; ++x) {
+                        const uint32_t sel = x ? 0x07060302u : 0x05040100u;
+                        const i2 a = {(int) perm(vr[b][1], vr[b][0], sel), (int) perm(vr[b][3], vr[b][2], sel)};
+#pragma unroll
+                        for (int k = 2; k >= 0; --k) o[b][x] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(h4, a), pc[k], o[b][x], 0, 0, 0);
+                    }
                 }
             }
         } else {

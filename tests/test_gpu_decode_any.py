@@ -104,3 +104,44 @@ def test_any_infinite_values_and_low_scores(p1a):
     O.kv_append_rows(pool.host_seq(0), k, v0, np.arange(n))
     ref = O.attn_rows(pool.host_seq(0), q, np.array([n - 2, n - 1], np.int32), Hq, SCALE, f64=True)
     close(got[:, :, keep], ref[:, :, keep], "the other dims")
+
+
+@pytest.mark.parametrize("kv_type", [O.KV_F16, O.KV_Q8_0, O.KV_Q4_0])
+@pytest.mark.parametrize("D,low", [(96, 60.0), (192, 43.0), (320, 30.0)])
+def test_any_weights_have_the_range_of_fp32(p1a, kv_type, D, low):
+    """one key with a small V beside thousands whose V is the largest f16 holds and whose weight is 2^-low of its own: what those
+    add is below, at and above an ulp of the result, and weights of any narrower range (f16 pieces end at 2^-24) make it more
+    than the result. The scores are twice the 2^5 of TOL, so twice TOL."""
+    Hq, Hkv, n = 4, 1, 8190
+    pool = Pool(p1a, kv_type, Hq, Hkv, D, 4, [n], seed=D, fill="none")
+    q, k, v, _ = I.qkv(D, n, 1, Hq, Hkv, D, f16_inputs=True)
+    q[:] = q[0, 0]
+    k[:] = -(low / 2.0 ** -4) * q[0, 0] / float(q[0, 0] @ q[0, 0])
+    k[4001] = 0.0
+    v[:] = 60000.0
+    v[4001] = (1.0 + 0.01 * np.arange(D)) * 2.0 ** -10
+    O.kv_append_rows(pool.host_seq(0), k, v, np.arange(n))
+    p1a.kv_append(pool.dev_seq(0), dev(k), dev(v), 0, n)
+    ref = O.attn_rows(pool.host_seq(0), q, np.array([n - 1], np.int32), Hq, SCALE, f64=True)
+    out = torch.empty((1, Hq, D), device="cuda")
+    p1a.attn_decode(dev(q), pool.dev_seq(0), out, 1, n - 1, Hq, SCALE)
+    rl = float(np.linalg.norm(out.cpu().numpy().astype(np.float64) - ref) / np.linalg.norm(ref))
+    assert rl <= 2 * TOL, (kv_type, D, low, rl)
+
+
+def test_any_infinite_value_under_equal_weights(p1a):
+    """f16: weights of a single bit (q = 0: every key the same) have nothing left for the lower pieces of a cut; an infinite V
+    stays infinite all the same, and the other dims are the mean"""
+    Hq, Hkv, D, n = 3, 1, 96, 128
+    pool = Pool(p1a, O.KV_F16, Hq, Hkv, D, 4, [n], seed=7, fill="none")
+    _, k, v, _ = I.qkv(9, n, 1, Hq, Hkv, D, f16_inputs=True)
+    v[50, 0, 3], v[7, 0, 90] = np.inf, -np.inf
+    O.kv_append_rows(pool.host_seq(0), k, v, np.arange(n))
+    p1a.kv_append(pool.dev_seq(0), dev(k), dev(v), 0, n)
+    out = torch.empty((1, Hq, D), device="cuda")
+    p1a.attn_decode(dev(np.zeros((1, Hq, D), np.float32)), pool.dev_seq(0), out, 1, n - 1, Hq, SCALE)
+    got = out.cpu().numpy()[0]
+    assert np.all(got[:, 3] == np.inf) and np.all(got[:, 90] == -np.inf)
+    keep = [d for d in range(D) if d not in (3, 90)]
+    mean = np.broadcast_to(v[:, 0].astype(np.float64).mean(0)[keep], (Hq, len(keep)))
+    close(got[:, keep], mean, "equal weights")
