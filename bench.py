@@ -190,7 +190,7 @@ def extras(p1a, torch, stream, Hq, Hkv, D, psh, scale, top, cpu):
     scr = torch.empty(p1a.prefill_scratch_bytes(Ts, p0s, Hq, Hkv, D), dtype=torch.uint8, device="cuda")
     sec = time_eager(torch, lambda: p1a.attn_prefill(q[:Ts], c, out[:Ts], Ts, p0s, Hq, scale, gate=gate[:Ts], scratch=scr), reps=5, group=10)
     ex["prefill_T128_p32640_q8_0_us"] = round(sec * 1e6, 1)
-    ex["prefill_T128_key_splits"] = p1a.prefill_key_splits(Ts, p0s, Hq)
+    ex["prefill_T128_key_splits"] = p1a.prefill_key_splits(Ts, p0s, Hq, Hkv)
     ex["prefill_T128_TFLOPs"] = round(4.0 * D * Hq * (p0s * Ts + Ts * (Ts + 1) / 2) / sec / 1e12, 1)
     del scr
     sec = time_eager(torch, lambda: p1a.kv_append(c, kc, vc, p0, T), reps=5, group=20)

@@ -188,18 +188,21 @@ int p1a_ew_quant(int op, const float *a, const float *b, float *y, void *qbuf, i
 int p1a_attn_prefill(const float *q, const p1a_kv *c, float *out, const float *gate, int T, int p0, int Hq,
                      float scale, void *scratch, size_t scratch_bytes, void *stream);
 /* bytes of scratch that enable the convert-once variant and hold the partials of a key-split call:
- * roundup(2 * roundup(p0 + T, 16) * Hkv * D * 2, 256) + (key splits > 1 ? roundup(T * Hq * splits * 8, 256) + T * Hq * splits * D * 4 : 0).
+ * roundup(2 * roundup(p0 + T, 16) * Hkv * D * 2, 256) + (splits > 1 ? roundup(T * Hq * splits * 8, 256) + T * Hq * splits * D * 4 : 0),
+ * splits = p1a_attn_prefill_call_splits(T, p0, Hq, Hkv).
  * Replaces attn_fold_scratch_bytes (src/fast/attn_fold.cuh:19). */
 size_t p1a_attn_prefill_scratch_bytes(int T, int p0, int Hq, int Hkv, int D);
-/* Key splits a prefill call of this shape takes at most on the current device (1 = none). A chunk of few query rows over a
+/* Key splits a prefill call of this shape takes on the current device (1 = none). A chunk of few query rows over a
  * long context (the last chunk of a prompt, a short turn of a long chat) would occupy T * Hq / 128 workgroups, each walking
- * every key; its keys are then dealt to several workgroups per (block of 128 rows, kv head) and the partials merged (the
- * nsplit of attn_fold, src/fast/attn_fold.cuh:19-26, chosen by the library). The count depends on (T, p0, Hq) and the
- * device's CU count only - what a call takes also on Hkv, which rounds its row blocks up - never on the scratch passed or on
- * the state of the stream; partials that do not fit the caller's scratch live in buffers the library keeps per (device,
- * stream) for this purpose (never freed before p1a_release). They cannot be allocated during stream capture: such a call
- * is refused with P1A_E_SCRATCH unless p1a_warmup_prefill (or an eager call of the shape) came first. */
+ * every key; its keys are then dealt to several workgroups per (block of 128, 64 or 32 rows, kv head) and the partials merged
+ * (the nsplit of attn_fold, src/fast/attn_fold.cuh:19-26, chosen by the library). The count depends on (T, p0, Hq, Hkv) and
+ * the device's CU count only, never on the scratch passed or on the state of the stream: _call_splits tells it, _key_splits
+ * the most it is for any Hkv (1: none whatever Hkv is). Partials that do not fit the caller's scratch live in buffers the
+ * library keeps per (device, stream) for this purpose (never freed before p1a_release). They cannot be allocated during
+ * stream capture: such a call is refused with P1A_E_SCRATCH unless p1a_warmup_prefill (or an eager call of the shape) came
+ * first. */
 int p1a_attn_prefill_key_splits(int T, int p0, int Hq);
+int p1a_attn_prefill_call_splits(int T, int p0, int Hq, int Hkv);
 /* Largest f16 staging copy the library keeps per (device, stream) for p1a_attn_prefill calls without caller scratch
  * (bytes; 0 = never: such calls convert inside the kernel). No counterpart in the reference. */
 void p1a_set_prefill_staging_limit(size_t bytes);
@@ -234,9 +237,9 @@ size_t p1a_decode_footprint_bytes(int Hq, int Hkv, int D);
 /* An identity of everything in this library that can change output BITS for a head shape on the current device: library
  * version and numerics revision, CU count, split-stream count (P1A_DEC_SPLIT / p1a_set_nsplit included). Two processes with
  * equal ids produce bit-identical attention outputs for equal inputs; the engine folds such switches into the numerics
- * hash of its session files (src/tp_model.cu:3697-3735). The prefill key-split plan is a function of (T, p0, Hq) and the
- * CU count, so it is covered. */
-#define P1A_NUMERICS_REV 7
+ * hash of its session files (src/tp_model.cu:3697-3735). The prefill key-split plan is a function of (T, p0, Hq, Hkv)
+ * and the CU count, so it is covered. */
+#define P1A_NUMERICS_REV 8
 uint64_t p1a_numerics_id(int Hq, int Hkv);
 /* Re-read the environment switch that is baked into captured graphs (P1A_DEC_SPLIT, the split-stream count); returns 1
  * when it differs from what was last read - the very first read included, as in the reference - (the caller must then drop

@@ -7,7 +7,7 @@ import os
 KV_F16, KV_Q4_0, KV_Q8_0 = 1, 2, 8
 
 EXPORTS = [
-    "p1a_kv_row_bytes", "p1a_kv_append", "p1a_kv_fill_random", "p1a_attn_prep", "p1a_attn_prep_mrope", "p1a_attn_decode", "p1a_attn_decode_a16", "p1a_attn_decode_noalloc", "p1a_a16_bytes", "p1a_ew_quant", "p1a_attn_prefill", "p1a_attn_prefill_scratch_bytes", "p1a_attn_prefill_key_splits",
+    "p1a_kv_row_bytes", "p1a_kv_append", "p1a_kv_fill_random", "p1a_attn_prep", "p1a_attn_prep_mrope", "p1a_attn_decode", "p1a_attn_decode_a16", "p1a_attn_decode_noalloc", "p1a_a16_bytes", "p1a_ew_quant", "p1a_attn_prefill", "p1a_attn_prefill_scratch_bytes", "p1a_attn_prefill_key_splits", "p1a_attn_prefill_call_splits",
     "p1a_sigmoid_mul", "p1a_warmup", "p1a_get_nsplit", "p1a_set_nsplit", "p1a_reload_env", "p1a_warmup_prefill", "p1a_set_prefill_staging_limit", "p1a_bench_decode_split_only", "p1a_bench_stream_read", "p1a_release", "p1a_last_error",
     "p1a_version", "p1a_decode_scratch_bytes", "p1a_decode_footprint_bytes", "p1a_numerics_id",
     # include/p1a_pool.h
@@ -85,6 +85,8 @@ def lib():
     L.p1a_kv_fill_random.argtypes = [kvp, i32, i32, ctypes.c_uint32, vp]
     L.p1a_attn_prefill_key_splits.restype = i32
     L.p1a_attn_prefill_key_splits.argtypes = [i32, i32, i32]
+    L.p1a_attn_prefill_call_splits.restype = i32
+    L.p1a_attn_prefill_call_splits.argtypes = [i32, i32, i32, i32]
     L.p1a_sigmoid_mul.restype = i32
     L.p1a_sigmoid_mul.argtypes = [vp, vp, sz, vp]
     L.p1a_warmup.restype = i32
@@ -315,7 +317,10 @@ def prefill_scratch_bytes(T, p0, Hq, Hkv, D):
     return int(lib().p1a_attn_prefill_scratch_bytes(T, p0, Hq, Hkv, D))
 
 
-def prefill_key_splits(T, p0, Hq):
+def prefill_key_splits(T, p0, Hq, Hkv=None):
+    """the key splits a call takes; without Hkv the most it takes for any"""
+    if Hkv is not None:
+        return int(lib().p1a_attn_prefill_call_splits(T, p0, Hq, Hkv))
     return int(lib().p1a_attn_prefill_key_splits(T, p0, Hq))
 
 

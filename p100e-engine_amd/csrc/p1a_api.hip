@@ -381,7 +381,7 @@ int p1a_warmup(int rows, int Hq, int Hkv, int D, void * stream) {
 int p1a_warmup_prefill(int T, int p0, int Hq, int Hkv, int D, void * stream) {
     if (T < 1 || p0 < 0 || Hq < 1 || Hkv < 1 || Hq % Hkv || D < 32) { set_error("p1a_warmup_prefill: bad shape"); return P1A_E_ARG; }
     size_t bo, bm;
-    prefill_part_need(T, p0, Hq, D, bo, bm);
+    prefill_part_need(T, p0, Hq, Hkv, D, bo, bm);
     // (the f16 staging copy of a quantized cache, when it is within the limit: optional, a call without it converts in the kernel)
     (void) stage_scratch((hipStream_t) stream, prefill_stage_bytes(p0 + T, Hkv, D));
     if (!bo) return P1A_OK;

@@ -153,7 +153,7 @@ bool split_scratch(hipStream_t s, size_t bytes_o, size_t bytes_ml, float *& o, f
 void * stage_scratch(hipStream_t s, size_t bytes);
 size_t prefill_stage_bytes(int n, int Hkv, int D);
 // bytes of partials a key-split prefill of this shape needs on the current device (0, 0 = one split)
-void prefill_part_need(int T, int p0, int Hq, int D, size_t & bytes_o, size_t & bytes_ml);
+void prefill_part_need(int T, int p0, int Hq, int Hkv, int D, size_t & bytes_o, size_t & bytes_ml);
 int cu_count();   // compute units of the current device
 int launch_sigmoid_mul(float * x, const float * g, size_t n, hipStream_t s);
 int launch_stream_read(const void * src, size_t bytes, hipStream_t s);   // benchmarks only

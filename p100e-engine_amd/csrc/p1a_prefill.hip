@@ -26,6 +26,7 @@
 // so they stream the same K/V tiles through one L2.
 #include "p1a_common.hpp"
 
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -996,7 +997,11 @@ __global__ void __launch_bounds__(256) dq_k(const char * kc, const char * vc, kv
 // partials merged. Chosen from the shape and the device alone (never from what scratch the caller brought: the result
 // bits depend on the split): the count that minimises, in units of a tile step, rounds of workgroups x (tiles per
 // workgroup + 6 for its set-up and partial stores) + the merge (its launch, 2, and its read of the partials, 1 per 6900
-// rows and split); a split is at least 8 tiles; 1 unless that saves 15 %.
+// rows and split); a split is at least 8 tiles; 1 unless that saves 15 %. (The figures are D = 256's, a workgroup to a CU; at
+// D <= 128, where the kernel on f16 tiles has two, they have not been taken.)
+// `units` are the row blocks the call really has, the last of each kv head full or not: planned for the blocks its rows could
+// fill, 12 / 12 heads, 1357 tokens behind 20453 - 132 of them, not 128 - got two splits and a second round of workgroups for
+// eight of 264: q8_0 of 256 658 us, five 488; f16 of 128 256 and 206.
 static int plan_splits(long units, int T, int p0, int Hq, int cus) {
     const long nt = (p0 + T - 1) / BN + 1;
     if (cus < 1) cus = 1;
@@ -1009,12 +1014,15 @@ static int plan_splits(long units, int T, int p0, int Hq, int cus) {
         if (cost(k) < cbest) { best = k; cbest = cost(k); }
     return cbest * 100 <= cost(1) * 85 ? (int) best : 1;
 }
-// The split slots a shape reserves, whatever its GQA: planned for the fewest row blocks T * Hq rows can make. The count a
-// call uses is planned from the blocks it really has (each kv head's last block need not be full): at most as many.
-int prefill_key_splits(int T, int p0, int Hq, int cus) { return plan_splits(((long) T * Hq + BM - 1) / BM, T, p0, Hq, cus); }
-static int used_key_splits(int T, int p0, int Hq, int Hkv, int cus) {
-    const int most = prefill_key_splits(T, p0, Hq, cus), k = plan_splits(((long) T * (Hq / Hkv) + BM - 1) / BM * Hkv, T, p0, Hq, cus);
-    return k < most ? k : most;
+int prefill_key_splits(int T, int p0, int Hq, int Hkv, int cus) {
+    return plan_splits(((long) T * (Hq / Hkv) + BM - 1) / BM * Hkv, T, p0, Hq, cus);
+}
+// the most any Hkv makes of it
+static int most_key_splits(int T, int p0, int Hq, int cus) {
+    int most = 1;
+    for (int h = 1; h <= Hq / h; ++h)
+        if (Hq % h == 0) most = std::max({most, prefill_key_splits(T, p0, Hq, h, cus), prefill_key_splits(T, p0, Hq, Hq / h, cus)});
+    return most;
 }
 // Rows of a block: 128, halved (down to 32) while the call would still leave half of the device without a workgroup. A
 // workgroup's set-up and epilogue are bound by its own CU's memory path (some 20 bytes a clock: 128 rows of q, gate and out
@@ -1040,8 +1048,8 @@ static bool convert_inside(const p1a_kv & c, int R, int n) {
 }
 size_t prefill_part_bytes_o(int T, int Hq, int D, int nks) { return nks > 1 ? (size_t) T * Hq * nks * D * 4 : 0; }
 size_t prefill_part_bytes_ml(int T, int Hq, int nks) { return nks > 1 ? (((size_t) T * Hq * nks * 2 * 4) + 255) & ~(size_t) 255 : 0; }
-void prefill_part_need(int T, int p0, int Hq, int D, size_t & bytes_o, size_t & bytes_ml) {
-    const int nks = prefill_key_splits(T, p0, Hq, cu_count());
+void prefill_part_need(int T, int p0, int Hq, int Hkv, int D, size_t & bytes_o, size_t & bytes_ml) {
+    const int nks = prefill_key_splits(T, p0, Hq, Hkv, cu_count());
     bytes_o = prefill_part_bytes_o(T, Hq, D, nks);
     bytes_ml = prefill_part_bytes_ml(T, Hq, nks);
 }
@@ -1073,7 +1081,7 @@ int launch_prefill(const p1a_kv & c, const float * q, float * out, const float *
     void * stage_own = nullptr;
     if (want_copy && !stage_caller) stage_own = stage_scratch(s, prefill_stage_bytes(n, c.Hkv, c.D));
     const bool stage = stage_caller || stage_own;
-    const int nks = used_key_splits(T, p0, Hq, c.Hkv, cu_count());
+    const int nks = prefill_key_splits(T, p0, Hq, c.Hkv, cu_count());
     if (nks > 1) {
         const size_t bo = prefill_part_bytes_o(T, Hq, c.D, nks), bm = prefill_part_bytes_ml(T, Hq, nks);
         if (aligned && scratch_bytes >= used + bm + bo) {
@@ -1130,12 +1138,17 @@ extern "C" size_t p1a_attn_prefill_scratch_bytes(int T, int p0, int Hq, int Hkv,
     // optional: with this much scratch a quantized cache is converted to f16 once per call instead of once per
     // workgroup, and the partials of a key-split call (few token blocks over a long context) live in it; with less (or
     // none) the kernel converts on the fly and the partials go to the library's own per-stream buffers
-    const int nks = Hq >= 1 ? p1a::prefill_key_splits(T, p0, Hq, p1a::cu_count()) : 1;
+    const int nks = Hq < 1 ? 1 : Hq % Hkv ? p1a::most_key_splits(T, p0, Hq, p1a::cu_count()) : p1a::prefill_key_splits(T, p0, Hq, Hkv, p1a::cu_count());
     return ((p1a::prefill_stage_bytes(p0 + T, Hkv, D) + 255) & ~(size_t) 255) + p1a::prefill_part_bytes_ml(T, Hq, nks) +
            p1a::prefill_part_bytes_o(T, Hq, D, nks);
 }
 
 extern "C" int p1a_attn_prefill_key_splits(int T, int p0, int Hq) {
     if (T < 1 || p0 < 0 || Hq < 1) return 1;
-    return p1a::prefill_key_splits(T, p0, Hq, p1a::cu_count());
+    return p1a::most_key_splits(T, p0, Hq, p1a::cu_count());
+}
+
+extern "C" int p1a_attn_prefill_call_splits(int T, int p0, int Hq, int Hkv) {
+    if (T < 1 || p0 < 0 || Hkv < 1 || Hq < Hkv || Hq % Hkv) return 1;
+    return p1a::prefill_key_splits(T, p0, Hq, Hkv, p1a::cu_count());
 }

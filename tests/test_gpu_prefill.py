@@ -266,6 +266,23 @@ def test_key_split_plan():
         assert (p0 + T - 1) // 64 + 1 >= 8 * ks or ks == 1
 
 
+def test_key_split_plan_counts_the_blocks_a_call_has():
+    """the plan's rounds of workgroups are those of the call's own row blocks, the last of each kv head rounded up: the count
+    chosen never costs more steps than none, also where the blocks are just over what fills the device (12 / 12 heads, 1357 tokens
+    behind 20453: 132 of them); the answer without Hkv covers every Hkv, and the scratch size holds that of its own"""
+    import importlib
+    p1a = importlib.import_module("p100e-engine_amd")
+    shapes = [(1357, 20453, 12)] + [(T, p0, Hq) for T in (17, 64, 130, 700, 1100, 1600, 2900) for p0 in (0, 900, 6000, 28000) for Hq in (4, 12, 24, 32)]
+    for T, p0, Hq in shapes:
+        tiles, most = (p0 + T - 1) // 64 + 1, p1a.prefill_key_splits(T, p0, Hq)
+        for Hkv in [h for h in range(1, Hq + 1) if Hq % h == 0]:
+            k, blocks = p1a.prefill_key_splits(T, p0, Hq, Hkv), -(-T * (Hq // Hkv) // 128) * Hkv
+            steps = lambda n: -(-blocks * n // 256) * (-(-tiles // n) + 6)
+            assert 1 <= k <= most and steps(k) <= steps(1), (T, p0, Hq, Hkv, k, most)
+            part = -(-T * Hq * k * 8 // 256) * 256 + T * Hq * k * 256 * 4 if k > 1 else 0
+            assert p1a.prefill_scratch_bytes(T, p0, Hq, Hkv, 256) == 4 * ((p0 + T + 15) // 16 * 16) * Hkv * 256 + part
+
+
 @pytest.mark.parametrize("kv_type", TYPES)
 @pytest.mark.parametrize("which", ["lower_lane_everywhere", "lower_half", "upper_half", "first_32", "all_but_one"])
 def test_row_maximum_spans_both_lane_halves(p1a, kv_type, which):
