@@ -417,17 +417,27 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
             voff_last[x][n] = (uint32_t) kl * (uint32_t) P.pg.rowb + co[n];
         }
     }
-    // FAST: the wave's 16 keys of a tile lie in one page (or the cache is contiguous): one table entry, one scalar base
+    // FAST: the wave's 16 keys of a tile lie in one page (or the cache is contiguous): one table entry, one scalar base;
+    // otherwise every item and scale block has an entry of its own
     constexpr bool FAST = GROUPED && IM::WAVE_MAJOR;
-    struct gpages { int pg; };
-    struct gbases { size_t go; };
+    struct gpages { int pg; int it[FAST ? 1 : S::NPT], sb; };
+    struct gbases { size_t go; gpages p; };
     // a group past the last position takes the base of the last one that holds a position: the LDS-direct loads then
     // fetch that group's 16 rows (all inside its page) instead of clamping row by row
     const int gclamp = DMA ? (pmax & ~15) : pmax;
     auto group_pages = [&](int tile) {
         gpages r;
         r.pg = 0;
-        if (FAST && ptab) {
+        if constexpr (!FAST) {
+            // asked for a step ahead of the tile, like the one entry of a 16-key group. (Looked up where the loads are made, a
+            // tile took a round trip to L2 per row: the entry of the next row stood behind the load of this one. Pages of
+            // 8, f16, 1000 tokens behind 2000, 24 / 4 heads of 256 312 -> 135 us, 32 / 8 of 128 162 -> 84; q8_0 252 -> 140.)
+            if (ptab) {
+#pragma unroll
+                for (int x = 0; x < S::NPT; ++x) r.it[x] = ptab[min(tile * BN + min(IM::key(x, tid), BN - 1), pmax) >> P.pg.psh];
+                if constexpr (S::SCALES_VIA_LDS) r.sb = ptab[min(tile * BN + 16 * wave + (lane & 15), pmax) >> P.pg.psh];
+            }
+        } else if (ptab) {
             // (a load from the constant address space at a wave-uniform address is an s_load_dword whose wait the compiler
             // places itself, before the first use; the table does not change while the kernel runs)
             const int32_t * e = ptab + (__builtin_amdgcn_readfirstlane(min(tile * BN + 16 * wave, gclamp)) >> P.pg.psh);
@@ -440,10 +450,13 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
     };
     auto group_bases = [&](int tile, gpages & gp) {
         gbases r;
+        if constexpr (!FAST) { r.go = 0; r.p = gp; return r; }
         const int p = __builtin_amdgcn_readfirstlane(min(tile * BN + 16 * wave, gclamp));
         r.go = (ptab ? (size_t) gp.pg * P.pg.pstride + (size_t) (p & pmask) * P.pg.rowb : (size_t) p * P.pg.rowb) + head_off;
         return r;
     };
+    // the head row of one position, whose page is known
+    auto row_off = [&](int pos, int page) { return (ptab ? (size_t) page * P.pg.pstride + (size_t) (pos & pmask) * P.pg.rowb : (size_t) pos * P.pg.rowb) + head_off; };
     // where item x of `tile` starts: base (scalar registers when GROUPED) + 32-bit offsets
     struct iaddr { gptr base; uint32_t vo[S::NOFF]; };
     auto item_addr = [&](const char * cache, int tile, const gbases & gb, int x) {
@@ -453,9 +466,9 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
             const bool is_last = tile == last_tile;
 #pragma unroll
             for (int n = 0; n < S::NOFF; ++n) r.vo[n] = is_last ? voff_last[x][n] : voff[x][n];
-        } else {   // pages shorter than a group (or items not dealt out wave by wave): every key looks its page up
+        } else {   // pages shorter than a group (or items not dealt out wave by wave)
             const int key = min(IM::key(x, tid), BN - 1);
-            r.base = (gptr) cache + (kv_off_tab(P.pg, ptab, min(tile * BN + key, pmax)) + head_off);
+            r.base = (gptr) cache + row_off(min(tile * BN + key, pmax), gb.p.it[x]);
 #pragma unroll
             for (int n = 0; n < S::NOFF; ++n) r.vo[n] = voff[x][n] - (uint32_t) (key & 15) * (uint32_t) P.pg.rowb;
         }
@@ -488,7 +501,7 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
         if constexpr (FAST) {
             off = gb.go + (tile == last_tile ? sb_last : sb_full);
         } else {
-            off = kv_off_tab(P.pg, ptab, min(tile * BN + lkey, pmax)) + head_off;
+            off = row_off(min(tile * BN + lkey, pmax), gb.p.sb);
         }
         const gptr p_ = (gptr) cache + off;
         if constexpr (S::SB == 16) { const u4 t = P1A_GLOAD(u4, p_); r.w[0] = t[0]; r.w[1] = t[1]; r.w[2] = t[2]; r.w[3] = t[3]; }

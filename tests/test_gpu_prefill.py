@@ -170,6 +170,28 @@ def test_small_heads_take_the_same_bits_whichever_way_tiles_come(p1a, kv_type, H
     check(outs[0], O.attn_rows(pool.host_seq(0), q, (p0 + np.arange(T)).astype(np.int32), Hq, D ** -0.5, gate=gate), f"small heads {kv_type} {Hq}/{Hkv}/{D} p0 {p0} T {T}")
 
 
+@pytest.mark.parametrize("kv_type", TYPES)
+@pytest.mark.parametrize("Hq,Hkv,D,p0,T", [(6, 2, 256, 0, 60), (4, 1, 256, 3000, 70), (8, 2, 128, 1500, 129), (4, 2, 64, 70, 33), (2, 1, 64, 4000, 5)])
+def test_pages_of_any_length_give_the_same_bits(p1a, kv_type, Hq, Hkv, D, p0, T):
+    """the table entries of a tile's keys are looked up a step ahead of it, one per key where pages are shorter than 16 positions:
+    one tile, tiles that wrap around, key splits; pages of 1, 4 and 8 positions against pages of 16"""
+    n, want = p0 + T, None
+    q, _, _, gate = I.qkv(n + D, 1, T, Hq, Hkv, D, f16_inputs=True)
+    for psh in (4, 3, 2, 0):
+        if (O.row_bytes(kv_type, Hkv, D) << psh) % 16:         # (refused: V would not be 16-byte aligned)
+            continue
+        pool = Pool(p1a, kv_type, Hq, Hkv, D, psh, [n, 21], seed=n + D)
+        p1a.set_prefill_staging_limit(0)
+        try:
+            out = run_prefill(p1a, pool.dev_seq(0), q, T, p0, Hq, D ** -0.5, gate=gate)
+        finally:
+            p1a.set_prefill_staging_limit(1 << 30)
+        if want is None:
+            want = out
+            check(out, O.attn_rows(pool.host_seq(0), q, (p0 + np.arange(T)).astype(np.int32), Hq, D ** -0.5, gate=gate), f"pages {kv_type} {Hq}/{Hkv}/{D} p0 {p0} T {T}")
+        assert np.array_equal(out, want), psh
+
+
 def test_f16_contiguous_and_small_pages_take_the_same_bits(p1a):
     """f16, D = 256: a contiguous cache that ends right behind the last position (whole 16-key groups cannot be fetched:
     the register-staged kernel runs), one with room (tiles loaded straight into LDS) and 16-position pages must agree
