@@ -15,13 +15,17 @@
 //   that is not zero is at least 1, it is cut into three f16 pieces, 11, 11 and the 2 to 4 bits left: exact (the last bit of
 //   such a P is 2^-23, f16 ends at 2^-24) and each above zero, so that an infinite V stays infinite. A tile with a smaller P
 //   takes fp32 matrix products, at a fifth of the rate: pieces would end at 2^-39 of the largest weight, where fp32 does not,
-//   and thousands of light keys with a large V are more than the result. (24 / 4 heads of 256 in pages of 4, 8 sequences x 4
-//   rows of 2500 keys, two pieces whatever P is 104 us, as it is 104, fp32 products throughout 122; 24 / 4 of 96 39 and 42.)
+//   and thousands of light keys with a large V are more than the result. (24 / 4 heads of 96, 8 sequences x 4 rows of 2500
+//   keys: two pieces whatever P is 37.6 us, as it is 40.9; 24 / 4 of 256 in pages of 4 cost the same both ways.)
 // Data movement
 //   A lane reads what it feeds to the products straight into registers: 8 consecutive values (16 / 8 / 4 bytes) of its key
 //   per K block, 2 consecutive dims (4 / 2 bytes; q4_0: one byte, dims c and c + 16) of 4 keys per V block. Only the
 //   block scales change lanes, through a small table in LDS. No LDS tile: such head rows are 2-byte aligned, which the
 //   LDS-direct loads of dec_mfma_k cannot take.
+// Builds: one for each number of 32-dim blocks a head can have. (Heads of other than 96 and 192 dims shared one for up to 8
+// blocks and one for up to 16: a branch per block keeps the loads and products of two blocks from being scheduled side by side, and
+// the LDS of the largest head keeps a second workgroup off the CU. 8 sequences x 4 rows of 2500 keys in pages of 8, q8_0,
+// 32 / 8 heads of 128 141 -> 74 us; 16 / 2 of 320 138 -> 66; 4 / 4 of 32 63 -> 27; 24 / 4 of 256 in pages of 4 121 -> 112.)
 // What bounds it: latency. At 24 / 4 heads, D = 96, q8_0 a context of 8190 is one tile per wave: positions, page entry, tile,
 // fold, each waiting for the one before. Two layers of it (prep, this kernel and the merge each) took 325 us and take 54, of
 // which the launches from Python are most; recorded, a layer of 2000 keys takes 15 us, one of 20000 keys (16 MB) 19 us.
@@ -76,16 +80,15 @@ __device__ __forceinline__ float below(float x) { return asf(__builtin_elementwi
 // two values to f16, towards zero
 __device__ __forceinline__ h2 cut2(float x, float y) { return __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(x, y)); }
 
-// NBM: the most 32-dim blocks of a head this build takes; EX: exactly that many
-template <uint32_t KT, int NBM, bool EX, int NW>
+template <uint32_t KT, int NB, int NW>
 __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
     constexpr bool F16 = KT == P1A_KV_F16, Q8 = KT == P1A_KV_Q8_0;
-    constexpr int OS = NBM * 32 + 4;                          // floats per parked column (padded)
+    constexpr int OS = NB * 32 + 4;                          // floats per parked column (padded)
     constexpr int PC = 8;                                     // columns parked at a time
     __shared__ __attribute__((aligned(16))) float parked[NW * PC * OS];
-    __shared__ __attribute__((aligned(16))) float stab[F16 ? 4 : NW * 2 * NBM * 16];   // per wave: K scales [block][key], V scales
+    __shared__ __attribute__((aligned(16))) float stab[F16 ? 4 : NW * 2 * NB * 16];   // per wave: K scales [block][key], V scales
     __shared__ float ml[NW][2][16];
-    const int nb = EX ? NBM : P.D >> 5, D = nb * 32;
+    constexpr int D = NB * 32;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
     // the kv heads of one split stream share cache lines: given the same index mod 8 they sit on one XCD, and
@@ -113,35 +116,34 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
         }
         return;
     }
-    const size_t hoff = (size_t) hk * head_bytes(KT, 32) * nb;
+    const size_t hoff = (size_t) hk * head_bytes(KT, 32) * NB;
     const int SC = Q8 ? 2 : 18;                               // distance of two block scales
 
     // Q^T operands of column c; the 8 k-slots of lane group g are dims 32 b + 8 g .., for q4_0 the low and the high
     // nibbles of bytes 4 g .. 4 g + 3. Asked for ahead of the first tile, converted behind its requests.
-    f4 qa[NBM][2];
+    f4 qa[NB][2];
     {
         const float * qr = P.q + (row0 + min(c, R - 1)) * D;
 #pragma unroll
-        for (int b = 0; b < NBM; ++b) {
-            if (!EX && b >= nb) continue;
+        for (int b = 0; b < NB; ++b) {
             const float * x = qr + 32 * b + (KT == P1A_KV_Q4_0 ? 4 : 8) * g;
             qa[b][0] = *reinterpret_cast<const f4 *>(x);
             qa[b][1] = *reinterpret_cast<const f4 *>(x + (KT == P1A_KV_Q4_0 ? 16 : 4));
         }
     }
-    f4 o[NBM][2];
+    f4 o[NB][2];
 #pragma unroll
-    for (int b = 0; b < NBM; ++b) o[b][0] = o[b][1] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < NB; ++b) o[b][0] = o[b][1] = f4{0.f, 0.f, 0.f, 0.f};
     float m = NEG_INF, l = 0.f;                               // l: over this lane's keys
-    float * const tk = stab + (F16 ? 0 : wave * 2 * NBM * 16), * const tv = tk + (F16 ? 0 : NBM * 16);
+    float * const tk = stab + (F16 ? 0 : wave * 2 * NB * 16), * const tv = tk + (F16 ? 0 : NB * 16);
 
     const int last = n - 1;
     // a tile's K operands, V values and block scales, all asked for before any of them is used
-    u4 kr[F16 ? NBM : 1];
-    uint64_t k8[Q8 ? NBM : 1];
-    uint32_t k4[!F16 && !Q8 ? NBM : 1];
-    uint32_t vr[NBM][4];
-    constexpr int NSC = (NBM + 3) / 4;
+    u4 kr[F16 ? NB : 1];
+    uint64_t k8[Q8 ? NB : 1];
+    uint32_t k4[!F16 && !Q8 ? NB : 1];
+    uint32_t vr[NB][4];
+    constexpr int NSC = (NB + 3) / 4;
     uint16_t sk[NSC], sv[NSC];
     auto request = [&](int ts) {
         // keys past the last one are read as the last one and weighted with nothing
@@ -162,24 +164,22 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
         if constexpr (!F16) {
 #pragma unroll
             for (int x = 0; x < NSC; ++x) {
-                const int b = min(4 * x + g, nb - 1);         // (lanes without a block of their own repeat the last one)
+                const int b = min(4 * x + g, NB - 1);         // (lanes without a block of their own repeat the last one)
                 sk[x] = ld<uint16_t>(kp + b * SC);
                 sv[x] = ld<uint16_t>(P.vc + ko + b * SC);
             }
         }
 #pragma unroll
-        for (int b = 0; b < NBM; ++b) {
-            if (!EX && b >= nb) continue;
+        for (int b = 0; b < NB; ++b) {
             if constexpr (F16) kr[b] = ld<u4>(kp + 64 * b + 16 * g);
-            else if constexpr (Q8) k8[b] = ld<uint64_t>(kp + 2 * nb + 32 * b + 8 * g);
+            else if constexpr (Q8) k8[b] = ld<uint64_t>(kp + 2 * NB + 32 * b + 8 * g);
             else k4[b] = ld<uint32_t>(kp + 18 * b + 2 + 4 * g);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const char * vp = P.vc + vo[i] + (F16 ? 4 * c : Q8 ? 2 * nb + 2 * c : 2 + c);
+            const char * vp = P.vc + vo[i] + (F16 ? 4 * c : Q8 ? 2 * NB + 2 * c : 2 + c);
 #pragma unroll
-            for (int b = 0; b < NBM; ++b) {
-                if (!EX && b >= nb) continue;
+            for (int b = 0; b < NB; ++b) {
                 if constexpr (F16) vr[b][i] = ld<uint32_t>(vp + 64 * b);
                 else if constexpr (Q8) vr[b][i] = ld<uint16_t>(vp + 32 * b);
                 else vr[b][i] = *reinterpret_cast<const uint8_t *>(vp + 18 * b);
@@ -188,10 +188,9 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
     };
     int ts = split * U + wave * 16;
     if (ts < n) request(ts);
-    h8 qf[NBM];
+    h8 qf[NB];
 #pragma unroll
-    for (int b = 0; b < NBM; ++b) {
-        if (!EX && b >= nb) continue;
+    for (int b = 0; b < NB; ++b) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) { qf[b][e] = (half_t) (qa[b][0][e] * P.qscale); qf[b][4 + e] = (half_t) (qa[b][1][e] * P.qscale); }
     }
@@ -201,7 +200,7 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
         if constexpr (!F16) {
 #pragma unroll
             for (int x = 0; x < NSC; ++x) {
-                const int b = min(4 * x + g, nb - 1);
+                const int b = min(4 * x + g, NB - 1);
                 tk[b * 16 + c] = (float) __builtin_bit_cast(half_t, sk[x]);
                 tv[b * 16 + c] = ts + c > last ? 0.f : (float) __builtin_bit_cast(half_t, sv[x]);
             }
@@ -210,8 +209,7 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
         // ---- S^T: this lane holds keys ts + 4 g + i of column c ----
         f4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int b = 0; b < NBM; ++b) {
-            if (!EX && b >= nb) continue;
+        for (int b = 0; b < NB; ++b) {
             if constexpr (F16) s = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, kr[b]), qf[b], s, 0, 0, 0);
             else {
                 uint32_t a[4];
@@ -240,7 +238,7 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
             const float alpha = m == mnew ? 1.f : __builtin_amdgcn_exp2f(m - mnew);   // (m = -inf: nothing accumulated yet, 0)
             l *= alpha;
 #pragma unroll
-            for (int b = 0; b < NBM; ++b) { if (!EX && b >= nb) continue; o[b][0] *= alpha; o[b][1] *= alpha; }
+            for (int b = 0; b < NB; ++b) { o[b][0] *= alpha; o[b][1] *= alpha; }
             m = mnew;
         }
         float p[4];
@@ -254,13 +252,12 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
                 for (int i = 0; i < 4; ++i)
                     if (ts + 4 * g + i > last) {
 #pragma unroll
-                        for (int b = 0; b < NBM; ++b) vr[b][i] = 0;
+                        for (int b = 0; b < NB; ++b) vr[b][i] = 0;
                     }
             }
             if (__builtin_expect(__any((p[0] < 1.f && p[0] > 0.f) || (p[1] < 1.f && p[1] > 0.f) || (p[2] < 1.f && p[2] > 0.f) || (p[3] < 1.f && p[3] > 0.f)), 0)) {
 #pragma unroll
-                for (int b = 0; b < NBM; ++b) {
-                    if (!EX && b >= nb) continue;
+                for (int b = 0; b < NB; ++b) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {             // keys 4 g + i of the four lane groups
                         uint32_t w = vr[b][i];
@@ -285,8 +282,7 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
                     }
                 }
 #pragma unroll
-                for (int b = 0; b < NBM; ++b) {
-                    if (!EX && b >= nb) continue;
+                for (int b = 0; b < NB; ++b) {
 #pragma unroll
                     for (int x = 0; x < 2; ++x) {
                         const uint32_t sel = x ? 0x07060302u : 0x05040100u;
@@ -298,8 +294,7 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
             }
         } else {
 #pragma unroll
-            for (int b = 0; b < NBM; ++b) {
-                if (!EX && b >= nb) continue;
+            for (int b = 0; b < NB; ++b) {
                 const f4 d = *reinterpret_cast<const f4 *>(tv + b * 16 + 4 * g);
                 float w0[4], w1[4], w2[4];
 #pragma unroll
@@ -337,8 +332,7 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
         if (c >= h0 && c < he) {
             float * dst = parked + (wave * PC + c - h0) * OS;
 #pragma unroll
-            for (int b = 0; b < NBM; ++b) {
-                if (!EX && b >= nb) continue;
+            for (int b = 0; b < NB; ++b) {
                 if constexpr (KT == P1A_KV_Q4_0) {            // row r of tile x: dim 32 b + 16 x + r
                     *reinterpret_cast<f4 *>(dst + 32 * b + 4 * g) = o[b][0];
                     *reinterpret_cast<f4 *>(dst + 32 * b + 16 + 4 * g) = o[b][1];
@@ -380,11 +374,12 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
 }
 
 template <uint32_t KT> void launch_kt(const any_params & P, dim3 grid, hipStream_t s) {
-    const int nb = P.D / 32;
-    if (nb == 3) dec_any_k<KT, 3, true, 8><<<grid, 512, 0, s>>>(P);
-    else if (nb == 6) dec_any_k<KT, 6, true, 8><<<grid, 512, 0, s>>>(P);
-    else if (nb <= 8) dec_any_k<KT, 8, false, 8><<<grid, 512, 0, s>>>(P);
-    else dec_any_k<KT, 16, false, 4><<<grid, 256, 0, s>>>(P);
+    switch (P.D / 32) {
+#define P1A_ANY(NB_) case NB_: dec_any_k<KT, NB_, NB_ <= 8 ? 8 : 4><<<grid, NB_ <= 8 ? 512 : 256, 0, s>>>(P); break
+        P1A_ANY(1); P1A_ANY(2); P1A_ANY(3); P1A_ANY(4); P1A_ANY(5); P1A_ANY(6); P1A_ANY(7); P1A_ANY(8);
+        P1A_ANY(9); P1A_ANY(10); P1A_ANY(11); P1A_ANY(12); P1A_ANY(13); P1A_ANY(14); P1A_ANY(15); P1A_ANY(16);
+#undef P1A_ANY
+    }
 }
 
 }   // namespace

@@ -24,7 +24,7 @@ def close(out, ref, what):
     print(f"[parity] {what}: rel_l2={rl:.2e}")
 
 
-# (type, q heads, kv heads, D, log2 of the page): every build (3, 6, up to 8, up to 16 blocks of 32 dims), one and more column
+# (type, q heads, kv heads, D, log2 of the page): builds of 8 and of 4 waves, one and more column
 # tiles (17 and 20 heads of a group), short pages, the 51- and 27-value-wide odd rows of D = 96 and one kv head
 SHAPES = [(O.KV_F16, 6, 1, 96, 4), (O.KV_Q8_0, 24, 4, 96, 8), (O.KV_Q4_0, 4, 1, 96, 4), (O.KV_Q8_0, 3, 1, 96, 0),
           (O.KV_F16, 16, 2, 192, 6), (O.KV_Q8_0, 16, 4, 192, 4), (O.KV_Q4_0, 8, 8, 192, 4),
@@ -64,6 +64,20 @@ def test_any_shape_vs_float64(p1a, kv_type, Hq, Hkv, D, psh):
     for s in (0, 2, 3, 4):
         close(got[s:s + 1], O.attn_rows(pool.host_seq(s), q[s:s + 1], pos[s:s + 1], Hq, SCALE, f64=True), f"slot {s}")
     assert np.all(np.isnan(got[1]))
+
+
+@pytest.mark.parametrize("kv_type", [O.KV_F16, O.KV_Q8_0, O.KV_Q4_0])
+@pytest.mark.parametrize("D", range(32, 513, 32))
+def test_any_head_size(p1a, kv_type, D):
+    """a build for each number of 32-dim blocks: a unit's first wave alone, and several units with a ragged end"""
+    Hq, Hkv, psh, lens = 3, 1, 2, [5, 400]
+    pool = Pool(p1a, kv_type, Hq, Hkv, D, psh, lens, seed=D)
+    for s, n in enumerate(lens):
+        q, _, _, gate = I.qkv(3 * D + s, 1, 1, Hq, Hkv, D, f16_inputs=True)
+        ref = O.attn_rows(pool.host_seq(s), q, np.array([n - 1], np.int32), Hq, SCALE, gate=gate, f64=True)
+        out = torch.full((1, Hq, D), float("nan"), device="cuda")
+        p1a.attn_decode(dev(q), pool.dev_seq(s), out, 1, n - 1, Hq, SCALE, gate=dev(gate))
+        close(out.cpu().numpy(), ref, f"type {kv_type} D {D} n {n}")
 
 
 @pytest.mark.parametrize("kv_type", [O.KV_F16, O.KV_Q8_0, O.KV_Q4_0])
