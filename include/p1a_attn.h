@@ -228,8 +228,8 @@ void p1a_set_nsplit(int n);
 /* Bytes of split scratch one decode call of these arguments needs (accumulators rounded up to 256 bytes, then the (m, l)
  * pairs), and the bytes the library keeps per (device, stream) for a head shape - the larger of the two is what a first call
  * allocates. A cache the MFMA kernel cannot take (misaligned base or page stride, pages of fewer than 16 positions, head
- * sizes other than 64 / 128 / 256) takes the kernel for any shape, which is sized for more partials per row; both are covered. No GPU call is made
- * (without a device the plan of a 256-CU part is returned). No counterpart in the reference, whose scratch size is a
+ * sizes other than 64 / 128 / 256) takes the kernel for any shape, which has a split count of its own; both are covered. No
+ * GPU call is made (without a device the plan of a 256-CU part is returned). No counterpart in the reference, whose scratch size is a
  * compile-time constant (src/fast/attn_dec2.cu:452-464). rows_per_seq as for p1a_attn_decode (T for a call without
  * pos_rows). */
 size_t p1a_decode_scratch_bytes(const p1a_kv *c, int Hq, int T, int rows_per_seq);

@@ -150,8 +150,8 @@ void decode_footprint(int Hq, int Hkv, int D, size_t & need_o, size_t & need_ml)
     c.Hkv = Hkv; c.D = D;
     need_o = need_ml = 0;
     const uint32_t types[3] = {P1A_KV_F16, P1A_KV_Q8_0, P1A_KV_Q4_0};
-    // (a cache the MFMA kernel cannot take - a misaligned base, short pages - goes to the kernel for any shape, which is sized for more
-    // partials per row: both plans count, so that a warm-up also covers such caches)
+    // (a cache the MFMA kernel cannot take - a misaligned base, short pages - goes to the kernel for any shape, which has a plan of
+    // its own: both count, so that a warm-up also covers such caches)
     for (uintptr_t base : {(uintptr_t) 16, (uintptr_t) 2})
         for (uint32_t ty : types)
             for (int rg = 1; rg <= 4; ++rg) {

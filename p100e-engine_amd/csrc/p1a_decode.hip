@@ -989,8 +989,7 @@ __global__ void __launch_bounds__(256) sigmoid_mul_k(float * __restrict__ x, con
 struct dec_plan {
     bool mfma;
     int GQA, NW, NT, RG;
-    int nsplit;    // split streams
-    int NS;        // partials per output row the scratch is sized for (at least nsplit, what merge_k folds)
+    int nsplit;    // split streams: partials per output row
 };
 
 bool mfma_ok(const p1a_kv & c, int GQA) {
@@ -1010,14 +1009,14 @@ dec_plan make_plan(const p1a_kv & c, int Hq, int rows_per_group, int nsplit_req,
     if (!p.mfma) {
         p.NW = 4; p.NT = 1;
         p.RG = rows_per_group < 1 ? 1 : rows_per_group;   // no sharing here: the group only selects the page table
-        // the scratch such a call asks for (4 partials for every 2 CUs per q head) is part of what callers size and
-        // allocate by; one workgroup per CU needs no more of them than that
-        int n = nsplit_req > 0 ? nsplit_req : 2 * cus / Hq;
-        n = n < 1 ? 1 : (n > 1024 ? 1024 : n);
-        p.NS = n * 4;
-        if (nsplit_req <= 0) n = cus / c.Hkv < p.NS ? cus / c.Hkv : p.NS;
-        if (n >= 8) n &= ~7;
-        p.nsplit = n < 1 ? 1 : n;
+        // one workgroup per CU, and not more than 4 partials for every 2 CUs per q head
+        int n = nsplit_req;
+        if (n <= 0) {
+            const int most = 4 * (2 * cus / Hq < 1 ? 1 : (2 * cus / Hq > 1024 ? 1024 : 2 * cus / Hq));
+            n = cus / c.Hkv < most ? cus / c.Hkv : most;
+        }
+        n = n < 1 ? 1 : (nsplit_req > 1024 ? 1024 : n);
+        p.nsplit = n >= 8 ? n & ~7 : n;
         return p;
     }
     const int cap = 32 / p.GQA < 4 ? 32 / p.GQA : 4;
@@ -1035,10 +1034,7 @@ dec_plan make_plan(const p1a_kv & c, int Hq, int rows_per_group, int nsplit_req,
     return p;
 }
 
-void finish_plan(dec_plan & p) {
-    p.NT = p.RG * p.GQA <= 16 ? 1 : 2;
-    if (p.mfma) p.NS = p.nsplit;
-}
+void finish_plan(dec_plan & p) { p.NT = p.RG * p.GQA <= 16 ? 1 : 2; }
 
 template <uint32_t KT, int D, uint32_t KS = KT>
 int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hipStream_t s) {
@@ -1085,8 +1081,8 @@ void decode_scratch_need(const p1a_kv & c, int Hq, int rows, int rows_per_group,
                          size_t & bytes_o, size_t & bytes_ml) {
     dec_plan pl = make_plan(c, Hq, rows_per_group, nsplit_req, cus);
     finish_plan(pl);
-    bytes_o = (size_t) rows * Hq * pl.NS * c.D * sizeof(float);
-    bytes_ml = (size_t) rows * Hq * pl.NS * 2 * sizeof(float);
+    bytes_o = (size_t) rows * Hq * pl.nsplit * c.D * sizeof(float);
+    bytes_ml = (size_t) rows * Hq * pl.nsplit * 2 * sizeof(float);
 }
 
 int decode_rows_per_group(const p1a_kv & c, int Hq, int want) {
@@ -1099,8 +1095,8 @@ int launch_decode(const p1a_kv & c, const decode_args & a, hipStream_t s) {
     dec_plan pl = make_plan(c, a.Hq, a.rows_per_group, a.nsplit, a.cus);
     pl.RG = a.rows_per_group;
     finish_plan(pl);
-    // the partials of this launch: [T * Hq][NS][D] accumulators and [T * Hq][NS][2] (m, l) pairs
-    const size_t need_o = (size_t) a.T * a.Hq * pl.NS * c.D * sizeof(float), need_ml = (size_t) a.T * a.Hq * pl.NS * 2 * sizeof(float);
+    // the partials of this launch: [T * Hq][nsplit][D] accumulators and [T * Hq][nsplit][2] (m, l) pairs
+    const size_t need_o = (size_t) a.T * a.Hq * pl.nsplit * c.D * sizeof(float), need_ml = (size_t) a.T * a.Hq * pl.nsplit * 2 * sizeof(float);
     if (need_o > a.cap_o || need_ml > a.cap_ml) {
         set_error("p1a_attn_decode: split partials of %zu + %zu bytes do not fit the scratch of %zu + %zu", need_o, need_ml, a.cap_o, a.cap_ml);
         return P1A_E_SCRATCH;

@@ -81,7 +81,7 @@ def test_reload_env(p1a):
 
 def test_decode_scratch_need_never_exceeds_footprint(p1a):
     """The per-(device, stream) buffers are sized once, at the footprint of a head shape. Whatever cache a later call of
-    that head shape brings - short pages, a misaligned base or page stride (the generic kernel: more partials per row),
+    that head shape brings - short pages, a misaligned base or page stride (the kernel for any shape, with a plan of its own),
     any row grouping - its partials must fit that footprint. Host arithmetic only."""
     from importlib import import_module
     b = import_module("p100e-engine_amd.binding")

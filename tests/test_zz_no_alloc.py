@@ -70,3 +70,21 @@ def test_noalloc_rows_of_several_sequences_and_refusal(p1a):
     assert b"static buffer" in L.p1a_last_error()
     torch.cuda.synchronize()
     assert bool((o32 == 7.0).all())
+
+
+def test_noalloc_takes_what_the_documented_size_fits(p1a):
+    """32 rows of 4 / 4 heads of 256 in pages of 4 positions (the kernel for any shape): T * Hq * splits * (D + 2) * 4 = 8.5 MB of
+    partials, a quarter of the fixed array"""
+    L = p1a.lib()
+    Hq, Hkv, D, T, n = 4, 4, 256, 32, 700
+    pool = Pool(p1a, O.KV_Q4_0, Hq, Hkv, D, 2, [n], seed=530)
+    c = pool.dev_seq(0)
+    assert p1a.decode_scratch_bytes(c.struct(), Hq, T, T) <= T * Hq * p1a.get_nsplit(Hkv) * (D + 2) * 4
+    q, _, _, gate = I.qkv(531, 1, T, Hq, Hkv, D)
+    dq, dg = dev(q), dev(gate)
+    want, got = torch.zeros((T, Hq, D), device="cuda"), torch.zeros((T, Hq, D), device="cuda")
+    assert call(L, "p1a_attn_decode_a16", dq, c, want, dg, None, T, n - T, Hq) == 0
+    assert call(L, "p1a_attn_decode_noalloc", dq, c, got, dg, None, T, n - T, Hq) == 0, L.p1a_last_error()
+    torch.cuda.synchronize()
+    assert torch.equal(want, got)
+    check(got.cpu().numpy(), O.attn_rows(pool.host_seq(0), q, (n - T + np.arange(T)).astype(np.int32), Hq, 1 / 16, gate=gate), "noalloc, pages of 4")
