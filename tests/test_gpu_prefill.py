@@ -248,15 +248,54 @@ def test_key_split_chunks(p1a, kv_type, Hq, Hkv, D, p0, T):
         assert ma < 2e-3 and rl < 1e-3, (t, ma, rl)
 
 
-@pytest.mark.parametrize("Hq,Hkv,T,p0", [(10, 2, 26, 0), (10, 2, 25, 70), (7, 1, 37, 3), (12, 2, 64, 64), (16, 1, 9, 500), (3, 3, 129, 0), (24, 4, 22, 2100)])
-def test_row_blocks(p1a, Hq, Hkv, T, p0):
-    """a block of 128 query rows holds tokens x q heads of one kv head: blocks that end inside a token, last blocks of one to
-    all rows, groups of blocks that are not full, one head per kv head"""
+def rows_of_a_block(p1a, T, p0, Hq, Hkv):
+    """query rows of a workgroup's block on this device: 128, halved down to 32 while half of the CUs would get no workgroup"""
+    cus, R, ks = torch.cuda.get_device_properties(0).multi_processor_count, T * (Hq // Hkv), p1a.prefill_key_splits(T, p0, Hq, Hkv)
+    b = 128
+    while b > 32 and 2 * -(-R // b) * Hkv * ks <= cus:
+        b //= 2
+    return b
+
+
+@pytest.mark.parametrize("Hq,Hkv,T,p0,rows", [(10, 2, 26, 0, 32), (10, 2, 25, 70, 32), (7, 1, 37, 3, 32), (12, 2, 64, 64, 32), (16, 1, 9, 500, 32), (3, 3, 129, 0, 32), (24, 4, 22, 2100, 32),
+                                              (10, 2, 900, 0, 64), (24, 4, 351, 5, 64), (10, 2, 1700, 0, 128), (24, 4, 731, 61, 128), (3, 3, 5700, 0, 128)])
+def test_row_blocks(p1a, Hq, Hkv, T, p0, rows):
+    """a block of query rows holds tokens x q heads of one kv head: blocks of 32, 64 and 128 rows that end inside a token, last blocks
+    of two to all rows, groups of blocks that are not full, one head per kv head"""
+    assert rows_of_a_block(p1a, T, p0, Hq, Hkv) == rows
     pool = Pool(p1a, O.KV_F16, Hq, Hkv, 256, 4, [p0 + T], seed=T + p0)
     q, _, _, gate = I.qkv(T, 1, T, Hq, Hkv, 256, f16_inputs=True)
-    ref = O.attn_rows(pool.host_seq(0), q, (p0 + np.arange(T)).astype(np.int32), Hq, 1 / 16, gate=gate)
+    at = np.arange(T) if T < 200 else np.unique(np.r_[0, 1, 126:132, I.rng(T).integers(0, T, 12), T - 40, T - 3:T])
+    ref = O.attn_rows(pool.host_seq(0), q[at], (p0 + at).astype(np.int32), Hq, 1 / 16, gate=gate[at])
     out = run_prefill(p1a, pool.dev_seq(0), q, T, p0, Hq, 1 / 16, gate=gate)
-    check(out, ref, f"row blocks {Hq}/{Hkv} p0 {p0} T {T}")
+    assert np.isfinite(out).all()
+    check(out[at], ref, f"row blocks {Hq}/{Hkv} p0 {p0} T {T}")
+
+
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("Hq,Hkv,D,p0,T,split", [(32, 8, 128, 0, 603, False), (32, 8, 128, 61, 603, False), (16, 2, 64, 61, 1101, False), (6, 3, 64, 0, 2870, False),
+                                                 (32, 8, 128, 6000, 301, True), (16, 2, 64, 5000, 501, True)])
+def test_full_blocks_of_small_heads(p1a, Hq, Hkv, D, p0, T, split, gated):
+    """D = 64 / 128 in calls that fill the device: blocks of 128 rows, 32 to each of four independent waves, whose lanes store
+    their rows from registers - with and without the gate, and as partials of a key split: the oracle's values on sampled
+    rows, the bits of 8-position pages (tiles staged through registers, pairs of waves, rows through LDS), nothing of what lies
+    past the last position (NaN here)"""
+    assert rows_of_a_block(p1a, T, p0, Hq, Hkv) == 128 and (p1a.prefill_key_splits(T, p0, Hq, Hkv) > 1) == split
+    n, outs = p0 + T, []
+    q, _, _, gate = I.qkv(n, 1, T, Hq, Hkv, D, f16_inputs=True)
+    gate = gate if gated else None
+    for psh in (4, 3):
+        pool = Pool(p1a, O.KV_F16, Hq, Hkv, D, psh, [n], seed=n + D, n_layers=1, layer=0)
+        c, rb, ps = pool.dev_seq(0), O.row_bytes(O.KV_F16, Hkv, D), 1 << psh
+        page, first = int(pool.tabs[(n - 1) >> psh]), ((n - 1) & (ps - 1)) + 1
+        for base in (0, ps * rb):
+            o = page * c.pstride + base + first * rb
+            pool.dpool[o:o + (ps - first) * rb] = 0x7e
+        outs.append(run_prefill(p1a, c, q, T, p0, Hq, D ** -0.5, gate=gate))
+    assert np.array_equal(outs[0], outs[1]) and np.isfinite(outs[0]).all()
+    at = np.unique(np.r_[0, 1, 31:33, 127:129, I.rng(T).integers(0, T, 12), T - 40, T - 3:T])
+    ref = O.attn_rows(pool.host_seq(0), q[at], (p0 + at).astype(np.int32), Hq, D ** -0.5, gate=gate[at] if gated else None)
+    check(outs[0][at], ref, f"full blocks {Hq}/{Hkv}/{D} p0 {p0} T {T} gate {gated}")
 
 
 @pytest.mark.parametrize("Hq,Hkv,D,p0,T", [(3, 1, 64, 4000, 33), (2, 2, 64, 33000, 1), (5, 1, 128, 3000, 7), (1, 1, 256, 40000, 130), (24, 4, 256, 3500, 512)])
