@@ -418,9 +418,13 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
         }
     }
     // FAST: the wave's 16 keys of a tile lie in one page (or the cache is contiguous): one table entry, one scalar base;
-    // otherwise every item and scale block has an entry of its own
-    constexpr bool FAST = GROUPED && IM::WAVE_MAJOR;
-    struct gpages { int pg; int it[FAST ? 1 : S::NPT], sb; };
+    // otherwise every item and scale block has an entry of its own, asked for a step ahead of the tile too (AHEAD). (Looked up where
+    // the loads are made, a tile took a round trip to L2 per row: the entry of the next row stood behind the load of this one.
+    // Pages of 8, 1000 tokens behind 2000: f16, 24 / 4 heads of 256 312 -> 135 us, 32 / 8 of 128 162 -> 84; q8_0 of 256 252
+    // -> 140; q4_0 of 128, one item a thread, 99 -> 81.) The build whose items are not dealt out wave by wave - q4_0 at D = 64, half an
+    // item a thread - has no such chain, and it is faster looking up on the spot (4096 tokens behind 4096, 16 / 2 heads 216 us, 234 ahead).
+    constexpr bool FAST = GROUPED && IM::WAVE_MAJOR, AHEAD = !FAST && IM::WAVE_MAJOR;
+    struct gpages { int pg; int it[AHEAD ? S::NPT : 1], sb; };
     struct gbases { size_t go; gpages p; };
     // a group past the last position takes the base of the last one that holds a position: the LDS-direct loads then
     // fetch that group's 16 rows (all inside its page) instead of clamping row by row
@@ -429,12 +433,9 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
         gpages r;
         r.pg = 0;
         if constexpr (!FAST) {
-            // asked for a step ahead of the tile, like the one entry of a 16-key group. (Looked up where the loads are made, a
-            // tile took a round trip to L2 per row: the entry of the next row stood behind the load of this one. Pages of
-            // 8, f16, 1000 tokens behind 2000, 24 / 4 heads of 256 312 -> 135 us, 32 / 8 of 128 162 -> 84; q8_0 252 -> 140.)
-            if (ptab) {
+            if (AHEAD && ptab) {
 #pragma unroll
-                for (int x = 0; x < S::NPT; ++x) r.it[x] = ptab[min(tile * BN + min(IM::key(x, tid), BN - 1), pmax) >> P.pg.psh];
+                for (int x = 0; x < S::NPT; ++x) r.it[AHEAD ? x : 0] = ptab[min(tile * BN + IM::key(x, tid), pmax) >> P.pg.psh];
                 if constexpr (S::SCALES_VIA_LDS) r.sb = ptab[min(tile * BN + 16 * wave + (lane & 15), pmax) >> P.pg.psh];
             }
         } else if (ptab) {
@@ -467,8 +468,8 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
 #pragma unroll
             for (int n = 0; n < S::NOFF; ++n) r.vo[n] = is_last ? voff_last[x][n] : voff[x][n];
         } else {   // pages shorter than a group (or items not dealt out wave by wave)
-            const int key = min(IM::key(x, tid), BN - 1);
-            r.base = (gptr) cache + row_off(min(tile * BN + key, pmax), gb.p.it[x]);
+            const int key = min(IM::key(x, tid), BN - 1), pos = min(tile * BN + key, pmax);
+            r.base = (gptr) cache + (AHEAD ? row_off(pos, gb.p.it[AHEAD ? x : 0]) : kv_off_tab(P.pg, ptab, pos) + head_off);
 #pragma unroll
             for (int n = 0; n < S::NOFF; ++n) r.vo[n] = voff[x][n] - (uint32_t) (key & 15) * (uint32_t) P.pg.rowb;
         }
