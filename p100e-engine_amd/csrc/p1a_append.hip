@@ -208,6 +208,38 @@ __device__ __forceinline__ int pair_pos(const mrope_view & mr, const int32_t * p
     else return 0;
     return mr.p[(size_t) st * mr.stride + t];
 }
+// What both prep kernels do to a head, in one place: a token's rows are the same bits whichever of them a call takes.
+// sum of squares of a head whose lanes (lanes past it hold zeros) are an aligned group of G
+template <int G> __device__ __forceinline__ float head_ss(const float (&a)[4]) {
+    float ss = a[0] * a[0];
+    ss = ss + a[1] * a[1];
+    ss = ss + a[2] * a[2];
+    ss = ss + a[3] * a[3];
+    ss = ss + dpp<0xB1>(ss);                               // lane ^ 1
+    ss = ss + dpp<0x4E>(ss);                               // lane ^ 2
+    ss = ss + dpp<0x141>(ss);                              // the other quad of 8
+    if constexpr (G >= 16) ss = ss + dpp<0x140>(ss);       // the other 8 of 16
+    if constexpr (G >= 32) ss = ss + __shfl_xor(ss, 16);
+    if constexpr (G >= 64) ss = ss + __shfl_xor(ss, 32);
+    return ss;
+}
+// one dim of a rotated pair: x is the lower (lo) or the upper of the two
+__device__ __forceinline__ float rotate(float x, float other, float c, float sn, bool lo) {
+    const float x0 = lo ? x : other, x1 = lo ? other : x;
+    const float p0 = x0 * (lo ? c : sn), p1 = x1 * (lo ? sn : c);
+    return lo ? p0 - p1 : p0 + p1;
+}
+// dims 4 i .. 4 i + 3 of a head to its place in the cache
+template <uint32_t KT> __device__ __forceinline__ void write_head(char * row, int h, int D, int i, bool live, float4 x) {
+    const int nb = D / 32, blk = i >> 3, j8 = i & 7;
+    if constexpr (KT == P1A_KV_F16) {
+        if (live) reinterpret_cast<h4 *>(row + (size_t) h * D * 2)[i] = h4{(half_t) x.x, (half_t) x.y, (half_t) x.z, (half_t) x.w};
+    } else if constexpr (KT == P1A_KV_Q8_0) {
+        if (live) q8_block(x, j8, row + (size_t) h * nb * 34, blk, nb);
+    } else {
+        if (live) q4_block(x, j8, row + ((size_t) h * nb + blk) * 18);
+    }
+}
 template <uint32_t KT>
 __global__ void __launch_bounds__(64) prep_k(const float * __restrict__ qg, const float * __restrict__ k,
                                              const float * __restrict__ v, const float * __restrict__ qn,
@@ -219,22 +251,11 @@ __global__ void __launch_bounds__(64) prep_k(const float * __restrict__ qg, cons
     const bool live = 4 * i < D;                               // dead lanes form whole 8-lane groups (D % 32 == 0)
     const int row = p0 < 0 ? pos[t] : p0 + t;                  // cache position of token t (src/fast/fused.cu:520)
     const size_t o = kv_off_tab(pg, kv_tab(pg, t), row);
-    const int nb = D / 32, blk = i >> 3, j8 = i & 7;
-    auto write_head = [&](char * cache, int h, float4 x) {
-        if constexpr (KT == P1A_KV_F16) {
-            if (live) reinterpret_cast<h4 *>(cache + o + (size_t) h * D * 2)[i] = h4{(half_t) x.x, (half_t) x.y, (half_t) x.z, (half_t) x.w};
-        } else if constexpr (KT == P1A_KV_Q8_0) {
-            if (live) q8_block(x, j8, cache + o + (size_t) h * nb * 34, blk, nb);
-            else xor8_max(0.f);
-        } else {
-            if (live) q4_block(x, j8, cache + o + ((size_t) h * nb + blk) * 18);
-        }
-    };
     if (b >= Hq + Hkv) {                                       // v head: the plain quantizing write
         const int h = b - Hq - Hkv;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
         if (live) x = reinterpret_cast<const float4 *>(v + (size_t) t * ldv + (size_t) h * D)[i];
-        write_head(vc, h, x);
+        write_head<KT>(vc + o, h, D, i, live, x);
         return;
     }
     const bool isq = b < Hq;
@@ -267,16 +288,7 @@ __global__ void __launch_bounds__(64) prep_k(const float * __restrict__ qg, cons
         }
     }
     if (isq && live) reinterpret_cast<float4 *>(gate + ((size_t) t * Hq + h) * D)[i] = gt;
-    float ss = a.x * a.x;
-    ss = ss + a.y * a.y;
-    ss = ss + a.z * a.z;
-    ss = ss + a.w * a.w;
-    ss = ss + dpp<0xB1>(ss);          // lane ^ 1
-    ss = ss + dpp<0x4E>(ss);          // lane ^ 2
-    ss = ss + dpp<0x141>(ss);         // the other quad of 8
-    ss = ss + dpp<0x140>(ss);         // the other 8 of 16
-    ss = ss + __shfl_xor(ss, 16);
-    ss = ss + __shfl_xor(ss, 32);
+    const float ss = head_ss<64>({a.x, a.y, a.z, a.w});
     const float sc = 1.0f / sqrtf(ss / (float) D + eps);
     float x[4] = {a.x * sc, a.y * sc, a.z * sc, a.w * sc};
     if (w && live) {
@@ -288,18 +300,13 @@ __global__ void __launch_bounds__(64) prep_k(const float * __restrict__ qg, cons
         const int jj = rot ? 4 * (lo ? i : i - hl) + e : 0;
         const float c0 = __shfl(tc[0], jj & 63), c1 = __shfl(tc[1], jj & 63);
         const float s0 = __shfl(tsn[0], jj & 63), s1 = __shfl(tsn[1], jj & 63);
-        if (rot) {
-            const float c = jj < 64 ? c0 : c1, sn = jj < 64 ? s0 : s1;
-            const float x0 = lo ? x[e] : other, x1 = lo ? other : x[e];
-            const float p0_ = x0 * (lo ? c : sn), p1_ = x1 * (lo ? sn : c);
-            x[e] = lo ? p0_ - p1_ : p0_ + p1_;
-        }
+        if (rot) x[e] = rotate(x[e], other, jj < 64 ? c0 : c1, jj < 64 ? s0 : s1, lo);
     }
     const float4 r = make_float4(x[0], x[1], x[2], x[3]);
     if (isq) {
         if (live) reinterpret_cast<float4 *>(q + ((size_t) t * Hq + h) * D)[i] = r;
     } else {
-        write_head(kc, h, r);
+        write_head<KT>(kc + o, h, D, i, live, r);
     }
 }
 
@@ -347,7 +354,6 @@ __global__ void __launch_bounds__(512) prep_rows_k(const float * __restrict__ qg
     }
     const int row = p0 < 0 ? pos[t] : p0 + t;
     const size_t o = kv_off_tab(pg, kv_tab(pg, t), row);
-    const int nb = D / 32, blk = i >> 3, j8 = i & 7;
     __syncthreads();
     const bool lo = i < hl, rot = i < 2 * hl;
     const int partner = (threadIdx.x & 63) - i + (rot ? (lo ? i + hl : i - hl) : i);
@@ -363,16 +369,7 @@ __global__ void __launch_bounds__(512) prep_rows_k(const float * __restrict__ qg
         const bool isq = b < Hq;
         float x[4] = {a[0], a[1], a[2], a[3]};
         if (b < Hq + Hkv) {
-            float ss = a[0] * a[0];
-            ss = ss + a[1] * a[1];
-            ss = ss + a[2] * a[2];
-            ss = ss + a[3] * a[3];
-            ss = ss + dpp<0xB1>(ss);      // lane ^ 1
-            ss = ss + dpp<0x4E>(ss);      // lane ^ 2
-            ss = ss + dpp<0x141>(ss);     // the other quad of 8
-            if constexpr (G >= 16) ss = ss + dpp<0x140>(ss);   // the other 8 of 16
-            if constexpr (G >= 32) ss = ss + __shfl_xor(ss, 16);
-            if constexpr (G >= 64) ss = ss + __shfl_xor(ss, 32);
+            const float ss = head_ss<G>(x);
             const float sc = 1.0f / sqrtf(ss / (float) D + eps);
 #pragma unroll
             for (int e = 0; e < 4; ++e) x[e] = x[e] * sc;
@@ -384,11 +381,7 @@ __global__ void __launch_bounds__(512) prep_rows_k(const float * __restrict__ qg
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float other = __shfl(x[e], partner);
-                if (rot) {
-                    const float x0 = lo ? x[e] : other, x1 = lo ? other : x[e];
-                    const float p0_ = x0 * (lo ? c4[e] : s4_[e]), p1_ = x1 * (lo ? s4_[e] : c4[e]);
-                    x[e] = lo ? p0_ - p1_ : p0_ + p1_;
-                }
+                if (rot) x[e] = rotate(x[e], other, c4[e], s4_[e], lo);
             }
         }
         const float4 r = make_float4(x[0], x[1], x[2], x[3]);
@@ -400,14 +393,7 @@ __global__ void __launch_bounds__(512) prep_rows_k(const float * __restrict__ qg
             }
         } else {
             const int h = b < Hq + Hkv ? b - Hq : b - Hq - Hkv;
-            char * const cache = b < Hq + Hkv ? kc : vc;
-            if constexpr (KT == P1A_KV_F16) {
-                if (live) reinterpret_cast<h4 *>(cache + o + (size_t) h * D * 2)[i] = h4{(half_t) r.x, (half_t) r.y, (half_t) r.z, (half_t) r.w};
-            } else if constexpr (KT == P1A_KV_Q8_0) {
-                if (live) q8_block(r, j8, cache + o + (size_t) h * nb * 34, blk, nb);
-            } else {
-                if (live) q4_block(r, j8, cache + o + ((size_t) h * nb + blk) * 18);
-            }
+            write_head<KT>((b < Hq + Hkv ? kc : vc) + o, h, D, i, live, r);
         }
         a = an;
         gt = gn;

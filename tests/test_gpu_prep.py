@@ -262,3 +262,24 @@ def test_mrope_in_a_call_of_many_tokens(p1a, Hq, D, n_rot):
     for x, y in zip(*out):
         for t in (0, 1, T - 2, T - 1):
             assert torch.equal(x[t], y[t]), t
+
+
+@pytest.mark.parametrize("kv_type,Hq,Hkv,D,n_rot", [(O.KV_Q8_0, 24, 4, 256, 64), (O.KV_F16, 32, 8, 128, 128), (O.KV_Q4_0, 40, 2, 192, 64)])
+def test_call_past_the_caches(p1a, kv_type, Hq, Hkv, D, n_rot):
+    """from 80 MB of q | gate rows on they are read past the caches: the bits of the same rows in two calls of half as many tokens"""
+    T = -(-(80 << 20) // (Hq * D * 8))
+    T += T & 1
+    g = torch.Generator(device="cuda").manual_seed(D)
+    qg, k, v = (torch.randn((T, n), generator=g, device="cuda") for n in (Hq * 2 * D, Hkv * D, Hkv * D))
+    qn, kn = (1 + 0.1 * torch.randn(D, generator=g, device="cuda") for _ in range(2))
+    pos, outs = torch.arange(T, dtype=torch.int32, device="cuda"), []
+    for step in (T, T // 2):
+        c = p1a.KVCache.contiguous(kv_type, T, Hkv, D)
+        q, gate = torch.zeros((T, Hq, D), device="cuda"), torch.zeros((T, Hq * D), device="cuda")
+        for a in range(0, T, step):
+            b = a + step
+            p1a.attn_prep(qg[a:b], k[a:b], v[a:b], qn, kn, pos[a:b], q[a:b], gate[a:b], c, a, step, Hq, n_rot, 1e6, 1e-6)
+        outs.append((q, gate, *c._keep))
+    for x, y in zip(*outs):
+        assert torch.equal(x, y)
+    assert torch.equal(outs[0][1].view(T, Hq, D), qg.view(T, Hq, 2 * D)[:, :, D:])
