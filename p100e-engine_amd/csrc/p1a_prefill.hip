@@ -1,29 +1,33 @@
 // Chunked causal prefill attention over a paged f16 / q8_0 / q4_0 KV cache for gfx950 (MI355X).
 //
-// One workgroup (4 waves, one per SIMD, 512 registers each) owns 128 consecutive query ROWS of one kv head - row r is token
-// r / GQA under q head r % GQA of the group; wave w owns 32 of them as the N = 32 columns of v_mfma_f32_32x32x16_f16 tiles.
+// One workgroup (4 waves) owns 128 consecutive query ROWS of one kv head (64 or 32 in a call of few) - row r is token r / GQA
+// under q head r % GQA of the group; wave w owns 32 (16, 8) of them as the N = 32 columns of v_mfma_f32_32x32x16_f16 tiles.
 // (Rows, not the tokens of one q head: a chunk of few tokens fills its blocks - 77 tokens under 6 heads are 4 blocks, not
 // 6 - and a block spans 128 / GQA tokens, so fewer of the keys it walks are behind the diagonal for most of its rows. 24 / 4
 // heads of 256, q8_0: 77 tokens behind 16000 88.7 -> 79.7 us for the whole call; a full chunk, 4096 behind 28672, the same.)
-// Keys are walked in tiles of 64, kept in LDS as f16 (two K and two V tiles). f16 rows of 512 bytes are moved from global memory straight into LDS
-// (global_load_lds_dwordx4); everything else is fetched into registers with 16-byte loads off a wave-uniform page base,
-// dequantized and stored to the same LDS places.
-//   S^T = K Q^T : A = K rows straight from LDS (ds_read_b128), B = Q^T held in accumulation registers (pre-multiplied
+// Keys are walked in tiles of 64, kept in LDS as f16 (two K and two V tiles). f16 rows in pages of 16 positions or more are
+// moved from global memory straight into LDS (global_load_lds_dwordx4); everything else is fetched into registers with
+// 16-byte loads, dequantized and stored to the same LDS places.
+//   S^T = K Q^T : A = K rows straight from LDS (ds_read_b128), B = Q^T held in registers for the whole kernel (pre-multiplied
 //                 by scale * log2 e, rounded to f16). A lane then holds 16 keys of ONE query row, so the row maximum
 //                 needs no cross-lane work beyond one half-wave swap.
 //   O^T = V^T P^T : A = V^T read with the transposing ds_read_b64_tr_b16, B = P^T straight from the S^T registers.
-//                 Waves pair up: each wave of a pair accumulates half the dims for the 64 rows of both, so a V^T
-//                 fragment feeds two MFMAs; the partner's P^T comes through LDS.
+// Two builds of that, chosen by where the registers and the LDS reads end (pf_solo):
+//   pairs (D = 256, and whatever is staged through registers): one wave per SIMD with 512 registers. Two waves share their
+//                 64 rows for O^T, each accumulating half the dims of both, so a V^T fragment feeds two MFMAs; the partner's
+//                 P^T comes through LDS.
+//   solo (D = 64 / 128, tiles straight into LDS): a wave accumulates all dims of its own rows in 256 registers, and a CU
+//                 holds two workgroups.
 // The loop is software-pipelined so that every iteration holds two independent instruction streams side by side: the
 // MFMAs of S^T for tile j+1 next to exp2 / f16 conversion of tile j, then the MFMAs of O^T for tile j next to masking and
-// the row maximum of tile j+1 (and the dequantization of the tiles that come after). With one wave per SIMD nothing
-// else can hide one pipe behind the other.
+// the row maximum of tile j+1 (and the dequantization of the tiles that come after). With one or two waves per SIMD little
+// else hides one pipe behind the other.
 // fp32 accumulation; the softmax denominator is a packed dot product of the rounded P with ones, so that it sums the same
 // rounded P that multiplies V. The reference maximum of a row moves lazily (only when the row maximum has grown
 // by more than 2^RESCALE_STEP), so the accumulators are rescaled a handful of times per row. Keys above a row's
 // diagonal are masked; the sigmoid output gate is applied in the epilogue.
-// Workgroup order: up to GQA consecutive row blocks of one kv head (128 tokens) get consecutive dispatch slots on the same XCD,
-// so they stream the same K/V tiles through one L2.
+// Workgroup order: up to GQA consecutive row blocks of one kv head (with key splits all of them) get consecutive dispatch slots
+// on the same XCD, so they stream the same K/V tiles through one L2.
 #include "p1a_common.hpp"
 
 #include <algorithm>
@@ -119,6 +123,10 @@ __device__ __forceinline__ pair32 deq4x4(uint32_t w, h2 dd) {
     const h2 b = __builtin_bit_cast(h2, perm_b(0x64646464u, w, 0x04030402u));
     return pair32{__builtin_bit_cast(uint32_t, (a - off) * dd), __builtin_bit_cast(uint32_t, (b - off) * dd)};
 }
+
+// sigmoid(g) through the hardware exponential and reciprocal (each within an ulp or two; exact at g = 0): the library's
+// full-range expf and IEEE division are some twenty instructions per value, 128 values per lane
+__device__ __forceinline__ float sigmoid(float g) { return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * g)); }
 
 constexpr float RESCALE_STEP = 8.0f;   // log2 units: the reference maximum of a row only moves in steps larger than this
 
@@ -233,11 +241,7 @@ template <class S> __device__ __forceinline__ void store_tile(const typename S::
 
 // GROUPED: pages hold at least 16 positions (or the cache is contiguous), so a 16-key group has one base
 __device__ __forceinline__ uint32_t lds_addr(const char * p) { return (uint32_t) (size_t) (const __attribute__((address_space(3))) char *) p; }
-// 64 lanes x 16 bytes, global (scalar base + 32-bit lane offset) -> LDS at `lds` + 16 * lane, no registers in between
-__device__ __forceinline__ void dma16(const char * sbase, uint32_t voff, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(voff), "s"(sbase), "s"(lds) : "memory", "m0");
-}
-// the same to `lds` + a constant: one scalar instruction per load
+// 64 lanes x 16 bytes, global (scalar base + 32-bit lane offset) -> LDS at `lds` + a constant + 16 * lane, no registers in between
 __device__ __forceinline__ void dma16_at(const char * sbase, uint32_t voff, uint32_t lds, int at) {
     asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(voff), "s"(sbase), "s"(lds), "i"(at) : "memory", "m0", "scc");
 }
@@ -852,8 +856,10 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
         ml[0] = m_run;
         ml[1] = l_own;
     }
-    // (a device full of workgroups, two on a CU: each lane the 16 bytes it holds of its row, which the other workgroup covers; 1 - 2 %
-    // better there than the way below, but 11.2 against 9.7 us for 40 tokens behind 100)
+    // Full blocks, two workgroups on a CU: each lane stores the 16 bytes it holds of its row, which the other workgroup's products
+    // cover. Against the way below: 2003 tokens, 16 / 2 heads of 64 28.5 -> 27.2 us, 8 / 8 of 128 35.2 -> 34.2; 32 / 8 of 128
+    // 54.1 -> 53.7; 24 / 4 of 128, 4096 tokens 116.9 -> 118.4, the one of thirty calls that loses more than the runs differ. (Short
+    // blocks are alone on their CU: 40 tokens behind 100 9.7 us below, 11.2 this way.)
     if (!PAIR && P.rpw == 32) {
         const float inv = part ? 1.0f : 1.0f / l_own;
         const size_t rr = row_index(min(my_row, P.R - 1));
@@ -872,7 +878,7 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
                     f4 v = {o[0][dt][4 * q4] * inv, o[0][dt][4 * q4 + 1] * inv, o[0][dt][4 * q4 + 2] * inv, o[0][dt][4 * q4 + 3] * inv};
                     if (P.gate && !part)
 #pragma unroll
-                        for (int x = 0; x < 4; ++x) v[x] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * gt[dt][q4][x]));
+                        for (int x = 0; x < 4; ++x) v[x] *= sigmoid(gt[dt][q4][x]);
                     *reinterpret_cast<f4 *>(orow + 32 * dt + 8 * q4 + 4 * g) = v;
                 }
         }
@@ -903,12 +909,10 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
 #pragma unroll
         for (int i = 0; i < N8; ++i) v[i] = *reinterpret_cast<const f4 *>(img + (i0 + i) * RPI * ORS);
         if (P.gate && !part) {
-            // sigmoid through the hardware exponential and reciprocal (each within an ulp or two; exact at g = 0): the
-            // library's full-range expf and IEEE division are some twenty instructions per value, 128 values per lane
 #pragma unroll
             for (int i = 0; i < N8; ++i)
 #pragma unroll
-                for (int x = 0; x < 4; ++x) v[i][x] *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * gt[i][x]));
+                for (int x = 0; x < 4; ++x) v[i][x] *= sigmoid(gt[i][x]);
         }
 #pragma unroll
         for (int i = 0; i < N8; ++i) {
@@ -922,9 +926,9 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
 template <uint32_t KT, int D, bool GROUPED, bool DMA = false>
 int launch_pf_g(const pf_params & P, hipStream_t s) {
     using L = pf_lay<D>;
-    const int lds = 2 * L::STAGE_B + (stager<KT, D>::SCALES_VIA_LDS ? 2 * 4 * 16 * stager<KT, D>::SB : 0) +
+    constexpr int lds = 2 * L::STAGE_B + (stager<KT, D>::SCALES_VIA_LDS ? 2 * 4 * 16 * stager<KT, D>::SB : 0) +
                     (pf_solo(D, DMA) ? (D == 64 ? BM * (2 * D + 16) : 0) : 4 * (BN / 16) * 64 * 16 + 4 * 32 * 4);
-    static_assert(BM * (4 * D + 16) <= 2 * L::STAGE_B + 4 * (BN / 16) * 64 * 16, "the output rows fit where the tiles and P^T were");
+    static_assert(BM * (4 * D + 16) <= lds, "the output rows fit where the tiles (and P^T) were");
     // (the attribute belongs to the function on ONE device: remembered per device, set again on another)
     static std::atomic<uint32_t> attr_set{0};
     int dev = 0;
@@ -1050,11 +1054,13 @@ static int block_rows(int R, int Hkv, int nks, int cus) {
 // A quantized cache is converted inside the kernel, without a copy, where few row blocks would share the copy: one block
 // makes every tile exactly once either way. A copy costs its bytes (about 0.5 us per million values of K and V each), the
 // conversion in the kernel some 1.5 us per tile of a workgroup (q8_0 a little more: two loads a key), and those are few only
-// while the splits spread them. Measured
-// copy / inside, us, q8_0 and q4_0: one block, 8 / 8 heads of 256 behind 28000 124 / 61 and 146 / 62, 24 / 4 behind 5000 41 / 38 and
-// 43 / 38, behind 2000 31 / 33 and 32 / 33; three, 24 / 4 behind 16000 63 / 56 and 69 / 56; four, 51 / 49 behind 10000 and 41 / 42
-// behind 5000; six, 86 / 90 behind 16000. At D <= 128 the kernel on a copy also has two workgroups to a CU: one block 44 / 34
-// (8 / 8 of 128 behind 16000), two (32 / 8) 55 / 70.
+// while the splits spread them. Copy / inside, us:
+//   D = 256, q8_0: level at 3 to 4 million values a block for up to four blocks (24 / 4 heads, 4 M: one block 36 / 36, three 52 / 48,
+//   four 66 / 65; 2.5 M: 35 / 37, 43 / 44, 50 / 50; 8 M: 44 / 41, 78 / 71, 107 / 103), behind with five (4 M: 86 / 90) and six (109 / 118).
+//   q4_0: level at 2 to 2.5 M (2.5 M: one 36 / 38, two 44 / 42, four 54 / 50; 8 M: 48 / 42, 60 / 49, 117 / 101); five and six gain little
+//   (4 M: 92 / 89, 116 / 116).
+//   D <= 128, where the kernel on a copy has two workgroups to a CU: one block from 2.5 M on (32 / 8 of 128 q8_0 26 / 25 and, at 5 M,
+//   30 / 27; q4_0 28 / 24 and 34 / 26). Two to four would gain too at 128 (12 M for four: 53 / 51 and 58 / 49), not at 64 (55 / 72).
 static bool convert_inside(const p1a_kv & c, int R, int n) {
     const int blocks = (R + BM - 1) / BM;
     if (c.pt && c.psh < 4) return false;                      // (a page lookup per key: measured nowhere as good)

@@ -1,4 +1,4 @@
-"""The decode kernels' register / LDS budget, read from the compiler's resource report (no GPU needed: hipcc cross-compiles).
+"""The kernels' register / LDS budget, read from the compiler's resource report (no GPU needed: hipcc cross-compiles).
 The design leans on it: a spill reload inside the key loop is a vector load that drains the whole tile queue, any scratch
 at all costs a launch about 0.7 us, and the single-buffered build only pays if two of its workgroups fit a CU (half the
 register file, 80 KB of LDS)."""
@@ -13,14 +13,13 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SRC = os.path.join(ROOT, "p100e-engine_amd", "csrc")
 
 
-def resource_report(tmp_path):
+def resource_report(tmp_path, source="p1a_decode.hip", flags=()):
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
         pytest.skip("no hipcc here")
     cmd = [hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-I" + os.path.join(ROOT, "include"), "-I" + SRC,
            "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument", "-Wno-inline-asm",
-           "-Rpass-analysis=kernel-resource-usage", "--cuda-device-only", "-c", os.path.join(SRC, "p1a_decode.hip"),
-           "-o", str(tmp_path / "dec.o")]
+           "-Rpass-analysis=kernel-resource-usage", "--cuda-device-only", *flags, "-c", os.path.join(SRC, source), "-o", str(tmp_path / "out.o")]
     r = subprocess.run(cmd, capture_output=True, text=True, timeout=900)
     assert r.returncode == 0, r.stderr[-2000:]
     kernels, cur = {}, None
@@ -53,3 +52,30 @@ def test_decode_kernels_fit_their_budget(tmp_path):
         waves = int(re.search(r"ELi(\d+)ELb1ELj\d+EEEv", name).group(1))
         assert r["LDS Size"] <= 80 * 1024, (name, r)                       # two workgroups in 160 KB
         assert r["Occupancy"] * 4 >= 2 * waves, (name, r)                   # two workgroups' waves on the 4 SIMDs
+
+
+VGPR_FORM = ("-mllvm", "-amdgpu-mfma-vgpr-form")               # (as the Makefile builds these two)
+
+
+def test_prefill_kernels_fit_their_budget(tmp_path):
+    """one workgroup of four waves to a CU, two where D <= 128 and the tiles come straight into LDS; nothing in memory. Scalar
+    registers do spill, to lanes of vector registers (reading the arguments again behind the key loop takes all of that out
+    and costs 0.3 us a call): not more than they do"""
+    ks = {k: v for k, v in resource_report(tmp_path, "p1a_prefill.hip", VGPR_FORM).items() if "prefill_k" in k}
+    assert len(ks) == 21, sorted(ks)
+    for name, r in ks.items():                                 # prefill_k<KT, D, GROUPED, DMA>
+        D, dma = int(re.search(r"ELi(\d+)ELb", name).group(1)), "ELb1ELb1E" in name
+        assert r.get("VGPRs Spill", 0) == 0 and r.get("ScratchSize", 0) == 0, (name, r)
+        assert r.get("SGPRs Spill", 0) <= (2 if dma else 19), (name, r)
+        assert r["Occupancy"] >= (2 if dma and D <= 128 else 1), (name, r)
+
+
+def test_any_shape_kernels_fit_their_budget(tmp_path):
+    """a build for each of 16 head sizes and three types, none of which spills; up to 256 dims eight waves, two to a SIMD, and LDS
+    for two workgroups on a CU"""
+    ks = {k: v for k, v in resource_report(tmp_path, "p1a_decode_any.hip", VGPR_FORM).items() if "dec_any_k" in k}
+    assert len(ks) == 48, sorted(ks)
+    for name, r in ks.items():                                 # dec_any_k<KT, blocks of 32 dims, waves>
+        blocks = int(re.search(r"ILj\d+ELi(\d+)ELi", name).group(1))
+        assert all(r.get(x, 0) == 0 for x in ("VGPRs Spill", "SGPRs Spill", "ScratchSize")), (name, r)
+        assert r["LDS Size"] <= 80 * 1024 and r["Occupancy"] >= (2 if blocks <= 8 else 1), (name, r)
