@@ -79,6 +79,9 @@ struct dec_params {
     float qscale;     // softmax scale * log2(e)
     int nsplit;       // split streams
     int GPS;          // row groups of a sequence
+    int RPS;          // rows of a sequence
+    int inner_sh;     // LIST: log2(GPS * Hkv) when that is a power of two, else -1
+    int rps_magic;    // LIST: 65536 / RPS + 1
     int hkv_sh;       // log2(Hkv) when Hkv is a power of two, else -1
     int npt;          // page-table entries of one sequence (ceil(n_ctx / page positions)); 0 = contiguous
 };
@@ -93,6 +96,9 @@ __device__ __forceinline__ size_t rfl64(size_t x) {
 
 // 4 int8 codes (one dword) -> (code * d) as two packed f16 pairs, returned as raw dwords so MFMA operands are built in place
 struct u2 { uint32_t lo, hi; };
+typedef int i8 __attribute__((ext_vector_type(8)));
+typedef int i8_a4 __attribute__((ext_vector_type(8), aligned(4)));
+typedef const __attribute__((address_space(4))) uint64_t * kargs;   // a kernel's arguments, as words
 __device__ __forceinline__ u2 deq4(uint32_t w, h2 d01, h2 d23) {
     const h2 off = {(half_t) 1152, (half_t) 1152};
     const uint32_t x = w ^ 0x80808080u;
@@ -109,6 +115,14 @@ __device__ __forceinline__ half_t scale_to_half(float q, float s) {
     asm volatile("" : "+v"(p));
     return (half_t) p;
 }
+
+// the lane's number, worked out anew wherever it is asked for (no register holds it in between)
+__device__ __forceinline__ int lane_id() {
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
+    return l;
+}
+__device__ __forceinline__ void put_lane(int & v, int x, int lane) { asm("v_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(x), "i"(lane)); }
 
 // the maximum over the four lanes that share (lane & 15): the two 16-lane rows of each half, then the two halves
 __device__ __forceinline__ float max_over_groups(float m) { return max_swap32(max_swap16(m)); }
@@ -156,6 +170,56 @@ template <int NR> __device__ __forceinline__ void wait_tiles(int newer) {
 __device__ __forceinline__ int sload_i32(const int32_t * p) {
     return *reinterpret_cast<const __attribute__((address_space(4))) int32_t *>(rfl64((size_t) p));
 }
+__device__ __forceinline__ i8 sload_i8(const int32_t * p) { return *reinterpret_cast<const __attribute__((address_space(4))) i8_a4 *>(rfl64((size_t) p)); }
+
+// The streams of a call's sequences that hold keys, those of two units and more (A) ahead of those of one (B): lane r (of the first 32)
+// gets how many the sequences up to and including row r's have, A in the low half and B in the high one. The positions come
+// through the scalar cache: a vector load would queue up behind the tiles that the other workgroup of the compute unit has asked
+// for (16 sequences of 20000 keys, 24 / 4 heads of 256, q8_0, two layers: 323 us, 317 so). rt: row r's page-table row, for T < 8.
+template <int U> __device__ __forceinline__ uint32_t live_streams(const dec_params & P, int lane, int & rt) {
+    const int T = P.T;
+    int pr = 0;
+    rt = 0;
+    auto single = [&](auto n_tag) {   // (rows past the last: that one once more)
+        constexpr int N = decltype(n_tag)::value;
+        int v[N], w[N];
+        const int32_t * rtab = P.pg.rtab ? P.pg.rtab : P.pos_rows;
+#pragma unroll
+        for (int k = 0; k < N; ++k) { v[k] = sload_i32(P.pos_rows + min(k, T - 1)); w[k] = sload_i32(rtab + min(k, T - 1)); }
+#pragma unroll
+        for (int k = 0; k < N; ++k) { put_lane(pr, v[k], k); put_lane(rt, w[k], k); }
+    };
+    if (T <= 4) single(std::integral_constant<int, 4>{});
+    else if (T < 8) single(std::integral_constant<int, 8>{});
+    else {
+        i8 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = sload_i8(P.pos_rows + min(8 * k, T - 8));   // (the last eight once more where there are none)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) put_lane(pr, v[k >> 3][k & 7], k);
+        if (T > 16) {
+#pragma unroll
+            for (int k = 16; k < 32; ++k) put_lane(pr, v[k >> 3][k & 7], k);
+        }
+        // (rows T - 8 .. T - 1 are in eight lanes from a multiple of eight on)
+        if (T & 7) pr = __builtin_amdgcn_ds_bpermute(4 * (lane < (T & ~7) ? lane : lane + 8 - (T & 7)), pr);
+    }
+    int n = lane < T && pr >= 0 ? pr / U + 1 : 0;              // units
+    if (P.RPS > 1) {                                           // the most of a sequence's rows, in its first one
+        const int n1 = n;
+        for (int k = 1; k < P.RPS; ++k) n = max(n, __builtin_amdgcn_ds_bpermute(4 * (lane + k), n1));
+        if (lane - (int) ((uint32_t) lane * (uint32_t) P.rps_magic >> 16) * P.RPS) n = 0;
+    }
+    const int na = min(max(n - P.nsplit, 0), P.nsplit);
+    int u = na | ((min(n, P.nsplit) - na) << 16);
+    // sums over the lanes up to this one
+    u += __builtin_amdgcn_update_dpp(0, u, 0x111, 0xf, 0xf, true);
+    u += __builtin_amdgcn_update_dpp(0, u, 0x112, 0xf, 0xf, true);
+    u += __builtin_amdgcn_update_dpp(0, u, 0x114, 0xf, 0xf, true);
+    u += __builtin_amdgcn_update_dpp(0, u, 0x118, 0xf, 0xf, true);
+    u += __builtin_amdgcn_update_dpp(0, u, 0x142, 0xa, 0xf, false);
+    return (uint32_t) u;
+}
 
 // SB ("single-buffered"): one K and one V slot per wave instead of two, so that two workgroups fit a CU's LDS (and register
 // file: 128 registers per lane) - for calls of many workgroups, where a second resident workgroup covers the start-up,
@@ -163,8 +227,12 @@ __device__ __forceinline__ int sload_i32(const int32_t * p) {
 // are done, V likewise; everything a lane computes, and the order it computes it in, is the same as in the double-buffered
 // kernel, so the partials are the same bits. One column tile only (NT == 1, at most 16 live columns).
 // KS (when it differs from KT = f16): the type the cache holds - its raw tiles are staged (raw_cfg) and converted to f16
-template <uint32_t KT, int D, int NT, int NWV, bool SB, uint32_t KS = KT>
-__global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const dec_params P) {
+// HOW = KS, and for calls of several sequences LIST (workgroups take the streams that hold keys), LIST | LOOP (one takes several)
+constexpr uint32_t LIST_ = 0x100, LOOP_ = 0x200;
+template <uint32_t KT, int D, int NT, int NWV, bool SB, uint32_t HOW = KT>
+__global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const dec_params P_) {
+    constexpr uint32_t KS = HOW & 0xff;
+    constexpr bool LIST = HOW & LIST_, LOOP = HOW & LOOP_;
     using C = tile_cfg<KT, D>;
     using RW = raw_cfg<KS, D>;
     constexpr bool STG = KS != KT;
@@ -196,30 +264,93 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     constexpr bool QLDS = (KT == P1A_KV_Q8_0 && NT == 2) || SB;
     __shared__ __attribute__((aligned(16))) char qtab[QLDS && !SB ? 32 * C::QRS : 16];
     __shared__ __attribute__((aligned(16))) char tabs[NWV * C::TAB_B];
+    __shared__ int wl[LOOP ? 32 : 1];                         // what live_streams() gave
     __shared__ __attribute__((aligned(16))) char vab[SB ? 16 : NWV * C::VA_B + 16];
 
-    const int lane = threadIdx.x & 63, wave = rfl(threadIdx.x >> 6);
-    const int c = lane & 15, g = lane >> 4;
+    constexpr int U = 32 * NWV;                               // positions per unit
+    const int wave = rfl(threadIdx.x >> 6);
     // blockIdx.x -> (split stream, head group). Workgroups are dealt to the 8 XCDs round-robin by linear index, so
-    // the kv heads of one split stream (which share cache lines) are given the same index mod 8. Sequence r of a batch
-    // starts on XCD r mod 8 (all of its row groups, which read the same keys): sequences fill the streams from 0 up, and
-    // with stream s on XCD s mod 8 in each of them the low XCDs had the work of all short ones. A layer of 32 sequences
-    // (24 / 4 heads of 256, q8_0, prep and merge included), each of 256 keys - 128 live workgroups, all on XCD 0 - 43 -> 29
-    // us, of 1024 keys 47 -> 39, of 2048 (eight streams) 51 both ways; of 300 ... 5000 keys 57 -> 48.
+    // the kv heads of one split stream (which share cache lines) are given the same index mod 8. (Sequence r of a batch starts on
+    // XCD r mod 8: sequences fill the streams from 0 up, and the low XCDs would have the work of all short ones.)
+    // LIST: an XCD deals its workgroups to its compute units in turn too, empty or not, so that one workgroup for every stream there
+    // could be puts the first streams of all sequences on the same few units (8 sequences of 1024 keys, 24 / 4 heads of 256: 128
+    // workgroups with keys on 32 of 256 units). The streams that hold keys are counted through instead, sequence by sequence,
+    // those of two units ahead of the others so that no unit gets two of them; number q goes to XCD q mod 8, one workgroup for every kv head and
+    // row group of it, and workgroups left over come last. (LOOP: one takes the numbers q, q + q_step, ...) Same partition of
+    // the keys, same bits. q8_0, 24 / 4 heads of 256, two layers with prep and merge: 8 sequences of 1024 keys 47 -> 38 us, 16 of 300 ... 5000
+    // 68 -> 58, 2 of 20000 74 -> 69, 32 of 256 61 -> 43; what it does not help costs at most 2 % (4 of 4000 ... 16000, two rows each 75 -> 77).
+    int hg = 0, gsub = 0, q = 0, q_step = 0, q_a = 0, q_end = 0, rt_lanes = 0;
+    uint32_t u_sum = 0;
+    if constexpr (LIST) {
+        const dec_params & P = P_;
+        const int lane = threadIdx.x & 63;
+        const int i = blockIdx.x, j = i >> 3, inner = P.Hkv * P.GPS;
+        const int jq = P.inner_sh >= 0 ? j >> P.inner_sh : j / inner, in = j - jq * inner;
+        q = jq * 8 + (i & 7);
+        if (LOOP) q_step = (P.inner_sh >= 0 ? (int) (gridDim.x >> 3) >> P.inner_sh : (int) (gridDim.x >> 3) / inner) * 8;
+        gsub = P.GPS == 1 ? 0 : in / P.Hkv;
+        hg = in - gsub * P.Hkv;
+        u_sum = live_streams<U>(P, lane, rt_lanes);
+        const uint32_t all = (uint32_t) __builtin_amdgcn_readlane((int) u_sum, 31);
+        q_a = (int) (all & 0xffff);
+        q_end = q_a + (int) (all >> 16);
+        if (q >= q_end) return;
+        if (LOOP && lane < 32) wl[lane] = u_sum;              // (every wave writes all of it, the same values: none reads it before it is there)
+    }
+    for (;;) {
+    // (LOOP: what hangs on the lane or on the kernel's arguments is worked out, or read, afresh for every item: kept from one to
+    // the next it would take the registers that the key loop needs)
+    const int tid = LOOP ? (wave << 6) | lane_id() : (int) threadIdx.x;
+    dec_params P_again;
+    if constexpr (LOOP) {
+        kargs kp = (kargs) __builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(kp));
+        struct words { uint64_t w[sizeof(dec_params) / 8]; } k;
+        static_assert(sizeof k == sizeof P_, "whole words");
+#pragma unroll
+        for (unsigned i = 0; i < sizeof(dec_params) / 8; ++i) k.w[i] = kp[i];
+        P_again = __builtin_bit_cast(dec_params, k);
+    }
+    const dec_params & P = LOOP ? P_again : P_;
+    const int lane = tid & 63;
+    const int c = lane & 15, g = lane >> 4;
     const int HG = P.Hkv;
-    int split, hg;
-    if ((P.nsplit & 7) == 0) {
-        const int i = blockIdx.x, j = i >> 3;
-        const int jq = P.hkv_sh >= 0 ? j >> P.hkv_sh : j / HG;
-        hg = j - jq * HG;
-        split = jq * 8 + ((i - (P.GPS == 1 ? (int) blockIdx.y : (int) blockIdx.y / P.GPS)) & 7);
+    auto next_item = [&]() {
+        if constexpr (!LOOP) return false;
+        q += q_step;
+        if (q >= q_end) return false;
+        u_sum = wl[lane_id() & 31];
+        return true;
+    };
+    int split, row0;
+    if constexpr (LIST) {
+        const bool in_a = q < q_a;
+        const uint32_t upto = in_a ? u_sum & 0xffff : u_sum >> 16;
+        const int at = in_a ? q : q - q_a;                     // place in its half of the list
+        const int first = __popcll(__ballot(lane < 32 && (int) upto <= at));   // the first row of the sequence
+        split = at - (first ? __builtin_amdgcn_readlane((int) upto, first - 1) : 0);
+        if (!in_a) {                                           // (behind the sequence's streams of two units)
+            const int a1 = __builtin_amdgcn_readlane((int) (u_sum & 0xffff), first), a0 = first ? __builtin_amdgcn_readlane((int) (u_sum & 0xffff), first - 1) : 0;
+            split += a1 - a0;
+        }
+        row0 = first + gsub * P.RG;
+        if (row0 >= P.T) {                                    // (a last sequence of fewer rows)
+            if (next_item()) continue;
+            return;
+        }
     } else {
-        split = blockIdx.x / HG;
-        hg = blockIdx.x - split * HG;
+        if ((P.nsplit & 7) == 0) {
+            const int i = blockIdx.x, j = i >> 3;
+            const int jq = P.hkv_sh >= 0 ? j >> P.hkv_sh : j / HG;
+            hg = j - jq * HG;
+            split = jq * 8 + ((i - (P.GPS == 1 ? (int) blockIdx.y : (int) blockIdx.y / P.GPS)) & 7);
+        } else {
+            split = blockIdx.x / HG;
+            hg = blockIdx.x - split * HG;
+        }
+        row0 = blockIdx.y * P.RG;
     }
     const int hk = hg, sub = wave;
-    constexpr int U = 32 * NWV;                               // positions per unit
-    const int row0 = blockIdx.y * P.RG;
     const int nr = min(P.RG, P.T - row0);                     // rows of this group
     const int R = nr * P.GQA;                                 // live MFMA columns
     // the page-table entry of this wave's first tile is asked for before anything else (it is the first link of the
@@ -227,7 +358,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     // (the group's first position and its page-table row hang on the kernel arguments only: both scalar loads are issued
     // before either value is used - one round trip for the two)
     const bool has_rt = P.pg.pt && P.pg.rtab;
-    const int rt0 = has_rt ? sload_i32(P.pg.rtab + (P.pos_rows ? row0 : 0)) : 0;
+    const int rt0 = !has_rt ? 0 : LIST && !LOOP && P.T < 8 ? __builtin_amdgcn_readlane(rt_lanes, row0) : sload_i32(P.pg.rtab + (P.pos_rows ? row0 : 0));
     const int pos_first = P.pos_rows ? sload_i32(P.pos_rows + row0) : 0;
     const int32_t * ptab = P.pg.pt ? P.pg.pt + rt0 : nullptr;
     // (n_ctx only bounds the read here: an entry fetched through a clamped index is fetched again, unclamped, once the
@@ -260,7 +391,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     // rows carry their own positions: merge_k then knows from those which streams to skip and never reads them.
     if (split * U >= n_max) {
         if (!P.pos_rows) {
-            for (int col = threadIdx.x; col < R; col += NWV * 64) {
+            for (int col = tid; col < R; col += NWV * 64) {
                 const int t = row_of(col), hh = col - t * P.GQA;
                 const size_t row = (size_t) (row0 + t) * P.Hq + (size_t) hg * P.GQA + hh;
                 float * pm = P.part_ml + (row * P.nsplit + split) * 2;
@@ -268,6 +399,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
                 pm[1] = 0.f;
             }
         }
+        if (next_item()) continue;
         return;
     }
 #pragma unroll
@@ -394,7 +526,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
         float4 a[NPC];
 #pragma unroll
         for (int k = 0; k < NPC; ++k) {
-            const int i = threadIdx.x + k * NWV * 64, col = i / (D / 4), d4 = i - col * (D / 4);
+            const int i = tid + k * NWV * 64, col = i / (D / 4), d4 = i - col * (D / 4);
             a[k] = make_float4(0.f, 0.f, 0.f, 0.f);
             if (col < R) {
                 const int t = row_of(col), hh = col - t * P.GQA;
@@ -403,7 +535,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
         }
 #pragma unroll
         for (int k = 0; k < NPC; ++k) {
-            const int i = threadIdx.x + k * NWV * 64, col = i / (D / 4), d4 = i - col * (D / 4);
+            const int i = tid + k * NWV * 64, col = i / (D / 4), d4 = i - col * (D / 4);
             const float s = P.qscale;
             if (col < 16) *reinterpret_cast<h4 *>(qown + col * C::QRS + d4 * 8) = h4{scale_to_half(a[k].x, s), scale_to_half(a[k].y, s), scale_to_half(a[k].z, s), scale_to_half(a[k].w, s)};
         }
@@ -430,7 +562,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
             float4 a[NPQ];
 #pragma unroll
             for (int k = 0; k < NPQ; ++k) {
-                const int i = threadIdx.x + k * NWV * 64, col = i / (D / 4);
+                const int i = tid + k * NWV * 64, col = i / (D / 4);
                 a[k] = make_float4(0.f, 0.f, 0.f, 0.f);
                 if (col < R) a[k] = *reinterpret_cast<const float4 *>(qown + (size_t) i * 16);
             }
@@ -438,12 +570,12 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
             const float s = P.qscale;
 #pragma unroll
             for (int k = 0; k < NPQ; ++k) {
-                const int i = threadIdx.x + k * NWV * 64, col = i / (D / 4), d = 4 * (i - col * (D / 4));
+                const int i = tid + k * NWV * 64, col = i / (D / 4), d = 4 * (i - col * (D / 4));
                 if (col < 8) *reinterpret_cast<h4 *>(qt + col * C::QRS + d * 2) = h4{scale_to_half(a[k].x, s), scale_to_half(a[k].y, s), scale_to_half(a[k].z, s), scale_to_half(a[k].w, s)};
             }
         }
     } else {
-    for (int i = threadIdx.x; i < (QLDS ? 32 : R) * (D / 4); i += NWV * 64) {
+    for (int i = tid; i < (QLDS ? 32 : R) * (D / 4); i += NWV * 64) {
         const int col = i / (D / 4), d = 4 * (i - col * (D / 4));
         float4 a = make_float4(0.f, 0.f, 0.f, 0.f);          // (columns past the live ones: zero operands)
         if (col < R) a = *reinterpret_cast<const float4 *>(kb1 + (size_t) i * 16);
@@ -476,13 +608,15 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     f4 o[NT][C::NDT];
     f4 ol[NT];
     float m_run[NT];
+    float zero = 0.f;
+    if constexpr (LOOP) asm volatile("" : "+v"(zero));        // (or four registers would carry it from item to item)
     const h4 ones = {(half_t) 1, (half_t) 1, (half_t) 1, (half_t) 1};
 #pragma unroll
     for (int r = 0; r < NT; ++r) {
         m_run[r] = NEG_INF;
-        ol[r] = f4{0.f, 0.f, 0.f, 0.f};
+        ol[r] = f4{zero, zero, zero, zero};
 #pragma unroll
-        for (int j = 0; j < C::NDT; ++j) o[r][j] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < C::NDT; ++j) o[r][j] = f4{zero, zero, zero, zero};
     }
 
     // one 16-key tile from slots (ks, vs); the loads of tile t + 1 into (ksn, vsn) are issued between its products
@@ -753,7 +887,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     constexpr int QD = D / 4;                                 // dims per quarter
     constexpr int PC = SB ? 8 : 16;                           // columns parked at a time
     // (lane coordinates worked out afresh: what is derived from them here need not live in registers through the key loop)
-    int tid_f = threadIdx.x;
+    int tid_f = LOOP ? (wave << 6) | lane_id() : (int) threadIdx.x;
     asm volatile("" : "+v"(tid_f));
     const int c_f = tid_f & 15, g_f = (tid_f >> 4) & 3;
     auto park = [&](int w, int k) -> float * {                // dim quarter k of wave w
@@ -838,6 +972,9 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
         };
         if (SB || he - h0 <= NWV) fold_round(std::integral_constant<int, 64>{}); else fold_round(std::integral_constant<int, 32>{});
         }
+    }
+    if (!next_item()) return;
+    __syncthreads();                                          // (the fold has been read: the tiles and tables are free)
     }
 }
 
@@ -1044,9 +1181,18 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hi
     P.p0 = a.p0; P.p0_dev = a.p0_dev; P.pos_rows = a.pos_rows;
     P.T = a.T; P.RG = pl.RG; P.Hq = a.Hq; P.Hkv = c.Hkv; P.GQA = pl.GQA;
     P.qscale = a.scale * 1.4426950408889634f; P.nsplit = pl.nsplit;
+    const int groups = (a.T + pl.RG - 1) / pl.RG;
+    P.RPS = a.rows_per_seq < a.T ? a.rows_per_seq : a.T;
     P.GPS = a.rows_per_seq > pl.RG ? a.rows_per_seq / pl.RG : 1;
-    P.hkv_sh = -1;
-    for (int sh = 0; sh < 16; ++sh) if ((1 << sh) == c.Hkv) P.hkv_sh = sh;
+    if (P.GPS > groups) P.GPS = groups;
+    const int nseq = (groups + P.GPS - 1) / P.GPS;
+    P.rps_magic = 65536 / P.RPS + 1;
+    const int inner = c.Hkv * P.GPS;
+    P.hkv_sh = P.inner_sh = -1;
+    for (int sh = 0; sh < 16; ++sh) {
+        if ((1 << sh) == c.Hkv) P.hkv_sh = sh;
+        if ((1 << sh) == inner) P.inner_sh = sh;
+    }
     P.npt = c.pt ? (int) (((long long) c.n_ctx + (1LL << c.psh) - 1) >> c.psh) : 0;
     constexpr bool big_tiles = KT == P1A_KV_F16 && D == 256;
     // A call of at least two workgroups per CU whose row groups fit one column tile takes the single-buffered variant, two
@@ -1056,20 +1202,30 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hi
     // for calls of many - measured slower on every shape tried, e.g. 8 x 4 rows q4_0 at 8 K 72 -> 60 us with one.)
     const long long wgs_all = (long long) pl.nsplit * c.Hkv * ((a.T + pl.RG - 1) / pl.RG);
     const bool sb = KS == KT && pl.NT == 1 && wgs_all >= 2LL * (a.cus > 0 ? a.cus : 256);
-    const dim3 grid(pl.nsplit * c.Hkv, (a.T + pl.RG - 1) / pl.RG);
-#define P1A_DEC(NT_, NW_) dec_mfma_k<KT, D, NT_, NW_, false, KS><<<grid, NW_ * 64, 0, s>>>(P)
-    if constexpr (KS != KT) {
-        if (pl.NT == 1) P1A_DEC(1, 8);
-        else P1A_DEC(2, 8);
-    } else if constexpr (big_tiles) {
-        if (sb) dec_mfma_k<KT, D, 1, 4, true><<<grid, 256, 0, s>>>(P);
-        else if (pl.NT == 1) P1A_DEC(1, 4);
-        else P1A_DEC(2, 4);
-    } else {
-        if (sb) dec_mfma_k<KT, D, 1, 8, true><<<grid, 512, 0, s>>>(P);
-        else if (pl.NT == 1) P1A_DEC(1, 8);
-        else P1A_DEC(2, 8);
-    }
+    const dim3 grid(pl.nsplit * c.Hkv, groups);
+    // The list (see dec_mfma_k) costs a workgroup some 0.2 us before its first request. Where two workgroups share a compute unit that hides,
+    // and every call of several sequences takes it (110 calls of 2 ... 32 sequences drawn over 4 ... 131072 keys, D = 256 and f16:
+    // 0.98 - 1.6 times as fast, 1.1 in the mean). Where one has a unit to itself (two column tiles, staged tiles) it shows: calls of
+    // four sequences and more whose page-table rows cannot hold the keys that half of the streams begin with (8 x 4 rows of 300
+    // ... 5000 keys, q8_0, 24 / 4 heads of 256, two layers 72.8 -> 62.1 us, 16 of 300 ... 5000, 32 / 8 of 128 104 -> 93; with every
+    // stream live 8 of 18797, q8_0, 24 / 4 of 128, four layers would go from 349 to 360).
+    const bool list = a.pos_rows && groups > 1 && (sb || (groups >= 4 && 2LL * c.n_ctx <= (long long) pl.nsplit * 32 * pl.NW));
+    long long nq = ((long long) nseq * pl.nsplit + 7) / 8;   // streams there could be, in eights
+    // More than 16 workgroups for every compute unit - 32 sequences - and most would find nothing to do, at 0.5 us for every 1000 of
+    // them: that many walk the list (32 sequences of 256 keys, q8_0, 24 / 4 heads of 256, two layers: 61 us, 49.5 with a workgroup
+    // for every stream, 43 so; of 300 ... 5000 99, 94.6, 90.5; f16, 32 / 8 of 128, 32 of 1024 91, 95, 89). Fewer would lose more where
+    // all streams are live (16 of 20000: 313, 304 with one workgroup a stream, 333 with two).
+    const long long most = 16LL * (a.cus > 0 ? a.cus : 256) / (8 * inner);
+    const bool loop = list && sb && nq > most;
+    if (loop) nq = most > 1 ? most : 1;
+    const unsigned lgrid = (unsigned) (8 * inner * nq);
+#define P1A_DEC(NT_, NW_, SB_) do { if (list) dec_mfma_k<KT, D, NT_, NW_, SB_, KS | LIST_><<<lgrid, NW_ * 64, 0, s>>>(P); else dec_mfma_k<KT, D, NT_, NW_, SB_, KS><<<grid, NW_ * 64, 0, s>>>(P); } while (0)
+    constexpr int NW = big_tiles ? 4 : 8;
+    if (pl.NT == 2) P1A_DEC(2, NW, false);
+    else if constexpr (KS != KT) P1A_DEC(1, NW, false);
+    else if (loop) dec_mfma_k<KT, D, 1, NW, true, KS | LIST_ | LOOP_><<<lgrid, NW * 64, 0, s>>>(P);
+    else if (sb) P1A_DEC(1, NW, true);
+    else P1A_DEC(1, NW, false);
 #undef P1A_DEC
     return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
 }

@@ -396,3 +396,45 @@ def test_staged_tiles_for_small_heads(p1a, kv_type, Hq, Hkv, D):
     for t in range(4):
         one = run_decode(p1a, pool.dev_seq(int(rtab[t] // pool.maxp)), q[t:t + 1], 1, int(pos[t]), Hq, scale, gate=gate[t:t + 1])
         assert np.array_equal(one[0], out[t].cpu().numpy()), t
+
+
+MIXED = [1, 255, 256, 257, 2304, 0, 700, 9000]                 # edges of a unit, an idle slot, more than every stream once (Hkv = 8)
+
+
+@pytest.mark.parametrize("kv_type,Hq,Hkv,D,psh,lens,rows", [
+    (O.KV_Q8_0, 24, 4, 256, 8, [300, 17000], 1), (O.KV_Q8_0, 24, 4, 256, 8, MIXED[:5], 1), (O.KV_Q4_0, 12, 4, 256, 8, MIXED[:4], 5),
+    (O.KV_F16, 16, 8, 128, 4, MIXED, 1), (O.KV_F16, 16, 8, 128, 4, MIXED[:3], 3), (O.KV_F16, 8, 8, 64, 6, MIXED + [3], 1),
+    (O.KV_F16, 16, 8, 128, 4, 2 * MIXED + [40], 1), (O.KV_F16, 8, 8, 64, 6, 4 * MIXED[:6], 1), (O.KV_F16, 8, 8, 64, 6, [4200 + 9 * i for i in range(32)], 1),
+    (O.KV_F16, 20, 5, 64, 6, 4 * MIXED[:7], 1), (O.KV_F16, 8, 8, 256, 6, 3 * MIXED[:7], 1), (O.KV_Q8_0, 8, 8, 64, 6, 4 * MIXED[:5], 1),
+    (O.KV_Q8_0, 16, 8, 128, 6, 2 * MIXED[:7], 2), (O.KV_Q8_0, 24, 4, 256, 8, MIXED[:5], 4), (O.KV_F16, 16, 4, 64, 6, MIXED[:4], 8),
+    (O.KV_F16, 16, 2, 64, 6, MIXED[:4], 8)])
+def test_rows_of_sequences_of_any_length(p1a, kv_type, Hq, Hkv, D, psh, lens, rows):
+    """Sequences of no key, one, a unit more or less and more than all streams hold once, in calls of every way the streams that hold
+    keys are found: up to 4, 7, 8, 16 and 32 rows, a number that is no multiple of eight, several rows and row groups a sequence,
+    head counts that are no power of two, workgroups that take one stream (all builds) and several (17 sequences and more); the
+    32 sequences of 4200 keys go round the list more than once. Every row == the row of the sequence's own call, bit for bit."""
+    n, scale, ps = len(lens), D ** -0.5, 1 << psh
+    g = torch.Generator(device="cuda").manual_seed(n * 1000 + rows)
+    need = [-(-max(x, 1) // ps) + 1 for x in lens]
+    maxp = max(need)
+    order = torch.randperm(sum(need), generator=g, device="cuda").to(torch.int32)
+    tab = torch.zeros(n * maxp, dtype=torch.int32, device="cuda")
+    for s in range(n):
+        tab[s * maxp:s * maxp + need[s]] = order[sum(need[:s]):sum(need[:s + 1])]
+    c = p1a.KVCache.paged(kv_type, Hkv, D, psh, sum(need), tab, maxp)
+    for s, x in enumerate(lens):
+        if x:
+            p1a.kv_append(c.slot(s, maxp), torch.randn((x, Hkv, D), generator=g, device="cuda"), torch.randn((x, Hkv, D), generator=g, device="cuda"), 0, x)
+    T = n * rows
+    q, gate = torch.randn((T, Hq, D), generator=g, device="cuda"), torch.randn((T, Hq, D), generator=g, device="cuda")
+    pos = [max(x - rows, -1) + r if x >= rows else x - 1 for x in lens for r in range(rows)]
+    rtab = torch.tensor([s * maxp for s in range(n) for _ in range(rows)], dtype=torch.int32, device="cuda")
+    out = torch.full((T, Hq, D), 7.0, device="cuda")
+    p1a.attn_decode_rows(q, c.with_rows(rtab), out, T, torch.tensor(pos, dtype=torch.int32, device="cuda"), Hq, scale, gate=gate, rows_per_seq=rows)
+    one = torch.empty((1, Hq, D), device="cuda")
+    for t in range(T):
+        if pos[t] < 0:
+            assert torch.isnan(out[t]).all()
+            continue
+        p1a.attn_decode(q[t:t + 1], c.slot(t // rows, maxp), one, 1, pos[t], Hq, scale, gate=gate[t:t + 1])
+        assert torch.equal(out[t:t + 1], one), (t, pos[t])
