@@ -97,6 +97,7 @@ struct pf_params {
     int nblk;     // row blocks (4 rpw rows) of a kv head
     int nbg;      // groups of row blocks
     int bpg;      // blocks of a group
+    int turn_a, turn_b;   // slots of an XCD taken in reverse order
     int run;      // key splits: consecutive workgroups of an XCD (0: groups in turn)
     // key splits: with nks > 1 workgroup (block, kv head, ks) walks its share of the block's tiles and leaves an unnormalised
     // partial (O relative to m, and (m, l)) per row in part_o [T*Hq][nks][D] / part_ml [T*Hq][nks][2] for the merge
@@ -270,7 +271,9 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
     // blockIdx.x -> (group of row blocks, kv head, block of the group): the blocks of a group share an XCD. Groups are dealt to
     // the XCDs in turn; with key splits a unit is (key split, kv head) with all of its row blocks, and an XCD may take a run of
     // `run` consecutive workgroups instead of whole units
-    const int id = blockIdx.x, xcd = id & 7, slot = id >> 3;
+    const int id = blockIdx.x, xcd = id & 7;
+    int slot = id >> 3;
+    if constexpr (!PAIR) { if (slot >= P.turn_a && slot < P.turn_b) slot = P.turn_a + P.turn_b - 1 - slot; }
     const int lin = P.run ? xcd * P.run + slot : ((slot / P.bpg) * 8 + xcd) * P.bpg + slot % P.bpg;
     const int vunit = lin / P.bpg, hh = lin - vunit * P.bpg;
     const int nunits = P.nbg * P.Hkv;
@@ -944,7 +947,17 @@ int launch_pf_g(const pf_params & P, hipStream_t s) {
     }
     const int units = P.nbg * P.Hkv * P.nks;
     const int slots = P.run ? P.run : ((units + 7) / 8) * P.bpg;
-    prefill_k<KT, D, GROUPED, DMA><<<slots * 8, NTHR, lds, s>>>(P);
+    pf_params Q = P;
+    Q.turn_a = Q.turn_b = 0;
+    // Two workgroups to a compute unit, which an XCD deals them to in turn: the unit of slot s also gets slot s + 32. Longest blocks first
+    // would give it two long ones (63 blocks of 1 ... 32 tiles: 32 + 16 ... 17 + 1 tiles); the second round is taken in reverse
+    // (33 each). First 2003 tokens, 32 / 8 heads of 128, f16, prep included 85.0 -> 81.2 us, 24 / 4 of 64 37.1 -> 34.5; what fits one round or
+    // takes many is as it was.
+    if (pf_solo(D, DMA) && P.nks == 1) {
+        const int per = std::max(cu_count() / 8, 1);          // compute units of an XCD
+        if (slots > per) { Q.turn_a = per; Q.turn_b = std::min(2 * per, slots); }
+    }
+    prefill_k<KT, D, GROUPED, DMA><<<slots * 8, NTHR, lds, s>>>(Q);
     return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
 }
 template <uint32_t KT, int D>
