@@ -160,4 +160,88 @@ int launch_stream_read(const void * src, size_t bytes, hipStream_t s);   // benc
 
 void set_error(const char * fmt, ...);
 
+// ---- wave-uniform values, scalar loads ----
+__device__ __forceinline__ int rfl(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ size_t rfl64(size_t x) {
+    const uint32_t lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) x);
+    const uint32_t hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (x >> 32));
+    return ((size_t) hi << 32) | lo;
+}
+typedef int i8 __attribute__((ext_vector_type(8)));
+typedef int i8_a4 __attribute__((ext_vector_type(8), aligned(4)));
+// A page-table entry through the scalar cache: a load from the constant address space at a wave-uniform address is an
+// s_load_dword, and the compiler itself places the wait for it before the first use of the value (a hand-written
+// s_load whose result the compiler may copy before a hand-written wait is a race). The table does not change while a
+// kernel runs.
+__device__ __forceinline__ int sload_i32(const int32_t * p) {
+    return *reinterpret_cast<const __attribute__((address_space(4))) int32_t *>(rfl64((size_t) p));
+}
+__device__ __forceinline__ i8 sload_i8(const int32_t * p) { return *reinterpret_cast<const __attribute__((address_space(4))) i8_a4 *>(rfl64((size_t) p)); }
+__device__ __forceinline__ void put_lane(int & v, int x, int lane) { asm("v_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(x), "i"(lane)); }
+
+// ---- calls of several sequences: the streams that hold keys ----
+// The streams of a call's sequences that hold keys, those of two units and more (A) ahead of those of one (B): lane r (of the first 32)
+// gets how many the sequences up to and including row r's have, A in the low half and B in the high one. The positions come
+// through the scalar cache: a vector load would queue up behind the tiles that the other workgroup of the compute unit has asked
+// for (16 sequences of 20000 keys, 24 / 4 heads of 256, q8_0, two layers: 323 us, 317 so). rt: row r's page-table row, for T < 8.
+// RPS: rows of a sequence (rps_magic = 65536 / RPS + 1); U: positions of a unit
+template <int U> __device__ __forceinline__ uint32_t live_streams(const int32_t * pos_rows, const int32_t * rtab_, int T, int RPS, int rps_magic, int nsplit, int lane, int & rt) {
+    int pr = 0;
+    rt = 0;
+    auto single = [&](auto n_tag) {   // (rows past the last: that one once more)
+        constexpr int N = decltype(n_tag)::value;
+        int v[N], w[N];
+        const int32_t * rtab = rtab_ ? rtab_ : pos_rows;
+#pragma unroll
+        for (int k = 0; k < N; ++k) { v[k] = sload_i32(pos_rows + min(k, T - 1)); w[k] = sload_i32(rtab + min(k, T - 1)); }
+#pragma unroll
+        for (int k = 0; k < N; ++k) { put_lane(pr, v[k], k); put_lane(rt, w[k], k); }
+    };
+    if (T <= 4) single(std::integral_constant<int, 4>{});
+    else if (T < 8) single(std::integral_constant<int, 8>{});
+    else {
+        i8 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = sload_i8(pos_rows + min(8 * k, T - 8));   // (the last eight once more where there are none)
+#pragma unroll
+        for (int k = 0; k < 16; ++k) put_lane(pr, v[k >> 3][k & 7], k);
+        if (T > 16) {
+#pragma unroll
+            for (int k = 16; k < 32; ++k) put_lane(pr, v[k >> 3][k & 7], k);
+        }
+        // (rows T - 8 .. T - 1 are in eight lanes from a multiple of eight on)
+        if (T & 7) pr = __builtin_amdgcn_ds_bpermute(4 * (lane < (T & ~7) ? lane : lane + 8 - (T & 7)), pr);
+    }
+    int n = lane < T && pr >= 0 ? pr / U + 1 : 0;              // units
+    if (RPS > 1) {                                           // the most of a sequence's rows, in its first one
+        const int n1 = n;
+        for (int k = 1; k < RPS; ++k) n = max(n, __builtin_amdgcn_ds_bpermute(4 * (lane + k), n1));
+        if (lane - (int) ((uint32_t) lane * (uint32_t) rps_magic >> 16) * RPS) n = 0;
+    }
+    const int na = min(max(n - nsplit, 0), nsplit);
+    int u = na | ((min(n, nsplit) - na) << 16);
+    // sums over the lanes up to this one
+    u += __builtin_amdgcn_update_dpp(0, u, 0x111, 0xf, 0xf, true);
+    u += __builtin_amdgcn_update_dpp(0, u, 0x112, 0xf, 0xf, true);
+    u += __builtin_amdgcn_update_dpp(0, u, 0x114, 0xf, 0xf, true);
+    u += __builtin_amdgcn_update_dpp(0, u, 0x118, 0xf, 0xf, true);
+    u += __builtin_amdgcn_update_dpp(0, u, 0x142, 0xa, 0xf, false);
+    return (uint32_t) u;
+}
+// number q of that list (q_a of them are A): the first row of its sequence, and the stream
+struct stream_at { int first, split; };
+__device__ __forceinline__ stream_at pick_stream(uint32_t u_sum, int q, int q_a, int lane) {
+    const bool in_a = q < q_a;
+    const uint32_t upto = in_a ? u_sum & 0xffff : u_sum >> 16;
+    const int at = in_a ? q : q - q_a;                         // place in its half of the list
+    stream_at r;
+    r.first = __popcll(__ballot(lane < 32 && (int) upto <= at));
+    r.split = at - (r.first ? __builtin_amdgcn_readlane((int) upto, r.first - 1) : 0);
+    if (!in_a) {                                               // (behind the sequence's streams of two units)
+        const int a1 = __builtin_amdgcn_readlane((int) (u_sum & 0xffff), r.first), a0 = r.first ? __builtin_amdgcn_readlane((int) (u_sum & 0xffff), r.first - 1) : 0;
+        r.split += a1 - a0;
+    }
+    return r;
+}
+
 }   // namespace p1a

@@ -87,17 +87,9 @@ struct dec_params {
 };
 
 __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) { return __builtin_amdgcn_perm(hi, lo, sel); }
-__device__ __forceinline__ int rfl(int x) { return __builtin_amdgcn_readfirstlane(x); }
-__device__ __forceinline__ size_t rfl64(size_t x) {
-    const uint32_t lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) x);
-    const uint32_t hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (x >> 32));
-    return ((size_t) hi << 32) | lo;
-}
 
 // 4 int8 codes (one dword) -> (code * d) as two packed f16 pairs, returned as raw dwords so MFMA operands are built in place
 struct u2 { uint32_t lo, hi; };
-typedef int i8 __attribute__((ext_vector_type(8)));
-typedef int i8_a4 __attribute__((ext_vector_type(8), aligned(4)));
 typedef const __attribute__((address_space(4))) uint64_t * kargs;   // a kernel's arguments, as words
 __device__ __forceinline__ u2 deq4(uint32_t w, h2 d01, h2 d23) {
     const h2 off = {(half_t) 1152, (half_t) 1152};
@@ -122,7 +114,6 @@ __device__ __forceinline__ int lane_id() {
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
     return l;
 }
-__device__ __forceinline__ void put_lane(int & v, int x, int lane) { asm("v_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(x), "i"(lane)); }
 
 // the maximum over the four lanes that share (lane & 15): the two 16-lane rows of each half, then the two halves
 __device__ __forceinline__ float max_over_groups(float m) { return max_swap32(max_swap16(m)); }
@@ -163,64 +154,6 @@ template <int NR> __device__ __forceinline__ void wait_tiles(int newer) {
     else if (newer == 2) wait_vm_imm<2 * NR>();
     else wait_vm_imm<3 * NR>();
 }
-// A page-table entry through the scalar cache: a load from the constant address space at a wave-uniform address is an
-// s_load_dword, and the compiler itself places the wait for it before the first use of the value (a hand-written
-// s_load whose result the compiler may copy before a hand-written wait is a race). The table does not change while a
-// kernel runs.
-__device__ __forceinline__ int sload_i32(const int32_t * p) {
-    return *reinterpret_cast<const __attribute__((address_space(4))) int32_t *>(rfl64((size_t) p));
-}
-__device__ __forceinline__ i8 sload_i8(const int32_t * p) { return *reinterpret_cast<const __attribute__((address_space(4))) i8_a4 *>(rfl64((size_t) p)); }
-
-// The streams of a call's sequences that hold keys, those of two units and more (A) ahead of those of one (B): lane r (of the first 32)
-// gets how many the sequences up to and including row r's have, A in the low half and B in the high one. The positions come
-// through the scalar cache: a vector load would queue up behind the tiles that the other workgroup of the compute unit has asked
-// for (16 sequences of 20000 keys, 24 / 4 heads of 256, q8_0, two layers: 323 us, 317 so). rt: row r's page-table row, for T < 8.
-template <int U> __device__ __forceinline__ uint32_t live_streams(const dec_params & P, int lane, int & rt) {
-    const int T = P.T;
-    int pr = 0;
-    rt = 0;
-    auto single = [&](auto n_tag) {   // (rows past the last: that one once more)
-        constexpr int N = decltype(n_tag)::value;
-        int v[N], w[N];
-        const int32_t * rtab = P.pg.rtab ? P.pg.rtab : P.pos_rows;
-#pragma unroll
-        for (int k = 0; k < N; ++k) { v[k] = sload_i32(P.pos_rows + min(k, T - 1)); w[k] = sload_i32(rtab + min(k, T - 1)); }
-#pragma unroll
-        for (int k = 0; k < N; ++k) { put_lane(pr, v[k], k); put_lane(rt, w[k], k); }
-    };
-    if (T <= 4) single(std::integral_constant<int, 4>{});
-    else if (T < 8) single(std::integral_constant<int, 8>{});
-    else {
-        i8 v[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = sload_i8(P.pos_rows + min(8 * k, T - 8));   // (the last eight once more where there are none)
-#pragma unroll
-        for (int k = 0; k < 16; ++k) put_lane(pr, v[k >> 3][k & 7], k);
-        if (T > 16) {
-#pragma unroll
-            for (int k = 16; k < 32; ++k) put_lane(pr, v[k >> 3][k & 7], k);
-        }
-        // (rows T - 8 .. T - 1 are in eight lanes from a multiple of eight on)
-        if (T & 7) pr = __builtin_amdgcn_ds_bpermute(4 * (lane < (T & ~7) ? lane : lane + 8 - (T & 7)), pr);
-    }
-    int n = lane < T && pr >= 0 ? pr / U + 1 : 0;              // units
-    if (P.RPS > 1) {                                           // the most of a sequence's rows, in its first one
-        const int n1 = n;
-        for (int k = 1; k < P.RPS; ++k) n = max(n, __builtin_amdgcn_ds_bpermute(4 * (lane + k), n1));
-        if (lane - (int) ((uint32_t) lane * (uint32_t) P.rps_magic >> 16) * P.RPS) n = 0;
-    }
-    const int na = min(max(n - P.nsplit, 0), P.nsplit);
-    int u = na | ((min(n, P.nsplit) - na) << 16);
-    // sums over the lanes up to this one
-    u += __builtin_amdgcn_update_dpp(0, u, 0x111, 0xf, 0xf, true);
-    u += __builtin_amdgcn_update_dpp(0, u, 0x112, 0xf, 0xf, true);
-    u += __builtin_amdgcn_update_dpp(0, u, 0x114, 0xf, 0xf, true);
-    u += __builtin_amdgcn_update_dpp(0, u, 0x118, 0xf, 0xf, true);
-    u += __builtin_amdgcn_update_dpp(0, u, 0x142, 0xa, 0xf, false);
-    return (uint32_t) u;
-}
-
 // SB ("single-buffered"): one K and one V slot per wave instead of two, so that two workgroups fit a CU's LDS (and register
 // file: 128 registers per lane) - for calls of many workgroups, where a second resident workgroup covers the start-up,
 // the fold and the memory round trips of the first. Tile t + 1 of K is then requested once the products with tile t of K
@@ -290,7 +223,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
         if (LOOP) q_step = (P.inner_sh >= 0 ? (int) (gridDim.x >> 3) >> P.inner_sh : (int) (gridDim.x >> 3) / inner) * 8;
         gsub = P.GPS == 1 ? 0 : in / P.Hkv;
         hg = in - gsub * P.Hkv;
-        u_sum = live_streams<U>(P, lane, rt_lanes);
+        u_sum = live_streams<U>(P.pos_rows, P.pg.rtab, P.T, P.RPS, P.rps_magic, P.nsplit, lane, rt_lanes);
         const uint32_t all = (uint32_t) __builtin_amdgcn_readlane((int) u_sum, 31);
         q_a = (int) (all & 0xffff);
         q_end = q_a + (int) (all >> 16);
@@ -324,16 +257,9 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     };
     int split, row0;
     if constexpr (LIST) {
-        const bool in_a = q < q_a;
-        const uint32_t upto = in_a ? u_sum & 0xffff : u_sum >> 16;
-        const int at = in_a ? q : q - q_a;                     // place in its half of the list
-        const int first = __popcll(__ballot(lane < 32 && (int) upto <= at));   // the first row of the sequence
-        split = at - (first ? __builtin_amdgcn_readlane((int) upto, first - 1) : 0);
-        if (!in_a) {                                           // (behind the sequence's streams of two units)
-            const int a1 = __builtin_amdgcn_readlane((int) (u_sum & 0xffff), first), a0 = first ? __builtin_amdgcn_readlane((int) (u_sum & 0xffff), first - 1) : 0;
-            split += a1 - a0;
-        }
-        row0 = first + gsub * P.RG;
+        const stream_at at = pick_stream(u_sum, q, q_a, lane);
+        split = at.split;
+        row0 = at.first + gsub * P.RG;
         if (row0 >= P.T) {                                    // (a last sequence of fewer rows)
             if (next_item()) continue;
             return;

@@ -50,14 +50,9 @@ struct any_params {
     float qscale;     // softmax scale * log2(e)
     int nsplit;
     int SQ;           // rows of a sequence (1 << 30: all rows are one sequence's)
+    int T, RPS, rps_magic, inner;   // list: rows, those of a sequence (at most T), 65536 / RPS + 1, workgroups of a stream
 };
 
-// a load through the scalar cache at a wave-uniform address (page tables and positions do not change while a kernel runs)
-__device__ __forceinline__ int sload_i32(const int32_t * p) {
-    const size_t a = (size_t) p;
-    const uint32_t lo = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) a), hi = (uint32_t) __builtin_amdgcn_readfirstlane((int) (uint32_t) (a >> 32));
-    return *reinterpret_cast<const __attribute__((address_space(4))) int32_t *>(((size_t) hi << 32) | lo);
-}
 template <typename T> __device__ __forceinline__ T ld(const char * p) {   // (any alignment)
     T x;
     __builtin_memcpy(&x, p, sizeof x);
@@ -80,8 +75,9 @@ __device__ __forceinline__ float below(float x) { return asf(__builtin_elementwi
 // two values to f16, towards zero
 __device__ __forceinline__ h2 cut2(float x, float y) { return __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(x, y)); }
 
-template <uint32_t KT, int NB, int NW>
-__global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
+// LIST: blockIdx.x counts the streams that hold keys (live_streams), the others behind them
+template <uint32_t KT, int NB, int NW, bool LIST>
+__device__ __forceinline__ void any_body(const any_params & P) {
     constexpr bool F16 = KT == P1A_KV_F16, Q8 = KT == P1A_KV_Q8_0;
     constexpr int OS = NB * 32 + 4;                          // floats per parked column (padded)
     constexpr int PC = 8;                                     // columns parked at a time
@@ -91,21 +87,42 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
     constexpr int D = NB * 32;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g = lane >> 4;
-    // the kv heads of one split stream share cache lines: given the same index mod 8 they sit on one XCD, and
-    // sequence r of a batch starts on XCD r mod 8 (short ones only fill the first streams: p1a_decode.hip)
-    int split, hk;
-    if ((P.nsplit & 7) == 0) {
-        const int i = blockIdx.x, j = i >> 3, jq = j / P.Hkv;
-        hk = j - jq * P.Hkv;
-        split = jq * 8 + ((i - (int) blockIdx.z / P.SQ) & 7);
-    } else {
-        split = blockIdx.x / P.Hkv;
-        hk = blockIdx.x - split * P.Hkv;
-    }
+    // the kv heads of one split stream share cache lines: given the same index mod 8 they sit on one XCD, and sequence r of a batch
+    // starts on XCD r mod 8 (short ones only fill the first streams; the reasons for that and for the list are p1a_decode.hip's)
     constexpr int U = 16 * NW;
-    const int t = blockIdx.z, col0 = blockIdx.y * 16, R = min(16, P.GQA - col0);
+    int split, hk, t, ct, rt = 0;
+    const bool has_rt = P.pg.pt && P.pg.rtab;
+    if constexpr (LIST) {
+        const int i = blockIdx.x, j = i >> 3, jq = j / P.inner, q = jq * 8 + (i & 7);
+        int in = j - jq * P.inner, rt_lanes;
+        const int rest = in / P.Hkv, nct = (P.GQA + 15) / 16;
+        hk = in - rest * P.Hkv;
+        const int sub = rest / nct;
+        ct = rest - sub * nct;
+        const uint32_t u_sum = live_streams<U>(P.pos_rows, P.pg.rtab, P.T, P.RPS, P.rps_magic, P.nsplit, lane, rt_lanes);
+        const uint32_t all = (uint32_t) __builtin_amdgcn_readlane((int) u_sum, 31);
+        const int q_a = (int) (all & 0xffff);
+        if (q >= q_a + (int) (all >> 16)) return;
+        const stream_at at = pick_stream(u_sum, q, q_a, lane);
+        split = at.split;
+        t = at.first + sub;
+        if (t >= P.T) return;                                 // (a last sequence of fewer rows)
+        if (has_rt) rt = P.T < 8 ? __builtin_amdgcn_readlane(rt_lanes, t / P.RG * P.RG) : sload_i32(P.pg.rtab + t / P.RG * P.RG);
+    } else {
+        if ((P.nsplit & 7) == 0) {
+            const int i = blockIdx.x, j = i >> 3, jq = j / P.Hkv;
+            hk = j - jq * P.Hkv;
+            split = jq * 8 + ((i - (int) blockIdx.z / P.SQ) & 7);
+        } else {
+            split = blockIdx.x / P.Hkv;
+            hk = blockIdx.x - split * P.Hkv;
+        }
+        t = blockIdx.z;
+        ct = blockIdx.y;
+        if (has_rt) rt = sload_i32(P.pg.rtab + (P.pos_rows ? (t / P.RG) * P.RG : 0));
+    }
+    const int col0 = ct * 16, R = min(16, P.GQA - col0);
     const size_t row0 = (size_t) t * P.Hq + (size_t) hk * P.GQA + col0;   // the output row of column 0
-    const int rt = P.pg.pt && P.pg.rtab ? sload_i32(P.pg.rtab + (P.pos_rows ? (t / P.RG) * P.RG : 0)) : 0;
     const int n = (P.pos_rows ? sload_i32(P.pos_rows + t) : (P.p0_dev ? sload_i32(P.p0_dev) : P.p0) + t) + 1;
     const int32_t * ptab = P.pg.pt ? P.pg.pt + rt : nullptr;
     if (split * U >= n) {                                     // no key in this stream (with pos_rows the merge does not look at it)
@@ -373,9 +390,19 @@ __global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) {
     }
 }
 
-template <uint32_t KT> void launch_kt(const any_params & P, dim3 grid, hipStream_t s) {
+template <uint32_t KT, int NB, int NW>
+__global__ void __launch_bounds__(NW * 64) dec_any_k(const any_params P) { any_body<KT, NB, NW, false>(P); }
+template <uint32_t KT, int NB, int NW>
+__global__ void __launch_bounds__(NW * 64) dec_list_any_k(const any_params P) { any_body<KT, NB, NW, true>(P); }
+
+template <uint32_t KT, int NB> void launch_nb(const any_params & P, bool list, dim3 grid, hipStream_t s) {
+    constexpr int NW = NB <= 8 ? 8 : 4;
+    if constexpr (NB <= 8) { if (list) { dec_list_any_k<KT, NB, NW><<<grid, NW * 64, 0, s>>>(P); return; } }
+    dec_any_k<KT, NB, NW><<<grid, NW * 64, 0, s>>>(P);
+}
+template <uint32_t KT> void launch_kt(const any_params & P, bool list, dim3 grid, hipStream_t s) {
     switch (P.D / 32) {
-#define P1A_ANY(NB_) case NB_: dec_any_k<KT, NB_, NB_ <= 8 ? 8 : 4><<<grid, NB_ <= 8 ? 512 : 256, 0, s>>>(P); break
+#define P1A_ANY(NB_) case NB_: launch_nb<KT, NB_>(P, list, grid, s); break
         P1A_ANY(1); P1A_ANY(2); P1A_ANY(3); P1A_ANY(4); P1A_ANY(5); P1A_ANY(6); P1A_ANY(7); P1A_ANY(8);
         P1A_ANY(9); P1A_ANY(10); P1A_ANY(11); P1A_ANY(12); P1A_ANY(13); P1A_ANY(14); P1A_ANY(15); P1A_ANY(16);
 #undef P1A_ANY
@@ -393,10 +420,20 @@ int launch_decode_any(const p1a_kv & c, const decode_args & a, int rows_per_grou
     P.p0 = a.p0; P.p0_dev = a.p0_dev; P.pos_rows = a.pos_rows; P.RG = rows_per_group;
     P.Hq = a.Hq; P.Hkv = c.Hkv; P.GQA = a.Hq / c.Hkv; P.D = c.D; P.qscale = a.scale * 1.4426950408889634f; P.nsplit = nsplit;
     P.SQ = a.rows_per_seq;
-    const dim3 grid(nsplit * c.Hkv, (P.GQA + 15) / 16, a.T);
-    if (c.type == P1A_KV_F16) launch_kt<P1A_KV_F16>(P, grid, s);
-    else if (c.type == P1A_KV_Q8_0) launch_kt<P1A_KV_Q8_0>(P, grid, s);
-    else launch_kt<P1A_KV_Q4_0>(P, grid, s);
+    P.T = a.T;
+    P.RPS = a.rows_per_seq < a.T ? a.rows_per_seq : a.T;
+    P.rps_magic = 65536 / P.RPS + 1;
+    const int nct = (P.GQA + 15) / 16, nseq = (a.T + P.RPS - 1) / P.RPS;
+    P.inner = c.Hkv * nct * P.RPS;
+    // Four to 16 rows of several sequences: calls drawn over 4 ... 7600 keys are 0.95 - 1.27 times as fast, 1.1 in the mean (4 of 616, q8_0,
+    // 16 / 4 heads of 96, four layers 65.6 -> 57.9 us, 8 of 211 ... 3391, 4 / 1 of 192 86.7 -> 68.4). With 32 rows a grid of 8192 workgroups is mostly
+    // empty and each reads all positions before it knows (f16, 24 / 4 of 192, 8 x 4 rows of 11 ... 188 keys 37 us, 48 with the list); with two
+    // there is little to spread (16 / 2 of 96, 15 ... 246 keys 19.8 and 21.9).
+    const bool list = a.pos_rows && nseq > 1 && a.T >= 4 && a.T <= 16 && c.D <= 256;
+    const dim3 grid = list ? dim3((unsigned) (((long long) nseq * nsplit + 7) / 8 * 8 * P.inner)) : dim3(nsplit * c.Hkv, nct, a.T);
+    if (c.type == P1A_KV_F16) launch_kt<P1A_KV_F16>(P, list, grid, s);
+    else if (c.type == P1A_KV_Q8_0) launch_kt<P1A_KV_Q8_0>(P, list, grid, s);
+    else launch_kt<P1A_KV_Q4_0>(P, list, grid, s);
     return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
 }
 
