@@ -438,3 +438,24 @@ def test_long_contexts_of_few_row_blocks(p1a, kv_type, Hq, Hkv, D, p0, T):
     for o in outs[1:]:
         assert np.array_equal(o, outs[0])
     check(outs[0], O.attn_rows(pool.host_seq(0), q, (p0 + np.arange(T)).astype(np.int32), Hq, D ** -0.5, gate=gate), f"few blocks {kv_type} {Hq}/{Hkv}/{D} p0 {p0} T {T}")
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,T,p0", [(32, 8, 128, 1030, 0), (16, 8, 64, 1100, 7), (24, 4, 64, 2003, 0), (8, 8, 128, 4100, 50), (8, 8, 64, 4300, 0)])
+def test_second_round_in_reverse(p1a, Hq, Hkv, D, T, p0):
+    """Heads of 64 and 128 in calls of one row block past what a workgroup to every compute unit takes up to more than two of them
+    do: the second round's blocks are taken in reverse. Every row against fp32 attention over the f16 values the cache holds."""
+    n = p0 + T
+    g = torch.Generator(device="cuda").manual_seed(T)
+    k, v = torch.randn((n, Hkv, D), generator=g, device="cuda"), torch.randn((n, Hkv, D), generator=g, device="cuda")
+    q = torch.randn((T, Hq, D), generator=g, device="cuda")
+    c = p1a.KVCache.contiguous(O.KV_F16, (n + 15) & ~15, Hkv, D)
+    p1a.kv_append(c, k, v, 0, n)
+    out = torch.full((T, Hq, D), float("nan"), device="cuda")
+    p1a.attn_prefill(q, c, out, T, p0, Hq, D ** -0.5)
+    k, v = k.half().float(), v.half().float()
+    hidden = torch.arange(n, device="cuda")[None, :] > p0 + torch.arange(T, device="cuda")[:, None]
+    ref = torch.empty_like(out)
+    for h in range(Hq):
+        s = (q[:, h] @ k[:, h // (Hq // Hkv)].t().contiguous()) * D ** -0.5
+        ref[:, h] = torch.softmax(s.masked_fill(hidden, float("-inf")), -1) @ v[:, h // (Hq // Hkv)]
+    check(out.cpu().numpy(), ref.cpu().numpy(), f"second round D={D} T={T}")
