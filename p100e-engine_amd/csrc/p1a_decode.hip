@@ -1137,22 +1137,33 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hi
     // stream live 8 of 18797, q8_0, 24 / 4 of 128, four layers would go from 349 to 360).
     const bool list = a.pos_rows && groups > 1 && (sb || (groups >= 4 && 2LL * c.n_ctx <= (long long) pl.nsplit * 32 * pl.NW));
     long long nq = ((long long) nseq * pl.nsplit + 7) / 8;   // streams there could be, in eights
-    // More than 16 workgroups for every compute unit - 32 sequences - and most would find nothing to do, at 0.5 us for every 1000 of
-    // them: that many walk the list (32 sequences of 256 keys, q8_0, 24 / 4 heads of 256, two layers: 61 us, 49.5 with a workgroup
-    // for every stream, 43 so; of 300 ... 5000 99, 94.6, 90.5; f16, 32 / 8 of 128, 32 of 1024 91, 95, 89). Fewer would lose more where
-    // all streams are live (16 of 20000: 313, 304 with one workgroup a stream, 333 with two).
-    const long long most = 16LL * (a.cus > 0 ? a.cus : 256) / (8 * inner);
-    const bool loop = list && sb && nq > most;
+    // Where most workgroups would find nothing to do, at 0.5 us for every 1000 of them, fewer walk the list.
+    //   Two to a unit: more than 16 for every compute unit, i.e. 32 sequences (of 256 keys, q8_0, 24 / 4 heads of 256, two layers: 61 us, 49.5
+    //   with a workgroup for every stream, 43 so; of 300 ... 5000 99, 94.6, 90.5; f16, 32 / 8 of 128, 32 of 1024 91, 95, 89). Fewer would lose more where
+    //   all streams are live (16 of 20000: 313, 304 with one workgroup a stream, 333 with eight for every unit).
+    //   One to a unit: more than two for every compute unit; at least half of the streams are known to be empty there (start, a workgroup
+    //   for every stream, two for every unit: 8 x 4 rows of 300 ... 5000, q8_0, 24 / 4 of 256 73.6, 62.7, 56.5 us; 16 of 256, 32 / 8 of 128 53, 45, 39;
+    //   32 of 256 77, 71, 43; q4_0, 24 / 4 of 128, 16 of 60 ... 1500 58.5, 46.9, 40.3).
+    const long long most = (sb ? 16LL : 2LL) * (a.cus > 0 ? a.cus : 256) / (8 * inner);
+    constexpr bool can_loop_2 = !(KT == P1A_KV_Q4_0);   // (q4_0 with two column tiles has no register left for it)
+    const bool loop = list && nq > most && (pl.NT == 2 ? can_loop_2 : KS != KT || sb);
     if (loop) nq = most > 1 ? most : 1;
     const unsigned lgrid = (unsigned) (8 * inner * nq);
-#define P1A_DEC(NT_, NW_, SB_) do { if (list) dec_mfma_k<KT, D, NT_, NW_, SB_, KS | LIST_><<<lgrid, NW_ * 64, 0, s>>>(P); else dec_mfma_k<KT, D, NT_, NW_, SB_, KS><<<grid, NW_ * 64, 0, s>>>(P); } while (0)
-    constexpr int NW = big_tiles ? 4 : 8;
-    if (pl.NT == 2) P1A_DEC(2, NW, false);
-    else if constexpr (KS != KT) P1A_DEC(1, NW, false);
-    else if (loop) dec_mfma_k<KT, D, 1, NW, true, KS | LIST_ | LOOP_><<<lgrid, NW * 64, 0, s>>>(P);
-    else if (sb) P1A_DEC(1, NW, true);
-    else P1A_DEC(1, NW, false);
-#undef P1A_DEC
+    auto go = [&](auto nt, auto single, auto can_loop) {
+        constexpr int NT = decltype(nt)::value, NW = big_tiles ? 4 : 8;
+        constexpr bool SB = decltype(single)::value;
+        if constexpr (decltype(can_loop)::value) {
+            if (loop) { dec_mfma_k<KT, D, NT, NW, SB, KS | LIST_ | LOOP_><<<lgrid, NW * 64, 0, s>>>(P); return; }
+        }
+        if (list) dec_mfma_k<KT, D, NT, NW, SB, KS | LIST_><<<lgrid, NW * 64, 0, s>>>(P);
+        else dec_mfma_k<KT, D, NT, NW, SB, KS><<<grid, NW * 64, 0, s>>>(P);
+    };
+    constexpr std::true_type yes;
+    constexpr std::false_type no;
+    if (pl.NT == 2) go(std::integral_constant<int, 2>{}, no, std::bool_constant<can_loop_2>{});
+    else if constexpr (KS != KT) go(std::integral_constant<int, 1>{}, no, yes);
+    else if (sb) go(std::integral_constant<int, 1>{}, yes, yes);
+    else go(std::integral_constant<int, 1>{}, no, no);
     return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
 }
 
