@@ -2,6 +2,7 @@
 (src/fast/attn.cuh:34-70 of the reference tree): kv_append, kv_append_dev, attn_decode, attn_decode_dev,
 attn_decode_rows, attn_prefill; attn_prep is src/fast/fused.cuh:101-113."""
 import ctypes
+import importlib
 import os
 
 KV_F16, KV_Q4_0, KV_Q8_0 = 1, 2, 8
@@ -46,6 +47,21 @@ def lib_path():
 
 
 _lib = None
+_call = None      # the native side of the calls a step is made of (csrc/p1a_call.cpp)
+
+
+def _calls():
+    """Load _p1a_call.so (built with libp1a_attn.so) and hand it the library's entry points."""
+    global _call
+    if _call is None:
+        L = lib()
+        try:
+            m = importlib.import_module("._p1a_call", __package__)
+        except ImportError as e:
+            raise P1AError(f"_p1a_call.so is missing next to {lib_path()}: build it with `make -C p100e-engine_amd/csrc`") from e
+        m.bind(*(ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in ("p1a_attn_prep", "p1a_attn_decode_a16", "p1a_attn_prefill", "p1a_kv_append")), KVCache, _stream)
+        _call = m
+    return _call
 
 
 def lib():
@@ -255,7 +271,7 @@ class KVCache:
 
 def kv_append(c, k, v, p0, T):
     """src/fast/attn.cuh:37-38 of the reference: k, v [T][Hkv][D] f32 -> cache positions p0..p0+T-1."""
-    _check(lib().p1a_kv_append(ctypes.byref(c.struct()), _ptr(k), _ptr(v), p0, None, None, T, _stream()), "kv_append")
+    _check((_call or _calls()).append(c, k, v, p0, None, None, T), "kv_append")
 
 
 def kv_fill_random(c, p0, p1, seed):
@@ -265,13 +281,13 @@ def kv_fill_random(c, p0, p1, seed):
 
 def kv_append_dev(c, k, v, p0_dev, T):
     """src/fast/attn.cuh:58: the first position is read from device memory."""
-    _check(lib().p1a_kv_append(ctypes.byref(c.struct()), _ptr(k), _ptr(v), 0, _ptr(p0_dev), None, T, _stream()), "kv_append_dev")
+    _check((_call or _calls()).append(c, k, v, 0, p0_dev, None, T), "kv_append_dev")
 
 
 def kv_append_rows(c, k, v, pos_rows, T):
     """Cache-write half of attn_prep in device-position mode (src/fast/fused.cuh:101-113): row t -> pos_rows[t] of
     its own sequence (c.rtab)."""
-    _check(lib().p1a_kv_append(ctypes.byref(c.struct()), _ptr(k), _ptr(v), -1, None, _ptr(pos_rows), T, _stream()), "kv_append_rows")
+    _check((_call or _calls()).append(c, k, v, -1, None, pos_rows, T), "kv_append_rows")
 
 
 def attn_prep(qg, k, v, q_norm, k_norm, pos, q, gate, c, p0, T, Hq, n_rot, freq_base, eps, ldq=0, ldk=0, ldv=0, mrope=None):
@@ -284,24 +300,23 @@ def attn_prep(qg, k, v, q_norm, k_norm, pos, q, gate, c, p0, T, Hq, n_rot, freq_
                                          ctypes.byref(c.struct()), p0, T, Hq, n_rot, freq_base, eps, ldq, ldk, ldv,
                                          _ptr(mp), stride, s0, s1, s2, sect, _stream()), "attn_prep")
         return
-    _check(lib().p1a_attn_prep(_ptr(qg), _ptr(k), _ptr(v), _ptr(q_norm), _ptr(k_norm), _ptr(pos), _ptr(q), _ptr(gate), c.struct(), p0, T, Hq,
-                               n_rot, freq_base, eps, ldq, ldk, ldv, _stream()), "attn_prep")
+    _check((_call or _calls()).prep(qg, k, v, q_norm, k_norm, pos, q, gate, c, p0, T, Hq, n_rot, freq_base, eps, ldq, ldk, ldv), "attn_prep")
 
 
 def attn_decode(q, c, out, T, p0, Hq, scale, gate=None):
     """src/fast/attn.cuh:44."""
-    _check(lib().p1a_attn_decode(_ptr(q), ctypes.byref(c.struct()), _ptr(out), _ptr(gate), T, p0, None, None, 0, Hq, scale, _stream()), "attn_decode")
+    _check((_call or _calls()).decode(q, c, out, gate, None, T, p0, None, None, 0, Hq, scale), "attn_decode")
 
 
 def attn_decode_dev(q, c, out, T, p0_dev, max_n, Hq, scale, gate=None):
     """src/fast/attn.cuh:59-60 (max_n is accepted for signature parity; the grid never depends on the depth)."""
-    _check(lib().p1a_attn_decode(_ptr(q), ctypes.byref(c.struct()), _ptr(out), _ptr(gate), T, 0, _ptr(p0_dev), None, 0, Hq, scale, _stream()), "attn_decode_dev")
+    _check((_call or _calls()).decode(q, c, out, gate, None, T, 0, p0_dev, None, 0, Hq, scale), "attn_decode_dev")
 
 
 def attn_decode_rows(q, c, out, T, pos, Hq, scale, gate=None, rows_per_seq=1, qbuf=None):
     """src/fast/attn.cuh:64-65; rows_per_seq > 1: consecutive rows form verify blocks that share one KV read; qbuf: also
     emit the a16 activation buffer of the gated rows (src/fast/fused.cu:478-496)."""
-    _check(lib().p1a_attn_decode_a16(_ptr(q), ctypes.byref(c.struct()), _ptr(out), _ptr(gate), _ptr(qbuf), T, 0, None, _ptr(pos), rows_per_seq, Hq, scale, _stream()), "attn_decode_rows")
+    _check((_call or _calls()).decode(q, c, out, gate, qbuf, T, 0, None, pos, rows_per_seq, Hq, scale), "attn_decode_rows")
 
 
 def a16_bytes(T, n):
@@ -327,7 +342,7 @@ def prefill_key_splits(T, p0, Hq, Hkv=None):
 def attn_prefill(q, c, out, T, p0, Hq, scale, gate=None, scratch=None):
     """src/fast/attn.cuh:46-50 / src/fast/attn_fold.cuh:19-26."""
     nbytes = 0 if scratch is None else scratch.numel() * scratch.element_size()
-    _check(lib().p1a_attn_prefill(_ptr(q), ctypes.byref(c.struct()), _ptr(out), _ptr(gate), T, p0, Hq, scale, _ptr(scratch), nbytes, _stream()), "attn_prefill")
+    _check((_call or _calls()).prefill(q, c, out, gate, T, p0, Hq, scale, scratch, nbytes), "attn_prefill")
 
 
 def sigmoid_mul(x, g):

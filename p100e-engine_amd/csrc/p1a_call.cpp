@@ -1,0 +1,176 @@
+// The Python side of a call in native code: arguments -> the C ABI of include/p1a_attn.h. A one-row step of a small model is
+// bound by what the host does around its three launches, and half of what was not the launches was the ctypes call: 19
+// arguments converted one by one, a descriptor built field by field, a stream looked up from Python. The calls a step is made of
+// come here instead; arguments are taken as ctypes takes them (whole numbers cut to 32 bits, floats, None for a null pointer, anything
+// with data_ptr() as a device pointer), and the GIL is released around the call. One token of 4 heads of 64, prep and decode from Python:
+// 18.1 us with ctypes, 15.6 so (7.7 of them the C calls, 3.5 the caller's own indexing); two layers of 24 / 4 heads of 96 34.4 -> 29.2.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <cstdint>
+#include <cstring>
+
+#include "p1a_attn.h"
+
+namespace {
+
+PyObject * s_data_ptr, * s_struct, * s_field[11];
+const char * const FIELDS[11] = {"type", "n_ctx", "Hkv", "D", "k", "v", "pt", "rtab", "psh", "pstride", "_pt_off"};
+// set by bind(): the library's entry points, the class whose fields are read directly, and how the current stream is found
+decltype(&p1a_attn_prep) f_prep;
+decltype(&p1a_attn_decode_a16) f_decode;
+decltype(&p1a_attn_prefill) f_prefill;
+decltype(&p1a_kv_append) f_append;
+PyObject * kv_class, * stream_of;
+
+// (each reader does nothing once an error is set, so that the callers test for one at the end)
+int as_int(PyObject * o) {
+    if (PyErr_Occurred()) return 0;
+    if (PyFloat_Check(o)) { PyErr_SetString(PyExc_TypeError, "int expected instead of float instance"); return 0; }
+    return (int) (uint32_t) PyLong_AsUnsignedLongMask(o);
+}
+size_t as_size(PyObject * o) {
+    if (PyErr_Occurred()) return 0;
+    if (PyFloat_Check(o)) { PyErr_SetString(PyExc_TypeError, "int expected instead of float instance"); return 0; }
+    return (size_t) PyLong_AsUnsignedLongMask(o);
+}
+float as_float(PyObject * o) { return PyErr_Occurred() ? 0.f : (float) PyFloat_AsDouble(o); }
+void * address(PyObject * o) { return o == Py_None ? nullptr : (void *) (uintptr_t) as_size(o); }
+void * data_ptr(PyObject * t) {
+    if (PyErr_Occurred() || t == Py_None) return nullptr;
+    PyObject * r = PyObject_CallMethodNoArgs(t, s_data_ptr);
+    if (!r) return nullptr;
+    void * p = address(r);
+    Py_DECREF(r);
+    return p;
+}
+template <typename T> T * ptr(PyObject * t) { return (T *) data_ptr(t); }
+
+// the cache's descriptor as it is now: a KVCache's fields, or what its struct() gives
+bool describe(PyObject * c, p1a_kv & kv) {
+    if (PyErr_Occurred()) return false;
+    if ((PyObject *) Py_TYPE(c) != kv_class) {
+        PyObject * st = PyObject_CallMethodNoArgs(c, s_struct);
+        if (!st) return false;
+        Py_buffer b;
+        const bool ok = PyObject_GetBuffer(st, &b, PyBUF_SIMPLE) == 0;
+        if (ok) {
+            if (b.len == (Py_ssize_t) sizeof kv) memcpy(&kv, b.buf, sizeof kv);
+            else PyErr_SetString(PyExc_TypeError, "struct() gave no p1a_kv");
+            PyBuffer_Release(&b);
+        }
+        Py_DECREF(st);
+        return !PyErr_Occurred();
+    }
+    PyObject * f[11] = {};
+    for (int i = 0; i < 11 && !PyErr_Occurred(); ++i) f[i] = PyObject_GetAttr(c, s_field[i]);
+    if (!PyErr_Occurred()) {
+        kv.type = (uint32_t) as_int(f[0]);
+        kv.n_ctx = as_int(f[1]); kv.Hkv = as_int(f[2]); kv.D = as_int(f[3]);
+        kv.k = address(f[4]); kv.v = address(f[5]);
+        const char * pt = ptr<char>(f[6]);
+        kv.pt = (const int32_t *) (f[6] == Py_None ? nullptr : pt + 4 * (ptrdiff_t) as_int(f[10]));
+        kv.rtab = ptr<int32_t>(f[7]);
+        kv.psh = as_int(f[8]);
+        kv.pstride = as_size(f[9]);
+    }
+    for (PyObject * x : f) Py_XDECREF(x);
+    return !PyErr_Occurred();
+}
+void * stream() {
+    if (PyErr_Occurred()) return nullptr;
+    PyObject * r = PyObject_CallNoArgs(stream_of);
+    if (!r) return nullptr;
+    void * p = address(r);
+    Py_DECREF(r);
+    return p;
+}
+bool takes(Py_ssize_t n, Py_ssize_t want) {
+    if (n != want) PyErr_Format(PyExc_TypeError, "%zd arguments expected, %zd given", want, n);
+    return n == want;
+}
+#define P1A_CALL(expr) do { if (PyErr_Occurred()) return nullptr; int rc_; Py_BEGIN_ALLOW_THREADS rc_ = (expr); Py_END_ALLOW_THREADS return PyLong_FromLong(rc_); } while (0)
+
+// (qg, k, v, q_norm, k_norm, pos, q, gate, cache, p0, T, Hq, n_rot, freq_base, eps, ldq, ldk, ldv)
+PyObject * prep(PyObject *, PyObject * const * a, Py_ssize_t n) {
+    if (!takes(n, 18)) return nullptr;
+    p1a_kv kv;
+    float * p[8];
+    for (int i = 0; i < 8; ++i) p[i] = ptr<float>(a[i]);
+    describe(a[8], kv);
+    const int p0 = as_int(a[9]), T = as_int(a[10]), Hq = as_int(a[11]), nr = as_int(a[12]);
+    const float base = as_float(a[13]), eps = as_float(a[14]);
+    const int lq = as_int(a[15]), lk = as_int(a[16]), lv = as_int(a[17]);
+    void * s = stream();
+    P1A_CALL(f_prep(p[0], p[1], p[2], p[3], p[4], (const int32_t *) p[5], p[6], p[7], &kv, p0, T, Hq, nr, base, eps, lq, lk, lv, s));
+}
+// (q, cache, out, gate, qbuf, T, p0, p0_dev, pos, rows_per_seq, Hq, scale)
+PyObject * decode(PyObject *, PyObject * const * a, Py_ssize_t n) {
+    if (!takes(n, 12)) return nullptr;
+    p1a_kv kv;
+    const float * q = ptr<float>(a[0]);
+    describe(a[1], kv);
+    float * out = ptr<float>(a[2]);
+    const float * gate = ptr<float>(a[3]);
+    void * qbuf = data_ptr(a[4]);
+    const int T = as_int(a[5]), p0 = as_int(a[6]);
+    const int32_t * p0_dev = ptr<int32_t>(a[7]), * pos = ptr<int32_t>(a[8]);
+    const int rps = as_int(a[9]), Hq = as_int(a[10]);
+    const float scale = as_float(a[11]);
+    void * s = stream();
+    P1A_CALL(f_decode(q, &kv, out, gate, qbuf, T, p0, p0_dev, pos, rps, Hq, scale, s));
+}
+// (q, cache, out, gate, T, p0, Hq, scale, scratch, scratch_bytes)
+PyObject * prefill(PyObject *, PyObject * const * a, Py_ssize_t n) {
+    if (!takes(n, 10)) return nullptr;
+    p1a_kv kv;
+    const float * q = ptr<float>(a[0]);
+    describe(a[1], kv);
+    float * out = ptr<float>(a[2]);
+    const float * gate = ptr<float>(a[3]);
+    const int T = as_int(a[4]), p0 = as_int(a[5]), Hq = as_int(a[6]);
+    const float scale = as_float(a[7]);
+    void * scratch = data_ptr(a[8]);
+    const size_t bytes = as_size(a[9]);
+    void * s = stream();
+    P1A_CALL(f_prefill(q, &kv, out, gate, T, p0, Hq, scale, scratch, bytes, s));
+}
+// (cache, k, v, p0, p0_dev, pos, T)
+PyObject * append(PyObject *, PyObject * const * a, Py_ssize_t n) {
+    if (!takes(n, 7)) return nullptr;
+    p1a_kv kv;
+    describe(a[0], kv);
+    const float * k = ptr<float>(a[1]), * v = ptr<float>(a[2]);
+    const int p0 = as_int(a[3]);
+    const int32_t * p0_dev = ptr<int32_t>(a[4]), * pos = ptr<int32_t>(a[5]);
+    const int T = as_int(a[6]);
+    void * s = stream();
+    P1A_CALL(f_append(&kv, k, v, p0, p0_dev, pos, T, s));
+}
+// (addresses of p1a_attn_prep, p1a_attn_decode_a16, p1a_attn_prefill, p1a_kv_append; the cache class; the current stream's handle)
+PyObject * bind(PyObject *, PyObject * const * a, Py_ssize_t n) {
+    if (!takes(n, 6)) return nullptr;
+    f_prep = (decltype(f_prep)) address(a[0]);
+    f_decode = (decltype(f_decode)) address(a[1]);
+    f_prefill = (decltype(f_prefill)) address(a[2]);
+    f_append = (decltype(f_append)) address(a[3]);
+    if (PyErr_Occurred()) return nullptr;
+    Py_INCREF(a[4]); Py_XSETREF(kv_class, a[4]);
+    Py_INCREF(a[5]); Py_XSETREF(stream_of, a[5]);
+    Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {
+    {"bind", (PyCFunction) (void (*)(void)) bind, METH_FASTCALL, nullptr}, {"prep", (PyCFunction) (void (*)(void)) prep, METH_FASTCALL, nullptr},
+    {"decode", (PyCFunction) (void (*)(void)) decode, METH_FASTCALL, nullptr}, {"prefill", (PyCFunction) (void (*)(void)) prefill, METH_FASTCALL, nullptr},
+    {"append", (PyCFunction) (void (*)(void)) append, METH_FASTCALL, nullptr}, {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module_ = {PyModuleDef_HEAD_INIT, "_p1a_call", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}   // namespace
+
+PyMODINIT_FUNC PyInit__p1a_call(void) {
+    s_data_ptr = PyUnicode_InternFromString("data_ptr");
+    s_struct = PyUnicode_InternFromString("struct");
+    for (int i = 0; i < 11; ++i) s_field[i] = PyUnicode_InternFromString(FIELDS[i]);
+    return PyModule_Create(&module_);
+}

@@ -1,0 +1,87 @@
+"""The native side of the Python calls (csrc/p1a_call.cpp): every argument reaches the C ABI as ctypes would hand it over. The library's
+entry points are stood in for by callbacks that note what they get; no GPU."""
+import ctypes
+import importlib
+
+import pytest
+
+p1a = importlib.import_module("p100e-engine_amd")
+b = importlib.import_module("p100e-engine_amd.binding")
+VP, I, F, SZ = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_size_t
+KV = ctypes.POINTER(b.p1a_kv)
+SIGNATURES = {"p1a_attn_prep": [VP] * 8 + [KV, I, I, I, I, F, F, I, I, I, VP], "p1a_attn_decode_a16": [VP, KV, VP, VP, VP, I, I, VP, VP, I, I, F, VP],
+              "p1a_attn_prefill": [VP, KV, VP, VP, I, I, I, F, VP, SZ, VP], "p1a_kv_append": [KV, VP, VP, I, VP, VP, I, VP]}
+
+
+class Tensor:
+    def __init__(self, at, n=0):
+        self.at, self.n = at, n
+
+    def data_ptr(self):
+        return self.at
+
+    def numel(self):
+        return self.n
+
+    def element_size(self):
+        return 4
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    got = []
+
+    def stand_in(types):
+        def f(*a):
+            got.append([{n: getattr(x.contents, n) for n, _ in b.p1a_kv._fields_} if isinstance(x, KV) else x for x in a])
+            return 0
+        return ctypes.CFUNCTYPE(I, *types)(f)
+    kept = {n: stand_in(t) for n, t in SIGNATURES.items()}
+    m = b._calls()
+    m.bind(*(ctypes.cast(kept[n], VP).value for n in SIGNATURES), b.KVCache, lambda: 0x7770)
+    yield got
+    b._call = None
+    b._calls()                                                 # the library's own entry points again
+
+
+def test_arguments_reach_the_library(calls):
+    big = 0x7fff12345678
+    c = p1a.KVCache(p1a.KV_Q8_0, 4096, 4, 256, big, big + 64, Tensor(0x5000), Tensor(0x6000), 8, 1 << 33)
+    want = dict(type=8, n_ctx=4096, Hkv=4, D=256, k=big, v=big + 64, pt=0x5000, rtab=0x6000, psh=8, pstride=1 << 33)
+    slot = c.slot(3, 17)
+    want_slot = dict(want, pt=0x5000 + 4 * 3 * 17, rtab=None)
+    flat = p1a.KVCache(p1a.KV_F16, 100, 2, 64, 0x100, 0x200)
+    want_flat = dict(type=1, n_ctx=100, Hkv=2, D=64, k=0x100, v=0x200, pt=None, rtab=None, psh=0, pstride=0)
+    t = [Tensor(0x1000 + 16 * i) for i in range(8)]
+    at = [x.at for x in t]
+    p1a.attn_prep(*t, c, -1, 5, 24, 64, 1e6, 1e-6, ldq=7, ldk=8, ldv=9)
+    p1a.attn_decode(t[0], slot, t[1], 2, 77, 24, 0.0625)
+    p1a.attn_decode_dev(t[0], flat, t[1], 2, t[2], 999, 4, 0.125, gate=t[3])
+    p1a.attn_decode_rows(t[0], c, t[1], 4, t[2], 24, 0.5, gate=t[3], rows_per_seq=2, qbuf=t[4])
+    p1a.attn_prefill(t[0], slot, t[1], 100, 3, 24, 0.25, gate=t[2], scratch=Tensor(0x9000, 1 << 32))
+    p1a.attn_prefill(t[0], flat, t[1], 100, 3, 24, 0.25)
+    p1a.kv_append(slot, t[0], t[1], 9, 10)
+    p1a.kv_append_dev(c, t[0], t[1], t[2], 10)
+    p1a.kv_append_rows(c, t[0], t[1], t[2], 10)
+    p1a.attn_decode(t[0], b.KVDesc(slot.struct()), t[1], True, 77, 24, 1)
+    f = lambda x: ctypes.c_float(x).value
+    s = 0x7770
+    assert calls == [
+        at + [want, -1, 5, 24, 64, f(1e6), f(1e-6), 7, 8, 9, s],
+        [at[0], want_slot, at[1], None, None, 2, 77, None, None, 0, 24, f(0.0625), s],
+        [at[0], want_flat, at[1], at[3], None, 2, 0, at[2], None, 0, 4, f(0.125), s],
+        [at[0], want, at[1], at[3], at[4], 4, 0, None, at[2], 2, 24, f(0.5), s],
+        [at[0], want_slot, at[1], at[2], 100, 3, 24, f(0.25), 0x9000, 1 << 34, s],
+        [at[0], want_flat, at[1], None, 100, 3, 24, f(0.25), None, 0, s],
+        [want_slot, at[0], at[1], 9, None, None, 10, s],
+        [want, at[0], at[1], 0, at[2], None, 10, s],
+        [want, at[0], at[1], -1, None, at[2], 10, s],
+        [at[0], want_slot, at[1], None, None, 1, 77, None, None, 0, 24, 1.0, s]]
+
+
+@pytest.mark.parametrize("change", [dict(T=1.5), dict(T=None), dict(q=3), dict(scale="x"), dict(c=object()), dict(c=None)])
+def test_what_is_no_argument_is_refused(calls, change):
+    a = dict(q=Tensor(16), c=p1a.KVCache(p1a.KV_F16, 100, 2, 64, 0x100, 0x200), out=Tensor(32), T=1, p0=0, Hq=4, scale=1.0)
+    with pytest.raises((TypeError, AttributeError, ctypes.ArgumentError)):
+        p1a.attn_decode(**{**a, **change})
+    assert not calls
