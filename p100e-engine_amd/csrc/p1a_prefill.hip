@@ -100,7 +100,8 @@ struct pf_params {
     int turn_a, turn_b;   // slots of an XCD taken in reverse order
     int run;      // key splits: consecutive workgroups of an XCD (0: groups in turn)
     // key splits: with nks > 1 workgroup (block, kv head, ks) walks its share of the block's tiles and leaves an unnormalised
-    // partial (O relative to m, and (m, l)) per row in part_o [T*Hq][nks][D] / part_ml [T*Hq][nks][2] for the merge
+    // partial (O relative to m, and (m, l)) per row in part_o [T*Hq][nks][D] / part_ml [T*Hq][nks][2] for the merge; out is part_o
+    // then, and gate null
     int nks;
     float * part_o;
     float * part_ml;
@@ -867,19 +868,19 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
         const float inv = part ? 1.0f : 1.0f / l_own;
         const size_t rr = row_index(min(my_row, P.R - 1));
         f4 gt[HD][4];
-        if (P.gate && !part)
+        if (P.gate)
 #pragma unroll
             for (int dt = 0; dt < HD; ++dt)
 #pragma unroll
                 for (int q4 = 0; q4 < 4; ++q4) gt[dt][q4] = *reinterpret_cast<const f4 *>(P.gate + rr * D + 32 * dt + 8 * q4 + 4 * g);
         if (live) {
-            float * orow = part ? P.part_o + (rr * P.nks + ksp) * D : P.out + rr * D;
+            float * orow = P.out + (part ? rr * P.nks + ksp : rr) * D;
 #pragma unroll
             for (int dt = 0; dt < HD; ++dt)
 #pragma unroll
                 for (int q4 = 0; q4 < 4; ++q4) {
                     f4 v = {o[0][dt][4 * q4] * inv, o[0][dt][4 * q4 + 1] * inv, o[0][dt][4 * q4 + 2] * inv, o[0][dt][4 * q4 + 3] * inv};
-                    if (P.gate && !part)
+                    if (P.gate)
 #pragma unroll
                         for (int x = 0; x < 4; ++x) v[x] *= sigmoid(gt[dt][q4][x]);
                     *reinterpret_cast<f4 *>(orow + 32 * dt + 8 * q4 + 4 * g) = v;
@@ -904,23 +905,42 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
 #pragma unroll
     for (int i0 = 0; i0 < NRI; i0 += N8) {
         f4 gt[N8], v[N8];
-        if (P.gate && !part) {
+        if (P.gate) {
 #pragma unroll
             for (int i = 0; i < N8; ++i) gt[i] = *reinterpret_cast<const f4 *>(P.gate + row_index(wrow0 + min(row_at(i0 + i), wlast)) * D + d4);
         }
         if (PAIR && i0 == 0) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
         for (int i = 0; i < N8; ++i) v[i] = *reinterpret_cast<const f4 *>(img + (i0 + i) * RPI * ORS);
-        if (P.gate && !part) {
+        if (P.gate) {
 #pragma unroll
             for (int i = 0; i < N8; ++i)
 #pragma unroll
                 for (int x = 0; x < 4; ++x) v[i][x] *= sigmoid(gt[i][x]);
         }
+        // (f16 tiles, D = 256: results, which nothing here reads again, go past the caches: 600 tokens behind 300, 24 / 4 heads, f16 53.9 -> 51.1 us, 2000, 32 / 8, q8_0
+        // 157 -> 151. Not partials, which the merge reads at once: q4_0, 77 behind 16000 71.6 -> 73.2.)
+        if constexpr (DMA && PAIR) {
+            f4 * po[N8];
 #pragma unroll
-        for (int i = 0; i < N8; ++i) {
-            const size_t row = row_index(wrow0 + row_at(i0 + i));
-            if (row_at(i0 + i) < wrows) *reinterpret_cast<f4 *>((part ? P.part_o + (row * P.nks + ksp) * D : P.out + row * D) + d4) = v[i];
+            for (int i = 0; i < N8; ++i) {
+                const size_t row = row_index(wrow0 + row_at(i0 + i));
+                po[i] = reinterpret_cast<f4 *>(P.out + (part ? row * P.nks + ksp : row) * D + d4);
+            }
+            if (!part) {
+#pragma unroll
+                for (int i = 0; i < N8; ++i) if (row_at(i0 + i) < wrows) __builtin_nontemporal_store(v[i], po[i]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < N8; ++i) if (row_at(i0 + i) < wrows) *po[i] = v[i];
+                asm volatile("");                             // (or the two would be merged into one, through the caches)
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < N8; ++i) {
+                const size_t row = row_index(wrow0 + row_at(i0 + i));
+                if (row_at(i0 + i) < wrows) *reinterpret_cast<f4 *>(P.out + (part ? row * P.nks + ksp : row) * D + d4) = v[i];
+            }
         }
         if ((i0 + N8) * RPI >= wrows) break;
     }
@@ -1126,6 +1146,7 @@ int launch_prefill(const p1a_kv & c, const float * q, float * out, const float *
         } else if (!split_scratch(s, bo, bm, P.part_o, P.part_ml)) return P1A_E_SCRATCH;   // (the split count fixes the result bits: never fewer splits for want of room)
     }
     P.nks = nks;
+    if (nks > 1) { P.out = P.part_o; P.gate = nullptr; }
     P.rpw = block_rows(P.R, c.Hkv, nks, cu_count()) / 4;
     P.nblk = (P.R + 4 * P.rpw - 1) / (4 * P.rpw);
     // Groups of at most GQA blocks, as even as can be: a group's missing blocks are workgroups that find nothing to do, but
