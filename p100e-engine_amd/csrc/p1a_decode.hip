@@ -1135,19 +1135,22 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hi
     // four sequences and more whose page-table rows cannot hold the keys that half of the streams begin with (8 x 4 rows of 300
     // ... 5000 keys, q8_0, 24 / 4 heads of 256, two layers 72.8 -> 62.1 us, 16 of 300 ... 5000, 32 / 8 of 128 104 -> 93; with every
     // stream live 8 of 18797, q8_0, 24 / 4 of 128, four layers would go from 349 to 360).
-    const bool list = a.pos_rows && groups > 1 && (sb || (groups >= 4 && 2LL * c.n_ctx <= (long long) pl.nsplit * 32 * pl.NW));
+    const long long once = (long long) pl.nsplit * 32 * pl.NW;   // the keys that every stream holds a unit of
+    const bool list = a.pos_rows && groups > 1 && (sb || (groups >= 4 && 2LL * c.n_ctx <= once));
     long long nq = ((long long) nseq * pl.nsplit + 7) / 8;   // streams there could be, in eights
     // Where most workgroups would find nothing to do, at 0.5 us for every 1000 of them, fewer walk the list.
     //   Two to a unit: more than 16 for every compute unit, i.e. 32 sequences (of 256 keys, q8_0, 24 / 4 heads of 256, two layers: 61 us, 49.5
     //   with a workgroup for every stream, 43 so; of 300 ... 5000 99, 94.6, 90.5; f16, 32 / 8 of 128, 32 of 1024 91, 95, 89). Fewer would lose more where
-    //   all streams are live (16 of 20000: 313, 304 with one workgroup a stream, 333 with eight for every unit).
+    //   all streams are live (16 of 20000: 313, 304 with one workgroup a stream, 333 with eight for every unit); but four for every unit where
+    //   page-table rows hold a quarter of that at most (32 of 1024, f16, 16 / 4 of 64: 45 us with 16, 39 with four; 24 / 4 of 256, q8_0 68 and 64; where
+    //   they hold half, f16, 8 / 8 of 256, 2000 keys 212 and 220).
     //   One to a unit: more than two for every compute unit; at least half of the streams are known to be empty there (start, a workgroup
     //   for every stream, two for every unit: 8 x 4 rows of 300 ... 5000, q8_0, 24 / 4 of 256 73.6, 62.7, 56.5 us; 16 of 256, 32 / 8 of 128 53, 45, 39;
     //   32 of 256 77, 71, 43; q4_0, 24 / 4 of 128, 16 of 60 ... 1500 58.5, 46.9, 40.3).
     const long long most = (sb ? 16LL : 2LL) * (a.cus > 0 ? a.cus : 256) / (8 * inner);
     constexpr bool can_loop_2 = !(KT == P1A_KV_Q4_0);   // (q4_0 with two column tiles has no register left for it)
     const bool loop = list && nq > most && (pl.NT == 2 ? can_loop_2 : KS != KT || sb);
-    if (loop) nq = most > 1 ? most : 1;
+    if (loop) nq = sb && 4LL * c.n_ctx <= once ? (most + 3) / 4 : most > 1 ? most : 1;
     const unsigned lgrid = (unsigned) (8 * inner * nq);
     auto go = [&](auto nt, auto single, auto can_loop) {
         constexpr int NT = decltype(nt)::value, NW = big_tiles ? 4 : 8;
