@@ -213,9 +213,16 @@ template <int U> __device__ __forceinline__ uint32_t live_streams(const int32_t 
         if (T & 7) pr = __builtin_amdgcn_ds_bpermute(4 * (lane < (T & ~7) ? lane : lane + 8 - (T & 7)), pr);
     }
     int n = lane < T && pr >= 0 ? pr / U + 1 : 0;              // units
-    if (RPS > 1) {                                           // the most of a sequence's rows, in its first one
-        const int n1 = n;
-        for (int k = 1; k < RPS; ++k) n = max(n, __builtin_amdgcn_ds_bpermute(4 * (lane + k), n1));
+    if (RPS > 1) {                                             // the most of a sequence's rows, in its first one
+        if ((RPS & (RPS - 1)) == 0 && RPS <= 16) {             // (lane i from lanes i + 1, + 2, ...: its sixteen lanes hold whole sequences)
+            n = max(n, __builtin_amdgcn_update_dpp(0, n, 0x101, 0xf, 0xf, true));
+            if (RPS > 2) n = max(n, __builtin_amdgcn_update_dpp(0, n, 0x102, 0xf, 0xf, true));
+            if (RPS > 4) n = max(n, __builtin_amdgcn_update_dpp(0, n, 0x104, 0xf, 0xf, true));
+            if (RPS > 8) n = max(n, __builtin_amdgcn_update_dpp(0, n, 0x108, 0xf, 0xf, true));
+        } else {
+            const int n1 = n;
+            for (int k = 1; k < RPS; ++k) n = max(n, __builtin_amdgcn_ds_bpermute(4 * (lane + k), n1));
+        }
         if (lane - (int) ((uint32_t) lane * (uint32_t) rps_magic >> 16) * RPS) n = 0;
     }
     const int na = min(max(n - nsplit, 0), nsplit);
