@@ -429,7 +429,9 @@ int launch_decode_any(const p1a_kv & c, const decode_args & a, int rows_per_grou
     // 16 / 4 heads of 96, four layers 65.6 -> 57.9 us, 8 of 211 ... 3391, 4 / 1 of 192 86.7 -> 68.4). With 32 rows a grid of 8192 workgroups is mostly
     // empty and each reads all positions before it knows (f16, 24 / 4 of 192, 8 x 4 rows of 11 ... 188 keys 37 us, 48 with the list); with two
     // there is little to spread (16 / 2 of 96, 15 ... 246 keys 19.8 and 21.9).
-    const bool list = a.pos_rows && nseq > 1 && a.T >= 4 && a.T <= 16 && c.D <= 256;
+    // Larger heads, a compute unit to a workgroup, only while few heads keep most streams empty (q8_0, 16 rows of 1000 keys, two layers: 16 / 2 of 192 1.25
+    // times as fast, 24 / 4 1.02, 32 / 8 0.98; f16 1.14, 0.94, 0.88, with 8 rows 1.22, 1.02, 0.94).
+    const bool list = a.pos_rows && nseq > 1 && a.T >= 4 && a.T <= 16 && (c.D <= 128 || (c.D <= 256 && c.Hkv * a.T <= 32));
     const dim3 grid = list ? dim3((unsigned) (((long long) nseq * nsplit + 7) / 8 * 8 * P.inner)) : dim3(nsplit * c.Hkv, nct, a.T);
     if (c.type == P1A_KV_F16) launch_kt<P1A_KV_F16>(P, list, grid, s);
     else if (c.type == P1A_KV_Q8_0) launch_kt<P1A_KV_Q8_0>(P, list, grid, s);
