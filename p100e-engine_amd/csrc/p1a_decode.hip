@@ -1144,8 +1144,8 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hi
     //   all streams are live (16 of 20000: 313, 304 with one workgroup a stream, 333 with eight for every unit); but four for every unit where
     //   page-table rows hold a quarter of that at most (32 of 1024, f16, 16 / 4 of 64: 45 us with 16, 39 with four; 24 / 4 of 256, q8_0 68 and 64; where
     //   they hold half, f16, 8 / 8 of 256, 2000 keys 212 and 220).
-    //   One to a unit: more than two for every compute unit; at least half of the streams are known to be empty there (start, a workgroup
-    //   for every stream, two for every unit: 8 x 4 rows of 300 ... 5000, q8_0, 24 / 4 of 256 73.6, 62.7, 56.5 us; 16 of 256, 32 / 8 of 128 53, 45, 39;
+    //   One to a unit: more than two for every compute unit; at least half of the streams are known to be empty there (without the list, a
+    //   workgroup for every stream, two for every unit: 8 x 4 rows of 300 ... 5000, q8_0, 24 / 4 of 256 73.6, 62.7, 56.5 us; 16 of 256, 32 / 8 of 128 53, 45, 39;
     //   32 of 256 77, 71, 43; q4_0, 24 / 4 of 128, 16 of 60 ... 1500 58.5, 46.9, 40.3).
     const long long most = (sb ? 16LL : 2LL) * (a.cus > 0 ? a.cus : 256) / (8 * inner);
     constexpr bool can_loop_2 = !(KT == P1A_KV_Q4_0);   // (q4_0 with two column tiles has no register left for it)
