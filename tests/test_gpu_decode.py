@@ -430,9 +430,9 @@ def test_rows_of_sequences_of_any_length(p1a, kv_type, Hq, Hkv, D, psh, lens, ro
     T = n * rows
     q, gate = torch.randn((T, Hq, D), generator=g, device="cuda"), torch.randn((T, Hq, D), generator=g, device="cuda")
     pos = [max(x - rows, -1) + r if x >= rows else x - 1 for x in lens for r in range(rows)]
-    rtab = torch.tensor([s * maxp for s in range(n) for _ in range(rows)], dtype=torch.int32, device="cuda")
+    rtab = torch.tensor([-1] + [s * maxp for s in range(n) for _ in range(rows)], dtype=torch.int32, device="cuda")[1:]   # (4-byte aligned, no more)
     out = torch.full((T, Hq, D), 7.0, device="cuda")
-    p1a.attn_decode_rows(q, c.with_rows(rtab), out, T, torch.tensor(pos, dtype=torch.int32, device="cuda"), Hq, scale, gate=gate, rows_per_seq=rows)
+    p1a.attn_decode_rows(q, c.with_rows(rtab), out, T, torch.tensor([-1] + pos, dtype=torch.int32, device="cuda")[1:], Hq, scale, gate=gate, rows_per_seq=rows)
     one = torch.empty((1, Hq, D), device="cuda")
     for t in range(T):
         if pos[t] < 0:
