@@ -26,6 +26,7 @@
 //   multiplies V. The waves of one head fold their (m, l, O) through LDS; one partial per (workgroup, head) goes to
 //   scratch and merge_k folds the splits in a fixed order and applies the sigmoid gate.
 #include "p1a_common.hpp"
+#include "p1a_plan.hpp"
 
 #include <cstdlib>
 #include <type_traits>
@@ -1044,61 +1045,6 @@ __global__ void __launch_bounds__(256) sigmoid_mul_k(float * __restrict__ x, con
         x[i] *= 1.0f / (1.0f + expf(-g[i]));
 }
 
-// ---- launch plan: which kernel a shape takes, and how the keys are split ----
-// The MFMA kernel needs 16-byte aligned head rows (f16: D in {64, 128, 256}; q8_0 / q4_0: D == 256), 16-byte aligned
-// bases and strides, pages of >= 16 positions and GQA <= 16; q8_0 / q4_0 at D = 64 or 128 (head rows of whole dwords)
-// take its staged build, which fetches 4 bytes per lane and only needs 4-byte alignment. Everything else takes the
-// kernel of p1a_decode_any.hip.
-struct dec_plan {
-    bool mfma;
-    int GQA, NW, NT, RG;
-    int nsplit;    // split streams: partials per output row
-};
-
-bool mfma_ok(const p1a_kv & c, int GQA) {
-    if (GQA < 1 || GQA > 16) return false;
-    if (c.D != 64 && c.D != 128 && c.D != 256) return false;
-    const bool staged = c.type != P1A_KV_F16 && c.D != 256;   // q8_0 / q4_0 head rows are whole 16-byte chunks only at D = 256
-    const uintptr_t al = staged ? 3 : 15;
-    if (((uintptr_t) c.k | (uintptr_t) c.v) & al) return false;
-    if (c.pt && ((c.pstride & al) || c.psh < 4)) return false;
-    return true;
-}
-
-dec_plan make_plan(const p1a_kv & c, int Hq, int rows_per_group, int nsplit_req, int cus) {
-    dec_plan p;
-    p.GQA = Hq / c.Hkv;
-    p.mfma = mfma_ok(c, p.GQA);
-    if (!p.mfma) {
-        p.NW = 4; p.NT = 1;
-        p.RG = rows_per_group < 1 ? 1 : rows_per_group;   // no sharing here: the group only selects the page table
-        // one workgroup per CU, and not more than 4 partials for every 2 CUs per q head
-        int n = nsplit_req;
-        if (n <= 0) {
-            const int most = 4 * (2 * cus / Hq < 1 ? 1 : (2 * cus / Hq > 1024 ? 1024 : 2 * cus / Hq));
-            n = cus / c.Hkv < most ? cus / c.Hkv : most;
-        }
-        n = n < 1 ? 1 : (nsplit_req > 1024 ? 1024 : n);
-        p.nsplit = n >= 8 ? n & ~7 : n;
-        return p;
-    }
-    const int cap = 32 / p.GQA < 4 ? 32 / p.GQA : 4;
-    p.RG = rows_per_group < 1 ? 1 : (rows_per_group > cap ? cap : rows_per_group);
-    // One kv head per workgroup: its waves fold into ONE partial, which keeps the split traffic at a few percent of the KV
-    // bytes; the heads of a split stream are placed on one XCD so shared cache lines meet in its L2.
-    const bool big_tiles = c.type == P1A_KV_F16 && c.D == 256;   // 34 KB of LDS per wave
-    p.NW = big_tiles ? 4 : 8;
-    const int HG = c.Hkv;
-    // (one workgroup per CU for every variant: the four-wave one keeps 128 KB of f16 tiles in LDS; measured for f16 at
-    // 32 K: 64 streams 27.2 us, 128 streams - two rounds of workgroups - 30.2 us)
-    int n = nsplit_req > 0 ? nsplit_req : cus / HG;
-    if (n >= 8) n &= ~7;
-    p.nsplit = n < 1 ? 1 : (n > 1024 ? 1024 : n);
-    return p;
-}
-
-void finish_plan(dec_plan & p) { p.NT = p.RG * p.GQA <= 16 ? 1 : 2; }
-
 template <uint32_t KT, int D, uint32_t KS = KT>
 int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hipStream_t s) {
     dec_params P;
@@ -1107,11 +1053,10 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hi
     P.p0 = a.p0; P.p0_dev = a.p0_dev; P.pos_rows = a.pos_rows;
     P.T = a.T; P.RG = pl.RG; P.Hq = a.Hq; P.Hkv = c.Hkv; P.GQA = pl.GQA;
     P.qscale = a.scale * 1.4426950408889634f; P.nsplit = pl.nsplit;
-    const int groups = (a.T + pl.RG - 1) / pl.RG;
-    P.RPS = a.rows_per_seq < a.T ? a.rows_per_seq : a.T;
-    P.GPS = a.rows_per_seq > pl.RG ? a.rows_per_seq / pl.RG : 1;
-    if (P.GPS > groups) P.GPS = groups;
-    const int nseq = (groups + P.GPS - 1) / P.GPS;
+    constexpr bool big_tiles = KT == P1A_KV_F16 && D == 256;
+    const decode_grid gr = plan_grid(pl, KS, D, c.Hkv, c.n_ctx, a.T, a.rows_per_seq, a.pos_rows != nullptr, a.cus);
+    P.RPS = gr.RPS;
+    P.GPS = gr.GPS;
     P.rps_magic = 65536 / P.RPS + 1;
     const int inner = c.Hkv * P.GPS;
     P.hkv_sh = P.inner_sh = -1;
@@ -1120,52 +1065,22 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hi
         if ((1 << sh) == inner) P.inner_sh = sh;
     }
     P.npt = c.pt ? (int) (((long long) c.n_ctx + (1LL << c.psh) - 1) >> c.psh) : 0;
-    constexpr bool big_tiles = KT == P1A_KV_F16 && D == 256;
-    // A call of at least two workgroups per CU whose row groups fit one column tile takes the single-buffered variant, two
-    // workgroups to a CU (same partials, bit for bit; measured at 24 / 4 heads, D = 256: 8 q8_0 slots of 1 K ... 27 K 56 ->
-    // 47 us, 4 x 64 K q4_0 single rows 92 -> 73 us, 16 x 2 rows q4_0 at 16 K 143 -> 115 us, 32 slots of 2 ... 5 K 104 -> 71 us).
-    // (A workgroup walks ONE split stream whatever the call: letting it walk several in turn - fewer, longer workgroups
-    // for calls of many - measured slower on every shape tried, e.g. 8 x 4 rows q4_0 at 8 K 72 -> 60 us with one.)
-    const long long wgs_all = (long long) pl.nsplit * c.Hkv * ((a.T + pl.RG - 1) / pl.RG);
-    const bool sb = KS == KT && pl.NT == 1 && wgs_all >= 2LL * (a.cus > 0 ? a.cus : 256);
-    const dim3 grid(pl.nsplit * c.Hkv, groups);
-    // The list (see dec_mfma_k) costs a workgroup some 0.2 us before its first request. Where two workgroups share a compute unit that hides,
-    // and every call of several sequences takes it (110 calls of 2 ... 32 sequences drawn over 4 ... 131072 keys, D = 256 and f16:
-    // 0.98 - 1.6 times as fast, 1.1 in the mean). Where one has a unit to itself (two column tiles, staged tiles) it shows: calls of
-    // four sequences and more whose page-table rows cannot hold the keys that half of the streams begin with (8 x 4 rows of 300
-    // ... 5000 keys, q8_0, 24 / 4 heads of 256, two layers 72.8 -> 62.1 us, 16 of 300 ... 5000, 32 / 8 of 128 104 -> 93; with every
-    // stream live 8 of 18797, q8_0, 24 / 4 of 128, four layers would go from 349 to 360).
-    const long long once = (long long) pl.nsplit * 32 * pl.NW;   // the keys that every stream holds a unit of
-    const bool list = a.pos_rows && groups > 1 && (sb || (groups >= 4 && 2LL * c.n_ctx <= once));
-    long long nq = ((long long) nseq * pl.nsplit + 7) / 8;   // streams there could be, in eights
-    // Where most workgroups would find nothing to do, at 0.5 us for every 1000 of them, fewer walk the list.
-    //   Two to a unit: more than 16 for every compute unit, i.e. 32 sequences (of 256 keys, q8_0, 24 / 4 heads of 256, two layers: 61 us, 49.5
-    //   with a workgroup for every stream, 43 so; of 300 ... 5000 99, 94.6, 90.5; f16, 32 / 8 of 128, 32 of 1024 91, 95, 89). Fewer would lose more where
-    //   all streams are live (16 of 20000: 313, 304 with one workgroup a stream, 333 with eight for every unit); but four for every unit where
-    //   page-table rows hold a quarter of that at most (32 of 1024, f16, 16 / 4 of 64: 45 us with 16, 39 with four; 24 / 4 of 256, q8_0 68 and 64; where
-    //   they hold half, f16, 8 / 8 of 256, 2000 keys 212 and 220).
-    //   One to a unit: more than two for every compute unit; at least half of the streams are known to be empty there (without the list, a
-    //   workgroup for every stream, two for every unit: 8 x 4 rows of 300 ... 5000, q8_0, 24 / 4 of 256 73.6, 62.7, 56.5 us; 16 of 256, 32 / 8 of 128 53, 45, 39;
-    //   32 of 256 77, 71, 43; q4_0, 24 / 4 of 128, 16 of 60 ... 1500 58.5, 46.9, 40.3).
-    const long long most = (sb ? 16LL : 2LL) * (a.cus > 0 ? a.cus : 256) / (8 * inner);
-    constexpr bool can_loop_2 = !(KT == P1A_KV_Q4_0);   // (q4_0 with two column tiles has no register left for it)
-    const bool loop = list && nq > most && (pl.NT == 2 ? can_loop_2 : KS != KT || sb);
-    if (loop) nq = sb && 4LL * c.n_ctx <= once ? (most + 3) / 4 : most > 1 ? most : 1;
-    const unsigned lgrid = (unsigned) (8 * inner * nq);
+    const dim3 grid(gr.x, gr.y);
+    constexpr bool can_loop_2 = KT != P1A_KV_Q4_0;            // (plan_grid asks for no other)
     auto go = [&](auto nt, auto single, auto can_loop) {
         constexpr int NT = decltype(nt)::value, NW = big_tiles ? 4 : 8;
         constexpr bool SB = decltype(single)::value;
         if constexpr (decltype(can_loop)::value) {
-            if (loop) { dec_mfma_k<KT, D, NT, NW, SB, KS | LIST_ | LOOP_><<<lgrid, NW * 64, 0, s>>>(P); return; }
+            if (gr.loop) { dec_mfma_k<KT, D, NT, NW, SB, KS | LIST_ | LOOP_><<<grid, NW * 64, 0, s>>>(P); return; }
         }
-        if (list) dec_mfma_k<KT, D, NT, NW, SB, KS | LIST_><<<lgrid, NW * 64, 0, s>>>(P);
+        if (gr.list) dec_mfma_k<KT, D, NT, NW, SB, KS | LIST_><<<grid, NW * 64, 0, s>>>(P);
         else dec_mfma_k<KT, D, NT, NW, SB, KS><<<grid, NW * 64, 0, s>>>(P);
     };
     constexpr std::true_type yes;
     constexpr std::false_type no;
     if (pl.NT == 2) go(std::integral_constant<int, 2>{}, no, std::bool_constant<can_loop_2>{});
     else if constexpr (KS != KT) go(std::integral_constant<int, 1>{}, no, yes);
-    else if (sb) go(std::integral_constant<int, 1>{}, yes, yes);
+    else if (gr.sb) go(std::integral_constant<int, 1>{}, yes, yes);
     else go(std::integral_constant<int, 1>{}, no, no);
     return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
 }

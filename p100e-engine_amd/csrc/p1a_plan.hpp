@@ -1,0 +1,121 @@
+// The decode launch plan: which kernel a shape takes, how its keys are split and how large its grid is. Host arithmetic only, on the
+// descriptor and the call's numbers.
+#pragma once
+#include <algorithm>
+#include <cstddef>
+#include <cstdint>
+#include "p1a_attn.h"
+
+namespace p1a {
+
+// ---- launch plan: which kernel a shape takes, and how the keys are split ----
+// The MFMA kernel needs 16-byte aligned head rows (f16: D in {64, 128, 256}; q8_0 / q4_0: D == 256), 16-byte aligned
+// bases and strides, pages of >= 16 positions and GQA <= 16; q8_0 / q4_0 at D = 64 or 128 (head rows of whole dwords)
+// take its staged build, which fetches 4 bytes per lane and only needs 4-byte alignment. Everything else takes the
+// kernel of p1a_decode_any.hip.
+struct dec_plan {
+    bool mfma;
+    int GQA, NW, NT, RG;
+    int nsplit;    // split streams: partials per output row
+};
+
+inline bool mfma_ok(const p1a_kv & c, int GQA) {
+    if (GQA < 1 || GQA > 16) return false;
+    if (c.D != 64 && c.D != 128 && c.D != 256) return false;
+    const bool staged = c.type != P1A_KV_F16 && c.D != 256;   // q8_0 / q4_0 head rows are whole 16-byte chunks only at D = 256
+    const uintptr_t al = staged ? 3 : 15;
+    if (((uintptr_t) c.k | (uintptr_t) c.v) & al) return false;
+    if (c.pt && ((c.pstride & al) || c.psh < 4)) return false;
+    return true;
+}
+
+inline dec_plan make_plan(const p1a_kv & c, int Hq, int rows_per_group, int nsplit_req, int cus) {
+    dec_plan p;
+    p.GQA = Hq / c.Hkv;
+    p.mfma = mfma_ok(c, p.GQA);
+    if (!p.mfma) {
+        p.NW = 4; p.NT = 1;
+        p.RG = rows_per_group < 1 ? 1 : rows_per_group;   // no sharing here: the group only selects the page table
+        // one workgroup per CU, and not more than 4 partials for every 2 CUs per q head
+        int n = nsplit_req;
+        if (n <= 0) {
+            const int most = 4 * (2 * cus / Hq < 1 ? 1 : (2 * cus / Hq > 1024 ? 1024 : 2 * cus / Hq));
+            n = cus / c.Hkv < most ? cus / c.Hkv : most;
+        }
+        n = n < 1 ? 1 : (nsplit_req > 1024 ? 1024 : n);
+        p.nsplit = n >= 8 ? n & ~7 : n;
+        return p;
+    }
+    const int cap = 32 / p.GQA < 4 ? 32 / p.GQA : 4;
+    p.RG = rows_per_group < 1 ? 1 : (rows_per_group > cap ? cap : rows_per_group);
+    // One kv head per workgroup: its waves fold into ONE partial, which keeps the split traffic at a few percent of the KV
+    // bytes; the heads of a split stream are placed on one XCD so shared cache lines meet in its L2.
+    const bool big_tiles = c.type == P1A_KV_F16 && c.D == 256;   // 34 KB of LDS per wave
+    p.NW = big_tiles ? 4 : 8;
+    const int HG = c.Hkv;
+    // (one workgroup per CU for every variant: the four-wave one keeps 128 KB of f16 tiles in LDS; measured for f16 at
+    // 32 K: 64 streams 27.2 us, 128 streams - two rounds of workgroups - 30.2 us)
+    int n = nsplit_req > 0 ? nsplit_req : cus / HG;
+    if (n >= 8) n &= ~7;
+    p.nsplit = n < 1 ? 1 : (n > 1024 ? 1024 : n);
+    return p;
+}
+
+inline void finish_plan(dec_plan & p) { p.NT = p.RG * p.GQA <= 16 ? 1 : 2; }
+
+// The grid of the MFMA kernel: a workgroup for every (split stream, kv head) and row group, or - `list` - for every kv head and row
+// group of the streams that hold keys, counted through on the device: x = 8 * Hkv * GPS * nq, nq eights of streams (`loop`: a workgroup
+// takes the streams q, q + 8 nq, ...)
+struct decode_grid {
+    bool sb, list, loop;   // two workgroups to a compute unit; kinds of dec_mfma_k
+    int RPS, GPS;          // rows and row groups of a sequence
+    unsigned x, y;
+};
+
+inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv, int n_ctx, int T, int rows_per_seq, bool pos_rows, int cus_) {
+    decode_grid r;
+    const int cus = cus_ > 0 ? cus_ : 256, groups = (T + pl.RG - 1) / pl.RG;
+    const bool staged = type != P1A_KV_F16 && D != 256;
+    r.RPS = rows_per_seq < T ? rows_per_seq : T;
+    r.GPS = rows_per_seq > pl.RG ? rows_per_seq / pl.RG : 1;
+    if (r.GPS > groups) r.GPS = groups;
+    const int nseq = (groups + r.GPS - 1) / r.GPS, inner = Hkv * r.GPS;
+    // A call of at least two workgroups per CU whose row groups fit one column tile takes the single-buffered variant, two
+    // workgroups to a CU (same partials, bit for bit; measured at 24 / 4 heads, D = 256: 8 q8_0 slots of 1 K ... 27 K 56 ->
+    // 47 us, 4 x 64 K q4_0 single rows 92 -> 73 us, 16 x 2 rows q4_0 at 16 K 143 -> 115 us, 32 slots of 2 ... 5 K 104 -> 71 us).
+    // (A workgroup walks ONE split stream whatever the call: letting it walk several in turn - fewer, longer workgroups
+    // for calls of many - measured slower on every shape tried, e.g. 8 x 4 rows q4_0 at 8 K 72 -> 60 us with one.)
+    r.sb = !staged && pl.NT == 1 && (long long) pl.nsplit * Hkv * groups >= 2LL * cus;
+    // The list (see dec_mfma_k) costs a workgroup some 0.2 us before its first request. Where two workgroups share a compute unit that hides,
+    // and every call of several sequences takes it (110 calls of 2 ... 32 sequences drawn over 4 ... 131072 keys, D = 256 and f16:
+    // 0.98 - 1.6 times as fast, 1.1 in the mean). Where one has a unit to itself (two column tiles, staged tiles) it shows: calls of
+    // four sequences and more whose page-table rows cannot hold the keys that half of the streams begin with (8 x 4 rows of 300
+    // ... 5000 keys, q8_0, 24 / 4 heads of 256, two layers 72.8 -> 62.1 us, 16 of 300 ... 5000, 32 / 8 of 128 104 -> 93; with every
+    // stream live 8 of 18797, q8_0, 24 / 4 of 128, four layers would go from 349 to 360).
+    const long long once = (long long) pl.nsplit * 32 * pl.NW;   // the keys that every stream holds a unit of
+    r.list = pos_rows && groups > 1 && (r.sb || (groups >= 4 && 2LL * n_ctx <= once));
+    r.loop = false;
+    r.x = (unsigned) (pl.nsplit * Hkv);
+    r.y = (unsigned) groups;
+    if (!r.list) return r;
+    long long nq = ((long long) nseq * pl.nsplit + 7) / 8;   // streams there could be, in eights
+    // Where most workgroups would find nothing to do, at 0.5 us for every 1000 of them, fewer walk the list.
+    //   Two to a unit: more than 16 for every compute unit, i.e. 32 sequences (of 256 keys, q8_0, 24 / 4 heads of 256, two layers: 61 us, 49.5
+    //   with a workgroup for every stream, 43 so; of 300 ... 5000 99, 94.6, 90.5; f16, 32 / 8 of 128, 32 of 1024 91, 95, 89). Fewer would lose more where
+    //   all streams are live (16 of 20000: 313, 304 with one workgroup a stream, 333 with eight for every unit); but four for every unit where
+    //   page-table rows hold a quarter of that at most (32 of 1024, f16, 16 / 4 of 64: 45 us with 16, 39 with four; 24 / 4 of 256, q8_0 68 and 64; where
+    //   they hold half, f16, 8 / 8 of 256, 2000 keys 212 and 220).
+    //   One to a unit: more than two for every compute unit; at least half of the streams are known to be empty there (without the list, a
+    //   workgroup for every stream, two for every unit: 8 x 4 rows of 300 ... 5000, q8_0, 24 / 4 of 256 73.6, 62.7, 56.5 us; 16 of 256, 32 / 8 of 128 53, 45, 39;
+    //   32 of 256 77, 71, 43; q4_0, 24 / 4 of 128, 16 of 60 ... 1500 58.5, 46.9, 40.3).
+    const long long most = (r.sb ? 16LL : 2LL) * cus / (8 * inner);
+    const bool can_loop = pl.NT == 2 ? staged || type != P1A_KV_Q4_0 : staged || r.sb;   // (q4_0 with two column tiles has no register left for it)
+    r.loop = can_loop && nq > most;
+    // (never none: 8 * inner workgroups are more than that where kv heads and row groups are many)
+    if (r.loop) nq = std::max(1LL, r.sb && 4LL * n_ctx <= once ? (most + 3) / 4 : most);
+    r.x = (unsigned) (8 * inner * nq);
+    r.y = 1;
+    return r;
+}
+
+}   // namespace p1a

@@ -408,6 +408,7 @@ MIXED = [1, 255, 256, 257, 2304, 0, 700, 9000]                 # edges of a unit
     (O.KV_F16, 20, 5, 64, 6, 4 * MIXED[:7], 1), (O.KV_F16, 8, 8, 256, 6, 3 * MIXED[:7], 1), (O.KV_Q8_0, 8, 8, 64, 6, 4 * MIXED[:5], 1),
     (O.KV_Q8_0, 16, 8, 128, 6, 2 * MIXED[:7], 2), (O.KV_Q8_0, 24, 4, 256, 8, MIXED[:5], 4), (O.KV_F16, 16, 4, 64, 6, MIXED[:4], 8),
     (O.KV_F16, 16, 2, 64, 6, MIXED[:4], 8),
+    (O.KV_F16, 32, 32, 128, 4, [300], 17), (O.KV_F16, 64, 64, 128, 4, [200, 90], 11), (O.KV_Q8_0, 32, 32, 256, 4, [257], 31),   # (row groups of one row, more (group, kv head) pairs than two a unit)
     (O.KV_Q8_0, 24, 4, 96, 8, MIXED[:5], 1), (O.KV_F16, 8, 8, 96, 6, MIXED + [3], 1), (O.KV_Q4_0, 40, 2, 192, 6, MIXED[:4], 3), (O.KV_F16, 16, 8, 192, 6, MIXED[:3], 2), (O.KV_F16, 20, 5, 96, 2, 4 * MIXED[:7], 1),
     (O.KV_Q8_0, 16, 8, 320, 6, 2 * MIXED[:7], 2)])
 def test_rows_of_sequences_of_any_length(p1a, kv_type, Hq, Hkv, D, psh, lens, rows):
