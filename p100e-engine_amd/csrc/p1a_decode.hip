@@ -92,6 +92,8 @@ __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel)
 // 4 int8 codes (one dword) -> (code * d) as two packed f16 pairs, returned as raw dwords so MFMA operands are built in place
 struct u2 { uint32_t lo, hi; };
 typedef const __attribute__((address_space(4))) uint64_t * kargs;   // a kernel's arguments, as words
+// the pointer, known to the compiler as one to device memory
+template <typename T> __device__ __forceinline__ void in_memory(T *& p) { p = (T *) (__attribute__((address_space(1))) T *) (uintptr_t) p; }
 __device__ __forceinline__ u2 deq4(uint32_t w, h2 d01, h2 d23) {
     const h2 off = {(half_t) 1152, (half_t) 1152};
     const uint32_t x = w ^ 0x80808080u;
@@ -244,6 +246,10 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
 #pragma unroll
         for (unsigned i = 0; i < sizeof(dec_params) / 8; ++i) k.w[i] = kp[i];
         P_again = __builtin_bit_cast(dec_params, k);
+        // (pointers made of words are generic ones, and what goes through them FLAT: an access that may count as memory or as LDS,
+        // after which only a wait for everything is defined - but the tiles are waited for by count, behind the last item's stores)
+        in_memory(P_again.q); in_memory(P_again.kc); in_memory(P_again.vc); in_memory(P_again.part_o); in_memory(P_again.part_ml);
+        in_memory(P_again.pg.pt); in_memory(P_again.pg.rtab); in_memory(P_again.p0_dev); in_memory(P_again.pos_rows);
     }
     const dec_params & P = LOOP ? P_again : P_;
     const int lane = tid & 63;

@@ -65,6 +65,29 @@ def test_decode_list_kernels_fit_their_budget(tmp_path):
         assert r["LDS Size"] <= 160 * 1024, (name, r)
 
 
+def test_decode_kernels_make_no_flat_access(tmp_path):
+    """tiles are waited for by count; a FLAT access in flight (a pointer the compiler does not know to be one to device memory) leaves
+    only the wait for everything defined"""
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    if not os.path.exists(hipcc):
+        pytest.skip("no hipcc here")
+    out = tmp_path / "decode.s"
+    r = subprocess.run([hipcc, "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-I" + os.path.join(ROOT, "include"), "-Xclang", "-target-feature", "-Xclang",
+                        "-packed-fp32-ops", "-Wno-unused-command-line-argument", "-Wno-inline-asm", "--cuda-device-only", "-S",
+                        os.path.join(SRC, "p1a_decode.hip"), "-o", str(out)], capture_output=True, text=True, timeout=900)
+    assert r.returncode == 0, r.stderr[-2000:]
+    kernel, flat, seen = "", set(), set()
+    for line in out.read_text().splitlines():
+        m = re.match(r"(_ZN\S*dec_mfma_k\S*):", line)
+        if m or re.match(r"\S+:", line) and not line.startswith("."):
+            kernel = m.group(1) if m else ""
+        if kernel:
+            seen.add(kernel)
+            if re.match(r"\s+flat_", line):
+                flat.add(kernel)
+    assert len(seen) >= 40 and not flat, (len(seen), sorted(flat))
+
+
 VGPR_FORM = ("-mllvm", "-amdgpu-mfma-vgpr-form")               # (as the Makefile builds these two)
 
 
