@@ -28,8 +28,9 @@ struct kv_view {
     size_t rowb;            // bytes of one position (all kv heads)
 };
 
+// (a row table without a page table means nothing and may be anything: no kernel gets to see it)
 inline kv_view view_of(const p1a_kv & c) {
-    return kv_view{c.pt, c.rtab, c.psh, c.pstride, p1a_kv_row_bytes(c.type, c.Hkv, c.D)};
+    return kv_view{c.pt, c.pt ? c.rtab : nullptr, c.psh, c.pstride, p1a_kv_row_bytes(c.type, c.Hkv, c.D)};
 }
 
 __device__ __forceinline__ const int32_t * kv_tab(const kv_view & g, int t) {

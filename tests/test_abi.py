@@ -57,6 +57,29 @@ def test_cpp_mirror_header_compiles():
     assert r.returncode == 0, r.stderr[-2000:]
 
 
+def test_row_tables_count_only_with_a_page_table(tmp_path):
+    """pt == NULL: a contiguous cache, whatever rtab holds (include/p1a_attn.h). The kernels' view of such a cache has no row table, so
+    that no kernel can read through it. Host code only: the library's internal header, compiled into a program of its own."""
+    import subprocess
+    src = '''#include "p1a_common.hpp"
+extern "C" size_t p1a_kv_row_bytes(uint32_t, int, int) { return 1088; }
+int main() {
+    p1a_kv c = {};
+    c.type = P1A_KV_Q8_0; c.n_ctx = 100; c.Hkv = 4; c.D = 256; c.rtab = (const int32_t *) 0x40;
+    const p1a::kv_view flat = p1a::view_of(c);
+    c.pt = (const int32_t *) 0x1000;
+    const p1a::kv_view paged = p1a::view_of(c);
+    return !flat.pt && !flat.rtab && paged.pt == c.pt && paged.rtab == c.rtab ? 0 : 1;
+}
+'''
+    (tmp_path / "view.hip").write_text(src)
+    r = subprocess.run(["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-inline-asm",
+                        "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(ROOT, "p100e-engine_amd", "csrc"), str(tmp_path / "view.hip"), "-o", str(tmp_path / "view")],
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+    assert subprocess.run([str(tmp_path / "view")], timeout=60).returncode == 0
+
+
 def test_reload_env(p1a):
     """attn_dec2_reload_env (src/fast/attn_dec2.cuh:21): true exactly when the baked-in switch changed"""
     import os
