@@ -411,7 +411,7 @@ int launch_append(const p1a_kv & c, const float * k, const float * v, int p0, co
     if (c.type == P1A_KV_F16) append_k<P1A_KV_F16><<<grid, 256, 0, s>>>(k, v, kc, vc, p0, p0_dev, pos_rows, c.Hkv, c.D, pg);
     else if (c.type == P1A_KV_Q8_0) append_k<P1A_KV_Q8_0><<<grid, 256, 0, s>>>(k, v, kc, vc, p0, p0_dev, pos_rows, c.Hkv, c.D, pg);
     else append_k<P1A_KV_Q4_0><<<grid, 256, 0, s>>>(k, v, kc, vc, p0, p0_dev, pos_rows, c.Hkv, c.D, pg);
-    return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+    return launched();
 }
 
 namespace {
@@ -458,7 +458,7 @@ int launch_fill_random(const p1a_kv & c, int p0, int p1, uint32_t seed, hipStrea
     const size_t nw = (size_t) (p1 - p0) * row_words;
     const unsigned blocks = (unsigned) (nw / 256 + 1 < 4096 ? nw / 256 + 1 : 4096);
     fill_random_k<<<blocks, 256, 0, s>>>((uint16_t *) c.k, (uint16_t *) c.v, view_of(c), c.type, c.D, p0, nw, row_words, head_words, seed);
-    return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+    return launched();
 }
 
 namespace {
@@ -484,7 +484,7 @@ int launch_ew_quant(int op, const float * a, const float * b, float * y, void * 
     const dim3 grid((n / 4 + 255) / 256, T);
     if (op == 0) ew_q_k<0><<<grid, 256, 0, s>>>(a, b, y, qbuf, n, lda, ldb);
     else ew_q_k<1><<<grid, 256, 0, s>>>(a, b, y, qbuf, n, lda, ldb);
-    return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+    return launched();
 }
 
 int launch_prep(const p1a_kv & c, const float * qg, const float * k, const float * v, const float * q_norm, const float * k_norm,
@@ -510,7 +510,7 @@ int launch_prep(const p1a_kv & c, const float * qg, const float * k, const float
 #undef P1A_PREP_ROWS_G
 #undef P1A_PREP_ARGS
 #undef P1A_PREP_ROWS
-        return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+        return launched();
     }
     const dim3 grid(H, T);
 #define P1A_PREP(KT_) prep_k<KT_><<<grid, 64, 0, s>>>(qg, k, v, q_norm, k_norm, pos, q, gate, kc, vc, p0, Hq, c.Hkv, c.D, n_rot, \
@@ -519,7 +519,7 @@ int launch_prep(const p1a_kv & c, const float * qg, const float * k, const float
     else if (c.type == P1A_KV_Q8_0) P1A_PREP(P1A_KV_Q8_0);
     else P1A_PREP(P1A_KV_Q4_0);
 #undef P1A_PREP
-    return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+    return launched();
 }
 
 }   // namespace p1a

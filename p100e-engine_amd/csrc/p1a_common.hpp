@@ -160,6 +160,13 @@ int launch_sigmoid_mul(float * x, const float * g, size_t n, hipStream_t s);
 int launch_stream_read(const void * src, size_t bytes, hipStream_t s);   // benchmarks only
 
 void set_error(const char * fmt, ...);
+// what became of the launches since the last such question; an error is taken (left standing, the next call's launch would be blamed for it)
+inline int launched() {
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) return P1A_OK;
+    set_error("launch failed: %s", hipGetErrorString(e));
+    return P1A_E_LAUNCH;
+}
 
 // ---- wave-uniform values, scalar loads ----
 __device__ __forceinline__ int rfl(int x) { return __builtin_amdgcn_readfirstlane(x); }

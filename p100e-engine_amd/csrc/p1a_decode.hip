@@ -1088,7 +1088,7 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hi
     else if constexpr (KS != KT) go(std::integral_constant<int, 1>{}, no, yes);
     else if (gr.sb) go(std::integral_constant<int, 1>{}, yes, yes);
     else go(std::integral_constant<int, 1>{}, no, no);
-    return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+    return launched();
 }
 
 }   // namespace
@@ -1135,13 +1135,13 @@ int launch_decode(const p1a_kv & c, const decode_args & a, hipStream_t s) {
     if (rc != P1A_OK || a.skip_merge) return rc;
     merge_k<<<dim3(a.T * a.Hq, (c.D + MRG_DIMS - 1) / MRG_DIMS), 256, 0, s>>>(a.part_o, a.part_ml, a.out, a.gate, pl.nsplit, c.D, a.qbuf, a.Hq, a.T,
                                                        a.pos_rows, pl.mfma ? 32 * pl.NW : decode_any_unit(c.D));
-    return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+    return launched();
 }
 
 int launch_merge(const float * part_o, const float * part_ml, float * out, const float * gate, int NS, int D, int Hq, int T, hipStream_t s) {
     const int rpw = 256 / (D / 4), rows = T * Hq;             // (D is 64, 128 or 256 here)
     merge_rows_k<<<(rows + rpw - 1) / rpw, 256, 0, s>>>(part_o, part_ml, out, gate, NS, D, rows);
-    return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+    return launched();
 }
 
 
@@ -1170,13 +1170,13 @@ int launch_stream_read(const void * src, size_t bytes, hipStream_t s) {
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) (void) hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     stream_read_k<<<4 * (cus > 0 ? cus : 256), 512, 0, s>>>(reinterpret_cast<const f4 *>(src), bytes / 16);
-    return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+    return launched();
 }
 
 int launch_sigmoid_mul(float * x, const float * g, size_t n, hipStream_t s) {
     const size_t nb = (n + 255) / 256;
     sigmoid_mul_k<<<(unsigned) (nb > 4096 ? 4096 : (nb ? nb : 1)), 256, 0, s>>>(x, g, n);
-    return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+    return launched();
 }
 
 }   // namespace p1a

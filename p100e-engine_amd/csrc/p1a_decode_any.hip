@@ -436,7 +436,7 @@ int launch_decode_any(const p1a_kv & c, const decode_args & a, int rows_per_grou
     if (c.type == P1A_KV_F16) launch_kt<P1A_KV_F16>(P, list, grid, s);
     else if (c.type == P1A_KV_Q8_0) launch_kt<P1A_KV_Q8_0>(P, list, grid, s);
     else launch_kt<P1A_KV_Q4_0>(P, list, grid, s);
-    return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+    return launched();
 }
 
 }   // namespace p1a

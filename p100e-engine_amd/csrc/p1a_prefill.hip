@@ -978,7 +978,7 @@ int launch_pf_g(const pf_params & P, hipStream_t s) {
         if (slots > per) { Q.turn_a = per; Q.turn_b = std::min(2 * per, slots); }
     }
     prefill_k<KT, D, GROUPED, DMA><<<slots * 8, NTHR, lds, s>>>(Q);
-    return hipPeekAtLastError() == hipSuccess ? P1A_OK : P1A_E_LAUNCH;
+    return launched();
 }
 template <uint32_t KT, int D>
 int launch_pf(const pf_params & P, hipStream_t s) {
@@ -1175,7 +1175,7 @@ int launch_prefill(const p1a_kv & c, const float * q, float * out, const float *
         const unsigned blocks = (unsigned) ((items + 255) / 256);
         if (c.type == P1A_KV_Q8_0) dq_k<P1A_KV_Q8_0><<<blocks, 256, 0, s>>>(P.kc, P.vc, P.pg, n, c.Hkv, c.D, ko, vo);
         else dq_k<P1A_KV_Q4_0><<<blocks, 256, 0, s>>>(P.kc, P.vc, P.pg, n, c.Hkv, c.D, ko, vo);
-        if (hipPeekAtLastError() != hipSuccess) return P1A_E_LAUNCH;
+        if (launched() != P1A_OK) return P1A_E_LAUNCH;
         P.kc = ko; P.vc = vo;
         P.pg.pt = nullptr; P.pg.rtab = nullptr; P.pg.psh = 0; P.pg.pstride = 0;
         P.pg.rowb = (size_t) c.Hkv * c.D * 2;

@@ -57,6 +57,42 @@ def test_cpp_mirror_header_compiles():
     assert r.returncode == 0, r.stderr[-2000:]
 
 
+def test_a_refused_launch_is_told_once(tmp_path, p1a):
+    """P1A_E_LAUNCH comes with a diagnostic, and the runtime's error does not stand to be found by the next call. The runtime's launch is
+    stood in for by one that fails when told to; no GPU. In a process of its own, where the stand-in is loaded first."""
+    import subprocess
+    import sys
+    (tmp_path / "hip.c").write_text('''
+static int standing;
+int fail;
+struct d3 { unsigned x, y, z; };
+int __hipPushCallConfiguration(struct d3 g, struct d3 b, unsigned long lds, void *s) { return 0; }
+int __hipPopCallConfiguration(struct d3 *g, struct d3 *b, unsigned long *lds, void **s) { return 0; }
+int hipLaunchKernel(const void *f, unsigned long long gxy, unsigned gz, unsigned long long bxy, unsigned bz, void **a, unsigned long lds, void *s) { if (fail) standing = 9; return fail ? 9 : 0; }
+int hipPeekAtLastError(void) { return standing; }
+int hipGetLastError(void) { int e = standing; standing = 0; return e; }
+''')
+    subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "hip.c"), "-o", str(tmp_path / "hip.so")], check=True, timeout=60)
+    code = f'''
+import ctypes, importlib, sys
+sys.path.insert(0, {ROOT!r})
+H = ctypes.CDLL({str(tmp_path / "hip.so")!r}, mode=ctypes.RTLD_GLOBAL)
+p1a = importlib.import_module("p100e-engine_amd")
+b = importlib.import_module("p100e-engine_amd.binding")
+kv = b.p1a_kv(8, 100, 4, 256, 4096, 4096)
+L = p1a.lib()
+append = lambda: L.p1a_kv_append(ctypes.byref(kv), 4096, 4096, 0, None, None, 1, None)
+fail = ctypes.c_int.in_dll(H, "fail")
+assert append() == 0
+fail.value = 1
+assert append() == -4 and b"launch failed" in L.p1a_last_error(), L.p1a_last_error()
+fail.value = 0
+assert append() == 0 and H.hipPeekAtLastError() == 0
+'''
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr[-2000:]
+
+
 def test_row_tables_count_only_with_a_page_table(tmp_path):
     """pt == NULL: a contiguous cache, whatever rtab holds (include/p1a_attn.h). The kernels' view of such a cache has no row table, so
     that no kernel can read through it. Host code only: the library's internal header, compiled into a program of its own."""
