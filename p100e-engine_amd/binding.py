@@ -59,7 +59,8 @@ def _calls():
             m = importlib.import_module("._p1a_call", __package__)
         except ImportError as e:
             raise P1AError(f"_p1a_call.so is missing next to {lib_path()}: build it with `make -C p100e-engine_amd/csrc`") from e
-        m.bind(*(ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in ("p1a_attn_prep", "p1a_attn_decode_a16", "p1a_attn_prefill", "p1a_kv_append")), KVCache, _stream)
+        m.bind(*(ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in ("p1a_attn_prep", "p1a_attn_decode_a16", "p1a_attn_prefill", "p1a_kv_append")), KVCache, _stream,
+               ctypes.c_int, ctypes.c_uint32, ctypes.c_size_t, ctypes.c_float, ctypes.c_void_p, p1a_kv)
         _call = m
     return _call
 

@@ -1,8 +1,8 @@
 // The Python side of a call in native code: arguments -> the C ABI of include/p1a_attn.h. A one-row step of a small model is
 // bound by what the host does around its three launches, and half of what was not the launches was the ctypes call: 19
 // arguments converted one by one, a descriptor built field by field, a stream looked up from Python. The calls a step is made of
-// come here instead; arguments are taken as ctypes takes them (whole numbers cut to 32 bits, floats, None for a null pointer, anything
-// with data_ptr() as a device pointer), and the GIL is released around the call. One token of 4 heads of 64, prep and decode from Python:
+// come here instead; arguments are taken as ctypes takes them (whole numbers cut to 32 bits, floats, ctypes numbers of the parameter's
+// type, what _as_parameter_ stands for, None for a null pointer, anything with data_ptr() as a device pointer), and the GIL is released around the call. One token of 4 heads of 64, prep and decode from Python:
 // 18.1 us with ctypes, 15.6 so (7.7 of them the C calls, 3.5 the caller's own indexing); two layers of 24 / 4 heads of 96 34.4 -> 29.2.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -14,7 +14,7 @@
 
 namespace {
 
-PyObject * s_data_ptr, * s_struct, * s_field[11];
+PyObject * s_data_ptr, * s_struct, * s_value, * s_as_parameter, * s_field[11];
 const char * const FIELDS[11] = {"type", "n_ctx", "Hkv", "D", "k", "v", "pt", "rtab", "psh", "pstride", "_pt_off"};
 // set by bind(): the library's entry points, the class whose fields are read directly, and how the current stream is found
 decltype(&p1a_attn_prep) f_prep;
@@ -22,29 +22,81 @@ decltype(&p1a_attn_decode_a16) f_decode;
 decltype(&p1a_attn_prefill) f_prefill;
 decltype(&p1a_kv_append) f_append;
 PyObject * kv_class, * stream_of;
+enum { INT, UINT, SIZE, FLOAT, POINTER, DESC, NCLASS };
+PyObject * classes[NCLASS];   // ctypes' c_int, c_uint32, c_size_t, c_float, c_void_p, and the descriptor's Structure
 
 // (each reader does nothing once an error is set, so that the callers test for one at the end)
-int as_int(PyObject * o) {
-    if (PyErr_Occurred()) return 0;
-    if (PyFloat_Check(o)) { PyErr_SetString(PyExc_TypeError, "int expected instead of float instance"); return 0; }
-    return (int) (uint32_t) PyLong_AsUnsignedLongMask(o);
+// The value of a ctypes number, for a parameter of just that type; else null. of: its class (c_int, c_float, ...)
+PyObject * plain(PyObject * o, int of) {
+    if (PyErr_Occurred()) return nullptr;
+    const int is = PyObject_IsInstance(o, classes[of]);
+    return is == 1 ? PyObject_GetAttr(o, s_value) : nullptr;
 }
-size_t as_size(PyObject * o) {
-    if (PyErr_Occurred()) return 0;
-    if (PyFloat_Check(o)) { PyErr_SetString(PyExc_TypeError, "int expected instead of float instance"); return 0; }
-    return (size_t) PyLong_AsUnsignedLongMask(o);
+// what an argument says it stands for, or null (and the error there was stays)
+PyObject * stand_in(PyObject * o, bool argument) {
+    if (!argument || !PyErr_ExceptionMatches(PyExc_TypeError)) return nullptr;
+    PyObject * t, * v, * tb;
+    PyErr_Fetch(&t, &v, &tb);
+    PyObject * r = PyObject_GetAttr(o, s_as_parameter);
+    if (!r) { PyErr_Clear(); PyErr_Restore(t, v, tb); return nullptr; }
+    Py_XDECREF(t); Py_XDECREF(v); Py_XDECREF(tb);
+    return r;
 }
-float as_float(PyObject * o) { return PyErr_Occurred() ? 0.f : (float) PyFloat_AsDouble(o); }
-void * address(PyObject * o) { return o == Py_None ? nullptr : (void *) (uintptr_t) as_size(o); }
+uint64_t whole(PyObject * o, int of, bool argument = true) {
+    if (PyErr_Occurred()) return 0;
+    if (PyLong_CheckExact(o)) return (uint64_t) PyLong_AsUnsignedLongMask(o);
+    uint64_t r = 0;
+    if (PyObject * v = plain(o, of)) { r = whole(v, of, false); Py_DECREF(v); return r; }
+    if (PyErr_Occurred()) return 0;
+    if (PyFloat_Check(o)) PyErr_SetString(PyExc_TypeError, "int expected instead of float instance");
+    else r = (uint64_t) PyLong_AsUnsignedLongMask(o);
+    if (PyErr_Occurred())
+        if (PyObject * v = stand_in(o, argument)) { r = Py_EnterRecursiveCall(" in a call's argument") ? 0 : (r = whole(v, of), Py_LeaveRecursiveCall(), r); Py_DECREF(v); }
+    return r;
+}
+int as_int(PyObject * o) { return (int) (uint32_t) whole(o, INT); }
+size_t as_size(PyObject * o) { return (size_t) whole(o, SIZE); }
+float as_float(PyObject * o) {
+    if (PyErr_Occurred()) return 0.f;
+    if (PyFloat_CheckExact(o)) return (float) PyFloat_AS_DOUBLE(o);
+    float r = 0.f;
+    if (PyObject * v = plain(o, FLOAT)) { r = as_float(v); Py_DECREF(v); return r; }
+    if (PyErr_Occurred()) return 0.f;
+    r = (float) PyFloat_AsDouble(o);
+    if (PyErr_Occurred())
+        if (PyObject * v = stand_in(o, true)) { r = Py_EnterRecursiveCall(" in a call's argument") ? 0.f : (r = as_float(v), Py_LeaveRecursiveCall(), r); Py_DECREF(v); }
+    return r;
+}
+// a pointer: None, a Python int, a c_void_p
+void * address(PyObject * o) {
+    if (PyErr_Occurred() || o == Py_None) return nullptr;
+    if (PyLong_Check(o)) return (void *) (uintptr_t) PyLong_AsUnsignedLongMask(o);
+    void * r = nullptr;
+    if (PyObject * v = plain(o, POINTER)) { r = address(v); Py_DECREF(v); }
+    else if (!PyErr_Occurred()) PyErr_Format(PyExc_TypeError, "address expected instead of %s instance", Py_TYPE(o)->tp_name);
+    return r;
+}
+PyObject * data_ptr_of(PyObject * t) { return PyErr_Occurred() ? nullptr : PyObject_CallMethodNoArgs(t, s_data_ptr); }
 void * data_ptr(PyObject * t) {
     if (PyErr_Occurred() || t == Py_None) return nullptr;
-    PyObject * r = PyObject_CallMethodNoArgs(t, s_data_ptr);
+    PyObject * r = data_ptr_of(t);
     if (!r) return nullptr;
     void * p = address(r);
     Py_DECREF(r);
     return p;
 }
 template <typename T> T * ptr(PyObject * t) { return (T *) data_ptr(t); }
+// the page table from its entry `off` on
+const int32_t * table(PyObject * t, PyObject * off) {
+    if (PyErr_Occurred() || t == Py_None) return nullptr;
+    PyObject * r = data_ptr_of(t);
+    if (!r) return nullptr;
+    const char * p = nullptr;
+    if (PyLong_Check(r) && PyLong_Check(off)) p = (const char *) (uintptr_t) PyLong_AsUnsignedLongMask(r) + 4 * (ptrdiff_t) PyLong_AsUnsignedLongMask(off);
+    else PyErr_SetString(PyExc_TypeError, "the page table's address and offset are whole numbers");
+    Py_DECREF(r);
+    return (const int32_t *) p;
+}
 
 // the cache's descriptor as it is now: a KVCache's fields, or what its struct() gives
 bool describe(PyObject * c, p1a_kv & kv) {
@@ -53,10 +105,10 @@ bool describe(PyObject * c, p1a_kv & kv) {
         PyObject * st = PyObject_CallMethodNoArgs(c, s_struct);
         if (!st) return false;
         Py_buffer b;
-        const bool ok = PyObject_GetBuffer(st, &b, PyBUF_SIMPLE) == 0;
-        if (ok) {
-            if (b.len == (Py_ssize_t) sizeof kv) memcpy(&kv, b.buf, sizeof kv);
-            else PyErr_SetString(PyExc_TypeError, "struct() gave no p1a_kv");
+        const int is = PyObject_IsInstance(st, classes[DESC]);
+        if (is == 0) PyErr_SetString(PyExc_TypeError, "struct() gave no p1a_kv");
+        if (is == 1 && PyObject_GetBuffer(st, &b, PyBUF_SIMPLE) == 0) {
+            memcpy(&kv, b.buf, sizeof kv);
             PyBuffer_Release(&b);
         }
         Py_DECREF(st);
@@ -65,14 +117,13 @@ bool describe(PyObject * c, p1a_kv & kv) {
     PyObject * f[11] = {};
     for (int i = 0; i < 11 && !PyErr_Occurred(); ++i) f[i] = PyObject_GetAttr(c, s_field[i]);
     if (!PyErr_Occurred()) {
-        kv.type = (uint32_t) as_int(f[0]);
-        kv.n_ctx = as_int(f[1]); kv.Hkv = as_int(f[2]); kv.D = as_int(f[3]);
+        kv.type = (uint32_t) whole(f[0], UINT, false);
+        kv.n_ctx = (int) whole(f[1], INT, false); kv.Hkv = (int) whole(f[2], INT, false); kv.D = (int) whole(f[3], INT, false);
         kv.k = address(f[4]); kv.v = address(f[5]);
-        const char * pt = ptr<char>(f[6]);
-        kv.pt = (const int32_t *) (f[6] == Py_None ? nullptr : pt + 4 * (ptrdiff_t) as_int(f[10]));
+        kv.pt = table(f[6], f[10]);
         kv.rtab = ptr<int32_t>(f[7]);
-        kv.psh = as_int(f[8]);
-        kv.pstride = as_size(f[9]);
+        kv.psh = (int) whole(f[8], INT, false);
+        kv.pstride = (size_t) whole(f[9], SIZE, false);
     }
     for (PyObject * x : f) Py_XDECREF(x);
     return !PyErr_Occurred();
@@ -147,9 +198,10 @@ PyObject * append(PyObject *, PyObject * const * a, Py_ssize_t n) {
     void * s = stream();
     P1A_CALL(f_append(&kv, k, v, p0, p0_dev, pos, T, s));
 }
-// (addresses of p1a_attn_prep, p1a_attn_decode_a16, p1a_attn_prefill, p1a_kv_append; the cache class; the current stream's handle)
+// (addresses of p1a_attn_prep, p1a_attn_decode_a16, p1a_attn_prefill, p1a_kv_append; the cache class; the current stream's handle; the
+// ctypes classes)
 PyObject * bind(PyObject *, PyObject * const * a, Py_ssize_t n) {
-    if (!takes(n, 6)) return nullptr;
+    if (!takes(n, 6 + NCLASS)) return nullptr;
     f_prep = (decltype(f_prep)) address(a[0]);
     f_decode = (decltype(f_decode)) address(a[1]);
     f_prefill = (decltype(f_prefill)) address(a[2]);
@@ -157,6 +209,7 @@ PyObject * bind(PyObject *, PyObject * const * a, Py_ssize_t n) {
     if (PyErr_Occurred()) return nullptr;
     Py_INCREF(a[4]); Py_XSETREF(kv_class, a[4]);
     Py_INCREF(a[5]); Py_XSETREF(stream_of, a[5]);
+    for (int i = 0; i < NCLASS; ++i) { Py_INCREF(a[6 + i]); Py_XSETREF(classes[i], a[6 + i]); }
     Py_RETURN_NONE;
 }
 
@@ -171,6 +224,8 @@ PyModuleDef module_ = {PyModuleDef_HEAD_INIT, "_p1a_call", nullptr, -1, methods,
 PyMODINIT_FUNC PyInit__p1a_call(void) {
     s_data_ptr = PyUnicode_InternFromString("data_ptr");
     s_struct = PyUnicode_InternFromString("struct");
+    s_value = PyUnicode_InternFromString("value");
+    s_as_parameter = PyUnicode_InternFromString("_as_parameter_");
     for (int i = 0; i < 11; ++i) s_field[i] = PyUnicode_InternFromString(FIELDS[i]);
     return PyModule_Create(&module_);
 }

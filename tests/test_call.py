@@ -2,7 +2,9 @@
 entry points are stood in for by callbacks that note what they get; no GPU."""
 import ctypes
 import importlib
+from fractions import Fraction
 
+import numpy as np
 import pytest
 
 p1a = importlib.import_module("p100e-engine_amd")
@@ -27,18 +29,22 @@ class Tensor:
         return 4
 
 
+class Calls(list):
+    pass
+
+
 @pytest.fixture
 def calls(monkeypatch):
-    got = []
+    got = Calls()
 
     def stand_in(types):
         def f(*a):
             got.append([{n: getattr(x.contents, n) for n, _ in b.p1a_kv._fields_} if isinstance(x, KV) else x for x in a])
             return 0
         return ctypes.CFUNCTYPE(I, *types)(f)
-    kept = {n: stand_in(t) for n, t in SIGNATURES.items()}
+    kept = got.kept = {n: stand_in(t) for n, t in SIGNATURES.items()}
     m = b._calls()
-    m.bind(*(ctypes.cast(kept[n], VP).value for n in SIGNATURES), b.KVCache, lambda: 0x7770)
+    m.bind(*(ctypes.cast(kept[n], VP).value for n in SIGNATURES), b.KVCache, lambda: 0x7770, I, ctypes.c_uint32, SZ, F, VP, b.p1a_kv)
     yield got
     b._call = None
     b._calls()                                                 # the library's own entry points again
@@ -85,3 +91,61 @@ def test_what_is_no_argument_is_refused(calls, change):
     with pytest.raises((TypeError, AttributeError, ctypes.ArgumentError)):
         p1a.attn_decode(**{**a, **change})
     assert not calls
+
+
+class Stands:
+    def __init__(self, x):
+        self._as_parameter_ = x
+
+
+class Sub(b.p1a_kv):
+    pass
+
+
+NUMBERS = [3, True, -1, (1 << 40) + 5, np.int32(7), np.int64(-2), np.uint8(200), I(9), I(-9), ctypes.c_long(4), ctypes.c_uint32(4), ctypes.c_short(4), F(2.0), VP(64), Stands(11),
+           Stands(Stands(12)), Stands(I(13)), Stands(1.5), 1.5, np.float32(2), np.float64(2), None, "3", b"3", [3], Fraction(3), ctypes.c_size_t(1 << 40)]
+REALS = [0.5, 1, True, np.float32(0.25), np.float64(0.75), F(1.5), ctypes.c_double(1.5), I(1), Stands(0.5), Stands(F(2.5)), Fraction(1, 4), None, "0.5", [1.0], 1e300]
+ADDRESSES = [0x1000, 0, True, -16, None, VP(0x2000), VP(None), np.int64(0x3000), 1.0, I(5)]
+
+
+def same(what, by_ctypes, ours, calls):
+    """both go through, with the same arguments, or both raise"""
+    def go(f):
+        del calls[:]
+        try:
+            f()
+        except (TypeError, ctypes.ArgumentError):
+            assert not calls
+            return "refused"
+        return calls[:]
+    want = go(by_ctypes)
+    assert go(ours) == want, what
+    return want != "refused"
+
+
+def test_arguments_are_taken_as_ctypes_takes_them(calls):
+    """ctypes itself is the oracle: the same call through its own prototype and, for the descriptor, its Structure. Whole numbers (cut to
+    the parameter's width), ctypes numbers of the very type, what _as_parameter_ stands for; all else refused."""
+    ctype = calls.kept
+    t = [Tensor(0x1000 + 16 * i) for i in range(8)]
+    c = p1a.KVCache(p1a.KV_F16, 100, 2, 64, 0x100, 0x200)
+    s, kv = 0x7770, ctypes.byref(c.struct())
+    taken = 0
+    for x in NUMBERS:                                          # c_int and c_size_t parameters
+        taken += same(("T", x), lambda: ctype["p1a_attn_decode_a16"](0x1000, kv, 0x1010, None, None, x, 0, None, None, 0, 4, 1.0, s), lambda: p1a.attn_decode(t[0], c, t[1], x, 0, 4, 1.0), calls)
+        same(("bytes", x), lambda: ctype["p1a_attn_prefill"](0x1000, kv, 0x1010, None, 5, 0, 4, 1.0, 0x1020, x, s), lambda: b._calls().prefill(t[0], c, t[1], None, 5, 0, 4, 1.0, t[2], x), calls)
+    for x in REALS:
+        taken += same(("scale", x), lambda: ctype["p1a_attn_decode_a16"](0x1000, kv, 0x1010, None, None, 1, 0, None, None, 0, 4, x, s), lambda: p1a.attn_decode(t[0], c, t[1], 1, 0, 4, x), calls)
+    for x in ADDRESSES:                                        # what data_ptr() gives
+        taken += same(("data_ptr", x), lambda: ctype["p1a_attn_decode_a16"](x, kv, 0x1010, None, None, 1, 0, None, None, 0, 4, 1.0, s), lambda: p1a.attn_decode(Tensor(x), c, t[1], 1, 0, 4, 1.0), calls)
+    decode = ctype["p1a_attn_decode_a16"]
+    fields = [("type", NUMBERS), ("n_ctx", NUMBERS), ("D", NUMBERS), ("psh", NUMBERS), ("pstride", NUMBERS), ("k", ADDRESSES), ("v", ADDRESSES),
+              ("pt", [Tensor(x) for x in ADDRESSES] + [None]), ("rtab", [Tensor(x) for x in ADDRESSES] + [None]), ("_pt_off", [0, 5, True, -3, 1 << 33, np.int64(2), I(2), 1.0, None])]
+    for name, values in fields:
+        for x in values:
+            d = p1a.KVCache(p1a.KV_F16, 100, 2, 64, 0x100, 0x200, Tensor(0x5000), None, 4, 4096)
+            setattr(d, name, x)
+            taken += same((name, x), lambda: decode(0x1000, ctypes.byref(d.struct()), 0x1010, None, None, 1, 0, None, None, 0, 4, 1.0, s), lambda: p1a.attn_decode(t[0], d, t[1], 1, 0, 4, 1.0), calls)
+    for x in [c.struct(), Sub(1, 2, 3, 64, 16, 16), bytes(64), bytearray(64), (ctypes.c_uint8 * 64)(), None, 5]:   # what struct() gives
+        taken += same(("struct", x), lambda: decode(0x1000, ctypes.byref(x), 0x1010, None, None, 1, 0, None, None, 0, 4, 1.0, s), lambda: p1a.attn_decode(t[0], b.KVDesc(x), t[1], 1, 0, 4, 1.0), calls)
+    assert taken > 90
