@@ -2,7 +2,7 @@
 (src/fast/attn.cuh:34-70 of the reference tree): kv_append, kv_append_dev, attn_decode, attn_decode_dev,
 attn_decode_rows, attn_prefill; attn_prep is src/fast/fused.cuh:101-113."""
 import ctypes
-import importlib
+import importlib.util
 import os
 
 KV_F16, KV_Q4_0, KV_Q8_0 = 1, 2, 8
@@ -46,6 +46,10 @@ def lib_path():
     return os.path.join(os.path.dirname(os.path.abspath(__file__)), "libp1a_attn.so")
 
 
+def call_path():
+    return os.path.join(os.path.dirname(os.path.abspath(__file__)), "_p1a_call.so")
+
+
 _lib = None
 _call = None      # the native side of the calls a step is made of (csrc/p1a_call.cpp)
 
@@ -55,10 +59,12 @@ def _calls():
     global _call
     if _call is None:
         L = lib()
-        try:
-            m = importlib.import_module("._p1a_call", __package__)
+        try:                                                   # (by its path, as the library: this file is also loaded outside the package)
+            spec = importlib.util.spec_from_file_location("_p1a_call", call_path())
+            m = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(m)
         except ImportError as e:
-            raise P1AError(f"_p1a_call.so is missing next to {lib_path()}: build it with `make -C p100e-engine_amd/csrc`") from e
+            raise P1AError(f"{call_path()} is missing or not for this Python: build it with `make -C p100e-engine_amd/csrc`") from e
         m.bind(*(ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in ("p1a_attn_prep", "p1a_attn_decode_a16", "p1a_attn_prefill", "p1a_kv_append")), KVCache, _stream,
                ctypes.c_int, ctypes.c_uint32, ctypes.c_size_t, ctypes.c_float, ctypes.c_void_p, p1a_kv)
         _call = m

@@ -2,6 +2,9 @@
 entry points are stood in for by callbacks that note what they get; no GPU."""
 import ctypes
 import importlib
+import os
+import subprocess
+import sys
 from fractions import Fraction
 
 import numpy as np
@@ -149,3 +152,27 @@ def test_arguments_are_taken_as_ctypes_takes_them(calls):
     for x in [c.struct(), Sub(1, 2, 3, 64, 16, 16), bytes(64), bytearray(64), (ctypes.c_uint8 * 64)(), None, 5]:   # what struct() gives
         taken += same(("struct", x), lambda: decode(0x1000, ctypes.byref(x), 0x1010, None, None, 1, 0, None, None, 0, 4, 1.0, s), lambda: p1a.attn_decode(t[0], b.KVDesc(x), t[1], 1, 0, 4, 1.0), calls)
     assert taken > 90
+
+
+def test_the_binding_alone():
+    """binding.py loaded by its path, outside the package, finds its native side as it finds the library, and each of two that are
+    loaded keeps its own"""
+    code = f"""
+import importlib, importlib.util, sys
+sys.path.insert(0, {os.path.dirname(os.path.dirname(os.path.abspath(b.__file__)))!r})
+spec = importlib.util.spec_from_file_location("alone", {b.__file__!r})
+m = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(m)
+for x in (m, importlib.import_module("p100e-engine_amd.binding")):
+    x._stream = lambda: None                                   # (no GPU here)
+first = importlib.import_module("p100e-engine_amd.binding")
+for x in (first, m, first):                                    # each with its own classes, in turn
+    try:
+        x.attn_decode(None, x.KVDesc(x.p1a_kv(8, 100, 4, 256, 4096, 4096)), None, 1, 0, 24, 1.0)
+    except x.P1AError as e:
+        assert "null q/out" in str(e), e
+    else:
+        assert False
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr[-2000:]
