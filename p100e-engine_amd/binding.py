@@ -2,8 +2,10 @@
 (src/fast/attn.cuh:34-70 of the reference tree): kv_append, kv_append_dev, attn_decode, attn_decode_dev,
 attn_decode_rows, attn_prefill; attn_prep is src/fast/fused.cuh:101-113."""
 import ctypes
+import importlib.machinery
 import importlib.util
 import os
+import sys
 
 KV_F16, KV_Q4_0, KV_Q8_0 = 1, 2, 8
 
@@ -47,7 +49,8 @@ def lib_path():
 
 
 def call_path():
-    return os.path.join(os.path.dirname(os.path.abspath(__file__)), "_p1a_call.so")
+    """the native side of the calls as built for this Python (the name says which: under another one it is missing, not misread)"""
+    return os.path.join(os.path.dirname(os.path.abspath(__file__)), "_p1a_call" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
 
 _lib = None
@@ -55,7 +58,7 @@ _call = None      # the native side of the calls a step is made of (csrc/p1a_cal
 
 
 def _calls():
-    """Load _p1a_call.so (built with libp1a_attn.so) and hand it the library's entry points."""
+    """Load the _p1a_call module (built with libp1a_attn.so) and hand it the library's entry points."""
     global _call
     if _call is None:
         L = lib()
@@ -64,7 +67,7 @@ def _calls():
             m = importlib.util.module_from_spec(spec)
             spec.loader.exec_module(m)
         except ImportError as e:
-            raise P1AError(f"{call_path()} is missing or not for this Python: build it with `make -C p100e-engine_amd/csrc`") from e
+            raise P1AError(f"{call_path()} is missing or not for this Python: build it with `make -C p100e-engine_amd/csrc PYTHON={sys.executable}`") from e
         m.bind(*(ctypes.cast(getattr(L, n), ctypes.c_void_p).value for n in ("p1a_attn_prep", "p1a_attn_decode_a16", "p1a_attn_prefill", "p1a_kv_append")), KVCache, _stream,
                ctypes.c_int, ctypes.c_uint32, ctypes.c_size_t, ctypes.c_float, ctypes.c_void_p, p1a_kv)
         _call = m

@@ -5,6 +5,7 @@ import importlib
 import os
 import subprocess
 import sys
+import sysconfig
 from fractions import Fraction
 
 import numpy as np
@@ -176,3 +177,13 @@ for x in (first, m, first):                                    # each with its o
 """
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stderr[-2000:]
+
+
+def test_the_native_side_is_named_for_its_python(tmp_path):
+    """an extension module without an ABI tag would also be loaded by a Python whose objects are laid out differently"""
+    assert b.call_path().endswith(sysconfig.get_config_var("EXT_SUFFIX")) and os.path.exists(b.call_path())
+    other = tmp_path / "python"
+    other.write_text("#!/bin/sh\ncase \"$2\" in *EXTENSION_SUFFIXES*) echo .cpython-399-other.so ;; *) echo /nowhere ;; esac\n")
+    other.chmod(0o755)
+    r = subprocess.run(["make", "-n", "-B", "-C", os.path.join(os.path.dirname(b.__file__), "csrc"), f"PYTHON={other}"], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and "-I/nowhere" in r.stdout and "-o ../_p1a_call.cpython-399-other.so" in r.stdout, r.stdout + r.stderr
