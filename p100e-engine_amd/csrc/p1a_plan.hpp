@@ -87,9 +87,13 @@ inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv,
     // for calls of many - measured slower on every shape tried, e.g. 8 x 4 rows q4_0 at 8 K 72 -> 60 us with one.)
     r.sb = !staged && pl.NT == 1 && (long long) pl.nsplit * Hkv * groups >= 2LL * cus;
     // The list (see dec_mfma_k) costs a workgroup some 0.2 us before its first request. Where two workgroups share a compute unit that hides,
-    // and every call of several sequences takes it (110 calls of 2 ... 32 sequences drawn over 4 ... 131072 keys, D = 256 and f16:
-    // 0.98 - 1.6 times as fast, 1.1 in the mean). Where one has a unit to itself (two column tiles, staged tiles) it shows: calls of
-    // four sequences and more whose page-table rows cannot hold the keys that half of the streams begin with (8 x 4 rows of 300
+    // and every call of several row groups takes it. Several sequences (110 calls of 2 ... 32 drawn over 4 ... 131072 keys, D = 256 and f16):
+    // 0.98 - 1.6 times as fast, 1.1 in the mean. One sequence of 5 ... 32 rows (200 calls over 200, 3000 and 20000 keys, six head shapes):
+    // 0.84 - 1.6, 1.1 in the mean - the row groups of a stream are side by side on an XCD, which long sequences gain from (f16, 32 / 8 of 128, 13 rows
+    // of 20000 keys 150 -> 98 us, 8 rows 33 -> 26; 200 keys 14.1 -> 11.9); what loses most are row counts that only groups of one
+    // divide (q4_0, 16 / 16 of 256, 31 rows of 3000 keys 143 -> 166, f16, 16 / 4 of 64, 20000 keys 80 -> 95). Where one has a unit to itself (two
+    // column tiles, staged tiles) it shows: calls of four row groups and more whose page-table rows - as wide as n_ctx says, whatever
+    // the sequences hold - cannot hold the keys that half of the streams begin with (8 x 4 rows of 300
     // ... 5000 keys, q8_0, 24 / 4 heads of 256, two layers 72.8 -> 62.1 us, 16 of 300 ... 5000, 32 / 8 of 128 104 -> 93; with every
     // stream live 8 of 18797, q8_0, 24 / 4 of 128, four layers would go from 349 to 360).
     const long long once = (long long) pl.nsplit * 32 * pl.NW;   // the keys that every stream holds a unit of
