@@ -8,6 +8,7 @@ import torch
 import _inputs as I
 import _oracle as O
 from _gpu import Pool, check, dev
+from _plan import plan
 
 pytestmark = pytest.mark.gpu
 TYPES = [O.KV_F16, O.KV_Q8_0, O.KV_Q4_0]
@@ -414,8 +415,13 @@ MIXED = [1, 255, 256, 257, 2304, 0, 700, 9000]                 # edges of a unit
 def test_rows_of_sequences_of_any_length(p1a, kv_type, Hq, Hkv, D, psh, lens, rows):
     """Sequences of no key, one, a unit more or less and more than all streams hold once, in calls of every way the streams that hold
     keys are found: up to 4, 7, 8, 16 and 32 rows, a number that is no multiple of eight, several rows and row groups a sequence,
-    head counts that are no power of two, workgroups that take one stream (all builds, the any-shape kernel's too) and several (17 sequences and more); the
-    32 sequences of 4200 keys go round the list more than once. Every row == the row of the sequence's own call, bit for bit."""
+    head counts that are no power of two, workgroups that take one stream (all builds, the any-shape kernel's too) and may take several
+    (test_workgroups_that_take_several_streams holds that they do). Every row == the row of the sequence's own call, bit for bit."""
+    rows_against_calls_of_their_own(p1a, kv_type, Hq, Hkv, D, psh, lens, rows)
+
+
+def rows_against_calls_of_their_own(p1a, kv_type, Hq, Hkv, D, psh, lens, rows, cut=0):
+    """sequences of `lens` keys, `rows` rows each, in one call - the last sequence without its last `cut` rows"""
     n, scale, ps = len(lens), D ** -0.5, 1 << psh
     g = torch.Generator(device="cuda").manual_seed(n * 1000 + rows)
     need = [-(-max(x, 1) // ps) + 1 for x in lens]
@@ -428,10 +434,10 @@ def test_rows_of_sequences_of_any_length(p1a, kv_type, Hq, Hkv, D, psh, lens, ro
     for s, x in enumerate(lens):
         if x:
             p1a.kv_append(c.slot(s, maxp), torch.randn((x, Hkv, D), generator=g, device="cuda"), torch.randn((x, Hkv, D), generator=g, device="cuda"), 0, x)
-    T = n * rows
+    T = n * rows - cut
     q, gate = torch.randn((T, Hq, D), generator=g, device="cuda"), torch.randn((T, Hq, D), generator=g, device="cuda")
-    pos = [max(x - rows, -1) + r if x >= rows else x - 1 for x in lens for r in range(rows)]
-    rtab = torch.tensor([-1] + [s * maxp for s in range(n) for _ in range(rows)], dtype=torch.int32, device="cuda")[1:]   # (4-byte aligned, no more)
+    pos = [max(x - rows, -1) + r if x >= rows else x - 1 for x in lens for r in range(rows)][:T]
+    rtab = torch.tensor([-1] + [s * maxp for s in range(n) for _ in range(rows)][:T], dtype=torch.int32, device="cuda")[1:]   # (4-byte aligned, no more)
     out = torch.full((T, Hq, D), 7.0, device="cuda")
     p1a.attn_decode_rows(q, c.with_rows(rtab), out, T, torch.tensor([-1] + pos, dtype=torch.int32, device="cuda")[1:], Hq, scale, gate=gate, rows_per_seq=rows)
     one = torch.empty((1, Hq, D), device="cuda")
@@ -441,3 +447,38 @@ def test_rows_of_sequences_of_any_length(p1a, kv_type, Hq, Hkv, D, psh, lens, ro
             continue
         p1a.attn_decode(q[t:t + 1], c.slot(t // rows, maxp), one, 1, pos[t], Hq, scale, gate=gate[t:t + 1])
         assert torch.equal(out[t:t + 1], one), (t, pos[t])
+
+
+@pytest.mark.parametrize("kv_type,Hq,Hkv,D,psh,lens,rows,cut", [
+    (O.KV_Q4_0, 12, 4, 256, 8, MIXED[:4], 5, 4), (O.KV_F16, 8, 8, 64, 6, [900, 300, 5000], 6, 4), (O.KV_F16, 16, 8, 128, 4, [700, 60], 3, 2),   # one stream a workgroup
+    (O.KV_Q8_0, 8, 8, 64, 6, [3900 - 11 * i for i in range(5)], 6, 4), (O.KV_Q8_0, 40, 8, 256, 6, [3900 - 11 * i for i in range(8)], 4, 3),   # several
+    (O.KV_Q4_0, 40, 2, 192, 6, MIXED[1:5], 3, 2), (O.KV_Q8_0, 24, 4, 96, 8, [300, 2000, 700], 4, 3)])                                        # the any-shape kernel's list
+def test_last_sequence_of_fewer_rows(p1a, kv_type, Hq, Hkv, D, psh, lens, rows, cut):
+    """T that is no multiple of rows_per_seq: whole row groups of the last sequence are missing, or rows of its
+    last group are"""
+    rows_against_calls_of_their_own(p1a, kv_type, Hq, Hkv, D, psh, lens, rows, cut)
+
+
+@pytest.mark.parametrize("kv_type,Hq,Hkv,D,psh,n,rows", [(O.KV_F16, 16, 4, 64, 6, 700, 31), (O.KV_Q8_0, 8, 8, 256, 8, 3000, 32), (O.KV_F16, 32, 8, 128, 4, 520, 13), (O.KV_Q4_0, 16, 16, 256, 8, 9000, 7),
+                                                         (O.KV_Q8_0, 8, 8, 64, 6, 1500, 24), (O.KV_Q8_0, 24, 4, 96, 8, 4000, 16)])
+def test_many_rows_of_one_sequence(p1a, kv_type, Hq, Hkv, D, psh, n, rows):
+    rows_against_calls_of_their_own(p1a, kv_type, Hq, Hkv, D, psh, [n], rows)
+
+
+# every build of dec_mfma_k whose workgroups take several streams: two to a compute unit, staged tiles, two column tiles
+LONG, SHORT = [3900 - 11 * i for i in range(8)], [1900 - 7 * i for i in range(32)]
+SEVERAL = [(O.KV_Q8_0, 8, 8, 256, 6, SHORT, 1), (O.KV_Q4_0, 8, 8, 256, 6, SHORT, 1), (O.KV_F16, 8, 8, 128, 4, SHORT, 1), (O.KV_F16, 8, 8, 64, 4, SHORT, 1),
+           (O.KV_F16, 8, 8, 256, 5, [x // 2 for x in SHORT], 1), (O.KV_Q8_0, 40, 8, 256, 6, LONG, 4), (O.KV_F16, 40, 8, 256, 6, [x // 2 for x in LONG], 4),
+           (O.KV_F16, 40, 8, 128, 6, LONG, 4), (O.KV_F16, 40, 8, 64, 6, LONG, 4)]
+SEVERAL += [(kv, Hq, 8, D, 6, LONG, rows) for kv in (O.KV_Q8_0, O.KV_Q4_0) for D in (128, 64) for Hq, rows in ((16, 1), (40, 4))]
+
+
+@pytest.mark.parametrize("kv_type,Hq,Hkv,D,psh,lens,rows", SEVERAL)
+def test_workgroups_that_take_several_streams(p1a, kv_type, Hq, Hkv, D, psh, lens, rows):
+    """more streams hold keys than the grid takes at once, in each of the 17 looping builds: a second item reuses the LDS of the first and
+    reads the arguments again"""
+    need = max(-(-x // (1 << psh)) + 1 for x in lens)
+    p = plan(kv_type, Hq, Hkv, D, need << psh, len(lens) * rows, rows, cus=torch.cuda.get_device_properties(0).multi_processor_count)
+    live = sum(min(-(-x // (32 * p["NW"])), p["nsplit"]) for x in lens)
+    assert p["list"] and p["loop"] and live > p["x"] // (Hkv * p["GPS"]), (p, live)
+    rows_against_calls_of_their_own(p1a, kv_type, Hq, Hkv, D, psh, lens, rows)
