@@ -2,7 +2,7 @@
 
 The product is the C-ABI shared library ``libp1a_attn.so`` (sources in ``csrc/``, declarations in
 ``include/p1a_attn.h``) and its C++ mirror of the reference surface (``include/p100e_fast_attn.hpp``).
-This Python package is only the ctypes binding the tests, the smoke check and the benchmark use to drive that
+This Python package is only the binding the tests, the smoke check and the benchmark use to drive that
 library with torch tensors as device memory. It never computes anything itself: if the library is missing or a
 call is refused, it raises.
 """

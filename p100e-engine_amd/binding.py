@@ -1,4 +1,4 @@
-"""ctypes binding of include/p1a_attn.h. Function names follow the reference's C++ surface
+"""Python binding of include/p1a_attn.h: ctypes, and for the calls of a step a native module (csrc/p1a_call.cpp). Function names follow the reference's C++ surface
 (src/fast/attn.cuh:34-70 of the reference tree): kv_append, kv_append_dev, attn_decode, attn_decode_dev,
 attn_decode_rows, attn_prefill; attn_prep is src/fast/fused.cuh:101-113."""
 import ctypes

@@ -1,7 +1,8 @@
 // Split-K paged-KV decode / MTP-verify attention for gfx950 (MI355X).
 //
 // Work decomposition
-//   grid = (nsplit * kv heads, row groups), block = NW waves (8, or 4 when a tile is large). A row group is up to 4
+//   grid = (nsplit * kv heads, row groups) - calls of several row groups also count through the streams that hold keys instead
+//   (plan_grid, p1a_plan.hpp) -, block = NW waves (8, or 4 when a tile is large). A row group is up to 4
 //   query rows of ONE sequence (the tokens of a verify block); its GQA * rows query rows are the columns of 16-wide
 //   MFMA tiles, so the group's KV is read once. A workgroup owns one kv head; in unit u (32 * NW positions) wave w owns
 //   the 32 consecutive positions 32 w .., which it walks as two 16-key tiles; split stream s owns the units s,
@@ -214,7 +215,8 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     // those of two units ahead of the others so that no unit gets two of them; number q goes to XCD q mod 8, one workgroup for every kv head and
     // row group of it, and workgroups left over come last. (LOOP: one takes the numbers q, q + q_step, ...) Same partition of
     // the keys, same bits. q8_0, 24 / 4 heads of 256, two layers with prep and merge: 8 sequences of 1024 keys 47 -> 38 us, 16 of 300 ... 5000
-    // 68 -> 58, 2 of 20000 74 -> 69, 32 of 256 61 -> 43; what it does not help costs at most 2 % (4 of 4000 ... 16000, two rows each 75 -> 77).
+    // 68 -> 58, 2 of 20000 74 -> 69, 32 of 256 61 -> 43; what it does not help costs 2 ... 6 % (4 of 4000 ... 16000, two rows each 75 -> 77; 4 x 4 rows of 4252, 272 live workgroups
+    // for 256 units), a sequence of many rows that only groups of one divide up to 16 (plan_grid).
     int hg = 0, gsub = 0, q = 0, q_step = 0, q_a = 0, q_end = 0, rt_lanes = 0;
     uint32_t u_sum = 0;
     if constexpr (LIST) {

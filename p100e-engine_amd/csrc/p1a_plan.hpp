@@ -83,8 +83,6 @@ inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv,
     // A call of at least two workgroups per CU whose row groups fit one column tile takes the single-buffered variant, two
     // workgroups to a CU (same partials, bit for bit; measured at 24 / 4 heads, D = 256: 8 q8_0 slots of 1 K ... 27 K 56 ->
     // 47 us, 4 x 64 K q4_0 single rows 92 -> 73 us, 16 x 2 rows q4_0 at 16 K 143 -> 115 us, 32 slots of 2 ... 5 K 104 -> 71 us).
-    // (A workgroup walks ONE split stream whatever the call: letting it walk several in turn - fewer, longer workgroups
-    // for calls of many - measured slower on every shape tried, e.g. 8 x 4 rows q4_0 at 8 K 72 -> 60 us with one.)
     r.sb = !staged && pl.NT == 1 && (long long) pl.nsplit * Hkv * groups >= 2LL * cus;
     // The list (see dec_mfma_k) costs a workgroup some 0.2 us before its first request. Where two workgroups share a compute unit that hides,
     // and every call of several row groups takes it. Several sequences (110 calls of 2 ... 32 drawn over 4 ... 131072 keys, D = 256 and f16):
@@ -112,6 +110,8 @@ inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv,
     //   One to a unit: more than two for every compute unit; at least half of the streams are known to be empty there (without the list, a
     //   workgroup for every stream, two for every unit: 8 x 4 rows of 300 ... 5000, q8_0, 24 / 4 of 256 73.6, 62.7, 56.5 us; 16 of 256, 32 / 8 of 128 53, 45, 39;
     //   32 of 256 77, 71, 43; q4_0, 24 / 4 of 128, 16 of 60 ... 1500 58.5, 46.9, 40.3).
+    // All of these are times with page-table rows as wide as the sequences. Rows of 32768 positions, a server's limit, take the other route
+    // whatever the sequences hold: 72.2, 53.9, 78.3 and 58.6 us for the last four, 45.8 for 32 of 1024 (f16, 16 / 4 of 64).
     const long long most = (r.sb ? 16LL : 2LL) * cus / (8 * inner);
     const bool can_loop = pl.NT == 2 ? staged || type != P1A_KV_Q4_0 : staged || r.sb;   // (q4_0 with two column tiles has no register left for it)
     r.loop = can_loop && nq > most;

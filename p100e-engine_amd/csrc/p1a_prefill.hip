@@ -919,7 +919,10 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
                 for (int x = 0; x < 4; ++x) v[i][x] *= sigmoid(gt[i][x]);
         }
         // (f16 tiles, D = 256: results, which nothing here reads again, go past the caches: 600 tokens behind 300, 24 / 4 heads, f16 53.9 -> 51.1 us, 2000, 32 / 8, q8_0
-        // 157 -> 151. Not partials, which the merge reads at once: q4_0, 77 behind 16000 71.6 -> 73.2.)
+        // 157 -> 151. What reads them next gives most of it back: the first 4096 of 24 / 4, f16, alone 252 -> 239, with a cast to f16 behind the call 271.8
+        // and 272.5, with that and a product of 5120 columns 525.8 and 524.8; seven calls of 600 ... 4096 tokens alone 1.02 times as fast in the
+        // mean, with the cast 0.996 (0.988 - 1.009), with both 1.004 (0.997 - 1.018).
+        // Not partials, which the merge reads at once: q4_0, 77 behind 16000 71.6 -> 73.2.)
         if constexpr (DMA && PAIR) {
             f4 * po[N8];
 #pragma unroll
@@ -969,10 +972,10 @@ int launch_pf_g(const pf_params & P, hipStream_t s) {
     const int slots = P.run ? P.run : ((units + 7) / 8) * P.bpg;
     pf_params Q = P;
     Q.turn_a = Q.turn_b = 0;
-    // Two workgroups to a compute unit, which an XCD deals them to in turn: the unit of slot s also gets slot s + 32. Longest blocks first
+    // Two workgroups to a compute unit, which an XCD deals them to in turn: the unit of slot s also gets slot s + per. Longest blocks first
     // would give it two long ones (63 blocks of 1 ... 32 tiles: 32 + 16 ... 17 + 1 tiles); the second round is taken in reverse
-    // (33 each). First 2003 tokens, 32 / 8 heads of 128, f16, prep included 85.0 -> 81.2 us, 24 / 4 of 64 37.1 -> 34.5; what fits one round or
-    // takes many is as it was.
+    // (33 each). First 2003 tokens, 32 / 8 heads of 128, f16, prep included 85.0 -> 81.2 us, 24 / 4 of 64 37.1 -> 34.5. What fits
+    // one round is as it was; calls of more than two have their second one reversed too and are level (70 drawn prefills 0.98 - 1.10).
     if (pf_solo(D, DMA) && P.nks == 1) {
         const int per = std::max(cu_count() / 8, 1);          // compute units of an XCD
         if (slots > per) { Q.turn_a = per; Q.turn_b = std::min(2 * per, slots); }

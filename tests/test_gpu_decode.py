@@ -253,8 +253,8 @@ def test_widest_row_groups(p1a, kv_type, Hq, Hkv, rows):
 
 
 def test_descriptor_n_ctx_only_bounds(p1a):
-    """n_ctx of the descriptor is the caller's word; the kernel uses it to bound an early page-table read, never to pick a
-    page: an understated (or missing) n_ctx gives the same bits"""
+    """n_ctx of the descriptor is the caller's word: it bounds an early page-table read and chooses how a call of several rows is dealt to
+    the device, never a page: an understated (or missing) n_ctx gives the same bits"""
     Hq, Hkv, D, psh, n = 24, 4, 256, 5, 3000
     pool = Pool(p1a, O.KV_Q8_0, Hq, Hkv, D, psh, [n], seed=71)
     dq = dev(I.normal(I.rng(72), (2, Hq, D)))
@@ -463,6 +463,30 @@ def test_last_sequence_of_fewer_rows(p1a, kv_type, Hq, Hkv, D, psh, lens, rows, 
                                                          (O.KV_Q8_0, 8, 8, 64, 6, 1500, 24), (O.KV_Q8_0, 24, 4, 96, 8, 4000, 16)])
 def test_many_rows_of_one_sequence(p1a, kv_type, Hq, Hkv, D, psh, n, rows):
     rows_against_calls_of_their_own(p1a, kv_type, Hq, Hkv, D, psh, [n], rows)
+
+
+@pytest.mark.parametrize("kv_type,Hq,D,lens", [(O.KV_Q8_0, 8, 256, [2400 - 31 * i for i in range(24)]), (O.KV_Q8_0, 16, 128, [4100, 30, 5000, 777, 4800])])
+def test_understated_n_ctx_of_several_sequences(p1a, kv_type, Hq, D, lens):
+    """the grids that n_ctx chooses between (one stream a workgroup, several, fewer workgroups still; no list) give the same bits"""
+    n, Hkv, psh = len(lens), 8, 6
+    g = torch.Generator(device="cuda").manual_seed(D)
+    maxp = max(-(-x // 64) for x in lens)
+    tab = torch.randperm(n * maxp, generator=g, device="cuda").to(torch.int32)
+    c = p1a.KVCache.paged(kv_type, Hkv, D, psh, n * maxp, tab, maxp)
+    for s, x in enumerate(lens):
+        p1a.kv_append(c.slot(s, maxp), torch.randn((x, Hkv, D), generator=g, device="cuda"), torch.randn((x, Hkv, D), generator=g, device="cuda"), 0, x)
+    q = torch.randn((n, Hq, D), generator=g, device="cuda")
+    pos = dev(np.array(lens, np.int32) - 1)
+    rows = c.with_rows(dev(np.arange(n, dtype=np.int32) * maxp))
+    outs, grids = [], set()
+    for n_ctx in (c.n_ctx, 4000, 2000, 100, 0):
+        rows.n_ctx = min(n_ctx, c.n_ctx)
+        p = plan(kv_type, Hq, Hkv, D, rows.n_ctx, n, cus=torch.cuda.get_device_properties(0).multi_processor_count)
+        grids.add((p["list"], p["loop"], p["x"]))
+        outs.append(torch.empty_like(q))
+        p1a.attn_decode_rows(q, rows, outs[-1], n, pos, Hq, D ** -0.5)
+        assert torch.equal(outs[-1], outs[0]), n_ctx
+    assert len(grids) > 1, grids
 
 
 # every build of dec_mfma_k whose workgroups take several streams: two to a compute unit, staged tiles, two column tiles
