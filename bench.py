@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the paged-KV attention hot path on one MI355X.
 
-Workload (N = 1): configs[1] of the baseline description - 27B-shape decode, batch 1, one full-attention layer: 24 q heads / 4 kv
+Workload (N = 1): 27B-shape decode, batch 1, one full-attention layer: 24 q heads / 4 kv
 heads, head_dim 256, context 32768, q8_0 KV in 256-token pages scattered by a random permutation page table, fused
 sigmoid gate. A "step" is one p1a_attn_decode call (split-K kernel + merge) on inputs resident in HBM. The K timed
 steps are captured once into a hipGraph (the engine replays its decode step as a graph as well) and walk over the KV of
@@ -135,7 +135,7 @@ def extras(p1a, torch, stream, Hq, Hkv, D, psh, scale, top, cpu):
         x = torch.randn(shape, generator=g, device="cuda")
         return x * torch.rsqrt((x * x).mean(-1, keepdim=True) + 1e-6)
 
-    # configs[4]: chunked prefill, T = 4096 after 28672 tokens, q8_0, append of the chunk then attention + gate
+    # chunked prefill, T = 4096 after 28672 tokens, q8_0, append of the chunk then attention + gate
     p0, T = 28672, 4096
     kv, ppseq = build_pool(p1a, torch, p1a.KV_Q8_0, Hq, Hkv, D, psh, p0 + T, 1, seed=21)
     c = kv.slot(0, ppseq)
@@ -158,7 +158,7 @@ def extras(p1a, torch, stream, Hq, Hkv, D, psh, scale, top, cpu):
         "bound": "mfma", "achieved": round(flop / sec / 1e12, 1), "peak": MFMA_F16_PEAK_TFLOPS, "unit": "TFLOP/s",
         "frac": round(flop / sec / 1e12 / MFMA_F16_PEAK_TFLOPS, 4), "traffic": prefill_traffic(), "kernel": "prefill_k<f16, 256, grouped, lds-direct>",
         "call_ms": round(sec * 1e3, 4),
-        "note": "configs[4]: T = 4096 after 28672 tokens, q8_0, fused gate; flops = 4 D Hq (p0 T + T (T + 1) / 2); time = the "
+        "note": "T = 4096 after 28672 tokens, q8_0, fused gate; flops = 4 D Hq (p0 T + T (T + 1) / 2); time = the "
                 "whole p1a_attn_prefill call with caller scratch (the convert-once pass of about 40 us included), median of 9 "
                 "after 12 untimed calls; traffic = HBM-side bytes per call read from the committed rocprofv3 counter summary "
                 "(profiles/prefill_f16_staged_cfg5_traffic.json), not measured in this run"}
@@ -253,7 +253,7 @@ def prefill_traffic():
 
 
 def verify_config(p1a, torch, stream, Hq, Hkv, D, psh, scale, reps=20):
-    """configs[3]: MTP verify, 4 sequences x 4 rows (causal inside the block), q4_0, ctx 65536, each sequence's KV read once"""
+    """MTP verify, 4 sequences x 4 rows (causal inside the block), q4_0, ctx 65536, each sequence's KV read once"""
     n4 = 65536
     g = torch.Generator(device="cuda").manual_seed(6)
     kv, ppseq = build_pool(p1a, torch, p1a.KV_Q4_0, Hq, Hkv, D, psh, n4, 4, seed=22)
@@ -272,7 +272,7 @@ def verify_config(p1a, torch, stream, Hq, Hkv, D, psh, scale, reps=20):
     vb = 4 * n4 * 2 * p1a.kv_row_bytes(p1a.KV_Q4_0, Hkv, D)
     return {"verify_4x4_q4_0_64K_us": round(sec * 1e6, 2), "verify_GBs": round(vb / sec / 1e9, 1),
             "verify_kernel_us": round(sec_k * 1e6, 2), "verify_kernel_frac_of_hbm_peak": round(vb / sec_k / 1e9 / HBM_PEAK_GBS, 4),
-            "roofline_verify": {"bound": "hbm", "workload": "configs[3]: 4 sequences x 4 rows, q4_0, ctx 65536", "bytes": vb,
+            "roofline_verify": {"bound": "hbm", "workload": "4 sequences x 4 rows, q4_0, ctx 65536", "bytes": vb,
                                 "kernel": "dec_mfma_k<q4_0, 256, 2, 8>", "kernel_us": round(sec_k * 1e6, 2),
                                 "achieved": round(vb / sec_k / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                 "frac": round(vb / sec_k / 1e9 / HBM_PEAK_GBS, 4), "call_us": round(sec * 1e6, 2),
@@ -280,7 +280,7 @@ def verify_config(p1a, torch, stream, Hq, Hkv, D, psh, scale, reps=20):
 
 
 def batched_config(p1a, torch, stream, Hq, Hkv, D, psh, scale, reps=20):
-    """configs[2]: 8 slots, one row each, ctx log-uniform in [1024, 32768], q8_0, one shared pool"""
+    """8 slots, one row each, ctx log-uniform in [1024, 32768], q8_0, one shared pool"""
     import math
     g = torch.Generator(device="cuda").manual_seed(9)
     rs = torch.Generator().manual_seed(8)
@@ -299,7 +299,7 @@ def batched_config(p1a, torch, stream, Hq, Hkv, D, psh, scale, reps=20):
         sec_k = time_graph(torch, stream, [lambda: p1a.bench_decode_split_only(q, cr, out, 8, 0, Hq, scale, pos=pos)] * reps, 2)
     bb = sum(lens) * 2 * p1a.kv_row_bytes(p1a.KV_Q8_0, Hkv, D)
     res = {"batched_8slots_q8_0_us": round(sec * 1e6, 2), "batched_GBs": round(bb / sec / 1e9, 1), "batched_ctx": lens,
-           "roofline_batched": {"bound": "hbm", "workload": "configs[2]: 8 slots, 1 row each, q8_0, ctx log-uniform in [1024, 32768]",
+           "roofline_batched": {"bound": "hbm", "workload": "8 slots, 1 row each, q8_0, ctx log-uniform in [1024, 32768]",
                                 "bytes": bb, "kernel": "dec_mfma_k<q8_0, 256, 1, 8, two workgroups per CU>",
                                 "kernel_us": round(sec_k * 1e6, 2), "achieved": round(bb / sec_k / 1e9, 1), "peak": HBM_PEAK_GBS,
                                 "unit": "GB/s", "frac": round(bb / sec_k / 1e9 / HBM_PEAK_GBS, 4), "call_us": round(sec * 1e6, 2),
@@ -484,7 +484,7 @@ def cpu_prefill(torch, kv, ppseq, q, gate, out_gpu, p0, T, Hq, Hkv, D, psh, scal
     ma, rl = I.errors(out_gpu.cpu().numpy()[rows], ref)
     model, ncpu = host_cpu()
     return {"value": round(flop / dt / 1e12, 4), "unit": "TFLOP/s", "cores": int(O.lib().orc_num_threads()), "kind": "port",
-            "sample": f"{len(rows)} of {T} rows (every {every}th) of configs[4] on the C oracle with OpenMP, {dt:.1f} s; the full "
+            "sample": f"{len(rows)} of {T} rows (every {every}th) of the prefill chunk on the C oracle with OpenMP, {dt:.1f} s; the full "
                       f"chunk would take about {dt * T / len(rows):.0f} s",
             "cpu_model": model, "nproc": ncpu,
             "gpu_output_check": {"max_abs": float(f"{ma:.3e}"), "rel_l2": float(f"{rl:.3e}"), "tol": [I.MAX_ABS_TOL, I.REL_L2_TOL],
@@ -580,7 +580,7 @@ def main():
         "metric": "decode-attn HBM GB/s @27B q8_0 32K (paged, B=1, fused gate)", "value": round(gbs, 1), "unit": "GB/s",
         "n_gpus": 1, "steps": K, "warmup": W, "ms_per_step": round(sec * 1e3, 5), "higher_is_better": True,
         "scaling": "weak", "vs_baseline": None, "dtype": "q8_0 KV -> f16 MFMA, f32 accumulate", "data": "synthetic",
-        "config": {"workload": "configs[1]: decode 24/4 heads, head_dim 256, ctx 32768, q8_0, 256-token pages, random page table",
+        "config": {"workload": "decode 24/4 heads, head_dim 256, ctx 32768, q8_0, 256-token pages, random page table",
                    "kv_bytes_per_step": step_bytes, "layers_rotated": n_pools,
                    "launch": f"hipGraph of K steps, replayed {REPLAYS} times, median replay"},
         "replay_ms_per_step": [round(x * 1e3, 5) for x in samples],
