@@ -238,14 +238,14 @@ template <int U> __device__ __forceinline__ uint32_t live_streams(const int32_t 
         if (lane - (int) ((uint32_t) lane * (uint32_t) rps_magic >> 16) * RPS) n = 0;
     }
     const int na = min(max(n - nsplit, 0), nsplit);
-    int u = na | ((min(n, nsplit) - na) << 16);
+    uint32_t u = (uint32_t) na | (uint32_t) (min(n, nsplit) - na) << 16;   // (32 rows of 1024 streams: 2^31 in the sum)
     // sums over the lanes up to this one
-    u += __builtin_amdgcn_update_dpp(0, u, 0x111, 0xf, 0xf, true);
-    u += __builtin_amdgcn_update_dpp(0, u, 0x112, 0xf, 0xf, true);
-    u += __builtin_amdgcn_update_dpp(0, u, 0x114, 0xf, 0xf, true);
-    u += __builtin_amdgcn_update_dpp(0, u, 0x118, 0xf, 0xf, true);
-    u += __builtin_amdgcn_update_dpp(0, u, 0x142, 0xa, 0xf, false);
-    return (uint32_t) u;
+    u += (uint32_t) __builtin_amdgcn_update_dpp(0, (int) u, 0x111, 0xf, 0xf, true);
+    u += (uint32_t) __builtin_amdgcn_update_dpp(0, (int) u, 0x112, 0xf, 0xf, true);
+    u += (uint32_t) __builtin_amdgcn_update_dpp(0, (int) u, 0x114, 0xf, 0xf, true);
+    u += (uint32_t) __builtin_amdgcn_update_dpp(0, (int) u, 0x118, 0xf, 0xf, true);
+    u += (uint32_t) __builtin_amdgcn_update_dpp(0, (int) u, 0x142, 0xa, 0xf, false);
+    return u;
 }
 // number q of that list (q_a of them are A): the first row of its sequence, and the stream
 struct stream_at { int first, split; };
