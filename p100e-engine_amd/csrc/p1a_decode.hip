@@ -320,20 +320,10 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     }
     n_max = rfl(n_max);
     p_min = rfl(p_min);
-    // A workgroup none of whose streams holds a visible key (a short sequence in a batch: stream s is empty once s units
-    // cover the sequence) is done before it asks for anything else - a wide call of short sequences launches several of
-    // these for every workgroup that has work. It leaves the empty partials its stream would have ended with, unless the
-    // rows carry their own positions: merge_k then knows from those which streams to skip and never reads them.
+    // A workgroup none of whose streams holds a visible key (a short sequence: stream s is empty once s units cover the sequence) is done
+    // before it asks for anything else - a wide call of short sequences launches several of these for every workgroup that has
+    // work. It leaves nothing: merge_k knows from the rows' positions which streams to skip.
     if (split * U >= n_max) {
-        if (!P.pos_rows) {
-            for (int col = tid; col < R; col += NWV * 64) {
-                const int t = row_of(col), hh = col - t * P.GQA;
-                const size_t row = (size_t) (row0 + t) * P.Hq + (size_t) hg * P.GQA + hh;
-                float * pm = P.part_ml + (row * P.nsplit + split) * 2;
-                pm[0] = NEG_INF;
-                pm[1] = 0.f;
-            }
-        }
         if (next_item()) continue;
         return;
     }
@@ -919,20 +909,22 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
 // ... in order and the 8 slices are then added in order, so the result depends on nothing but the partials. A wave holds
 // two slices, so each of its loads covers two contiguous half-rows of 512 bytes. The (m, l) pairs are fetched once per
 // wave - lane i brings the pair of split i - and handed round by lane shuffles; the maximum is a wave reduction.
-// pos_rows / U (optional): row t of a batched call sits at position pos_rows[t] and its split stream s holds keys only when
-// s units of U positions do not cover the sequence yet - the streams past that are known to be empty and are not fetched.
+// Row t sits at position pos_rows[t], *p0_dev + t or p0 + t, and its split stream s holds keys only when s units of 2^u_sh positions do not
+// cover the sequence yet: the streams past that are known to be empty and are not fetched (nobody writes them). Calls of one sequence used to fetch every
+// stream's (m, l): few kv heads have many (one, 256), and one row over 500 keys (f16, 4 / 1 heads of 64, two layers with prep, recorded) took
+// 34.4 us, 27.5 so; 16 / 2 of 256 (q4_0) 37.4 and 34.8.
 constexpr int MRG_DIMS = 128;
 __global__ void __launch_bounds__(256) merge_k(const float * __restrict__ part_o, const float * __restrict__ part_ml,
                                                float * __restrict__ out, const float * __restrict__ gate, int NS_all, int D,
-                                               void * qbuf, int Hq, int T, const int32_t * __restrict__ pos_rows, int U) {
+                                               void * qbuf, int Hq, int T, const int32_t * __restrict__ pos_rows,
+                                               const int32_t * __restrict__ p0_dev, int p0, int u_sh) {
     __shared__ f4 sacc[8][32];
     __shared__ float sden[8];
-    const size_t row = blockIdx.x;
+    const int t_row = blockIdx.z;
+    const size_t row = (size_t) t_row * Hq + blockIdx.x;
     const int NS_row = NS_all;                                // (the row stride of the partials)
-    int NS = NS_all;
-    // (a row at a negative position - an idle slot - sees no key: no stream is read, and 0 / 0 gives the NaN row the
+    // (a row at a negative position - an idle slot - sees no key: no stream counts, and 0 / 0 gives the NaN row the
     // reference's combine gives for n = 0)
-    if (pos_rows && U > 0) { const int pr_ = pos_rows[row / Hq]; NS = pr_ < 0 ? 0 : min(NS_all, pr_ / U + 1); }
     const int tid = threadIdx.x, lane = tid & 63, qd = tid & 31, sl = tid >> 5;
     const int d = blockIdx.y * MRG_DIMS + qd * 4;
     const bool live = d < D;
@@ -946,14 +938,26 @@ __global__ void __launch_bounds__(256) merge_k(const float * __restrict__ part_o
     // the maximum over all splits first: batches of 64 pairs, lane i of every wave the pair of split s0 + i
     float M = NEG_INF;
     float2 pr = make_float2(NEG_INF, 0.f);                    // the pair of split `lane` of the first batch
+    // The first batch of partials (all of them when NS <= 64) is requested before anything is known about the maximum - and, where one
+    // sequence's position is in memory, about the position: its round trip in front of them costs more than what is fetched for nothing (16 / 2 heads, 32000 keys 41.9 us,
+    // 42.4 behind it); what no stream has written is dropped.
+    const bool beside = p0_dev && !pos_rows;
+    auto streams = [&](int at) { return at < 0 ? 0 : min(NS_all, (at >> u_sh) + 1); };
+    int NS = NS_all;
+    if (!beside) NS = streams(pos_rows ? sload_i32(pos_rows + t_row) : p0 + t_row);
     if (lane < NS) pr = *reinterpret_cast<const float2 *>(ml + 2 * lane);
-    // the first batch of partials (all of them when NS <= 64) is requested before anything is known about the maximum
     f4 a[CH];
 #pragma unroll
     for (int k = 0; k < CH; ++k) {
         const int s = sl + 8 * k;
         a[k] = f4{0.f, 0.f, 0.f, 0.f};
         if (s < NS && live) a[k] = *reinterpret_cast<const f4 *>(part_o + (row * NS_row + s) * D + d);
+    }
+    if (beside) {
+        // (asked for once those are on their way: scalar loads come back in no order, and the wait for one is a wait for all)
+        asm volatile("" : "+s"(p0_dev) :: "memory");
+        NS = streams(sload_i32(p0_dev) + t_row);
+        if (lane >= NS) pr = make_float2(NEG_INF, 0.f);
     }
     M = pr.x;
     for (int s0 = 64; s0 < NS; s0 += 64) if (s0 + lane < NS) M = fmaxf(M, ml[2 * (s0 + lane)]);
@@ -995,8 +999,7 @@ __global__ void __launch_bounds__(256) merge_k(const float * __restrict__ part_o
         // 8 consecutive lanes of slice 0 hold one 32-value group of the output row: its a16 activation quantize rides
         // along (what the engine's ew_quant emits for the output projection, src/fast/fused.cu:478-496)
         if (qbuf) {
-            const int t = (int) (row / Hq), h = (int) (row - (size_t) t * Hq);
-            a16_quant8(r, qd & 7, qbuf, t, h * (D >> 5) + (d >> 5), (Hq * D) >> 5, T, live);
+            a16_quant8(r, qd & 7, qbuf, t_row, (int) blockIdx.x * (D >> 5) + (d >> 5), (Hq * D) >> 5, T, live);
         }
     }
 }
@@ -1135,8 +1138,8 @@ int launch_decode(const p1a_kv & c, const decode_args & a, hipStream_t s) {
         rc = launch_decode_any(c, a, pl.RG, pl.nsplit, s);
     }
     if (rc != P1A_OK || a.skip_merge) return rc;
-    merge_k<<<dim3(a.T * a.Hq, (c.D + MRG_DIMS - 1) / MRG_DIMS), 256, 0, s>>>(a.part_o, a.part_ml, a.out, a.gate, pl.nsplit, c.D, a.qbuf, a.Hq, a.T,
-                                                       a.pos_rows, pl.mfma ? 32 * pl.NW : decode_any_unit(c.D));
+    merge_k<<<dim3(a.Hq, (c.D + MRG_DIMS - 1) / MRG_DIMS, a.T), 256, 0, s>>>(a.part_o, a.part_ml, a.out, a.gate, pl.nsplit, c.D, a.qbuf, a.Hq, a.T,
+                                                       a.pos_rows, a.p0_dev, a.p0, __builtin_ctz(pl.mfma ? 32 * pl.NW : decode_any_unit(c.D)));
     return launched();
 }
 

@@ -125,14 +125,7 @@ __device__ __forceinline__ void any_body(const any_params & P) {
     const size_t row0 = (size_t) t * P.Hq + (size_t) hk * P.GQA + col0;   // the output row of column 0
     const int n = (P.pos_rows ? sload_i32(P.pos_rows + t) : (P.p0_dev ? sload_i32(P.p0_dev) : P.p0) + t) + 1;
     const int32_t * ptab = P.pg.pt ? P.pg.pt + rt : nullptr;
-    if (split * U >= n) {                                     // no key in this stream (with pos_rows the merge does not look at it)
-        if (!P.pos_rows && threadIdx.x < R) {
-            float * pm = P.part_ml + ((row0 + threadIdx.x) * P.nsplit + split) * 2;
-            pm[0] = NEG_INF;
-            pm[1] = 0.f;
-        }
-        return;
-    }
+    if (split * U >= n) return;                               // no key in this stream (the merge does not look at it)
     const size_t hoff = (size_t) hk * head_bytes(KT, 32) * NB;
     const int SC = Q8 ? 2 : 18;                               // distance of two block scales
 

@@ -268,6 +268,32 @@ def test_descriptor_n_ctx_only_bounds(p1a):
         assert torch.equal(out, ref), n_ctx
 
 
+@pytest.mark.parametrize("kv_type,Hq,Hkv,D,psh", [(O.KV_F16, 4, 1, 64, 4), (O.KV_F16, 6, 1, 256, 6), (O.KV_Q4_0, 16, 2, 256, 6), (O.KV_Q8_0, 8, 1, 128, 5), (O.KV_Q8_0, 24, 4, 256, 8),
+                                                  (O.KV_Q8_0, 4, 1, 96, 4)])
+def test_short_calls_behind_a_long_one(p1a, kv_type, Hq, Hkv, D, psh):
+    """one sequence: only the streams its position fills count, whatever a longer call has left in the others' partials - positions on both sides of a
+    unit's end, in the call, in device memory and by rows; a negative position in device memory sees no key"""
+    n = 9000
+    pool = Pool(p1a, kv_type, Hq, Hkv, D, psh, [n], seed=29)
+    c, host = pool.dev_seq(0), pool.host_seq(0)
+    qs = I.normal(I.rng(30), (3, Hq, D))
+    q, scale = dev(qs), D ** -0.5
+    for T in (1, 3):
+        for p0 in (0, 62, 127, 253, 255, 256, 510, 700, 2303):
+            run_decode(p1a, c, qs, 3, n - 3, Hq, scale)                # every stream's partials are some other call's
+            want = run_decode(p1a, c, qs[:T], T, p0, Hq, scale)
+            check(want, O.attn_rows(host, qs[:T], np.arange(p0, p0 + T), Hq, scale), f"T {T} at {p0}")
+            got = torch.full((T, Hq, D), float("nan"), device="cuda")
+            run_decode(p1a, c, qs, 3, n - 3, Hq, scale)
+            p1a.attn_decode_dev(q[:T].contiguous(), c, got, T, dev(np.array([p0], np.int32)), n, Hq, scale)
+            assert np.array_equal(got.cpu().numpy(), want), (T, p0)
+            rows = torch.full((T, Hq, D), float("nan"), device="cuda")
+            p1a.attn_decode_rows(q[:T].contiguous(), pool.devkv.with_rows(dev(np.zeros(T, np.int32))), rows, T, dev(np.arange(p0, p0 + T, dtype=np.int32)), Hq, scale)
+            assert np.array_equal(rows.cpu().numpy(), want), (T, p0)
+    p1a.attn_decode_dev(q[:1].contiguous(), c, got, 1, dev(np.array([-1], np.int32)), n, Hq, scale)
+    assert torch.isnan(got[0]).all()
+
+
 def test_other_shapes_and_refusals(p1a):
     # GQA 4 / D 128 f16, GQA 8 / D 64 f16 (MFMA path), q8_0 at D 128 (generic path)
     for kv_type, Hq, Hkv, D in [(O.KV_F16, 8, 2, 128), (O.KV_F16, 8, 1, 64), (O.KV_Q8_0, 8, 2, 128), (O.KV_Q4_0, 6, 3, 96)]:
