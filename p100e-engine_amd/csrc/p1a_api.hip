@@ -181,6 +181,7 @@ int decode_call(const float * q, const p1a_kv * c, float * out, const float * ga
     if (!pos_rows && !p0_dev && p0 < 0) { set_error("p1a_attn_decode: negative p0"); return P1A_E_ARG; }
     decode_args a;
     a.q = q; a.out = out; a.gate = gate; a.T = T; a.p0 = p0; a.p0_dev = p0_dev; a.pos_rows = pos_rows;
+    a.host_n = pos_rows || p0_dev ? 0 : (long long) p0 + T;
     a.Hq = Hq; a.scale = scale;
     a.rows_per_group = decode_rows_per_group(*c, Hq, pos_rows ? (rows_per_seq < 1 ? 1 : rows_per_seq) : T);
     // a sequence's rows must split into whole groups, or a group would mix two sequences

@@ -117,6 +117,7 @@ struct decode_args {
     int T, p0;
     const int32_t * p0_dev;
     const int32_t * pos_rows;
+    long long host_n;     // positions the last row sees where the host knows it, else 0
     int rows_per_group;   // rows sharing one KV read
     int rows_per_seq;     // rows of one sequence (1 << 30 without per-row positions: all of them)
     int Hq;

@@ -86,15 +86,46 @@ struct dec_params {
     int rps_magic;    // LIST: 65536 / RPS + 1
     int hkv_sh;       // log2(Hkv) when Hkv is a power of two, else -1
     int npt;          // page-table entries of one sequence (ceil(n_ctx / page positions)); 0 = contiguous
+    float * out;      // DIRECT: where the results go, the gate, the a16 values
+    const float * gate;
+    void * qbuf;
 };
+
+// the pointer, known to the compiler as one to device memory
+template <typename T> __device__ __forceinline__ void in_memory(T *& p) { p = (T *) (__attribute__((address_space(1))) T *) (uintptr_t) p; }
+
+// sum / denominator, gate, result and a16 values of dims d .. d + 3 of head h of row t: 8 consecutive lanes hold one 32-value group of the
+// row (what the engine's ew_quant emits for the output projection, src/fast/fused.cu:478-496). A row that sees no key is 0 / 0: the NaN row the
+// reference's combine gives for n = 0.
+__device__ __forceinline__ void finish_row(const f4 n, float dn, const f4 gt, float * out, bool gated, void * qbuf, int t, int h, int d, int Hq, int D, int T, bool live) {
+    in_memory(out); in_memory(qbuf);
+    f4 r = {n[0] / dn, n[1] / dn, n[2] / dn, n[3] / dn};
+    if (gated) {
+#pragma unroll
+        for (int x = 0; x < 4; ++x) r[x] *= 1.0f / (1.0f + expf(-gt[x]));
+    }
+    if (live) *reinterpret_cast<f4 *>(out + ((size_t) t * Hq + h) * D + d) = r;
+    if (qbuf) a16_quant8(r, (d >> 2) & 7, qbuf, t, h * (D >> 5) + (d >> 5), (Hq * D) >> 5, T, live);
+}
+// a kernel's arguments, read where they are wanted (kept from the kernel's start they would take registers from the key loop)
+typedef const __attribute__((address_space(4))) char * kargb;
+__device__ __forceinline__ kargb args_again() {
+    kargb kp = (kargb) __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(kp));
+    return kp;
+}
+#define P1A_ARG(kp, field) (*reinterpret_cast<const __attribute__((address_space(4))) decltype(dec_params::field) *>((kp) + offsetof(dec_params, field)))
+// two floats that another wave of this workgroup has stored, past the caches of the compute unit
+__device__ __forceinline__ float2 get2(const float * p) {
+    const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return make_float2(__builtin_bit_cast(float, (uint32_t) v), __builtin_bit_cast(float, (uint32_t) (v >> 32)));
+}
 
 __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) { return __builtin_amdgcn_perm(hi, lo, sel); }
 
 // 4 int8 codes (one dword) -> (code * d) as two packed f16 pairs, returned as raw dwords so MFMA operands are built in place
 struct u2 { uint32_t lo, hi; };
 typedef const __attribute__((address_space(4))) uint64_t * kargs;   // a kernel's arguments, as words
-// the pointer, known to the compiler as one to device memory
-template <typename T> __device__ __forceinline__ void in_memory(T *& p) { p = (T *) (__attribute__((address_space(1))) T *) (uintptr_t) p; }
 __device__ __forceinline__ u2 deq4(uint32_t w, h2 d01, h2 d23) {
     const h2 off = {(half_t) 1152, (half_t) 1152};
     const uint32_t x = w ^ 0x80808080u;
@@ -164,12 +195,15 @@ template <int NR> __device__ __forceinline__ void wait_tiles(int newer) {
 // are done, V likewise; everything a lane computes, and the order it computes it in, is the same as in the double-buffered
 // kernel, so the partials are the same bits. One column tile only (NT == 1, at most 16 live columns).
 // KS (when it differs from KT = f16): the type the cache holds - its raw tiles are staged (raw_cfg) and converted to f16
-// HOW = KS, and for calls of several sequences LIST (workgroups take the streams that hold keys), LIST | LOOP (one takes several)
-constexpr uint32_t LIST_ = 0x100, LOOP_ = 0x200;
+// HOW = KS, and for calls of several sequences LIST (workgroups take the streams that hold keys), LIST | LOOP (one takes several);
+// DIRECT for calls whose rows see one unit at most, as far as the host knows: a workgroup for every (row group, kv head) writes the
+// results itself
+constexpr uint32_t LIST_ = 0x100, LOOP_ = 0x200, DIRECT_ = 0x400;
 template <uint32_t KT, int D, int NT, int NWV, bool SB, uint32_t HOW = KT>
 __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const dec_params P_) {
     constexpr uint32_t KS = HOW & 0xff;
-    constexpr bool LIST = HOW & LIST_, LOOP = HOW & LOOP_;
+    constexpr bool LIST = HOW & LIST_, LOOP = HOW & LOOP_, DIRECT = HOW & DIRECT_, AGAIN = LOOP || DIRECT;
+    static_assert(!DIRECT || (!SB && !LIST), "such calls have a workgroup to a CU at most");
     using C = tile_cfg<KT, D>;
     using RW = raw_cfg<KS, D>;
     constexpr bool STG = KS != KT;
@@ -217,7 +251,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     // the keys, same bits. q8_0, 24 / 4 heads of 256, two layers with prep and merge: 8 sequences of 1024 keys 47 -> 38 us, 16 of 300 ... 5000
     // 68 -> 58, 2 of 20000 74 -> 69, 32 of 256 61 -> 43; what it does not help costs 2 ... 6 % (4 of 4000 ... 16000, two rows each 75 -> 77; 4 x 4 rows of 4252, 272 live workgroups
     // for 256 units), a sequence of many rows that only groups of one divide up to 16 (plan_grid).
-    int hg = 0, gsub = 0, q = 0, q_step = 0, q_a = 0, q_end = 0, rt_lanes = 0;
+    int split = 0, hg = 0, gsub = 0, q = 0, q_step = 0, q_a = 0, q_end = 0, rt_lanes = 0;
     uint32_t u_sum = 0;
     if constexpr (LIST) {
         const dec_params & P = P_;
@@ -236,11 +270,11 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
         if (LOOP && lane < 32) wl[lane] = u_sum;              // (every wave writes all of it, the same values: none reads it before it is there)
     }
     for (;;) {
-    // (LOOP: what hangs on the lane or on the kernel's arguments is worked out, or read, afresh for every item: kept from one to
+    // (LOOP, DIRECT: what hangs on the lane or on the kernel's arguments is worked out, or read, afresh for every item: kept from one to
     // the next it would take the registers that the key loop needs)
-    const int tid = LOOP ? (wave << 6) | lane_id() : (int) threadIdx.x;
+    const int tid = AGAIN ? (wave << 6) | lane_id() : (int) threadIdx.x;
     dec_params P_again;
-    if constexpr (LOOP) {
+    if constexpr (AGAIN) {
         kargs kp = (kargs) __builtin_amdgcn_kernarg_segment_ptr();
         asm volatile("" : "+s"(kp));
         struct words { uint64_t w[sizeof(dec_params) / 8]; } k;
@@ -253,19 +287,26 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
         in_memory(P_again.q); in_memory(P_again.kc); in_memory(P_again.vc); in_memory(P_again.part_o); in_memory(P_again.part_ml);
         in_memory(P_again.pg.pt); in_memory(P_again.pg.rtab); in_memory(P_again.p0_dev); in_memory(P_again.pos_rows);
     }
-    const dec_params & P = LOOP ? P_again : P_;
+    const dec_params & P = AGAIN ? P_again : P_;
     const int lane = tid & 63;
     const int c = lane & 15, g = lane >> 4;
     const int HG = P.Hkv;
+    int n_max = 0;                                            // positions the group sees
     auto next_item = [&]() {
+        if constexpr (DIRECT) return ++split < min(P1A_ARG(args_again(), nsplit), (n_max + U - 1) / U);
         if constexpr (!LOOP) return false;
         q += q_step;
         if (q >= q_end) return false;
         u_sum = wl[lane_id() & 31];
         return true;
     };
-    int split, row0;
-    if constexpr (LIST) {
+    int row0;
+    if constexpr (DIRECT) {                                   // (the heads of a group on one XCD)
+        const int i = blockIdx.x, j = i >> 3, jg = j / HG;
+        hg = j - jg * HG;
+        row0 = (jg * 8 + (i & 7)) * P.RG;
+        if (row0 >= P.T) return;
+    } else if constexpr (LIST) {
         const stream_at at = pick_stream(u_sum, q, q_a, lane);
         split = at.split;
         row0 = at.first + gsub * P.RG;
@@ -312,7 +353,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     auto row_of = [&](int col) { return (col >= P.GQA) + (col >= 2 * P.GQA) + (col >= 3 * P.GQA); };
     // visible-position limit of each of this lane's columns, and the group's maximum
     int plim[NT];
-    int n_max = 0, p_min = 0x7fffffff;
+    int p_min = 0x7fffffff;
     for (int t = 0; t < nr; ++t) {
         const int pt_ = P.pos_rows ? (t ? P.pos_rows[row0 + t] : pos_first) : p0v + row0 + t;
         n_max = max(n_max, pt_ + 1);
@@ -324,9 +365,18 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     // before it asks for anything else - a wide call of short sequences launches several of these for every workgroup that has
     // work. It leaves nothing: merge_k knows from the rows' positions which streams to skip.
     if (split * U >= n_max) {
-        if (next_item()) continue;
+        if constexpr (DIRECT) {                               // (idle rows)
+            for (int i = tid; i < R * (D / 4); i += NWV * 64) {
+                const int col = i / (D / 4), t = row_of(col);
+                const kargb kp = args_again();
+                finish_row(f4{0.f, 0.f, 0.f, 0.f}, 0.f, f4{0.f, 0.f, 0.f, 0.f}, P1A_ARG(kp, out), P1A_ARG(kp, gate) != nullptr, P1A_ARG(kp, qbuf), row0 + t, hg * P.GQA + col - t * P.GQA,
+                           4 * (i % (D / 4)), P1A_ARG(kp, Hq), D, P1A_ARG(kp, T), true);
+            }
+        }
+        if (!DIRECT && next_item()) continue;
         return;
     }
+    const bool only = DIRECT && n_max <= U;                   // (no other stream has keys of these rows)
 #pragma unroll
     for (int r = 0; r < NT; ++r) {
         const int col = 16 * r + c;
@@ -534,7 +584,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     f4 ol[NT];
     float m_run[NT];
     float zero = 0.f;
-    if constexpr (LOOP) asm volatile("" : "+v"(zero));        // (or four registers would carry it from item to item)
+    if constexpr (AGAIN) asm volatile("" : "+v"(zero));        // (or four registers would carry it from item to item)
     const h4 ones = {(half_t) 1, (half_t) 1, (half_t) 1, (half_t) 1};
 #pragma unroll
     for (int r = 0; r < NT; ++r) {
@@ -812,7 +862,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     constexpr int QD = D / 4;                                 // dims per quarter
     constexpr int PC = SB ? 8 : 16;                           // columns parked at a time
     // (lane coordinates worked out afresh: what is derived from them here need not live in registers through the key loop)
-    int tid_f = LOOP ? (wave << 6) | lane_id() : (int) threadIdx.x;
+    int tid_f = AGAIN ? (wave << 6) | lane_id() : (int) threadIdx.x;
     asm volatile("" : "+v"(tid_f));
     const int c_f = tid_f & 15, g_f = (tid_f >> 4) & 3;
     auto park = [&](int w, int k) -> float * {                // dim quarter k of wave w
@@ -874,7 +924,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
             }
             const int col = 16 * r + cc;
             const int t = row_of(col), hh = col - t * P.GQA;
-            const size_t row = (size_t) (row0 + t) * P.Hq + (size_t) hg * P.GQA + hh;
+            const size_t row = (size_t) (row0 + t) * (DIRECT ? P1A_ARG(args_again(), Hq) : P.Hq) + (size_t) hg * P.GQA + hh;
 #pragma unroll
             for (int it = 0; it < NIT; ++it) {
                 const int d4 = dl + it * LPC;
@@ -884,12 +934,29 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
                     for (int w = 0; w < NWV; ++w) acc += aw[it][w] * fw[w];
                     // (two column tiles = several rows per group: the partials are tens of megabytes and nothing here reads
                     // them again, so they go past the cache - measured -3 ... -5 % on 4-row verify calls, +6 % on a single row)
-                    f4 * const po = reinterpret_cast<f4 *>(P.part_o + (row * P.nsplit + split) * D + 4 * d4);
+                    if (only) {                               // what merge_k makes of one stream: 2^0 times it, added to zeros
+                        const bool none = M == NEG_INF || l == 0.f;
+                        const f4 zero4 = {0.f, 0.f, 0.f, 0.f};
+                        f4 gt = zero4;
+                        const kargb kp = args_again();
+                        const float * gate = P1A_ARG(kp, gate);
+                        in_memory(gate);
+                        if (gate) gt = *reinterpret_cast<const f4 *>(gate + row * D + 4 * d4);
+                        finish_row(none ? zero4 : acc + zero4, none ? 0.f : l, gt, P1A_ARG(kp, out), gate != nullptr, P1A_ARG(kp, qbuf), row0 + t, hg * P.GQA + hh, 4 * d4, P1A_ARG(kp, Hq), D, P1A_ARG(kp, T), true);
+                        continue;
+                    }
+                    float * part_o = P.part_o;
+                    int nsp = P.nsplit;
+                    if constexpr (DIRECT) { const kargb kp = args_again(); part_o = P1A_ARG(kp, part_o); nsp = P1A_ARG(kp, nsplit); in_memory(part_o); }
+                    f4 * const po = reinterpret_cast<f4 *>(part_o + (row * nsp + split) * D + 4 * d4);
                     if (M != NEG_INF) { if constexpr (NT == 2) __builtin_nontemporal_store(acc, po); else *po = acc; }
                 }
             }
-            if (dl == 0) {
-                float * pm = P.part_ml + (row * P.nsplit + split) * 2;
+            if (dl == 0 && !only) {
+                float * part_ml = P.part_ml;
+                int nsp = P.nsplit;
+                if constexpr (DIRECT) { const kargb kp = args_again(); part_ml = P1A_ARG(kp, part_ml); nsp = P1A_ARG(kp, nsplit); in_memory(part_ml); }
+                float * pm = part_ml + (row * nsp + split) * 2;
                 pm[0] = M;
                 pm[1] = l;
             }
@@ -898,7 +965,50 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
         if (SB || he - h0 <= NWV) fold_round(std::integral_constant<int, 64>{}); else fold_round(std::integral_constant<int, 32>{});
         }
     }
-    if (!next_item()) return;
+    if (!next_item()) {
+        if constexpr (DIRECT) {
+            // More streams than n_ctx had said (it is never what results depend on): merged here, in merge_k's order, one row and 4
+            // dims to a thread
+            if (n_max <= U) return;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            const kargb kp = args_again();
+            const int nsp = P1A_ARG(kp, nsplit), GQA = P1A_ARG(kp, GQA), Hq = P1A_ARG(kp, Hq), NS = min(nsp, (n_max + U - 1) / U);
+            const float * pml = P1A_ARG(kp, part_ml), * ppo = P1A_ARG(kp, part_o), * gate = P1A_ARG(kp, gate);
+            in_memory(pml); in_memory(ppo); in_memory(gate);
+#pragma unroll 1
+            for (int i = (wave << 6) | lane_id(); i < R * (D / 4); i += NWV * 64) {
+                const int col = i / (D / 4), d = 4 * (i % (D / 4)), t = (col >= GQA) + (col >= 2 * GQA) + (col >= 3 * GQA), h = hg * GQA + col - t * GQA;
+                const size_t row = (size_t) (row0 + t) * Hq + h;
+                const float * const ml = pml + row * nsp * 2, * const po = ppo + row * nsp * D + d;
+                float M = NEG_INF;
+#pragma unroll 1
+                for (int s = 0; s < NS; ++s) M = fmaxf(M, get2(ml + 2 * s).x);
+                f4 n = {0.f, 0.f, 0.f, 0.f};
+                float dn = 0.f;
+#pragma unroll 1
+                for (int k = 0; k < 8; ++k) {
+                    f4 num = {0.f, 0.f, 0.f, 0.f};
+                    float den = 0.f;
+#pragma unroll 1
+                    for (int s = k; s < NS; s += 8) {
+                        const float2 p = get2(ml + 2 * s);
+                        if (p.x == NEG_INF || p.y == 0.f) continue;
+                        const float f = __builtin_amdgcn_exp2f(p.x - M);
+                        const float2 x = get2(po + (size_t) s * D), y = get2(po + (size_t) s * D + 2);
+                        den = fmaf(f, p.y, den);
+                        num[0] = fmaf(f, x.x, num[0]); num[1] = fmaf(f, x.y, num[1]);
+                        num[2] = fmaf(f, y.x, num[2]); num[3] = fmaf(f, y.y, num[3]);
+                    }
+                    if (k == 0) { n = num; dn = den; } else { n += num; dn += den; }
+                }
+                f4 gt = {0.f, 0.f, 0.f, 0.f};
+                if (gate) gt = *reinterpret_cast<const f4 *>(gate + row * D + d);
+                finish_row(n, dn, gt, P1A_ARG(kp, out), gate != nullptr, P1A_ARG(kp, qbuf), row0 + t, h, d, Hq, D, P1A_ARG(kp, T), true);
+            }
+        }
+        return;
+    }
     __syncthreads();                                          // (the fold has been read: the tiles and tables are free)
     }
 }
@@ -990,17 +1100,7 @@ __global__ void __launch_bounds__(256) merge_k(const float * __restrict__ part_o
         float dn = sden[0];
 #pragma unroll
         for (int k = 1; k < 8; ++k) { n += sacc[k][qd]; dn += sden[k]; }
-        f4 r = {n[0] / dn, n[1] / dn, n[2] / dn, n[3] / dn};
-        if (gate) {
-#pragma unroll
-            for (int x = 0; x < 4; ++x) r[x] *= 1.0f / (1.0f + expf(-gt[x]));
-        }
-        if (live) *reinterpret_cast<f4 *>(out + row * D + d) = r;
-        // 8 consecutive lanes of slice 0 hold one 32-value group of the output row: its a16 activation quantize rides
-        // along (what the engine's ew_quant emits for the output projection, src/fast/fused.cu:478-496)
-        if (qbuf) {
-            a16_quant8(r, qd & 7, qbuf, t_row, (int) blockIdx.x * (D >> 5) + (d >> 5), (Hq * D) >> 5, T, live);
-        }
+        finish_row(n, dn, gt, out, gate != nullptr, qbuf, t_row, (int) blockIdx.x, d, Hq, D, T, live);
     }
 }
 
@@ -1057,7 +1157,7 @@ __global__ void __launch_bounds__(256) sigmoid_mul_k(float * __restrict__ x, con
 }
 
 template <uint32_t KT, int D, uint32_t KS = KT>
-int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hipStream_t s) {
+int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, bool & direct, hipStream_t s) {
     dec_params P;
     P.q = a.q; P.kc = (const char *) c.k; P.vc = (const char *) c.v;
     P.part_o = a.part_o; P.part_ml = a.part_ml; P.pg = view_of(c);
@@ -1065,7 +1165,8 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hi
     P.T = a.T; P.RG = pl.RG; P.Hq = a.Hq; P.Hkv = c.Hkv; P.GQA = pl.GQA;
     P.qscale = a.scale * 1.4426950408889634f; P.nsplit = pl.nsplit;
     constexpr bool big_tiles = KT == P1A_KV_F16 && D == 256;
-    const decode_grid gr = plan_grid(pl, KS, D, c.Hkv, c.n_ctx, a.T, a.rows_per_seq, a.pos_rows != nullptr, a.cus);
+    const decode_grid gr = plan_grid(pl, KS, D, c.Hkv, c.n_ctx, a.T, a.rows_per_seq, a.pos_rows != nullptr, a.cus, a.skip_merge ? -1 : a.host_n);
+    direct = gr.direct;
     P.RPS = gr.RPS;
     P.GPS = gr.GPS;
     P.rps_magic = 65536 / P.RPS + 1;
@@ -1075,12 +1176,16 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, hi
         if ((1 << sh) == c.Hkv) P.hkv_sh = sh;
         if ((1 << sh) == inner) P.inner_sh = sh;
     }
+    P.out = a.out; P.gate = a.gate; P.qbuf = a.qbuf;
     P.npt = c.pt ? (int) (((long long) c.n_ctx + (1LL << c.psh) - 1) >> c.psh) : 0;
     const dim3 grid(gr.x, gr.y);
     constexpr bool can_loop_2 = KT != P1A_KV_Q4_0;            // (plan_grid asks for no other)
     auto go = [&](auto nt, auto single, auto can_loop) {
         constexpr int NT = decltype(nt)::value, NW = big_tiles ? 4 : 8;
         constexpr bool SB = decltype(single)::value;
+        if constexpr (!SB && (NT == 1 || KT != P1A_KV_Q4_0)) {   // (plan_grid asks for no other)
+            if (gr.direct) { dec_mfma_k<KT, D, NT, NW, false, KS | DIRECT_><<<grid, NW * 64, 0, s>>>(P); return; }
+        }
         if constexpr (decltype(can_loop)::value) {
             if (gr.loop) { dec_mfma_k<KT, D, NT, NW, SB, KS | LIST_ | LOOP_><<<grid, NW * 64, 0, s>>>(P); return; }
         }
@@ -1124,20 +1229,21 @@ int launch_decode(const p1a_kv & c, const decode_args & a, hipStream_t s) {
         return P1A_E_SCRATCH;
     }
     int rc;
+    bool direct = false;                                      // (the kernel writes the results itself)
     if (pl.mfma) {
-        if (c.type == P1A_KV_Q8_0 && c.D == 256) rc = launch_mfma<P1A_KV_Q8_0, 256>(c, a, pl, s);
-        else if (c.type == P1A_KV_Q4_0 && c.D == 256) rc = launch_mfma<P1A_KV_Q4_0, 256>(c, a, pl, s);
-        else if (c.type == P1A_KV_Q8_0 && c.D == 128) rc = launch_mfma<P1A_KV_F16, 128, P1A_KV_Q8_0>(c, a, pl, s);
-        else if (c.type == P1A_KV_Q8_0) rc = launch_mfma<P1A_KV_F16, 64, P1A_KV_Q8_0>(c, a, pl, s);
-        else if (c.type == P1A_KV_Q4_0 && c.D == 128) rc = launch_mfma<P1A_KV_F16, 128, P1A_KV_Q4_0>(c, a, pl, s);
-        else if (c.type == P1A_KV_Q4_0) rc = launch_mfma<P1A_KV_F16, 64, P1A_KV_Q4_0>(c, a, pl, s);
-        else if (c.D == 256) rc = launch_mfma<P1A_KV_F16, 256>(c, a, pl, s);
-        else if (c.D == 128) rc = launch_mfma<P1A_KV_F16, 128>(c, a, pl, s);
-        else rc = launch_mfma<P1A_KV_F16, 64>(c, a, pl, s);
+        if (c.type == P1A_KV_Q8_0 && c.D == 256) rc = launch_mfma<P1A_KV_Q8_0, 256>(c, a, pl, direct, s);
+        else if (c.type == P1A_KV_Q4_0 && c.D == 256) rc = launch_mfma<P1A_KV_Q4_0, 256>(c, a, pl, direct, s);
+        else if (c.type == P1A_KV_Q8_0 && c.D == 128) rc = launch_mfma<P1A_KV_F16, 128, P1A_KV_Q8_0>(c, a, pl, direct, s);
+        else if (c.type == P1A_KV_Q8_0) rc = launch_mfma<P1A_KV_F16, 64, P1A_KV_Q8_0>(c, a, pl, direct, s);
+        else if (c.type == P1A_KV_Q4_0 && c.D == 128) rc = launch_mfma<P1A_KV_F16, 128, P1A_KV_Q4_0>(c, a, pl, direct, s);
+        else if (c.type == P1A_KV_Q4_0) rc = launch_mfma<P1A_KV_F16, 64, P1A_KV_Q4_0>(c, a, pl, direct, s);
+        else if (c.D == 256) rc = launch_mfma<P1A_KV_F16, 256>(c, a, pl, direct, s);
+        else if (c.D == 128) rc = launch_mfma<P1A_KV_F16, 128>(c, a, pl, direct, s);
+        else rc = launch_mfma<P1A_KV_F16, 64>(c, a, pl, direct, s);
     } else {
         rc = launch_decode_any(c, a, pl.RG, pl.nsplit, s);
     }
-    if (rc != P1A_OK || a.skip_merge) return rc;
+    if (rc != P1A_OK || a.skip_merge || direct) return rc;
     merge_k<<<dim3(a.Hq, (c.D + MRG_DIMS - 1) / MRG_DIMS, a.T), 256, 0, s>>>(a.part_o, a.part_ml, a.out, a.gate, pl.nsplit, c.D, a.qbuf, a.Hq, a.T,
                                                        a.pos_rows, a.p0_dev, a.p0, __builtin_ctz(pl.mfma ? 32 * pl.NW : decode_any_unit(c.D)));
     return launched();

@@ -67,12 +67,12 @@ inline void finish_plan(dec_plan & p) { p.NT = p.RG * p.GQA <= 16 ? 1 : 2; }
 // group of the streams that hold keys, counted through on the device: x = 8 * Hkv * GPS * nq, nq eights of streams (`loop`: a workgroup
 // takes the streams q, q + 8 nq, ...)
 struct decode_grid {
-    bool sb, list, loop;   // two workgroups to a compute unit; kinds of dec_mfma_k
+    bool sb, list, loop, direct;   // two workgroups to a compute unit; kinds of dec_mfma_k
     int RPS, GPS;          // rows and row groups of a sequence
     unsigned x, y;
 };
 
-inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv, int n_ctx, int T, int rows_per_seq, bool pos_rows, int cus_) {
+inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv, int n_ctx, int T, int rows_per_seq, bool pos_rows, int cus_, long long host_n = 0) {
     decode_grid r;
     const int cus = cus_ > 0 ? cus_ : 256, groups = (T + pl.RG - 1) / pl.RG;
     const bool staged = type != P1A_KV_F16 && D != 256;
@@ -80,6 +80,20 @@ inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv,
     r.GPS = rows_per_seq > pl.RG ? rows_per_seq / pl.RG : 1;
     if (r.GPS > groups) r.GPS = groups;
     const int nseq = (groups + r.GPS - 1) / r.GPS, inner = Hkv * r.GPS;
+    // One unit at most, as far as the host knows - from the positions (host_n of them; 0: they are in device memory, -1: partials are asked for) or from what a
+    // page-table row holds -, and no more workgroups than compute units: the workgroup of a (row group, kv head) writes the results, eights of row groups to the XCDs,
+    // and there is no merge behind it. Steps of two layers, prep included, with merge_k and so: q8_0, 24 / 4 heads of 256, one sequence of 250 keys 34.4 and 29.6 us,
+    // 32 of them 42.8 and 33.4; f16, 32 / 8 of 128 30.6 and 26.0, 32 of them 40.2 and 33.4; 8 x 4 rows of 250 (24 / 4) 48.1 and 42.0; plain calls of 100 keys 28.4 and 26.5.
+    // Not from two units on: whoever folds last would have to merge, and its stores, counter and loads past the L2s cost what merge_k does (500 keys
+    // 34.6 and 35.3, 2000 35.1 and 36.2, 8000 37 and 48).
+    r.sb = r.list = r.loop = false;
+    const long long sees = host_n ? host_n : n_ctx;
+    r.direct = sees > 0 && sees <= 32 * pl.NW && (long long) groups * Hkv <= cus && !(pl.NT == 2 && type == P1A_KV_Q4_0 && !staged);
+    if (r.direct) {
+        r.x = (unsigned) ((groups + 7) / 8 * 8 * Hkv);
+        r.y = 1;
+        return r;
+    }
     // A call of at least two workgroups per CU whose row groups fit one column tile takes the single-buffered variant, two
     // workgroups to a CU (same partials, bit for bit; measured at 24 / 4 heads, D = 256: 8 q8_0 slots of 1 K ... 27 K 56 ->
     // 47 us, 4 x 64 K q4_0 single rows 92 -> 73 us, 16 x 2 rows q4_0 at 16 K 143 -> 115 us, 32 slots of 2 ... 5 K 104 -> 71 us).

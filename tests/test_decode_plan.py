@@ -63,3 +63,22 @@ def test_drawn_calls():
             assert set(seen) == all_ and set(seen.values()) == {1}, p
             kinds.add((p["sb"], p["loop"], p["NT"]))
     assert len(kinds) >= 5, kinds                              # (two to a unit and one, one stream and several, one column tile and two)
+
+
+@pytest.mark.parametrize("kv_type,Hq,Hkv,D,T,rows", [(F16, 4, 1, 64, 1, 1), (Q8_0, 24, 4, 256, 32, 4), (F16, 24, 4, 256, 31, 1), (Q8_0, 32, 8, 128, 32, 1), (F16, 12, 6, 128, 9, 3), (Q4_0, 16, 2, 256, 2, 1)])
+def test_calls_of_one_unit(kv_type, Hq, Hkv, D, T, rows):
+    """a workgroup for every (row group, kv head) where the host knows that no row sees more than a unit - from the positions before n_ctx -, each taken once,
+    the heads of a group on one XCD; everything else has the grids above"""
+    unit = 128 if kv_type == F16 and D == 256 else 256
+    for n_ctx, host_n, direct in ((unit, 0, 1), (unit + 1, 0, 0), (0, 0, 0), (1 << 17, unit, 1), (1, unit + 1, 0), (unit, -1, 0)):
+        p = plan(kv_type, Hq, Hkv, D, n_ctx, T, rows, pos_rows=host_n == 0, host_n=host_n)
+        assert p["direct"] == direct, (n_ctx, host_n)
+        if not direct:
+            continue
+        groups = -(-T // p["RG"])
+        taken = [((i >> 3) // Hkv * 8 + (i & 7), (i >> 3) % Hkv, i & 7) for i in range(p["x"])]
+        live = [(g, h) for g, h, _ in taken if g * p["RG"] < T]
+        assert p["y"] == 1 and sorted(live) == [(g, h) for g in range(groups) for h in range(Hkv)]
+        assert all(len({x for g, _, x in taken if g == k}) == 1 for k in range(groups))
+    assert not plan(Q4_0, 24, 4, 256, 256, 8, 4)["direct"]     # (two column tiles of q4_0: no registers for it)
+    assert not plan(F16, 32, 32, 64, 256, 9, 1)["direct"]      # (more workgroups than compute units)

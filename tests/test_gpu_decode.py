@@ -294,6 +294,38 @@ def test_short_calls_behind_a_long_one(p1a, kv_type, Hq, Hkv, D, psh):
     assert torch.isnan(got[0]).all()
 
 
+@pytest.mark.parametrize("kv_type,Hq,Hkv,D,rows", [(O.KV_F16, 4, 1, 64, 1), (O.KV_F16, 32, 8, 128, 4), (O.KV_F16, 24, 4, 256, 1), (O.KV_F16, 24, 4, 256, 4), (O.KV_Q8_0, 24, 4, 256, 1), (O.KV_Q8_0, 24, 4, 256, 3),
+                                                   (O.KV_Q4_0, 16, 2, 256, 1), (O.KV_Q8_0, 8, 1, 128, 4), (O.KV_Q4_0, 4, 4, 64, 2), (O.KV_Q8_0, 6, 1, 64, 4), (O.KV_Q4_0, 24, 4, 128, 3)])
+def test_calls_of_one_unit(p1a, kv_type, Hq, Hkv, D, rows):
+    """sequences of one unit of keys, whose workgroups write the results themselves: the bits of the calls that go through partials, gate, a16 values and idle
+    slots included, and close to the oracle"""
+    unit = 128 if kv_type == O.KV_F16 and D == 256 else 256
+    lens = [rows, unit, unit - 1, 17 + rows, 33]
+    pool = Pool(p1a, kv_type, Hq, Hkv, D, 4, lens, seed=41)
+    pos = np.concatenate([np.arange(n - rows, n) for n in lens]).astype(np.int32)
+    pos[4 * rows:] = -1                                               # the last slot is idle
+    T = rows * len(lens)
+    q, gate = dev(I.normal(I.rng(42), (T, Hq, D))), dev(I.normal(I.rng(43), (T, Hq, D)))
+    kv = pool.devkv.with_rows(dev(np.repeat(np.arange(len(lens), dtype=np.int32) * pool.maxp, rows)))
+    got = []
+    for n_ctx in (unit, 0):                                           # (0: nothing is known)
+        kv.n_ctx = n_ctx
+        assert plan(kv_type, Hq, Hkv, D, n_ctx, T, rows)["direct"] == (n_ctx == unit)
+        for g in (gate, None):
+            out, a16 = torch.full((T, Hq, D), 7.0, device="cuda"), torch.full((p1a.a16_bytes(T, Hq * D) // 2,), 7.0, dtype=torch.float16, device="cuda")
+            p1a.attn_decode_rows(q, kv, out, T, dev(pos), Hq, D ** -0.5, gate=g, rows_per_seq=rows, qbuf=a16)
+            got.append((out.cpu(), a16.cpu()))
+    for a, b in zip(got[:2], got[2:]):
+        for x, y in zip(a, b):
+            nan = torch.isnan(x)                                      # (the idle slot's; a NaN has many bit patterns)
+            assert torch.equal(nan, torch.isnan(y)) and torch.equal(x[~nan].view(torch.int16), y[~nan].view(torch.int16))
+    out = got[1][0].numpy()
+    assert np.isnan(out[4 * rows:]).all()
+    for i in range(4):
+        r = slice(i * rows, (i + 1) * rows)
+        check(out[r], O.attn_rows(pool.host_seq(i), q[r].cpu().numpy(), pos[r], Hq, D ** -0.5), f"sequence {i}")
+
+
 def test_other_shapes_and_refusals(p1a):
     # GQA 4 / D 128 f16, GQA 8 / D 64 f16 (MFMA path), q8_0 at D 128 (generic path)
     for kv_type, Hq, Hkv, D in [(O.KV_F16, 8, 2, 128), (O.KV_F16, 8, 1, 64), (O.KV_Q8_0, 8, 2, 128), (O.KV_Q4_0, 6, 3, 96)]:
