@@ -903,11 +903,11 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
         auto fetch = [&](int i) { gt[i] = *reinterpret_cast<const f4 *>(P.gate + row_index(wrow0 + min(row_at(i), wlast)) * D + d4); };
 #pragma unroll
         for (int i = 0; i < N8; ++i) fetch(i);
-        if (P.rpw > 8) {
+        if (wrows > 8) {
 #pragma unroll
             for (int i = N8; i < 2 * N8; ++i) fetch(i);
         }
-        if (P.rpw > 16) {
+        if (wrows > 16) {
 #pragma unroll
             for (int i = 2 * N8; i < NRI; ++i) fetch(i);
         }
