@@ -67,6 +67,12 @@ template <uint32_t KS, int D> struct raw_cfg {
     static_assert(HB % 4 == 0, "raw head rows are whole dwords");
 };
 
+// f16 tiles: rows of D / 8 16-byte chunks without padding, every one of which starts in the same LDS bank (D = 64: every other). So chunk i of
+// row r lies where chunk i ^ swz(r) would - a lane of a tile fetch brings whichever chunk of its row belongs where it writes -, and what 16 rows are read
+// at together is spread over all banks. Two layers with prep: f16, 24 / 4 heads of 256, 4 sequences of 2000 ... 8000 keys 60.2 -> 55.7 us; tiles converted to f16, 24 / 4 of
+// 128, q4_0, 8 x 2 rows of 8000 ... 32000 162 -> 136, q8_0 (32 / 8) 234 -> 222; heads of 64 level.
+template <int D> __device__ __forceinline__ int swz(int row) { return D == 64 ? (row >> 1) & 7 : row & 15; }
+
 struct dec_params {
     const float * q;
     const char * kc;
@@ -206,7 +212,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     static_assert(!DIRECT || (!SB && !LIST), "such calls have a workgroup to a CU at most");
     using C = tile_cfg<KT, D>;
     using RW = raw_cfg<KS, D>;
-    constexpr bool STG = KS != KT;
+    constexpr bool STG = KS != KT, SWZ = KT == P1A_KV_F16;
     static_assert(!SB || NT == 1, "the single-buffered variant has one column tile");
     static_assert(!STG || (KT == P1A_KV_F16 && !SB && D <= 128), "staged tiles are converted to f16 and take the double-buffered build");
     constexpr int NLD = STG ? RW::NRND : C::NRND;             // vector-memory operations per tile fetch
@@ -401,7 +407,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     for (int rd = 0; rd < NLD; ++rd) {
         const int i = rd * 64 + lane;
         const int key = i / IPK, cir = i - key * IPK;
-        soff[rd] = (unsigned) (key * rowb + (int) head_off + cir * ISZ);
+        soff[rd] = (unsigned) (key * rowb + (int) head_off + (SWZ && !STG ? cir ^ swz<D>(key) : cir) * ISZ);
     }
 
     // Tile t of this wave (t = 0, 1, ...): unit split + (t >> 1) * nsplit, keys [ts, ts + 16) with
@@ -424,7 +430,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
                 off -= (uint32_t) (max(ii / C::CPK - last, 0) * rowb);
             } else {
                 const int key = i / IPK, cir = i - key * IPK;
-                off = (uint32_t) (min(key, last) * rowb + (int) head_off + cir * ISZ);
+                off = (uint32_t) (min(key, last) * rowb + (int) head_off + (SWZ && !STG ? cir ^ swz<D>(key) : cir) * ISZ);
             }
         }
         if constexpr (STG) { if (RW::NDW % 64 == 0 || i < RW::NDW) dma4(b0, off, lds_addr(slot) + rd * 256); }
@@ -445,7 +451,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
                 const uint32_t d16 = *reinterpret_cast<const uint16_t *>(row + 2 * (p8 >> 2));
                 const h2 dd = __builtin_bit_cast(h2, d16 | (d16 << 16));
                 const u2 a = deq4(w0, dd, dd), b = deq4(w1, dd, dd);
-                *reinterpret_cast<u4 *>(dst + key * (2 * D) + 16 * p8) = u4{a.lo, a.hi, b.lo, b.hi};
+                *reinterpret_cast<u4 *>(dst + key * (2 * D) + 16 * (p8 ^ swz<D>(key))) = u4{a.lo, a.hi, b.lo, b.hi};
             }
         } else if constexpr (STG) {
             // item = one 18-byte block of one key (2-byte aligned): values 0 .. 15 are its low nibbles, 16 .. 31 the high ones
@@ -465,8 +471,9 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
                         lo[q >> 1][2 * (q & 1)] = l.lo; lo[q >> 1][2 * (q & 1) + 1] = l.hi;
                         hi[q >> 1][2 * (q & 1)] = h.lo; hi[q >> 1][2 * (q & 1) + 1] = h.hi;
                     }
-                    u4 * o = reinterpret_cast<u4 *>(dst + key * (2 * D) + 64 * b);
-                    o[0] = lo[0]; o[1] = lo[1]; o[2] = hi[0]; o[3] = hi[1];
+                    u4 * o = reinterpret_cast<u4 *>(dst + key * (2 * D));
+                    const int sw = swz<D>(key);
+                    o[(4 * b) ^ sw] = lo[0]; o[(4 * b + 1) ^ sw] = lo[1]; o[(4 * b + 2) ^ sw] = hi[0]; o[(4 * b + 3) ^ sw] = hi[1];
                 }
             }
         }
@@ -616,9 +623,10 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
         for (int r = 0; r < NT; ++r) s[r] = f4{0.f, 0.f, 0.f, 0.f};
         const char * krow = ks + c * C::HB;
         if constexpr (KT == P1A_KV_F16) {
+            const int ksw = 16 * (g ^ swz<D>(c));
 #pragma unroll
             for (int m = 0; m < C::NMF; ++m) {
-                const h8 a = *reinterpret_cast<const h8 *>(krow + (4 * m + g) * 16);
+                const h8 a = *reinterpret_cast<const h8 *>(krow + (64 * m ^ ksw));
 #pragma unroll
                 for (int r = 0; r < NT; ++r) {
                     h8 qo;
@@ -741,10 +749,11 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
         // ---- O^T += V^T P^T: k-slot i of lane group g is key ts + 4 g + i, the key of this lane's P value i ----
         if constexpr (KT == P1A_KV_F16) {
             const int kk = c >> 2, jq = c & 3;
-            const char * vr0 = vs + (4 * g + kk) * C::HB + jq * 8;
+            const char * vr0 = vs + (4 * g + kk) * C::HB + 8 * (jq & 1);
+            const int vsw = 16 * ((jq >> 1) ^ swz<D>(4 * g + kk));
 #pragma unroll
             for (int j = 0; j < C::NDT; ++j) {
-                const s4 w = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s4 __attribute__((address_space(3))) *) (vr0 + j * 32));
+                const s4 w = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s4 __attribute__((address_space(3))) *) (vr0 + (32 * j ^ vsw)));
                 const h4 a = __builtin_bit_cast(h4, w);
 #pragma unroll
                 for (int r = 0; r < NT; ++r) o[r][j] = __builtin_amdgcn_mfma_f32_16x16x16f16(a, pb[r], o[r][j], 0, 0, 0);
