@@ -203,8 +203,8 @@ template <int NR> __device__ __forceinline__ void wait_tiles(int newer) {
 // KS (when it differs from KT = f16): the type the cache holds - its raw tiles are staged (raw_cfg) and converted to f16
 // HOW = KS, and for calls of several sequences LIST (workgroups take the streams that hold keys), LIST | LOOP (one takes several);
 // DIRECT for calls whose rows see one unit at most, as far as the host knows: a workgroup for every (row group, kv head) writes the
-// results itself
-constexpr uint32_t LIST_ = 0x100, LOOP_ = 0x200, DIRECT_ = 0x400;
+// results itself; STAGED_SB marks the single-buffered builds of staged tiles
+constexpr uint32_t LIST_ = 0x100, LOOP_ = 0x200, DIRECT_ = 0x400, STAGED_SB_ = 0x800;
 template <uint32_t KT, int D, int NT, int NWV, bool SB, uint32_t HOW = KT>
 __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const dec_params P_) {
     constexpr uint32_t KS = HOW & 0xff;
@@ -214,22 +214,23 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     using RW = raw_cfg<KS, D>;
     constexpr bool STG = KS != KT, SWZ = KT == P1A_KV_F16;
     static_assert(!SB || NT == 1, "the single-buffered variant has one column tile");
-    static_assert(!STG || (KT == P1A_KV_F16 && !SB && D <= 128), "staged tiles are converted to f16 and take the double-buffered build");
+    static_assert(!STG || (KT == P1A_KV_F16 && D <= 128), "staged tiles are converted to f16");
     constexpr int NLD = STG ? RW::NRND : C::NRND;             // vector-memory operations per tile fetch
-    // STG: slot array 0 = the f16 K tile of every wave, 1 = the f16 V tile, 2 = two raw K tiles, 3 = two raw V tiles
+    // STG: slot array 0 = the f16 K tile of every wave, 1 = the f16 V tile, 2 = two raw K tiles, 3 = two raw V tiles (SB: the pool holds one f16 tile
+    // per wave, K first and then V, one raw K tile and one raw V tile)
     constexpr int SLOTX = STG ? (C::SLOT_B > 2 * RW::RAW_B ? C::SLOT_B : 2 * RW::RAW_B) : C::SLOT_B;
     // four tile slots per wave (K and V, two each), plus a small per-wave table. SB: one pool that holds one K slot, one
     // V slot (and the q4_0 copy) per wave at the size of a tile, and is handed over to the fold as a whole afterwards:
     // wave w parks 8 columns at a time, dim quarter k at PARK_B (4 w + k)
     constexpr int SLB = SB ? C::TILE_B : SLOTX;                // bytes per slot
     constexpr int PARK_B = 8 * C::QDP * 4;                     // SB: one dim quarter of 8 parked columns
-    constexpr int POOL_T = NWV * (2 * C::TILE_B + C::VA_B), POOL_P = NWV * 4 * PARK_B;
+    constexpr int POOL_T = NWV * (STG ? C::TILE_B + 2 * RW::RAW_B : 2 * C::TILE_B + C::VA_B), POOL_P = NWV * 4 * PARK_B;
     __shared__ __attribute__((aligned(16))) char pool[SB ? (POOL_T > POOL_P ? POOL_T : POOL_P) : 16];
     // (one array, slot array k at k NWV SLOT_B: K slot 0, K slot 1, V slot 0, V slot 1 - the fold addresses them by number)
     __shared__ __attribute__((aligned(16))) char slots[SB ? 16 : 4 * NWV * SLOTX];
     __shared__ __attribute__((aligned(16))) char qown[SB ? 16 * C::QRS : 16];          // SB: the f16 Q table (first the fp32 copy of up to 8 rows)
     // (STG: "K slot 1" / "V slot 1" - where the Q copies go before any tile is converted - are the f16 tile arrays themselves)
-    char * const kb0 = SB ? pool : slots, * const vb0 = SB ? pool + NWV * C::TILE_B : STG ? slots + NWV * SLOTX : slots + 2 * NWV * SLOTX;
+    char * const kb0 = SB ? pool : slots, * const vb0 = SB ? pool + (STG ? 0 : NWV * C::TILE_B) : STG ? slots + NWV * SLOTX : slots + 2 * NWV * SLOTX;
     char * const kb1 = SB || STG ? kb0 : slots + NWV * SLOTX, * const vb1 = SB || STG ? vb0 : slots + 3 * NWV * SLOTX;
     static_assert(SB || (32 * D * 4 <= NWV * SLOTX && 32 * C::QRS <= NWV * SLOTX), "the Q copies (at most 32 columns) fit over the second K and V slots");
     static_assert(!SB || 8 * D * 4 <= 16 * C::QRS, "SB: the fp32 copy of 8 rows fits where the f16 table of 16 goes");
@@ -353,7 +354,8 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     char * const vs0 = vb0 + wave * SLB, * const vs1 = vb1 + wave * SLB;
     char * const tab = tabs + wave * C::TAB_B;
     char * const va = (SB ? pool + 2 * NWV * C::TILE_B : vab) + wave * C::VA_B;
-    char * const rawk = slots + (2 * NWV + wave) * SLOTX, * const rawv = slots + (3 * NWV + wave) * SLOTX;   // STG: two raw tiles each
+    char * const rawk = SB ? pool + NWV * C::TILE_B + wave * RW::RAW_B : slots + (2 * NWV + wave) * SLOTX;   // STG: two raw tiles each (SB: one)
+    char * const rawv = SB ? rawk + NWV * RW::RAW_B : slots + (3 * NWV + wave) * SLOTX;
 
     // column -> row of the group (at most 4 rows: three comparisons instead of a division)
     auto row_of = [&](int col) { return (col >= P.GQA) + (col >= 2 * P.GQA) + (col >= 3 * P.GQA); };
@@ -427,7 +429,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
             if constexpr (SB) {   // worked out from scratch rather than from values kept in registers through the key loop
                 int ii = i;
                 asm volatile("" : "+v"(ii));
-                off -= (uint32_t) (max(ii / C::CPK - last, 0) * rowb);
+                off -= (uint32_t) (max(ii / IPK - last, 0) * rowb);
             } else {
                 const int key = i / IPK, cir = i - key * IPK;
                 off = (uint32_t) (min(key, last) * rowb + (int) head_off + (SWZ && !STG ? cir ^ swz<D>(key) : cir) * ISZ);
@@ -604,7 +606,8 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     // one 16-key tile from slots (ks, vs); the loads of tile t + 1 into (ksn, vsn) are issued between its products
     auto step = [&](char * ks, char * vs, char * ksn_, char * vsn_, int t) {
         // (STG: ks / vs are the wave's f16 tiles; the raw tiles alternate between the two halves of its raw areas)
-        char * const ksn = STG ? rawk + ((t + 1) & 1) * RW::RAW_B : ksn_, * const vsn = STG ? rawv + ((t + 1) & 1) * RW::RAW_B : vsn_;
+        constexpr int RAW2 = SB ? 0 : RW::RAW_B;
+        char * const ksn = STG ? rawk + ((t + 1) & 1) * RAW2 : ksn_, * const vsn = STG ? rawv + ((t + 1) & 1) * RAW2 : vsn_;
         const int ts = tile_start(t);
         const int tn = tile_start(t + 1);
         const bool have_n = tn < n_max;
@@ -614,9 +617,16 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
         int pgn = 0;
         if (ptab && have_n) pgn = sload_i32(page_of(tn));
         wait_vm_imm<NLD>();                                   // K of tile t has landed (only its V is younger)
-        if constexpr (STG) convert(rawk + (t & 1) * RW::RAW_B, ks);
+        if constexpr (STG) convert(rawk + (t & 1) * RAW2, ks);
         const size_t on = have_n ? tile_off(tn, pgn) : 0;
         const char * const kn = P.kc + on, * const vn = P.vc + on;
+        // (SB: a slot is free once its last read has come back; a raw tile's are the conversion's)
+        auto refill = [&](char * slot, const char * b0) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int rd = 0; rd < NLD; ++rd) fetch_round(slot, b0, tn, rd);
+        };
+        if (SB && STG && have_n) refill(ksn, kn);
         // ---- S^T = K Q^T ----
         f4 s[NT];
 #pragma unroll
@@ -701,11 +711,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
 #pragma unroll
             for (int rd = (KT == P1A_KV_Q8_0 ? C::NMF / 2 : C::NMF); rd < NLD; ++rd) fetch_round(ksn, kn, tn, rd);
         }
-        if (SB && have_n) {    // the K slot is free once its last fragment has been read
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-            for (int rd = 0; rd < NLD; ++rd) fetch_round(ksn, kn, tn, rd);
-        }
+        if (SB && !STG && have_n) refill(ksn, kn);
 
         // ---- online softmax (log2 domain); column = query row, this lane holds keys ts + 4 g + i ----
         h4 pb[NT];
@@ -745,7 +751,8 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
         }
 
         if (have_n) wait_vm_imm<NLD>(); else wait_vm_imm<0>();   // V of tile t has landed (only K of t + 1 is younger)
-        if constexpr (STG) convert(rawv + (t & 1) * RW::RAW_B, vs);
+        if constexpr (STG) convert(rawv + (t & 1) * RAW2, vs);
+        if (SB && STG && have_n) refill(vsn, vn);
         // ---- O^T += V^T P^T: k-slot i of lane group g is key ts + 4 g + i, the key of this lane's P value i ----
         if constexpr (KT == P1A_KV_F16) {
             const int kk = c >> 2, jq = c & 3;
@@ -851,11 +858,7 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
             }
         }
         static_assert(KT == P1A_KV_F16 || NLD <= (KT == P1A_KV_Q8_0 ? C::NDT / 2 : C::NMF / 2), "the PV loop must have room for every V load");
-        if (SB && have_n) {    // the V slot likewise
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-            for (int rd = 0; rd < NLD; ++rd) fetch_round(vsn, vn, tn, rd);
-        }
+        if (SB && !STG && have_n) refill(vsn, vn);
 #pragma unroll
         for (int r = 0; r < NT; ++r) ol[r] = __builtin_amdgcn_mfma_f32_16x16x16f16(ones, pb[r], ol[r], 0, 0, 0);
     };
@@ -1192,20 +1195,23 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, bo
     auto go = [&](auto nt, auto single, auto can_loop) {
         constexpr int NT = decltype(nt)::value, NW = big_tiles ? 4 : 8;
         constexpr bool SB = decltype(single)::value;
+        constexpr uint32_t HOW = SB && KS != KT ? KS | STAGED_SB_ : KS;
         if constexpr (!SB && (NT == 1 || KT != P1A_KV_Q4_0)) {   // (plan_grid asks for no other)
             if (gr.direct) { dec_mfma_k<KT, D, NT, NW, false, KS | DIRECT_><<<grid, NW * 64, 0, s>>>(P); return; }
         }
         if constexpr (decltype(can_loop)::value) {
-            if (gr.loop) { dec_mfma_k<KT, D, NT, NW, SB, KS | LIST_ | LOOP_><<<grid, NW * 64, 0, s>>>(P); return; }
+            if (gr.loop) { dec_mfma_k<KT, D, NT, NW, SB, HOW | LIST_ | LOOP_><<<grid, NW * 64, 0, s>>>(P); return; }
         }
-        if (gr.list) dec_mfma_k<KT, D, NT, NW, SB, KS | LIST_><<<grid, NW * 64, 0, s>>>(P);
-        else dec_mfma_k<KT, D, NT, NW, SB, KS><<<grid, NW * 64, 0, s>>>(P);
+        if (gr.list) dec_mfma_k<KT, D, NT, NW, SB, HOW | LIST_><<<grid, NW * 64, 0, s>>>(P);
+        else dec_mfma_k<KT, D, NT, NW, SB, HOW><<<grid, NW * 64, 0, s>>>(P);
     };
     constexpr std::true_type yes;
     constexpr std::false_type no;
     if (pl.NT == 2) go(std::integral_constant<int, 2>{}, no, std::bool_constant<can_loop_2>{});
-    else if constexpr (KS != KT) go(std::integral_constant<int, 1>{}, no, yes);
-    else if (gr.sb) go(std::integral_constant<int, 1>{}, yes, yes);
+    else if constexpr (KS != KT) {                            // (heads of 64: one workgroup to a unit, see plan_grid)
+        if constexpr (D == 128) { if (gr.sb) { go(std::integral_constant<int, 1>{}, yes, yes); return launched(); } }
+        go(std::integral_constant<int, 1>{}, no, yes);
+    } else if (gr.sb) go(std::integral_constant<int, 1>{}, yes, yes);
     else go(std::integral_constant<int, 1>{}, no, no);
     return launched();
 }

@@ -97,7 +97,11 @@ inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv,
     // A call of at least two workgroups per CU whose row groups fit one column tile takes the single-buffered variant, two
     // workgroups to a CU (same partials, bit for bit; measured at 24 / 4 heads, D = 256: 8 q8_0 slots of 1 K ... 27 K 56 ->
     // 47 us, 4 x 64 K q4_0 single rows 92 -> 73 us, 16 x 2 rows q4_0 at 16 K 143 -> 115 us, 32 slots of 2 ... 5 K 104 -> 71 us).
-    r.sb = !staged && pl.NT == 1 && (long long) pl.nsplit * Hkv * groups >= 2LL * cus;
+    // Staged tiles, D = 128: so too where more workgroups than compute units can have keys (two layers with prep, one to a unit and two: q8_0, 32 / 8 heads, 16 sequences of 2000 ... 8000
+    // keys 161 and 112 us, 4 of 8000 ... 32000 120 and 101; q4_0, 24 / 4, 8 x 2 rows of 8000 ... 32000 136 and 108, 32 sequences of 1000 53 and 45; but 8 x 2 rows of 1000 36.7 and 38.3). Not at D = 64,
+    // whose conversions are half as long (q8_0, 16 / 4, 32 of 2000 ... 8000 79 and 85; q4_0, 8 / 8, 2 of 32000 54.4 and 53.5).
+    const bool two = !staged || (D == 128 && ((long long) n_ctx + 32 * pl.NW - 1) / (32 * pl.NW) * groups * Hkv > cus);
+    r.sb = pl.NT == 1 && two && (long long) pl.nsplit * Hkv * groups >= 2LL * cus;
     // The list (see dec_mfma_k) costs a workgroup some 0.2 us before its first request. Where two workgroups share a compute unit that hides,
     // and every call of several row groups takes it. Several sequences (110 calls of 2 ... 32 drawn over 4 ... 131072 keys, D = 256 and f16):
     // 0.98 - 1.6 times as fast, 1.1 in the mean. One sequence of 5 ... 32 rows (200 calls over 200, 3000 and 20000 keys, six head shapes):
@@ -126,11 +130,13 @@ inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv,
     //   32 of 256 77, 71, 43; q4_0, 24 / 4 of 128, 16 of 60 ... 1500 58.5, 46.9, 40.3).
     // All of these are times with page-table rows as wide as the sequences. Rows of 32768 positions, a server's limit, take the other route
     // whatever the sequences hold: 72.2, 53.9, 78.3 and 58.6 us for the last four, 45.8 for 32 of 1024 (f16, 16 / 4 of 64).
-    const long long most = (r.sb ? 16LL : 2LL) * cus / (8 * inner);
-    const bool can_loop = pl.NT == 2 ? staged || type != P1A_KV_Q4_0 : staged || r.sb;   // (q4_0 with two column tiles has no register left for it)
+    //   Staged tiles, two to a unit: two for every compute unit where page-table rows cannot hold half of it, as in the second kind.
+    const bool resident = !r.sb || (staged && 2LL * n_ctx <= once);
+    const long long most = (resident ? 2LL : 16LL) * cus / (8 * inner);
+    const bool can_loop = pl.NT == 2 ? staged || type != P1A_KV_Q4_0 : r.sb || staged;   // (q4_0 with two column tiles has no register left for it)
     r.loop = can_loop && nq > most;
     // (never none: 8 * inner workgroups are more than that where kv heads and row groups are many)
-    if (r.loop) nq = std::max(1LL, r.sb && 4LL * n_ctx <= once ? (most + 3) / 4 : most);
+    if (r.loop) nq = std::max(1LL, r.sb && !staged && 4LL * n_ctx <= once ? (most + 3) / 4 : most);
     r.x = (unsigned) (8 * inner * nq);
     r.y = 1;
     return r;

@@ -547,6 +547,28 @@ def test_understated_n_ctx_of_several_sequences(p1a, kv_type, Hq, D, lens):
     assert len(grids) > 1, grids
 
 
+@pytest.mark.parametrize("kv_type,Hq,Hkv,lens,rows,loop", [(O.KV_Q8_0, 32, 8, [9000, 1, 16, 17, 5000, 300], 1, 0), (O.KV_Q4_0, 48, 8, [8500, 2, 33, 6000], 2, 0), (O.KV_Q8_0, 12, 4, [17000, 4, 1000], 4, 0),
+                                                             (O.KV_Q4_0, 4, 4, [1100 - 9 * i for i in range(32)], 1, 1), (O.KV_Q8_0, 16, 2, [3000 - 100 * i for i in range(20)], 1, 1)])
+def test_staged_tiles_two_workgroups_to_a_unit(p1a, kv_type, Hq, Hkv, lens, rows, loop):
+    """one raw tile of K and of V a wave and one f16 tile for both: the bits of single rows, which take the build with two of each; up to eight columns, more, one stream a workgroup and several"""
+    n_ctx = (max(lens) + 63) // 64 * 64
+    p = plan(kv_type, Hq, Hkv, 128, n_ctx, len(lens) * rows, rows, cus=torch.cuda.get_device_properties(0).multi_processor_count)
+    assert p["sb"] and p["list"] and p["loop"] == loop, p
+    rows_against_calls_of_their_own(p1a, kv_type, Hq, Hkv, 128, 6, lens, rows)
+
+
+def test_staged_tiles_many_rows_of_one_call(p1a):
+    """the same without row positions: two workgroups to a unit and no list"""
+    Hq, Hkv, D, n = 32, 8, 128, 4000
+    pool = Pool(p1a, O.KV_Q8_0, Hq, Hkv, D, 6, [n], seed=51)
+    assert plan(O.KV_Q8_0, Hq, Hkv, D, n, 11, pos_rows=False)["sb"]
+    q = I.normal(I.rng(52), (11, Hq, D))
+    out = run_decode(p1a, pool.dev_seq(0), q, 11, n - 11, Hq, D ** -0.5)
+    check(out, O.attn_rows(pool.host_seq(0), q, np.arange(n - 11, n), Hq, D ** -0.5), "11 rows")
+    for t in range(11):
+        assert np.array_equal(run_decode(p1a, pool.dev_seq(0), q[t:t + 1], 1, n - 11 + t, Hq, D ** -0.5)[0], out[t]), t
+
+
 # every build of dec_mfma_k whose workgroups take several streams: two to a compute unit, staged tiles, two column tiles
 LONG, SHORT = [3900 - 11 * i for i in range(8)], [1900 - 7 * i for i in range(32)]
 SEVERAL = [(O.KV_Q8_0, 8, 8, 256, 6, SHORT, 1), (O.KV_Q4_0, 8, 8, 256, 6, SHORT, 1), (O.KV_F16, 8, 8, 128, 4, SHORT, 1), (O.KV_F16, 8, 8, 64, 4, SHORT, 1),
