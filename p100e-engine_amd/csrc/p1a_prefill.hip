@@ -340,11 +340,7 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
         for (int i = N8; i < NRI; ++i) a[i] = make_float4(0.f, 0.f, 0.f, 0.f);
         if (P.rpw > 8) {
 #pragma unroll
-            for (int i = N8; i < 2 * N8; ++i) fetch(i);
-        }
-        if (P.rpw > 16) {
-#pragma unroll
-            for (int i = 2 * N8; i < NRI; ++i) fetch(i);
+            for (int i = N8; i < NRI; ++i) fetch(i);
         }
         between();
         const float s = P.qscale;
@@ -896,8 +892,8 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
     constexpr int ORS = 4 * D + 16;
     const int d4 = 4 * (lane % LPF);
     // All of the wave's gate rows are asked for before the first result is put down: eight at a time, each batch behind the stores of the
-    // one before, a round trip to memory stood in front of every quarter of the rows (prep and prefill, with no more Q rows fetched than a block has: first 512 tokens, f16,
-    // 24 / 4 heads of 256 39.0 -> 37.5 us, 2000 (q8_0) 122.7 -> 117.8; 32 / 8 of 128, 512 30.5 -> 28.6)
+    // one before, a round trip to memory stood in front of every quarter of the rows (prep and prefill of the first 512 tokens, f16,
+    // 24 / 4 heads of 256 38.2 -> 37.1 us, 800 54.0 -> 52.0, 2000 (q8_0) 122.7 -> 118; 32 / 8 of 128, 512 29.6 -> 28.6)
     f4 gt[NRI];
     if (P.gate) {
         auto fetch = [&](int i) { gt[i] = *reinterpret_cast<const f4 *>(P.gate + row_index(wrow0 + min(row_at(i), wlast)) * D + d4); };
