@@ -25,7 +25,8 @@
 //   dim. Q is pre-multiplied by scale * log2(e) and rounded to f16, P = 2^(S - m) is rounded to f16, all accumulation
 //   is fp32. The softmax denominator is one more MFMA against an all-ones operand, so it sums exactly the P that
 //   multiplies V. The waves of one head fold their (m, l, O) through LDS; one partial per (workgroup, head) goes to
-//   scratch and merge_k folds the splits in a fixed order and applies the sigmoid gate.
+//   scratch and merge_k folds the splits in a fixed order and applies the sigmoid gate (a call whose rows see one unit at most has one
+//   partial a row: its workgroups write the results, DIRECT).
 #include "p1a_common.hpp"
 #include "p1a_plan.hpp"
 
