@@ -1037,10 +1037,22 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
 // stream's (m, l): few kv heads have many (one, 256), and one row over 500 keys (f16, 4 / 1 heads of 64, two layers with prep, recorded) took
 // 34.4 us, 27.5 so; 16 / 2 of 256 (q4_0) 37.4 and 34.8.
 constexpr int MRG_DIMS = 128;
-__global__ void __launch_bounds__(256) merge_k(const float * __restrict__ part_o, const float * __restrict__ part_ml,
-                                               float * __restrict__ out, const float * __restrict__ gate, int NS_all, int D,
-                                               void * qbuf, int Hq, int T, const int32_t * __restrict__ pos_rows,
-                                               const int32_t * __restrict__ p0_dev, int p0, int u_sh) {
+// (one kernel argument: the host pays for each. Plain steps of four layers, which the host bounds, with 13 arguments and so: f16, 4 / 1 heads of 64 61 and 54 us,
+// 32 / 8 of 128 60 and 52, q8_0, 24 / 4 of 256 62 and 58; recorded ones level.)
+struct merge_params {
+    const float * part_o, * part_ml;
+    float * out;
+    const float * gate;
+    void * qbuf;
+    const int32_t * pos_rows, * p0_dev;
+    int NS_all, D, Hq, T, p0, u_sh;
+};
+__global__ void __launch_bounds__(256) merge_k(const merge_params P) {
+    const float * __restrict__ const part_o = P.part_o, * __restrict__ const part_ml = P.part_ml, * __restrict__ const gate = P.gate;
+    float * __restrict__ const out = P.out;
+    const int32_t * __restrict__ const pos_rows = P.pos_rows, * __restrict__ p0_dev = P.p0_dev;
+    void * const qbuf = P.qbuf;
+    const int NS_all = P.NS_all, D = P.D, Hq = P.Hq, T = P.T, p0 = P.p0, u_sh = P.u_sh;
     __shared__ f4 sacc[8][32];
     __shared__ float sden[8];
     const int t_row = blockIdx.z;
@@ -1260,8 +1272,9 @@ int launch_decode(const p1a_kv & c, const decode_args & a, hipStream_t s) {
         rc = launch_decode_any(c, a, pl.RG, pl.nsplit, s);
     }
     if (rc != P1A_OK || a.skip_merge || direct) return rc;
-    merge_k<<<dim3(a.Hq, (c.D + MRG_DIMS - 1) / MRG_DIMS, a.T), 256, 0, s>>>(a.part_o, a.part_ml, a.out, a.gate, pl.nsplit, c.D, a.qbuf, a.Hq, a.T,
-                                                       a.pos_rows, a.p0_dev, a.p0, __builtin_ctz(pl.mfma ? 32 * pl.NW : decode_any_unit(c.D)));
+    const merge_params M{a.part_o, a.part_ml, a.out, a.gate, a.qbuf, a.pos_rows, a.p0_dev, pl.nsplit, c.D, a.Hq, a.T, a.p0,
+                         __builtin_ctz(pl.mfma ? 32 * pl.NW : decode_any_unit(c.D))};
+    merge_k<<<dim3(a.Hq, (c.D + MRG_DIMS - 1) / MRG_DIMS, a.T), 256, 0, s>>>(M);
     return launched();
 }
 
