@@ -241,12 +241,12 @@ template <uint32_t KT> __device__ __forceinline__ void write_head(char * row, in
     }
 }
 template <uint32_t KT>
-__global__ void __launch_bounds__(64) prep_k(const float * __restrict__ qg, const float * __restrict__ k,
-                                             const float * __restrict__ v, const float * __restrict__ qn,
-                                             const float * __restrict__ kn, const int32_t * __restrict__ pos,
-                                             float * __restrict__ q, float * __restrict__ gate, char * kc, char * vc, int p0,
-                                             int Hq, int Hkv, int D, int n_rot, double ln_base, float eps, int ldq, int ldk,
-                                             int ldv, kv_view pg, mrope_view mr) {
+__device__ __forceinline__ void prep_head(const float * __restrict__ qg, const float * __restrict__ k,
+                                          const float * __restrict__ v, const float * __restrict__ qn,
+                                          const float * __restrict__ kn, const int32_t * __restrict__ pos,
+                                          float * __restrict__ q, float * __restrict__ gate, char * kc, char * vc, int p0,
+                                          int Hq, int Hkv, int D, int n_rot, double ln_base, float eps, int ldq, int ldk,
+                                          int ldv, const kv_view & pg, const mrope_view & mr) {
     const int t = blockIdx.y, b = blockIdx.x, i = threadIdx.x;
     const bool live = 4 * i < D;                               // dead lanes form whole 8-lane groups (D % 32 == 0)
     const int row = p0 < 0 ? pos[t] : p0 + t;                  // cache position of token t (src/fast/fused.cu:520)
@@ -308,6 +308,23 @@ __global__ void __launch_bounds__(64) prep_k(const float * __restrict__ qg, cons
     } else {
         write_head<KT>(kc + o, h, D, i, live, r);
     }
+}
+struct prep_params {
+    const float * qg, * k, * v, * qn, * kn;
+    const int32_t * pos;
+    float * q, * gate;
+    char * kc, * vc;
+    double ln_base;
+    kv_view pg;
+    mrope_view mr;
+    int p0, Hq, Hkv, D, n_rot, ldq, ldk, ldv;
+    float eps;
+};
+// (one kernel argument: the host pays for each. Plain steps of four layers with 21 of them and so: f16, 4 / 1 heads of 64 54.6 and 53.2 us, 32 / 8 of 128 53.4 and
+// 52.0, recorded ones level.)
+template <uint32_t KT> __global__ void __launch_bounds__(64) prep_k(const prep_params P) {
+    prep_head<KT>(P.qg, P.k, P.v, P.qn, P.kn, P.pos, P.q, P.gate, P.kc, P.vc, P.p0, P.Hq, P.Hkv, P.D, P.n_rot, P.ln_base, P.eps, P.ldq, P.ldk,
+                  P.ldv, P.pg, P.mr);
 }
 
 // The same for calls of many tokens, which one wave per (head, token) spent on the angles - some 250 double operations,
@@ -513,12 +530,10 @@ int launch_prep(const p1a_kv & c, const float * qg, const float * k, const float
         return launched();
     }
     const dim3 grid(H, T);
-#define P1A_PREP(KT_) prep_k<KT_><<<grid, 64, 0, s>>>(qg, k, v, q_norm, k_norm, pos, q, gate, kc, vc, p0, Hq, c.Hkv, c.D, n_rot, \
-                                                      ln_base, eps, ldq, ldk, ldv, pg, mr)
-    if (c.type == P1A_KV_F16) P1A_PREP(P1A_KV_F16);
-    else if (c.type == P1A_KV_Q8_0) P1A_PREP(P1A_KV_Q8_0);
-    else P1A_PREP(P1A_KV_Q4_0);
-#undef P1A_PREP
+    const prep_params P{qg, k, v, q_norm, k_norm, pos, q, gate, kc, vc, ln_base, pg, mr, p0, Hq, c.Hkv, c.D, n_rot, ldq, ldk, ldv, eps};
+    if (c.type == P1A_KV_F16) prep_k<P1A_KV_F16><<<grid, 64, 0, s>>>(P);
+    else if (c.type == P1A_KV_Q8_0) prep_k<P1A_KV_Q8_0><<<grid, 64, 0, s>>>(P);
+    else prep_k<P1A_KV_Q4_0><<<grid, 64, 0, s>>>(P);
     return launched();
 }
 
