@@ -93,6 +93,7 @@ struct dec_params {
     int rps_magic;    // LIST: 65536 / RPS + 1
     int hkv_sh;       // log2(Hkv) when Hkv is a power of two, else -1
     int npt;          // page-table entries of one sequence (ceil(n_ctx / page positions)); 0 = contiguous
+    int deal_sh;      // DIRECT: log2 of the row groups that are dealt to the XCDs at a time
     float * out;      // DIRECT: where the results go, the gate, the a16 values
     const float * gate;
     void * qbuf;
@@ -309,10 +310,10 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
         return true;
     };
     int row0;
-    if constexpr (DIRECT) {                                   // (the heads of a group on one XCD)
-        const int i = blockIdx.x, j = i >> 3, jg = j / HG;
+    if constexpr (DIRECT) {
+        const int i = blockIdx.x, j = i >> P.deal_sh, jg = j / HG;
         hg = j - jg * HG;
-        row0 = (jg * 8 + (i & 7)) * P.RG;
+        row0 = ((jg << P.deal_sh) + (i & ((1 << P.deal_sh) - 1))) * P.RG;
         if (row0 >= P.T) return;
     } else if constexpr (LIST) {
         const stream_at at = pick_stream(u_sum, q, q_a, lane);
@@ -1192,6 +1193,7 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, bo
     constexpr bool big_tiles = KT == P1A_KV_F16 && D == 256;
     const decode_grid gr = plan_grid(pl, KS, D, c.Hkv, c.n_ctx, a.T, a.rows_per_seq, a.pos_rows != nullptr, a.cus, a.skip_merge ? -1 : a.host_n);
     direct = gr.direct;
+    P.deal_sh = gr.deal_sh;
     P.RPS = gr.RPS;
     P.GPS = gr.GPS;
     P.rps_magic = 65536 / P.RPS + 1;

@@ -69,6 +69,7 @@ inline void finish_plan(dec_plan & p) { p.NT = p.RG * p.GQA <= 16 ? 1 : 2; }
 struct decode_grid {
     bool sb, list, loop, direct;   // two workgroups to a compute unit; kinds of dec_mfma_k
     int RPS, GPS;          // rows and row groups of a sequence
+    int deal_sh;           // direct: log2 of the row groups that are dealt to the XCDs at a time
     unsigned x, y;
 };
 
@@ -80,17 +81,24 @@ inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv,
     r.GPS = rows_per_seq > pl.RG ? rows_per_seq / pl.RG : 1;
     if (r.GPS > groups) r.GPS = groups;
     const int nseq = (groups + r.GPS - 1) / r.GPS, inner = Hkv * r.GPS;
-    // One unit at most, as far as the host knows - from the positions (host_n of them; 0: they are in device memory, -1: partials are asked for) or from what a
-    // page-table row holds -, and no more workgroups than compute units: the workgroup of a (row group, kv head) writes the results, eights of row groups to the XCDs,
-    // and there is no merge behind it. Steps of two layers, prep included, with merge_k and so: q8_0, 24 / 4 heads of 256, one sequence of 250 keys 34.4 and 29.6 us,
-    // 32 of them 42.8 and 33.4; f16, 32 / 8 of 128 30.6 and 26.0, 32 of them 40.2 and 33.4; 8 x 4 rows of 250 (24 / 4) 48.1 and 42.0; plain calls of 100 keys 28.4 and 26.5.
-    // Not from two units on: whoever folds last would have to merge, and its stores, counter and loads past the L2s cost what merge_k does (500 keys
-    // 34.6 and 35.3, 2000 35.1 and 36.2, 8000 37 and 48).
+    // One unit at most, as far as the host knows - from the positions (host_n of them; 0: they are in device memory, -1: partials are asked for)
+    // or from what a page-table row holds: the workgroup of a (row group, kv head) writes the results, and there is no merge behind
+    // it. Steps of two layers, prep included, with merge_k and so: q8_0, 24 / 4 heads of 256, one sequence of 250 keys 34.4 and 29.6 us, 32
+    // of them 42.8 and 33.4; f16, 32 / 8 of 128 30.6 and 26.0, 32 of them 40.2 and 33.4; 8 x 4 rows of 250 (24 / 4) 48.1 and 42.0; plain
+    // calls of 100 keys 28.4 and 26.5.
+    // A workgroup has its compute unit to itself. All kv heads of a row group go to one XCD, eights of groups at a time, where no XCD gets more of them than it
+    // has units so; else workgroups go to the XCDs in turn. Rows of 250 keys, heads of 256 (q8_0), with merge_k, by groups and in turn: one row of 40 heads
+    // 33.8, 44.7, 28.7, of 128 36.8, 77.9, 32.5, 9 rows of 24 heads 47.9, 47.3, 35.5; but 8 rows of 24 38.8, 32.8, 34.6, 16 of 8 heads of
+    // 128 37.2, 30.2, 31.8 (cache lines that two heads share; f16 level).
+    // Not from two units on: whoever folds last would have to merge, and its stores, counter and loads past the L2s cost what merge_k does
+    // (500 keys 34.6 and 35.3, 2000 35.1 and 36.2, 8000 37 and 48).
     r.sb = r.list = r.loop = false;
+    r.deal_sh = 0;
     const long long sees = host_n ? host_n : n_ctx;
     r.direct = sees > 0 && sees <= 32 * pl.NW && (long long) groups * Hkv <= cus && !(pl.NT == 2 && type == P1A_KV_Q4_0 && !staged);
     if (r.direct) {
-        r.x = (unsigned) ((groups + 7) / 8 * 8 * Hkv);
+        r.deal_sh = (groups + 7) / 8 * Hkv <= cus / 8 ? 3 : 0;
+        r.x = (unsigned) (((groups + (1 << r.deal_sh) - 1) >> r.deal_sh << r.deal_sh) * Hkv);
         r.y = 1;
         return r;
     }

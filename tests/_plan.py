@@ -6,7 +6,7 @@ import subprocess
 import tempfile
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-FIELDS = ("mfma", "NW", "NT", "RG", "nsplit", "sb", "list", "loop", "RPS", "GPS", "x", "y", "direct")
+FIELDS = ("mfma", "NW", "NT", "RG", "nsplit", "sb", "list", "loop", "RPS", "GPS", "x", "y", "direct", "deal_sh")
 SHIM = '''
 #include <cstring>
 #include "p1a_plan.hpp"
@@ -21,7 +21,7 @@ extern "C" void plan(uint32_t type, int Hq, int Hkv, int D, int n_ctx, int T, in
     p.RG = rg;
     p1a::finish_plan(p);
     const p1a::decode_grid g = p1a::plan_grid(p, type, D, Hkv, n_ctx, T, pos_rows ? rps : 1 << 30, pos_rows, cus, host_n);
-    const long long v[] = {p.mfma, p.NW, p.NT, p.RG, p.nsplit, g.sb, g.list, g.loop, g.RPS, g.GPS, g.x, g.y, g.direct};
+    const long long v[] = {p.mfma, p.NW, p.NT, p.RG, p.nsplit, g.sb, g.list, g.loop, g.RPS, g.GPS, g.x, g.y, g.direct, g.deal_sh};
     memcpy(o, v, sizeof v);
 }
 '''

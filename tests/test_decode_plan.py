@@ -65,6 +65,12 @@ def test_drawn_calls():
     assert len(kinds) >= 5, kinds                              # (two to a unit and one, one stream and several, one column tile and two)
 
 
+def direct_items(p, Hkv):
+    """(row group, kv head, XCD) of each workgroup of a direct call, as dec_mfma_k takes them from blockIdx (workgroup i is on XCD i mod 8)"""
+    sh = p["deal_sh"]
+    return [(((i >> sh) // Hkv << sh) + (i & ((1 << sh) - 1)), (i >> sh) % Hkv, i & 7) for i in range(p["x"])]
+
+
 @pytest.mark.parametrize("kv_type,Hq,Hkv,D,T,rows", [(F16, 4, 1, 64, 1, 1), (Q8_0, 24, 4, 256, 32, 4), (F16, 24, 4, 256, 31, 1), (Q8_0, 32, 8, 128, 32, 1), (F16, 12, 6, 128, 9, 3), (Q4_0, 16, 2, 256, 2, 1)])
 def test_calls_of_one_unit(kv_type, Hq, Hkv, D, T, rows):
     """a workgroup for every (row group, kv head) where the host knows that no row sees more than a unit - from the positions before n_ctx -, each taken once,
@@ -76,9 +82,28 @@ def test_calls_of_one_unit(kv_type, Hq, Hkv, D, T, rows):
         if not direct:
             continue
         groups = -(-T // p["RG"])
-        taken = [((i >> 3) // Hkv * 8 + (i & 7), (i >> 3) % Hkv, i & 7) for i in range(p["x"])]
+        taken = direct_items(p, Hkv)
         live = [(g, h) for g, h, _ in taken if g * p["RG"] < T]
         assert p["y"] == 1 and sorted(live) == [(g, h) for g in range(groups) for h in range(Hkv)]
         assert all(len({x for g, _, x in taken if g == k}) == 1 for k in range(groups))
     assert not plan(Q4_0, 24, 4, 256, 256, 8, 4)["direct"]     # (two column tiles of q4_0: no registers for it)
     assert not plan(F16, 32, 32, 64, 256, 9, 1)["direct"]      # (more workgroups than compute units)
+
+
+@pytest.mark.parametrize("kv_type,D", [(F16, 64), (F16, 128), (F16, 256), (Q8_0, 128), (Q8_0, 256), (Q4_0, 256)])
+def test_calls_of_one_unit_fit_every_xcd(kv_type, D):
+    """no XCD gets more live workgroups than its compute units, whatever the number of heads: all kv heads of a row group are on one
+    XCD only where they fit so"""
+    rng, seen = random.Random(6), {0: 0, 3: 0}
+    calls = [(Hkv, 1, T, 1, 256) for Hkv, T in ((32, 1), (33, 1), (40, 1), (64, 1), (128, 1), (24, 8), (24, 9), (16, 16), (15, 17), (8, 32), (10, 24), (10, 25))]
+    for _ in range(400):
+        calls.append((rng.randint(1, 130), rng.choice([1, 2, 4, 6]), rng.randint(1, 32), rng.choice([1, 2, 3, 4]), rng.choice([256, 256, 304, 80])))
+    for Hkv, gqa, T, rows, cus in calls:
+        p = plan(kv_type, Hkv * gqa, Hkv, D, 100, T, rows, cus=cus)
+        if not p["direct"]:
+            continue
+        live = [(g, h, x) for g, h, x in direct_items(p, Hkv) if g * p["RG"] < T]
+        assert sorted(i[:2] for i in live) == [(g, h) for g in range(-(-T // p["RG"])) for h in range(Hkv)], (Hkv, gqa, T, rows, cus, p)
+        assert max(sum(x == k for _, _, x in live) for k in range(8)) <= cus // 8, (Hkv, gqa, T, rows, cus, p)
+        seen[p["deal_sh"]] += 1
+    assert min(seen.values()) > 10, seen

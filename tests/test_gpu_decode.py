@@ -295,7 +295,8 @@ def test_short_calls_behind_a_long_one(p1a, kv_type, Hq, Hkv, D, psh):
 
 
 @pytest.mark.parametrize("kv_type,Hq,Hkv,D,rows", [(O.KV_F16, 4, 1, 64, 1), (O.KV_F16, 32, 8, 128, 4), (O.KV_F16, 24, 4, 256, 1), (O.KV_F16, 24, 4, 256, 4), (O.KV_Q8_0, 24, 4, 256, 1), (O.KV_Q8_0, 24, 4, 256, 3),
-                                                   (O.KV_Q4_0, 16, 2, 256, 1), (O.KV_Q8_0, 8, 1, 128, 4), (O.KV_Q4_0, 4, 4, 64, 2), (O.KV_Q8_0, 6, 1, 64, 4), (O.KV_Q4_0, 24, 4, 128, 3)])
+                                                   (O.KV_Q4_0, 16, 2, 256, 1), (O.KV_Q8_0, 8, 1, 128, 4), (O.KV_Q4_0, 4, 4, 64, 2), (O.KV_Q8_0, 6, 1, 64, 4), (O.KV_Q4_0, 24, 4, 128, 3),
+                                                   (O.KV_F16, 40, 40, 64, 1), (O.KV_Q8_0, 96, 48, 128, 2), (O.KV_Q8_0, 51, 51, 256, 1), (O.KV_F16, 280, 40, 64, 4)])   # (more kv heads than an XCD has units)
 def test_calls_of_one_unit(p1a, kv_type, Hq, Hkv, D, rows):
     """sequences of one unit of keys, whose workgroups write the results themselves: the bits of the calls that go through partials, gate, a16 values and idle
     slots included, and close to the oracle"""
