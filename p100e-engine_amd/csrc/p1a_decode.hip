@@ -1191,7 +1191,7 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, bo
     P.T = a.T; P.RG = pl.RG; P.Hq = a.Hq; P.Hkv = c.Hkv; P.GQA = pl.GQA;
     P.qscale = a.scale * 1.4426950408889634f; P.nsplit = pl.nsplit;
     constexpr bool big_tiles = KT == P1A_KV_F16 && D == 256;
-    const decode_grid gr = plan_grid(pl, KS, D, c.Hkv, c.n_ctx, a.T, a.rows_per_seq, a.pos_rows != nullptr, a.cus, a.skip_merge ? -1 : a.host_n);
+    const decode_grid gr = plan_grid(pl, KS, D, c.Hkv, c.n_ctx, a.T, a.rows_per_seq, a.pos_rows != nullptr, a.cus, a.host_n, a.skip_merge);
     direct = gr.direct;
     P.deal_sh = gr.deal_sh;
     P.RPS = gr.RPS;

@@ -73,7 +73,8 @@ struct decode_grid {
     unsigned x, y;
 };
 
-inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv, int n_ctx, int T, int rows_per_seq, bool pos_rows, int cus_, long long host_n = 0) {
+inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv, int n_ctx, int T, int rows_per_seq, bool pos_rows, int cus_,
+                             long long host_n, bool partials) {
     decode_grid r;
     const int cus = cus_ > 0 ? cus_ : 256, groups = (T + pl.RG - 1) / pl.RG;
     const bool staged = type != P1A_KV_F16 && D != 256;
@@ -81,9 +82,9 @@ inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv,
     r.GPS = rows_per_seq > pl.RG ? rows_per_seq / pl.RG : 1;
     if (r.GPS > groups) r.GPS = groups;
     const int nseq = (groups + r.GPS - 1) / r.GPS, inner = Hkv * r.GPS;
-    // One unit at most, as far as the host knows - from the positions (host_n of them; 0: they are in device memory, -1: partials are asked for)
+    // One unit at most, as far as the host knows - from the positions (host_n of them; 0: they are in device memory)
     // or from what a page-table row holds: the workgroup of a (row group, kv head) writes the results, and there is no merge behind
-    // it. Steps of two layers, prep included, with merge_k and so: q8_0, 24 / 4 heads of 256, one sequence of 250 keys 34.4 and 29.6 us, 32
+    // it (`partials`: they are what the call is for). Steps of two layers, prep included, with merge_k and so: q8_0, 24 / 4 heads of 256, one sequence of 250 keys 34.4 and 29.6 us, 32
     // of them 42.8 and 33.4; f16, 32 / 8 of 128 30.6 and 26.0, 32 of them 40.2 and 33.4; 8 x 4 rows of 250 (24 / 4) 48.1 and 42.0; plain
     // calls of 100 keys 28.4 and 26.5.
     // A workgroup has its compute unit to itself. All kv heads of a row group go to one XCD, eights of groups at a time, where no XCD gets more of them than it
@@ -95,7 +96,7 @@ inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv,
     r.sb = r.list = r.loop = false;
     r.deal_sh = 0;
     const long long sees = host_n ? host_n : n_ctx;
-    r.direct = sees > 0 && sees <= 32 * pl.NW && (long long) groups * Hkv <= cus && !(pl.NT == 2 && type == P1A_KV_Q4_0 && !staged);
+    r.direct = !partials && sees > 0 && sees <= 32 * pl.NW && (long long) groups * Hkv <= cus && !(pl.NT == 2 && type == P1A_KV_Q4_0 && !staged);
     if (r.direct) {
         r.deal_sh = (groups + 7) / 8 * Hkv <= cus / 8 ? 3 : 0;
         r.x = (unsigned) (((groups + (1 << r.deal_sh) - 1) >> r.deal_sh << r.deal_sh) * Hkv);
@@ -105,11 +106,16 @@ inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv,
     // A call of at least two workgroups per CU whose row groups fit one column tile takes the single-buffered variant, two
     // workgroups to a CU (same partials, bit for bit; measured at 24 / 4 heads, D = 256: 8 q8_0 slots of 1 K ... 27 K 56 ->
     // 47 us, 4 x 64 K q4_0 single rows 92 -> 73 us, 16 x 2 rows q4_0 at 16 K 143 -> 115 us, 32 slots of 2 ... 5 K 104 -> 71 us).
-    // Staged tiles, D = 128: so too where more workgroups than compute units can have keys (two layers with prep, one to a unit and two: q8_0, 32 / 8 heads, 16 sequences of 2000 ... 8000
-    // keys 161 and 112 us, 4 of 8000 ... 32000 120 and 101; q4_0, 24 / 4, 8 x 2 rows of 8000 ... 32000 136 and 108, 32 sequences of 1000 53 and 45; but 8 x 2 rows of 1000 36.7 and 38.3). Not at D = 64,
-    // whose conversions are half as long (q8_0, 16 / 4, 32 of 2000 ... 8000 79 and 85; q4_0, 8 / 8, 2 of 32000 54.4 and 53.5).
-    const bool two = !staged || (D == 128 && ((long long) n_ctx + 32 * pl.NW - 1) / (32 * pl.NW) * groups * Hkv > cus);
-    r.sb = pl.NT == 1 && two && (long long) pl.nsplit * Hkv * groups >= 2LL * cus;
+    // Staged tiles, D = 128: so too where more workgroups than compute units can have keys - by the positions, or by what a page-table row holds (two layers with
+    // prep, one to a unit and two: q8_0, 32 / 8 heads, 16 sequences of 2000 ... 8000 keys 161 and 112 us, 4 of 8000 ... 32000 120 and 101; q4_0, 24 / 4, 8 x 2
+    // rows of 8000 ... 32000 136 and 108, 32 sequences of 1000 53 and 45; but 8 x 2 rows of 1000 36.7 and 38.3). Not at D = 64, whose conversions
+    // are half as long (q8_0, 16 / 4, 32 of 2000 ... 8000 79 and 85; q4_0, 8 / 8, 2 of 32000 54.4 and 53.5).
+    // One sequence's rows have a workgroup for every stream there could be, and from eight for every unit on half of the empty ones' time is worth it, whatever the
+    // keys (q8_0, 32 rows of 1000 keys, 32 / 8 heads 68.8 and 62.2, 16 / 4 56.2 and 50.7; with four for every unit, 16 rows, 16 / 4 41.0 and 45.9, 32 / 8
+    // 45.9 and 46.9, 8 / 8 44.1 and 41.7; with two, 8 rows of 32 / 8, 37.7 and 44.7).
+    const long long all = (long long) pl.nsplit * Hkv * groups;
+    const bool two = !staged || (D == 128 && ((sees + 32 * pl.NW - 1) / (32 * pl.NW) * groups * Hkv > cus || (!pos_rows && all >= 8LL * cus)));
+    r.sb = pl.NT == 1 && two && all >= 2LL * cus;
     // The list (see dec_mfma_k) costs a workgroup some 0.2 us before its first request. Where two workgroups share a compute unit that hides,
     // and every call of several row groups takes it. Several sequences (110 calls of 2 ... 32 drawn over 4 ... 131072 keys, D = 256 and f16):
     // 0.98 - 1.6 times as fast, 1.1 in the mean. One sequence of 5 ... 32 rows (200 calls over 200, 3000 and 20000 keys, six head shapes):

@@ -76,9 +76,10 @@ def test_calls_of_one_unit(kv_type, Hq, Hkv, D, T, rows):
     """a workgroup for every (row group, kv head) where the host knows that no row sees more than a unit - from the positions before n_ctx -, each taken once,
     the heads of a group on one XCD; everything else has the grids above"""
     unit = 128 if kv_type == F16 and D == 256 else 256
-    for n_ctx, host_n, direct in ((unit, 0, 1), (unit + 1, 0, 0), (0, 0, 0), (1 << 17, unit, 1), (1, unit + 1, 0), (unit, -1, 0)):
+    for n_ctx, host_n, direct in ((unit, 0, 1), (unit + 1, 0, 0), (0, 0, 0), (1 << 17, unit, 1), (1, unit + 1, 0)):
         p = plan(kv_type, Hq, Hkv, D, n_ctx, T, rows, pos_rows=host_n == 0, host_n=host_n)
         assert p["direct"] == direct, (n_ctx, host_n)
+        assert not plan(kv_type, Hq, Hkv, D, n_ctx, T, rows, pos_rows=host_n == 0, host_n=host_n, partials=True)["direct"]
         if not direct:
             continue
         groups = -(-T // p["RG"])
@@ -107,3 +108,16 @@ def test_calls_of_one_unit_fit_every_xcd(kv_type, D):
         assert max(sum(x == k for _, _, x in live) for k in range(8)) <= cus // 8, (Hkv, gqa, T, rows, cus, p)
         seen[p["deal_sh"]] += 1
     assert min(seen.values()) > 10, seen
+
+
+@pytest.mark.parametrize("kv_type", [F16, Q8_0, Q4_0])
+def test_positions_the_host_knows_count_before_n_ctx(kv_type):
+    """the grid of a call whose positions the host gives does not depend on how wide its page table is"""
+    rng, kinds = random.Random(7), set()
+    for _ in range(200):
+        D, Hkv, T, host_n = rng.choice([64, 128, 128, 256]), rng.choice([1, 2, 4, 8, 16]), rng.randint(1, 32), int(2 ** rng.uniform(5, 17))
+        for partials in (False, True):
+            grids = [plan(kv_type, 4 * Hkv, Hkv, D, n_ctx, T, T, pos_rows=False, host_n=max(host_n, T), partials=partials) for n_ctx in (0, 100, host_n, 1024, 1 << 17)]
+            assert all(g == grids[0] for g in grids), (D, Hkv, T, host_n, partials)
+        kinds.add((grids[0]["sb"], D))
+    assert (1, 128) in kinds and (0, 128) in kinds

@@ -562,7 +562,7 @@ def test_staged_tiles_many_rows_of_one_call(p1a):
     """the same without row positions: two workgroups to a unit and no list"""
     Hq, Hkv, D, n = 32, 8, 128, 4000
     pool = Pool(p1a, O.KV_Q8_0, Hq, Hkv, D, 6, [n], seed=51)
-    assert plan(O.KV_Q8_0, Hq, Hkv, D, n, 11, pos_rows=False)["sb"]
+    assert plan(O.KV_Q8_0, Hq, Hkv, D, n, 11, pos_rows=False, host_n=n)["sb"]
     q = I.normal(I.rng(52), (11, Hq, D))
     out = run_decode(p1a, pool.dev_seq(0), q, 11, n - 11, Hq, D ** -0.5)
     check(out, O.attn_rows(pool.host_seq(0), q, np.arange(n - 11, n), Hq, D ** -0.5), "11 rows")
