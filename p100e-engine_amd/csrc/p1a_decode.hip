@@ -205,8 +205,8 @@ template <int NR> __device__ __forceinline__ void wait_tiles(int newer) {
 // KS (when it differs from KT = f16): the type the cache holds - its raw tiles are staged (raw_cfg) and converted to f16
 // HOW = KS, and for calls of several sequences LIST (workgroups take the streams that hold keys), LIST | LOOP (one takes several);
 // DIRECT for calls whose rows see one unit at most, as far as the host knows: a workgroup for every (row group, kv head) writes the
-// results itself; STAGED_SB marks the single-buffered builds of staged tiles
-constexpr uint32_t LIST_ = 0x100, LOOP_ = 0x200, DIRECT_ = 0x400, STAGED_SB_ = 0x800;
+// results itself
+constexpr uint32_t LIST_ = 0x100, LOOP_ = 0x200, DIRECT_ = 0x400;
 template <uint32_t KT, int D, int NT, int NWV, bool SB, uint32_t HOW = KT>
 __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const dec_params P_) {
     constexpr uint32_t KS = HOW & 0xff;
@@ -1210,15 +1210,14 @@ int launch_mfma(const p1a_kv & c, const decode_args & a, const dec_plan & pl, bo
     auto go = [&](auto nt, auto single, auto can_loop) {
         constexpr int NT = decltype(nt)::value, NW = big_tiles ? 4 : 8;
         constexpr bool SB = decltype(single)::value;
-        constexpr uint32_t HOW = SB && KS != KT ? KS | STAGED_SB_ : KS;
         if constexpr (!SB && (NT == 1 || KT != P1A_KV_Q4_0)) {   // (plan_grid asks for no other)
             if (gr.direct) { dec_mfma_k<KT, D, NT, NW, false, KS | DIRECT_><<<grid, NW * 64, 0, s>>>(P); return; }
         }
         if constexpr (decltype(can_loop)::value) {
-            if (gr.loop) { dec_mfma_k<KT, D, NT, NW, SB, HOW | LIST_ | LOOP_><<<grid, NW * 64, 0, s>>>(P); return; }
+            if (gr.loop) { dec_mfma_k<KT, D, NT, NW, SB, KS | LIST_ | LOOP_><<<grid, NW * 64, 0, s>>>(P); return; }
         }
-        if (gr.list) dec_mfma_k<KT, D, NT, NW, SB, HOW | LIST_><<<grid, NW * 64, 0, s>>>(P);
-        else dec_mfma_k<KT, D, NT, NW, SB, HOW><<<grid, NW * 64, 0, s>>>(P);
+        if (gr.list) dec_mfma_k<KT, D, NT, NW, SB, KS | LIST_><<<grid, NW * 64, 0, s>>>(P);
+        else dec_mfma_k<KT, D, NT, NW, SB, KS><<<grid, NW * 64, 0, s>>>(P);
     };
     constexpr std::true_type yes;
     constexpr std::false_type no;

@@ -54,15 +54,38 @@ def test_decode_kernels_fit_their_budget(tmp_path):
         assert r["Occupancy"] * 4 >= 2 * waves, (name, r)                   # two workgroups' waves on the 4 SIMDs
 
 
-def test_decode_list_kernels_fit_their_budget(tmp_path):
-    """the builds for calls of several sequences, one stream a workgroup (every build) and several (the single-buffered and the staged
-    ones, two column tiles of f16 and q8_0), are there and spill nothing either (the test above holds the single-buffered ones to two workgroups on a CU)"""
-    ks = {k: v for k, v in resource_report(tmp_path).items() if re.search(r"dec_mfma_k.*ELj\d{3}EEEv", k)}   # (the last argument: 256 list, 512 loop)
-    loop = [k for k in ks if int(re.search(r"ELj(\d+)EEEv", k).group(1)) & 512]
-    assert len(loop) == 17 and len(ks) - len(loop) == 23, sorted(ks)
+LIST, LOOP, DIRECT = 256, 512, 1024                            # what the last argument holds beside the cache's type
+
+
+def builds(names):
+    """dec_mfma_k<KT, D, NT, NWV, SB, HOW> by mangled name: its arguments, HOW taken apart as the cache's type and the kind of build"""
+    out = {}
+    for name in names:
+        kt, D, nt, nwv, sb, how = (int(x) for x in re.search(r"dec_mfma_kILj(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELb([01])ELj(\d+)EEEv", name).groups())
+        assert not how & ~(255 | LIST | LOOP | DIRECT), name
+        out[name] = {"D": D, "NT": nt, "waves": nwv, "sb": sb, "staged": how & 255 != kt, "kind": how & ~255}
+    return out
+
+
+def test_every_kind_of_decode_build_fits_its_budget(tmp_path):
+    """the builds for a stream a workgroup, for calls of several sequences - a list of streams, one a workgroup (every build) and several (the single-buffered and the
+    staged ones, two column tiles of f16 and q8_0) - and for calls of one unit, each with the double-buffered, single-buffered and staged builds it has: none spills, and two
+    workgroups of a single-buffered one fit a CU, staged or not"""
+    ks = {k: v for k, v in resource_report(tmp_path).items() if "dec_mfma_k" in k}
+    of = builds(ks)
+    counts = {}
+    for b in of.values():
+        key = (b["kind"], b["sb"], b["staged"])
+        counts[key] = counts.get(key, 0) + 1
+    assert counts == {(0, 0, False): 10, (0, 0, True): 8, (0, 1, False): 5, (0, 1, True): 2,
+                      (LIST, 0, False): 10, (LIST, 0, True): 8, (LIST, 1, False): 5, (LIST, 1, True): 2,
+                      (LIST | LOOP, 0, False): 4, (LIST | LOOP, 0, True): 8, (LIST | LOOP, 1, False): 5, (LIST | LOOP, 1, True): 2,
+                      (DIRECT, 0, False): 9, (DIRECT, 0, True): 8}
     for name, r in ks.items():
         assert all(r.get(x, 0) == 0 for x in ("VGPRs Spill", "SGPRs Spill", "ScratchSize")), (name, r)
-        assert r["LDS Size"] <= 160 * 1024, (name, r)
+        two = of[name]["sb"]
+        assert r["LDS Size"] <= (80 if two else 160) * 1024, (name, r)
+        assert r["Occupancy"] * 4 >= (2 if two else 1) * of[name]["waves"], (name, r)
 
 
 def test_decode_kernels_make_no_flat_access(tmp_path):
