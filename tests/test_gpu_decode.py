@@ -266,6 +266,9 @@ def test_descriptor_n_ctx_only_bounds(p1a):
         out = torch.empty((2, Hq, D), device="cuda")
         p1a.attn_decode(dq, c, out, 2, n - 2, Hq, 1 / 16)
         assert torch.equal(out, ref), n_ctx
+        out.fill_(7.0)
+        p1a.attn_decode_dev(dq, c, out, 2, dev(np.array([n - 2], np.int32)), n_ctx, Hq, 1 / 16)
+        assert torch.equal(out, ref), n_ctx
 
 
 @pytest.mark.parametrize("kv_type,Hq,Hkv,D,psh", [(O.KV_F16, 4, 1, 64, 4), (O.KV_F16, 6, 1, 256, 6), (O.KV_Q4_0, 16, 2, 256, 6), (O.KV_Q8_0, 8, 1, 128, 5), (O.KV_Q8_0, 24, 4, 256, 8),
@@ -323,6 +326,55 @@ def test_calls_of_one_unit(p1a, kv_type, Hq, Hkv, D, rows):
     out = got[1][0].numpy()
     assert np.isnan(out[4 * rows:]).all()
     for i in range(4):
+        r = slice(i * rows, (i + 1) * rows)
+        check(out[r], O.attn_rows(pool.host_seq(i), q[r].cpu().numpy(), pos[r], Hq, D ** -0.5), f"sequence {i}")
+
+
+@pytest.mark.parametrize("nsplit", [0, 3])
+@pytest.mark.parametrize("kv_type,Hq,Hkv,D,rows", [(O.KV_F16, 4, 1, 64, 1), (O.KV_F16, 24, 2, 64, 2), (O.KV_F16, 32, 8, 128, 4), (O.KV_F16, 12, 2, 128, 4), (O.KV_F16, 24, 4, 256, 1),
+                                                   (O.KV_F16, 24, 4, 256, 4), (O.KV_Q8_0, 24, 4, 256, 1), (O.KV_Q8_0, 24, 4, 256, 3), (O.KV_Q4_0, 16, 2, 256, 1), (O.KV_Q4_0, 12, 2, 256, 2),
+                                                   (O.KV_Q8_0, 32, 8, 128, 1), (O.KV_Q8_0, 8, 1, 128, 4), (O.KV_Q4_0, 24, 4, 128, 3), (O.KV_Q8_0, 6, 1, 64, 4), (O.KV_Q4_0, 4, 4, 64, 2)])
+def test_calls_of_one_unit_that_hold_more(p1a, kv_type, Hq, Hkv, D, rows, nsplit):
+    """an n_ctx of one unit over sequences that hold more: the workgroup of a row group goes through their streams and merges its own partials - the bits of the calls with
+    merge_k, gate and a16 values included, rows of one unit and of two in a group, idle rows beside live ones, more units than streams"""
+    unit = 128 if kv_type == O.KV_F16 and D == 256 else 256
+    lens = [unit + 1, 2 * unit, unit - 3, 7 * unit + 40, 3 * unit + rows, rows]
+    pool = Pool(p1a, kv_type, Hq, Hkv, D, 5, lens, seed=81)
+    pos = np.concatenate([np.arange(n - rows, n) for n in lens]).astype(np.int32)
+    pos[0] = unit - 1                                                 # (with more rows than one: the last row of the group sees a second unit)
+    pos[4 * rows] = -1                                                # an idle row, beside live ones where there are any
+    T = rows * len(lens)
+    q, gate = dev(I.normal(I.rng(82), (T, Hq, D))), dev(I.normal(I.rng(83), (T, Hq, D)))
+    kv = pool.devkv.with_rows(dev(np.repeat(np.arange(len(lens), dtype=np.int32) * pool.maxp, rows)))
+    p1a.set_nsplit(nsplit)
+    try:
+        got = []
+        for n_ctx in (unit, unit - 60, 0):                            # (0: nothing is known)
+            kv.n_ctx = n_ctx
+            assert plan(kv_type, Hq, Hkv, D, n_ctx, T, rows, nsplit=nsplit)["direct"] == (n_ctx > 0)
+            for g in (gate, None):
+                out, a16 = torch.full((T, Hq, D), 7.0, device="cuda"), torch.full((p1a.a16_bytes(T, Hq * D) // 2,), 7.0, dtype=torch.float16, device="cuda")
+                p1a.attn_decode_rows(q, kv, out, T, dev(pos), Hq, D ** -0.5, gate=g, rows_per_seq=rows, qbuf=a16)
+                got.append((out.cpu(), a16.cpu()))
+        for a, b in zip(got[:4], got[4:] * 2):
+            for x, y in zip(a, b):
+                nan = torch.isnan(x)
+                assert torch.equal(nan, torch.isnan(y)) and torch.equal(x[~nan].view(torch.int16), y[~nan].view(torch.int16))
+        # one sequence, its position in device memory
+        c = pool.dev_seq(3)
+        for p0 in (unit - rows, unit - 1, unit, 3 * unit - 1, lens[3] - rows):
+            outs = []
+            for n_ctx in (unit, 0):
+                c.n_ctx = n_ctx
+                assert plan(kv_type, Hq, Hkv, D, n_ctx, rows, rows, pos_rows=False, nsplit=nsplit)["direct"] == (n_ctx > 0)
+                outs.append(torch.full((rows, Hq, D), 7.0, device="cuda"))
+                p1a.attn_decode_dev(q[:rows], c, outs[-1], rows, dev(np.array([p0], np.int32)), n_ctx, Hq, D ** -0.5, gate=gate[:rows])
+            assert torch.equal(*outs), p0
+    finally:
+        p1a.set_nsplit(0)
+    out = got[1][0].numpy()
+    assert np.isnan(out[4 * rows]).all() and not np.isnan(np.delete(out, 4 * rows, 0)).any()
+    for i in (0, 1, 3):
         r = slice(i * rows, (i + 1) * rows)
         check(out[r], O.attn_rows(pool.host_seq(i), q[r].cpu().numpy(), pos[r], Hq, D ** -0.5), f"sequence {i}")
 
@@ -541,11 +593,11 @@ def test_understated_n_ctx_of_several_sequences(p1a, kv_type, Hq, D, lens):
     for n_ctx in (c.n_ctx, 4000, 2000, 100, 0):
         rows.n_ctx = min(n_ctx, c.n_ctx)
         p = plan(kv_type, Hq, Hkv, D, rows.n_ctx, n, cus=torch.cuda.get_device_properties(0).multi_processor_count)
-        grids.add((p["list"], p["loop"], p["x"]))
+        grids.add((p["direct"], p["list"], p["loop"], p["x"]))
         outs.append(torch.empty_like(q))
         p1a.attn_decode_rows(q, rows, outs[-1], n, pos, Hq, D ** -0.5)
         assert torch.equal(outs[-1], outs[0]), n_ctx
-    assert len(grids) > 1, grids
+    assert len(grids) > 1 and {g[0] for g in grids} == {0, 1}, grids
 
 
 @pytest.mark.parametrize("kv_type,Hq,Hkv,lens,rows,loop", [(O.KV_Q8_0, 32, 8, [9000, 1, 16, 17, 5000, 300], 1, 0), (O.KV_Q4_0, 48, 8, [8500, 2, 33, 6000], 2, 0), (O.KV_Q8_0, 12, 4, [17000, 4, 1000], 4, 0),
