@@ -891,21 +891,24 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
     // through LDS, where a row is put together (4 D bytes and 16 of padding; the tiles are done with), to whole rows in memory
     constexpr int ORS = 4 * D + 16;
     const int d4 = 4 * (lane % LPF);
-    // All of the wave's gate rows are asked for before the first result is put down: eight at a time, each batch behind the stores of the
-    // one before, a round trip to memory stood in front of every quarter of the rows (prep and prefill of the first 512 tokens, f16,
-    // 24 / 4 heads of 256 38.2 -> 37.1 us, 800 54.0 -> 52.0, 2000 (q8_0) 122.7 -> 118; 32 / 8 of 128, 512 29.6 -> 28.6)
-    f4 gt[NRI];
-    if (P.gate) {
-        auto fetch = [&](int i) { gt[i] = *reinterpret_cast<const f4 *>(P.gate + row_index(wrow0 + min(row_at(i), wlast)) * D + d4); };
+    // f16 caches and copies: all of the wave's gate rows are asked for before the first result is put down: eight at a time, each batch
+    // behind the stores of the one before, a round trip to memory stood in front of every quarter of the rows (prep and prefill of the first
+    // 512 tokens, f16, 24 / 4 heads of 256 37.8 -> 36.1 us, pages of 4 47.1 -> 45.8; 32 / 8 of 128 31.1 -> 30.3). Not where tiles are converted
+    // inside: with that many more registers asked for behind it the compiler arranges their key loop otherwise, and slower, gate or none
+    // (150 tokens behind 17112, 8 / 8 heads of 256, q4_0 69.2 us, 71.9 so; 77 behind 17000, 24 / 4 71.0 and 73.3; q8_0 71.9 and 72.4).
+    constexpr bool GATES_AHEAD = KT == P1A_KV_F16;
+    f4 gt[GATES_AHEAD ? NRI : N8];
+    auto fetch_gate = [&](int i) { gt[GATES_AHEAD ? i : i % N8] = *reinterpret_cast<const f4 *>(P.gate + row_index(wrow0 + min(row_at(i), wlast)) * D + d4); };
+    if (GATES_AHEAD && P.gate) {
 #pragma unroll
-        for (int i = 0; i < N8; ++i) fetch(i);
+        for (int i = 0; i < N8; ++i) fetch_gate(i);
         if (wrows > 8) {
 #pragma unroll
-            for (int i = N8; i < 2 * N8; ++i) fetch(i);
+            for (int i = N8; i < 2 * N8; ++i) fetch_gate(i);
         }
         if (wrows > 16) {
 #pragma unroll
-            for (int i = 2 * N8; i < NRI; ++i) fetch(i);
+            for (int i = 2 * N8; i < NRI; ++i) fetch_gate(i);
         }
     }
 #pragma unroll
@@ -922,6 +925,10 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
 #pragma unroll
     for (int i0 = 0; i0 < NRI; i0 += N8) {
         f4 v[N8];
+        if (!GATES_AHEAD && P.gate) {
+#pragma unroll
+            for (int i = 0; i < N8; ++i) fetch_gate(i0 + i);
+        }
         if (PAIR && i0 == 0) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
         for (int i = 0; i < N8; ++i) v[i] = *reinterpret_cast<const f4 *>(img + (i0 + i) * RPI * ORS);
@@ -929,7 +936,7 @@ __global__ void __launch_bounds__(NTHR, pf_solo(D, DMA) ? 2 : 1) prefill_k(const
 #pragma unroll
             for (int i = 0; i < N8; ++i)
 #pragma unroll
-                for (int x = 0; x < 4; ++x) v[i][x] *= sigmoid(gt[i0 + i][x]);
+                for (int x = 0; x < 4; ++x) v[i][x] *= sigmoid(gt[GATES_AHEAD ? i0 + i : i][x]);
         }
         // (f16 tiles, D = 256: results, which nothing here reads again, go past the caches: 600 tokens behind 300, 24 / 4 heads, f16 53.9 -> 51.1 us, 2000, 32 / 8, q8_0
         // 157 -> 151. What reads them next gives most of it back: the first 4096 of 24 / 4, f16, alone 252 -> 239, with a cast to f16 behind the call 271.8
