@@ -54,10 +54,13 @@ extern "C" {
  *     q4_0 : per head D/32 ggml block_q4_0 (f16 d, 16 B: byte i = v[i] | v[i+16] << 4)   src/fast/attn.cuh:4-5
  * The layer is selected by the k / v base pointers, the slot by pt (or rtab[t]), the storage mode by type.
  * n_ctx is how many positions a page-table row (or the contiguous cache) holds. It is never used to address keys, and results do not
- * depend on it; p1a_attn_decode takes it for the most that a sequence may hold when it picks how a call is dealt to the
- * device. Rows cut to the sequences are served faster where those are short: 32 sequences of 256 keys (q8_0, 32 / 8 heads of 128, two layers) 42 us
- * with rows of 256 positions, 78 with rows of 8192 and more. It must not be larger than what the table holds (one that understates what
- * sequences hold is served with the same results, slowly: up to 256 positions, 128 for f16 of D = 256, one workgroup walks a sequence).
+ * depend on it; p1a_attn_decode takes it for the most that a sequence may hold when it picks how a call whose positions are in device
+ * memory is dealt to the device. Rows cut to the sequences are served faster where those are short: 32 sequences of 256 keys (q8_0,
+ * 32 / 8 heads of 128, two layers with prep) 32.5 us with rows of 256 positions, 40 with 512 ... 2048, 42.5 with 8192 and more. It must not
+ * be larger than what the table holds. One that understates what sequences hold is served with the same results, but where it is 1 ... 256
+ * (128 for f16 of D = 256) slowly: one workgroup a kv head then walks a sequence, at 3 ... 7 us for every 256 (128) keys and layer - one row of
+ * 1000 keys (q8_0, 24 / 4 heads of 256, two layers) takes 34.8 us with its own n_ctx and 78 with 100, of 8000 keys 37 and 499, of 32000 50
+ * and 1378.
  */
 typedef struct p1a_kv {
     uint32_t type;

@@ -320,8 +320,8 @@ struct prep_params {
     int p0, Hq, Hkv, D, n_rot, ldq, ldk, ldv;
     float eps;
 };
-// (one kernel argument: the host pays for each. Plain steps of four layers with 21 of them and so: f16, 4 / 1 heads of 64 54.6 and 53.2 us, 32 / 8 of 128 53.4 and
-// 52.0, recorded ones level.)
+// (one kernel argument: the host pays for each. Plain steps of four layers with 21 of them and so: f16, 4 / 1 heads of 64 54.6 and 53.2 us,
+// 32 / 8 of 128 53.4 and 52.0, recorded ones level.)
 template <uint32_t KT> __global__ void __launch_bounds__(64) prep_k(const prep_params P) {
     prep_head<KT>(P.qg, P.k, P.v, P.qn, P.kn, P.pos, P.q, P.gate, P.kc, P.vc, P.p0, P.Hq, P.Hkv, P.D, P.n_rot, P.ln_base, P.eps, P.ldq, P.ldk,
                   P.ldv, P.pg, P.mr);

@@ -69,9 +69,10 @@ template <uint32_t KS, int D> struct raw_cfg {
 };
 
 // f16 tiles: rows of D / 8 16-byte chunks without padding, every one of which starts in the same LDS bank (D = 64: every other). So chunk i of
-// row r lies where chunk i ^ swz(r) would - a lane of a tile fetch brings whichever chunk of its row belongs where it writes -, and what 16 rows are read
-// at together is spread over all banks. Two layers with prep: f16, 24 / 4 heads of 256, 4 sequences of 2000 ... 8000 keys 60.2 -> 55.7 us; tiles converted to f16, 24 / 4 of
-// 128, q4_0, 8 x 2 rows of 8000 ... 32000 162 -> 136, q8_0 (32 / 8) 234 -> 222; heads of 64 level.
+// row r lies where chunk i ^ swz(r) would - a lane of a tile fetch brings whichever chunk of its row belongs where it writes -, and what 16 rows
+// are read at together is spread over all banks. Two layers with prep: f16, 24 / 4 heads of 256, 4 sequences of 2000 ... 8000 keys 60.2 -> 55.7 us
+// (bank conflicts 19.5 -> 3.4 % of the units' cycles; 32 / 8 of 128 22 -> 3.2); tiles converted to f16, 24 / 4 of 128, q4_0, 8 x 2 rows of
+// 8000 ... 32000 162 -> 136, q8_0 (32 / 8) 234 -> 222; heads of 64 level.
 template <int D> __device__ __forceinline__ int swz(int row) { return D == 64 ? (row >> 1) & 7 : row & 15; }
 
 struct dec_params {
@@ -105,7 +106,8 @@ template <typename T> __device__ __forceinline__ void in_memory(T *& p) { p = (T
 // sum / denominator, gate, result and a16 values of dims d .. d + 3 of head h of row t: 8 consecutive lanes hold one 32-value group of the
 // row (what the engine's ew_quant emits for the output projection, src/fast/fused.cu:478-496). A row that sees no key is 0 / 0: the NaN row the
 // reference's combine gives for n = 0.
-__device__ __forceinline__ void finish_row(const f4 n, float dn, const f4 gt, float * out, bool gated, void * qbuf, int t, int h, int d, int Hq, int D, int T, bool live) {
+__device__ __forceinline__ void finish_row(const f4 n, float dn, const f4 gt, float * out, bool gated, void * qbuf, int t, int h, int d, int Hq,
+                                           int D, int T, bool live) {
     in_memory(out); in_memory(qbuf);
     f4 r = {n[0] / dn, n[1] / dn, n[2] / dn, n[3] / dn};
     if (gated) {
@@ -257,9 +259,10 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
     // workgroups with keys on 32 of 256 units). The streams that hold keys are counted through instead, sequence by sequence,
     // those of two units ahead of the others so that no unit gets two of them; number q goes to XCD q mod 8, one workgroup for every kv head and
     // row group of it, and workgroups left over come last. (LOOP: one takes the numbers q, q + q_step, ...) Same partition of
-    // the keys, same bits. q8_0, 24 / 4 heads of 256, two layers with prep and merge: 8 sequences of 1024 keys 47 -> 38 us, 16 of 300 ... 5000
-    // 68 -> 58, 2 of 20000 74 -> 69, 32 of 256 61 -> 43; what it does not help costs 2 ... 6 % (4 of 4000 ... 16000, two rows each 75 -> 77; 4 x 4 rows of 4252, 272 live workgroups
-    // for 256 units), a sequence of many rows that only groups of one divide up to 16 (plan_grid).
+    // the keys, same bits. q8_0, 24 / 4 heads of 256, two layers with prep and merge: 8 sequences of 1024 keys 46.5 -> 38.3 us, 16 of
+    // 300 ... 5000 61.4 -> 54.1, 2 of 20000 65.2 -> 60.0, 32 of 500 66.4 -> 44.2; what it does not help costs 2 ... 6 % (4 of 4000 ... 16000, two
+    // rows each 75 -> 77; 4 x 4 rows of 4252, 272 live workgroups for 256 units), a sequence of many rows that only groups of one divide up
+    // to 16 (plan_grid).
     int split = 0, hg = 0, gsub = 0, q = 0, q_step = 0, q_a = 0, q_end = 0, rt_lanes = 0;
     uint32_t u_sum = 0;
     if constexpr (LIST) {
@@ -379,8 +382,9 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
             for (int i = tid; i < R * (D / 4); i += NWV * 64) {
                 const int col = i / (D / 4), t = row_of(col);
                 const kargb kp = args_again();
-                finish_row(f4{0.f, 0.f, 0.f, 0.f}, 0.f, f4{0.f, 0.f, 0.f, 0.f}, P1A_ARG(kp, out), P1A_ARG(kp, gate) != nullptr, P1A_ARG(kp, qbuf), row0 + t, hg * P.GQA + col - t * P.GQA,
-                           4 * (i % (D / 4)), P1A_ARG(kp, Hq), D, P1A_ARG(kp, T), true);
+                const f4 zero4 = {0.f, 0.f, 0.f, 0.f};
+                finish_row(zero4, 0.f, zero4, P1A_ARG(kp, out), P1A_ARG(kp, gate) != nullptr, P1A_ARG(kp, qbuf), row0 + t,
+                           hg * P.GQA + col - t * P.GQA, 4 * (i % (D / 4)), P1A_ARG(kp, Hq), D, P1A_ARG(kp, T), true);
             }
         }
         if (!DIRECT && next_item()) continue;
@@ -956,7 +960,8 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
                         const float * gate = P1A_ARG(kp, gate);
                         in_memory(gate);
                         if (gate) gt = *reinterpret_cast<const f4 *>(gate + row * D + 4 * d4);
-                        finish_row(none ? zero4 : acc + zero4, none ? 0.f : l, gt, P1A_ARG(kp, out), gate != nullptr, P1A_ARG(kp, qbuf), row0 + t, hg * P.GQA + hh, 4 * d4, P1A_ARG(kp, Hq), D, P1A_ARG(kp, T), true);
+                        finish_row(none ? zero4 : acc + zero4, none ? 0.f : l, gt, P1A_ARG(kp, out), gate != nullptr, P1A_ARG(kp, qbuf),
+                                   row0 + t, hg * P.GQA + hh, 4 * d4, P1A_ARG(kp, Hq), D, P1A_ARG(kp, T), true);
                         continue;
                     }
                     float * part_o = P.part_o;
@@ -1038,8 +1043,8 @@ __global__ void __launch_bounds__(NWV * 64, SB ? NWV / 2 : 1) dec_mfma_k(const d
 // stream's (m, l): few kv heads have many (one, 256), and one row over 500 keys (f16, 4 / 1 heads of 64, two layers with prep, recorded) took
 // 34.4 us, 27.5 so; 16 / 2 of 256 (q4_0) 37.4 and 34.8.
 constexpr int MRG_DIMS = 128;
-// (one kernel argument: the host pays for each. Plain steps of four layers, which the host bounds, with 13 arguments and so: f16, 4 / 1 heads of 64 61 and 54 us,
-// 32 / 8 of 128 60 and 52, q8_0, 24 / 4 of 256 62 and 58; recorded ones level.)
+// (One kernel argument: the host pays for each. Plain steps of four layers over 500 keys, which the host bounds, with 11 of them - and prep_k's
+// 21, p1a_append.hip - and so: f16, 4 / 1 heads of 64 64.5 and 61.9 us, 32 / 8 of 128 63.9 and 61.7, q8_0, 24 / 4 of 256 64.0 and 63.5.)
 struct merge_params {
     const float * part_o, * part_ml;
     float * out;
@@ -1075,8 +1080,8 @@ __global__ void __launch_bounds__(256) merge_k(const merge_params P) {
     float M = NEG_INF;
     float2 pr = make_float2(NEG_INF, 0.f);                    // the pair of split `lane` of the first batch
     // The first batch of partials (all of them when NS <= 64) is requested before anything is known about the maximum - and, where one
-    // sequence's position is in memory, about the position: its round trip in front of them costs more than what is fetched for nothing (16 / 2 heads, 32000 keys 41.9 us,
-    // 42.4 behind it); what no stream has written is dropped.
+    // sequence's position is in memory, about the position: its round trip in front of them costs more than what is fetched for nothing (16 / 2
+    // heads, 32000 keys 41.9 us, 42.4 behind it); what no stream has written is dropped.
     const bool beside = p0_dev && !pos_rows;
     auto streams = [&](int at) { return at < 0 ? 0 : min(NS_all, (at >> u_sh) + 1); };
     int NS = NS_all;

@@ -84,9 +84,10 @@ inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv,
     const int nseq = (groups + r.GPS - 1) / r.GPS, inner = Hkv * r.GPS;
     // One unit at most, as far as the host knows - from the positions (host_n of them; 0: they are in device memory)
     // or from what a page-table row holds: the workgroup of a (row group, kv head) writes the results, and there is no merge behind
-    // it (`partials`: they are what the call is for). Steps of two layers, prep included, with merge_k and so: q8_0, 24 / 4 heads of 256, one sequence of 250 keys 34.4 and 29.6 us, 32
-    // of them 42.8 and 33.4; f16, 32 / 8 of 128 30.6 and 26.0, 32 of them 40.2 and 33.4; 8 x 4 rows of 250 (24 / 4) 48.1 and 42.0; plain
-    // calls of 100 keys 28.4 and 26.5.
+    // it (`partials`: they are what the call is for). Steps of two layers, prep included, with merge_k and so: q8_0, 24 / 4 heads of 256,
+    // one sequence of 250 keys 34.4 and 29.6 us, 32 of them 42.8 and 33.4; f16, 32 / 8 of 128 30.6 and 26.0, 32 of them 40.2 and 33.4;
+    // 8 x 4 rows of 250 (24 / 4) 48.1 and 42.0; plain calls of 100 keys 28.4 and 26.5. (Positions in device memory behind table rows of a
+    // server's context limit go by merge_k: 32 of 256, q8_0, 32 / 8 of 128 32.5 with rows of 256 positions, 40 with 512, 42.5 with 32768.)
     // A workgroup has its compute unit to itself. All kv heads of a row group go to one XCD, eights of groups at a time, where no XCD gets more of them than it
     // has units so; else workgroups go to the XCDs in turn. Rows of 250 keys, heads of 256 (q8_0), with merge_k, by groups and in turn: one row of 40 heads
     // 33.8, 44.7, 28.7, of 128 36.8, 77.9, 32.5, 9 rows of 24 heads 47.9, 47.3, 35.5; but 8 rows of 24 38.8, 32.8, 34.6, 16 of 8 heads of
@@ -122,10 +123,10 @@ inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv,
     // 0.84 - 1.6, 1.1 in the mean - the row groups of a stream are side by side on an XCD, which long sequences gain from (f16, 32 / 8 of 128, 13 rows
     // of 20000 keys 150 -> 98 us, 8 rows 33 -> 26; 200 keys 14.1 -> 11.9); what loses most are row counts that only groups of one
     // divide (q4_0, 16 / 16 of 256, 31 rows of 3000 keys 143 -> 166, f16, 16 / 4 of 64, 20000 keys 80 -> 95). Where one has a unit to itself (two
-    // column tiles, staged tiles) it shows: calls of four row groups and more whose page-table rows - as wide as n_ctx says, whatever
-    // the sequences hold - cannot hold the keys that half of the streams begin with (8 x 4 rows of 300
-    // ... 5000 keys, q8_0, 24 / 4 heads of 256, two layers 72.8 -> 62.1 us, 16 of 300 ... 5000, 32 / 8 of 128 104 -> 93; with every
-    // stream live 8 of 18797, q8_0, 24 / 4 of 128, four layers would go from 349 to 360).
+    // column tiles, staged tiles that do not go two to a unit) it shows: calls of four row groups and more whose page-table rows - as wide as n_ctx
+    // says, whatever the sequences hold - cannot hold the keys that half of the streams begin with (without it, with a workgroup for every
+    // stream: 8 x 4 rows of 300 ... 5000 keys, q8_0, 24 / 4 heads of 256, two layers 71.0 and 61.1 us, 16 of 300 ... 5000, 16 / 4 of 64
+    // 49.9 and 41.5). With every stream live it costs what it takes: 8 of 18797, q8_0, 24 / 4 of 128, four layers 233 and 235.5.
     const long long once = (long long) pl.nsplit * 32 * pl.NW;   // the keys that every stream holds a unit of
     r.list = pos_rows && groups > 1 && (r.sb || (groups >= 4 && 2LL * n_ctx <= once));
     r.loop = false;
@@ -133,18 +134,20 @@ inline decode_grid plan_grid(const dec_plan & pl, uint32_t type, int D, int Hkv,
     r.y = (unsigned) groups;
     if (!r.list) return r;
     long long nq = ((long long) nseq * pl.nsplit + 7) / 8;   // streams there could be, in eights
-    // Where most workgroups would find nothing to do, at 0.5 us for every 1000 of them, fewer walk the list.
-    //   Two to a unit: more than 16 for every compute unit, i.e. 32 sequences (of 256 keys, q8_0, 24 / 4 heads of 256, two layers: 61 us, 49.5
-    //   with a workgroup for every stream, 43 so; of 300 ... 5000 99, 94.6, 90.5; f16, 32 / 8 of 128, 32 of 1024 91, 95, 89). Fewer would lose more where
-    //   all streams are live (16 of 20000: 313, 304 with one workgroup a stream, 333 with eight for every unit); but four for every unit where
-    //   page-table rows hold a quarter of that at most (32 of 1024, f16, 16 / 4 of 64: 45 us with 16, 39 with four; 24 / 4 of 256, q8_0 68 and 64; where
-    //   they hold half, f16, 8 / 8 of 256, 2000 keys 212 and 220).
-    //   One to a unit: more than two for every compute unit; at least half of the streams are known to be empty there (without the list, a
-    //   workgroup for every stream, two for every unit: 8 x 4 rows of 300 ... 5000, q8_0, 24 / 4 of 256 73.6, 62.7, 56.5 us; 16 of 256, 32 / 8 of 128 53, 45, 39;
-    //   32 of 256 77, 71, 43; q4_0, 24 / 4 of 128, 16 of 60 ... 1500 58.5, 46.9, 40.3).
-    // All of these are times with page-table rows as wide as the sequences. Rows of 32768 positions, a server's limit, take the other route
-    // whatever the sequences hold: 72.2, 53.9, 78.3 and 58.6 us for the last four, 45.8 for 32 of 1024 (f16, 16 / 4 of 64).
-    //   Staged tiles, two to a unit: two for every compute unit where page-table rows cannot hold half of it, as in the second kind.
+    // Where most workgroups would find nothing to do, at 0.5 us for every 1000 of them, fewer walk the list. (Three times each: without the list,
+    // with a workgroup for every stream, so; two layers with prep, page-table rows as wide as the sequences.)
+    //   Two to a unit: more than 16 for every compute unit, i.e. 32 sequences (q8_0, 24 / 4 heads of 256, 500 keys 66.4, 56.5, 44.2 us, 300 ... 5000
+    //   88.1, 83.9, 77.6; f16, 32 / 8 of 128, 1024 76.2, 81.3, 71.2). Fewer would lose more where all streams are live (16 of 20000: 314, 306 with a
+    //   workgroup for every stream, 333 with eight for every unit); but four for every unit where page-table rows hold a quarter of that at most
+    //   (32 of 1024, f16, 16 / 4 of 64 54.9, 56.4, 39.4 - with 16, behind rows of 32768 positions, 45.2; 24 / 4 of 256, q8_0 73.6, 68.8, 56.6;
+    //   where they hold half, f16, 8 / 8 of 256, 2000 keys 212 with 16 and 220 with four).
+    //   One to a unit: more than two for every compute unit; at least half of the streams are known to be empty there (8 x 4 rows of 300 ... 5000,
+    //   q8_0, 24 / 4 of 256 71.0, 61.1, 54.2; 16 / 4 of 64, 32 of 500 54.3, 45.2, 33.2, 16 of 300 ... 5000 49.9, 41.5, 37.5; 32 / 8 of 128,
+    //   16 of 500 57.8, 51.4, 39.1).
+    //   Staged tiles, two to a unit: two for every compute unit where page-table rows cannot hold half of it, as in the second kind (q8_0,
+    //   32 / 8 of 128, 32 of 500 67.8, 60.0, 46.7).
+    // Rows of 32768 positions, a server's limit, take the other route whatever the sequences hold: 71.2 us for the 8 x 4 rows, 49.6 for the 16 of
+    // 16 / 4 heads, 52.5 for the last.
     const bool resident = !r.sb || (staged && 2LL * n_ctx <= once);
     const long long most = (resident ? 2LL : 16LL) * cus / (8 * inner);
     const bool can_loop = pl.NT == 2 ? staged || type != P1A_KV_Q4_0 : r.sb || staged;   // (q4_0 with two column tiles has no register left for it)
